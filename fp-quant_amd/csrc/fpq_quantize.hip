@@ -440,6 +440,188 @@ __device__ __forceinline__ uint32_t fix_zero_nibbles(uint32_t w) {
   return w;
 }
 
+// One lane's chunk of EPL consecutive elements, rotated in place: the butterflies with stride < EPL stay in the
+// lane's registers, a wider rotation takes one or two exchanges with the neighbouring lanes that hold the rest
+// of the block (lane % (G / EPL) is the chunk's place in it).
+template <int EPL, int G, int ROT>
+__device__ __forceinline__ void rotate_chunk(float (&v)[EPL], float norm, uint32_t lane) {
+  if (ROT == FPQ_ROT_HADAMARD || ROT == FPQ_ROT_GSR) {
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) v[i] *= norm;
+#pragma unroll
+    for (int s = 1; s < (G < EPL ? G : EPL); s *= 2) {
+      __builtin_amdgcn_sched_barrier(0);  // keep the stages in place: EPL live values, no more
+#pragma unroll
+      for (int i = 0; i < EPL; ++i) {
+        if ((i & s) == 0) {
+          const float a = v[i], b = v[i + s];
+          v[i] = a + b;
+          v[i + s] = a - b;
+        }
+      }
+    }
+    if (G > EPL) {
+      // stride EPL: the two halves of a rotation block sit in lanes 2u and 2u + 1.  The even
+      // lane needs a + b, the odd one a - b = (value of the even lane) + (-own value).
+      __builtin_amdgcn_sched_barrier(0);
+      const uint32_t flip = (lane & 1u) << 31;
+#pragma unroll
+      for (int i = 0; i < EPL; ++i) {
+        const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(
+            (int)__float_as_uint(v[i]), 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, true));
+        v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ flip);
+      }
+      if (G > 2 * EPL) {
+        // stride 2 EPL (a 128-wide rotation with EPL = 32): the quarters of a block sit in lanes
+        // 4u .. 4u + 3 and the partner is lane ^ 2
+        static_assert(G <= 4 * EPL, "at most two exchanges between lanes");
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t flip2 = (lane & 2u) << 30;
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) {
+          const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(
+              (int)__float_as_uint(v[i]), 0x4E /* quad_perm [2,3,0,1] */, 0xF, 0xF, true));
+          v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ flip2);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (ROT == FPQ_ROT_GSR) {
+    // sequency order inside every G-block (G <= EPL here): a compile-time renaming of registers
+    static_assert(ROT != FPQ_ROT_GSR || G <= EPL, "GSR blocks must fit in one lane");
+    float w[EPL];
+#pragma unroll
+    for (int k = 0; k < EPL; ++k) w[k] = v[(k & ~(G - 1)) | gsr_source(k & (G - 1), G)];
+#pragma unroll
+    for (int k = 0; k < EPL; ++k) v[k] = w[k];
+  }
+}
+
+// E2M1 codes and scale bytes of one lane's rotated chunk (cw: CW dwords of codes; sbytes: the scale bytes, with
+// eight of them the first four in sb_lo).  Returns whether a group left the range in which the two-operation
+// division is proven: the caller then redoes the chunk with quantize_chunk_slow.
+template <int EPL, int FMT, int ZERO, bool QUEST>
+__device__ __forceinline__ bool quantize_chunk(const float (&v)[EPL], float gs, bool nv_fast,
+                                               const float2* __restrict__ lut, uint32_t (&cw)[EPL / 8],
+                                               uint32_t& sbytes, uint32_t& sb_lo) {
+  constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
+  constexpr int NG = EPL / GROUP;
+  bool need_slow = false;
+#pragma unroll
+  for (int gi = 0; gi < NG; ++gi) {
+    float a = 0.0f;
+    if (!QUEST) {
+#pragma unroll
+      for (int i = 0; i < GROUP; ++i) a = __builtin_fmaxf(a, __builtin_fabsf(v[gi * GROUP + i]));
+    }
+    uint32_t byte;
+    bool fast;
+    float k1, k2, cvt_scale;
+    if (QUEST) {
+      float os[4], oq[4];
+#pragma unroll
+      for (int o = 0; o < 4; ++o) {
+        const float* p = &v[gi * GROUP + 8 * o];
+        float sum = p[0], sq = p[0] * p[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) {
+          sum = sum + p[i];
+          sq = sq + p[i] * p[i];
+        }
+        os[o] = sum;
+        oq[o] = sq;
+      }
+      const float sum = (os[0] + os[1]) + (os[2] + os[3]), sq = (oq[0] + oq[1]) + (oq[2] + oq[3]);
+      const float mean = sum * 0.03125f, msq = sq * 0.03125f;
+      float var = msq - mean * mean;
+      var = var > 0.0f ? var : 0.0f;
+      const float sc = __builtin_sqrtf(var) * 0.48707976f + 1e-8f;   // fl32(2.92247856 / 6); >= 1e-8: normal
+      byte = (__float_as_uint(sc) >> 23) & 0xffu;
+      fast = true;
+      k1 = k2 = 0.0f;
+      cvt_scale = __uint_as_float(byte << 23);                         // s = 2^floor(log2(sc))
+    } else if (FMT == kFmtMx) {
+      const uint32_t bits = __float_as_uint(a);
+      byte = bits >> 23;
+      fast = (byte - 29u) <= 198u || bits == 0u;                       // -98 <= e <= 100, or all zero
+      k1 = 0.75f;
+      k2 = kKappa;
+      cvt_scale = __uint_as_float((bits & 0x7f800000u) - (2u << 23));  // 2^(e-2)
+      if (bits == 0u) {  // a zero group stores 2^-126 and zero codes
+        byte = 1u;
+        cvt_scale = 1.0f;
+      }
+    } else {
+      float t = div6_rn(a) * gs;
+      t = t > 448.0f ? 448.0f : t;
+      byte = e4m3_encode(t);
+      fast = nv_fast;
+      const float2 e = lut[byte & 0x7fu];
+      k1 = e.x;
+      k2 = e.y;
+      cvt_scale = 1.0f;
+    }
+    need_slow |= !fast;
+#pragma unroll
+    for (int d = 0; d < GROUP / 8; ++d) {
+      uint32_t w = 0u;
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const float x0 = v[gi * GROUP + d * 8 + 2 * h], x1 = v[gi * GROUP + d * 8 + 2 * h + 1];
+        float q0 = QUEST ? x0 : __builtin_fmaf(x0, k1, x0 * k2);
+        float q1 = QUEST ? x1 : __builtin_fmaf(x1, k1, x1 * k2);
+        if (ZERO == kZeroSigned && !QUEST) {  // x / s keeps the sign of x, also for -0
+          q0 = __builtin_copysignf(q0, x0);
+          q1 = __builtin_copysignf(q1, x1);
+        }
+        if (h == 0) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 0);
+        if (h == 1) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 1);
+        if (h == 2) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 2);
+        if (h == 3) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 3);
+      }
+      if (FMT == kFmtNv && ZERO == kZeroSigned) w = byte == 0u ? 0u : w;  // zero scale: +0 codes
+      cw[gi * (GROUP / 8) + d] = fix_zero_nibbles<ZERO>(w);
+    }
+    sbytes |= (byte & 0xffu) << (8 * (gi & 3));
+    if (NG == 8 && gi == 3) {  // eight scale bytes per chunk: park the first four
+      sb_lo = sbytes;
+      sbytes = 0u;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return need_slow;
+}
+
+template <int EPL, int FMT, int ZERO>
+__device__ __forceinline__ void quantize_chunk_slow(const float (&u)[EPL], float gs, float rg,
+                                                    uint32_t (&cw)[EPL / 8], uint32_t& sbytes) {
+  constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
+  constexpr int NG = EPL / GROUP;
+  sbytes = 0u;
+#pragma unroll 1
+  for (int gi = 0; gi < NG; ++gi) {
+    float a = 0.0f;
+#pragma unroll
+    for (int i = 0; i < GROUP; ++i) a = __builtin_fmaxf(a, __builtin_fabsf(u[gi * GROUP + i]));
+    const GroupScale g = FMT == kFmtMx ? mx_group_scale(a) : nv_group_scale(a, gs, rg);
+#pragma unroll
+    for (int d = 0; d < GROUP / 8; ++d) {
+      uint32_t w = 0u;
+#pragma unroll
+      for (int h = 0; h < 8; ++h) {
+        const float xv = u[gi * GROUP + d * 8 + h];
+        float q = scale_element(xv, g);
+        if (ZERO == kZeroSigned) q = __builtin_copysignf(q, xv);
+        if (FMT == kFmtNv) q = g.zero ? 0.0f : q;
+        w |= e2m1_code<ZERO>(q) << (4 * h);
+      }
+      cw[gi * (GROUP / 8) + d] = w;
+    }
+    sbytes |= (g.byte & 0xffu) << (8 * gi);
+  }
+}
+
 //
 // PACKED (EPL = 64, or 32 without a prologue) writes the operand layout of fpq_gemm_mxf4_packed /
 // fpq_gemm_nvf4_packed instead of row-major codes and scales.  A wave tile is then 32 rows x two
@@ -670,146 +852,14 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
         }
       }
     }
-    if (ROT == FPQ_ROT_HADAMARD || ROT == FPQ_ROT_GSR) {
-#pragma unroll
-      for (int i = 0; i < EPL; ++i) v[i] *= norm;
-#pragma unroll
-      for (int s = 1; s < (G < EPL ? G : EPL); s *= 2) {
-        __builtin_amdgcn_sched_barrier(0);  // keep the stages in place: EPL live values, no more
-#pragma unroll
-        for (int i = 0; i < EPL; ++i) {
-          if ((i & s) == 0) {
-            const float a = v[i], b = v[i + s];
-            v[i] = a + b;
-            v[i + s] = a - b;
-          }
-        }
-      }
-      if (G > EPL) {
-        // stride EPL: the two halves of a rotation block sit in lanes 2u and 2u + 1.  The even
-        // lane needs a + b, the odd one a - b = (value of the even lane) + (-own value).
-        __builtin_amdgcn_sched_barrier(0);
-        const uint32_t flip = (lane & 1u) << 31;
-#pragma unroll
-        for (int i = 0; i < EPL; ++i) {
-          const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(
-              (int)__float_as_uint(v[i]), 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, true));
-          v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ flip);
-        }
-        if (G > 2 * EPL) {
-          // stride 2 EPL (a 128-wide rotation with EPL = 32): the quarters of a block sit in lanes
-          // 4u .. 4u + 3 and the partner is lane ^ 2
-          static_assert(G <= 4 * EPL, "at most two exchanges between lanes");
-          __builtin_amdgcn_sched_barrier(0);
-          const uint32_t flip2 = (lane & 2u) << 30;
-#pragma unroll
-          for (int i = 0; i < EPL; ++i) {
-            const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(
-                (int)__float_as_uint(v[i]), 0x4E /* quad_perm [2,3,0,1] */, 0xF, 0xF, true));
-            v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ flip2);
-          }
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (ROT == FPQ_ROT_GSR) {
-      // sequency order inside every G-block (G <= EPL here): a compile-time renaming of registers
-      static_assert(ROT != FPQ_ROT_GSR || G <= EPL, "GSR blocks must fit in one lane");
-      float w[EPL];
-#pragma unroll
-      for (int k = 0; k < EPL; ++k) w[k] = v[(k & ~(G - 1)) | gsr_source(k & (G - 1), G)];
-#pragma unroll
-      for (int k = 0; k < EPL; ++k) v[k] = w[k];
-    }
+    rotate_chunk<EPL, G, ROT>(v, norm, lane);
     };
     float v[EPL];
     load_rotate(v);
 
     uint32_t cw[CW];
     uint32_t sbytes = 0u, sb_lo = 0u;
-    bool need_slow = false;
-#pragma unroll
-    for (int gi = 0; gi < NG; ++gi) {
-      float a = 0.0f;
-      if (!QUEST) {
-#pragma unroll
-        for (int i = 0; i < GROUP; ++i) a = __builtin_fmaxf(a, __builtin_fabsf(v[gi * GROUP + i]));
-      }
-      uint32_t byte;
-      bool fast;
-      float k1, k2, cvt_scale;
-      if (QUEST) {
-        float os[4], oq[4];
-#pragma unroll
-        for (int o = 0; o < 4; ++o) {
-          const float* p = &v[gi * GROUP + 8 * o];
-          float sum = p[0], sq = p[0] * p[0];
-#pragma unroll
-          for (int i = 1; i < 8; ++i) {
-            sum = sum + p[i];
-            sq = sq + p[i] * p[i];
-          }
-          os[o] = sum;
-          oq[o] = sq;
-        }
-        const float sum = (os[0] + os[1]) + (os[2] + os[3]), sq = (oq[0] + oq[1]) + (oq[2] + oq[3]);
-        const float mean = sum * 0.03125f, msq = sq * 0.03125f;
-        float var = msq - mean * mean;
-        var = var > 0.0f ? var : 0.0f;
-        const float sc = __builtin_sqrtf(var) * 0.48707976f + 1e-8f;   // fl32(2.92247856 / 6); >= 1e-8: normal
-        byte = (__float_as_uint(sc) >> 23) & 0xffu;
-        fast = true;
-        k1 = k2 = 0.0f;
-        cvt_scale = __uint_as_float(byte << 23);                         // s = 2^floor(log2(sc))
-      } else if (FMT == kFmtMx) {
-        const uint32_t bits = __float_as_uint(a);
-        byte = bits >> 23;
-        fast = (byte - 29u) <= 198u || bits == 0u;                       // -98 <= e <= 100, or all zero
-        k1 = 0.75f;
-        k2 = kKappa;
-        cvt_scale = __uint_as_float((bits & 0x7f800000u) - (2u << 23));  // 2^(e-2)
-        if (bits == 0u) {  // a zero group stores 2^-126 and zero codes
-          byte = 1u;
-          cvt_scale = 1.0f;
-        }
-      } else {
-        float t = div6_rn(a) * gs;
-        t = t > 448.0f ? 448.0f : t;
-        byte = e4m3_encode(t);
-        fast = nv_fast;
-        const float2 e = lut[byte & 0x7fu];
-        k1 = e.x;
-        k2 = e.y;
-        cvt_scale = 1.0f;
-      }
-      need_slow |= !fast;
-#pragma unroll
-      for (int d = 0; d < GROUP / 8; ++d) {
-        uint32_t w = 0u;
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const float x0 = v[gi * GROUP + d * 8 + 2 * h], x1 = v[gi * GROUP + d * 8 + 2 * h + 1];
-          float q0 = QUEST ? x0 : __builtin_fmaf(x0, k1, x0 * k2);
-          float q1 = QUEST ? x1 : __builtin_fmaf(x1, k1, x1 * k2);
-          if (ZERO == kZeroSigned && !QUEST) {  // x / s keeps the sign of x, also for -0
-            q0 = __builtin_copysignf(q0, x0);
-            q1 = __builtin_copysignf(q1, x1);
-          }
-          if (h == 0) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 0);
-          if (h == 1) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 1);
-          if (h == 2) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 2);
-          if (h == 3) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 3);
-        }
-        if (FMT == kFmtNv && ZERO == kZeroSigned) w = byte == 0u ? 0u : w;  // zero scale: +0 codes
-        cw[gi * (GROUP / 8) + d] = fix_zero_nibbles<ZERO>(w);
-      }
-      sbytes |= (byte & 0xffu) << (8 * (gi & 3));
-      if (NG == 8 && gi == 3) {  // eight scale bytes per chunk: park the first four
-        sb_lo = sbytes;
-        sbytes = 0u;
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
 
     if constexpr (PACKED) {
       // Scale exponents outside the fast range (tiny or huge values): redo the tile with the
@@ -817,28 +867,7 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
       if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
         float u[EPL];
         load_rotate(u);
-        sbytes = 0u;
-#pragma unroll 1
-        for (int gi = 0; gi < NG; ++gi) {
-          float a = 0.0f;
-#pragma unroll
-          for (int i = 0; i < GROUP; ++i) a = __builtin_fmaxf(a, __builtin_fabsf(u[gi * GROUP + i]));
-          const GroupScale g = FMT == kFmtMx ? mx_group_scale(a) : nv_group_scale(a, gs, rg);
-#pragma unroll
-          for (int d = 0; d < GROUP / 8; ++d) {
-            uint32_t w = 0u;
-#pragma unroll
-            for (int h = 0; h < 8; ++h) {
-              const float xv = u[gi * GROUP + d * 8 + h];
-              float q = scale_element(xv, g);
-              if (ZERO == kZeroSigned) q = __builtin_copysignf(q, xv);
-              if (FMT == kFmtNv) q = g.zero ? 0.0f : q;
-              w |= e2m1_code<ZERO>(q) << (4 * h);
-            }
-            cw[gi * (GROUP / 8) + d] = w;
-          }
-          sbytes |= (g.byte & 0xffu) << (8 * gi);
-        }
+        quantize_chunk_slow<EPL, FMT, ZERO>(u, gs, rg, cw, sbytes);
       }
       const uint32_t r = P32 ? lane >> 2 : lane >> 1, ksl = lane & 1u;
       const bool row_ok = r < valid;
@@ -1475,6 +1504,7 @@ __global__ __launch_bounds__(256) void row_inv_rms_kernel(const uint4* __restric
 // them in that kernel's order) and quantizes the row with the generic kernel's arithmetic into the
 // packed operand layout.  Workgroups past `rows` (the padding of the last 32-row tile) write zeros.
 constexpr uint32_t kRowsKernelMaxChunks = 2048;   // cols <= 16384
+constexpr int64_t kTileKernelMaxCols = 16384;     // rmsnorm_tile_quantize_kernel: a row in a wave's registers, four in LDS
 template <int G, int FMT, int ROT, int ZERO>
 __global__ __launch_bounds__(1024) void rmsnorm_rows_quantize_kernel(const uint4* __restrict__ x,
                                                                     uint32_t* __restrict__ codes,
@@ -1524,6 +1554,138 @@ __global__ __launch_bounds__(1024) void rmsnorm_rows_quantize_kernel(const uint4
     const uint32_t chunk = in ? row * cpr + cc : 0xffffffffu;
     lane8_process<G, FMT, ROT, ZERO, false, kProRmsNorm>(x, codes, scales, chunk, real && in, lane, cpr, 0u, norm, gs,
                                                          rg, nullptr, nullptr, nullptr, pro, rs);
+  }
+}
+
+// RMSNorm + rotate + quantize of many rows in ONE pass over x: a workgroup owns four neighbouring rows and a wave
+// reads one of them into registers (lane l takes the octets l, l + 64, ... -- the order of row_inv_rms_kernel, so
+// the statistic keeps its bits), normalises it there, stores the by-product as whole kilobytes and leaves the bf16
+// row in LDS; then lanes own 32-element chunks (4 rows x 16 chunks per wave) and rotate, quantize and store them in
+// the packed operand layout as runs of 64 bytes.  The 16-byte pieces of a chunk sit in LDS XOR-swizzled by the
+// chunk so that the chunk reads hit every bank group once.  Rows past `rows` (the padding of the last 32-row tile)
+// get zero codes and scale bytes.
+// Memory bounds it: x in, by-product and codes out, 152 MB for 8192 x 4096 (30.2 us = 5.0 TB/s, a device copy's
+// rate; 23.9 us without the by-product).  The statistic in a launch of its own, with a second pass over x, took
+// 46.6 (39.1) us; 2048 rows 16.6 -> 9.6, 128 rows 9.3 -> 5.8, 8192 x 2048 25.0 -> 16.9, 3000 x 8192 37.7 -> 25.8.
+// Four rows and four waves, 32 KB of LDS for 4096 columns, five workgroups per CU whose loads, arithmetic and stores
+// overlap: eight rows and eight waves take 30.8 us there but 7.3 against 6.6 at 512 rows and 44.9 against 40.0 for
+// 8192 x 5120; four rows and eight waves 34.6.
+constexpr int kTileRows = 4;   // rows, and waves, of a workgroup
+template <int G, int FMT, int ROT, int ZERO, int MAXO>
+__global__ __launch_bounds__(64 * kTileRows) void rmsnorm_tile_quantize_kernel(
+    const uint4* __restrict__ x, uint8_t* __restrict__ codes, uint8_t* __restrict__ scales, uint32_t rows, float norm,
+    float cols_f, float eps, float* __restrict__ inv_rms_out, const float* __restrict__ global_scale, Prologue pro) {
+  constexpr int EPL = 32;
+  constexpr uint32_t R = kTileRows, CPL = 64 / R;   // chunks of a row that one wave step covers
+  extern __shared__ __attribute__((aligned(128))) uint8_t dyn_lds[];
+  __shared__ float2 lut[128];
+  const uint32_t cpr = pro.chunks_per_row, lane = threadIdx.x & 63u;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t row_bytes = cpr * 16u, row0 = blockIdx.x * R;
+  // byte of octet o of row rr of the workgroup
+  auto place = [&](uint32_t rr, uint32_t o) -> uint32_t {
+    const uint32_t b = o >> 2;
+    return rr * row_bytes + b * 64u + (((o & 3u) ^ ((b >> 2) & 3u)) * 16u);
+  };
+  float gs = 1.0f, rg = 1.0f;
+  bool nv_fast = true;
+  if (FMT == kFmtNv) {
+    gs = *global_scale;
+    rg = gs == 0.0f ? 0.0f : 1.0f / gs;
+    nv_fast = gs >= 8.673617379884035e-19f && gs <= 1.152921504606847e18f;   // as quantize_stream_kernel
+    if (threadIdx.x < 128) {
+      const float s = e4m3_decode(threadIdx.x) * rg;
+      float2 e = make_float2(0.0f, 0.0f);
+      if (s != 0.0f && nv_fast) {
+        const float y = 1.0f / s;
+        e = make_float2(y, __builtin_fmaf(-s, y, 1.0f) / s);
+      }
+      lut[threadIdx.x] = e;
+    }
+  }
+
+  if (const uint32_t rr = wave, row = row0 + rr; row < rows) {
+    const uint4* src = x + (size_t)row * pro.ld_first;
+    uint4 raw[MAXO];
+#pragma unroll
+    for (int i = 0; i < MAXO; ++i) {
+      const uint32_t o = lane + 64u * i;
+      raw[i] = o < cpr ? src[o] : make_uint4(0u, 0u, 0u, 0u);
+    }
+    float a = 0.0f;
+#pragma unroll
+    for (int i = 0; i < MAXO; ++i) {
+      float p[8];
+      unpack8(raw[i], p);
+      float s = p[0] * p[0];
+#pragma unroll
+      for (int k = 1; k < 8; ++k) s = s + p[k] * p[k];
+      a = lane + 64u * i < cpr ? a + s : a;
+    }
+#pragma unroll
+    for (int lm = 1; lm < 64; lm *= 2) a = a + __shfl_xor(a, lm, 64);
+    const float rs = 1.0f / __builtin_sqrtf(a / cols_f + eps);
+    if (inv_rms_out && lane == 0u) inv_rms_out[row] = rs;
+    uint8_t* out = pro.out ? (uint8_t*)(pro.out + (size_t)row * cpr) : nullptr;
+#pragma unroll
+    for (int i = 0; i < MAXO; ++i) {
+      const uint32_t o = lane + 64u * i;
+      if (o >= cpr) continue;
+      float p[8], q[8];
+      unpack8(raw[i], p);
+      unpack8(pro.col_scale[o], q);
+      uint32_t w[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t t = pack_bf16x2(p[2 * k] * rs, p[2 * k + 1] * rs);
+        w[k] = pack_bf16x2(bf16_lo(t) * q[2 * k], bf16_hi(t) * q[2 * k + 1]);
+      }
+      const uint4 v = make_uint4(w[0], w[1], w[2], w[3]);
+      *(uint4*)(dyn_lds + place(rr, o)) = v;
+      if (out) store16_nt(out + o * 16u, v);
+    }
+  }
+  __syncthreads();
+
+  const uint32_t r = lane / CPL, c = lane % CPL, chunks = cpr / 4u, units = cpr / 8u;
+  const uint32_t rt = row0 >> 5, rit = (row0 & 31u) + r;   // row tile, row inside it
+  const bool row_ok = row0 + r < rows;
+  for (uint32_t c0 = wave * CPL; c0 < chunks; c0 += kTileRows * CPL) {
+    const bool in = c0 + c < chunks;                       // (whole quads of lanes: chunks % 8 == 0)
+    const uint32_t b = in ? c0 + c : c;
+    auto load_rotate = [&](float (&v)[EPL]) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float e[8];
+        unpack8(*(const uint4*)(dyn_lds + place(r, 4u * b + k)), e);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[8 * k + i] = e[i];
+      }
+      rotate_chunk<EPL, G, ROT>(v, norm, lane);
+    };
+    float v[EPL];
+    load_rotate(v);
+    uint32_t cw[EPL / 8], sbytes = 0u, sb_lo = 0u;
+    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
+      float u[EPL];
+      load_rotate(u);
+      quantize_chunk_slow<EPL, FMT, ZERO>(u, gs, rg, cw, sbytes);
+    }
+    if (!row_ok) {
+      cw[0] = cw[1] = cw[2] = cw[3] = 0u;
+      sbytes = 0u;
+    }
+    if (in) {
+      const uint32_t unit = b >> 1, slot = (b & 1u) * 32u + rit;
+      store16_nt(codes + (((size_t)rt * units + unit) * 64u + slot) * 16u, make_uint4(cw[0], cw[1], cw[2], cw[3]));
+      if (FMT == kFmtMx) {
+        scales[((size_t)rt * (units / 4u) + (unit >> 2)) * 256u + slot * 4u + (unit & 3u)] = (uint8_t)sbytes;
+      } else {
+        *(uint16_t*)(scales + ((size_t)rt * (units / 4u) + (unit >> 2)) * 512u + slot * 8u + 2u * (unit & 3u)) =
+            (uint16_t)sbytes;
+      }
+    }
   }
 }
 
@@ -1770,6 +1932,67 @@ static int dispatch_rmsnorm_rows(const void* x, int64_t ld, const void* weight, 
 #undef FPQ_LAUNCH_ROWS
   return FPQ_E_ROTATION;
 }
+
+template <int FMT>
+static int dispatch_rmsnorm_tile(const void* x, int64_t ld, const void* weight, int64_t rows, int64_t cols, float eps,
+                                 int rot_kind, int g, float norm, float* inv_rms, void* normed, void* codes,
+                                 void* scales, int zero_policy, void* stream_, const float* gsp = nullptr) {
+  hipStream_t stream = (hipStream_t)stream_;
+  if (rows < 0 || cols < 0) return FPQ_E_SHAPE;
+  if (rows == 0 || cols == 0) return FPQ_OK;
+  if (!x || !weight || !codes || !scales) return FPQ_E_NULL;
+  if (FMT == kFmtNv && !gsp) return FPQ_E_NULL;
+  if (zero_policy != FPQ_ZERO_REFERENCE && zero_policy != FPQ_ZERO_SIGNED) return FPQ_E_POLICY;
+  if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
+  if (rot_kind != FPQ_ROT_IDENTITY && rot_kind != FPQ_ROT_HADAMARD) {
+    return (rot_kind == FPQ_ROT_GSR || rot_kind == FPQ_ROT_GENERAL) ? FPQ_E_UNSUPPORTED : FPQ_E_ROTATION;
+  }
+  if (g != 16 && g != 32 && g != 64 && g != 128) return FPQ_E_ROTATION;
+  if (cols % 256 != 0 || ld < cols || ld % 8 != 0 || ld >= (int64_t)1 << 24) return FPQ_E_SHAPE;
+  if (rows * ld >= (int64_t)1 << 34) return FPQ_E_SHAPE;
+  if (cols > kTileKernelMaxCols) return FPQ_E_LIMIT;
+  if (((uintptr_t)x & 15u) || ((uintptr_t)weight & 15u) || ((uintptr_t)normed & 15u) || ((uintptr_t)inv_rms & 3u) ||
+      ((uintptr_t)codes & 15u) || ((uintptr_t)scales & (FMT == kFmtNv ? 7u : 3u)) || ((uintptr_t)gsp & 3u)) {
+    return FPQ_E_ALIGN;
+  }
+  Prologue pro{};
+  pro.col_scale = (const uint4*)weight;
+  pro.out = (uint4*)normed;
+  pro.chunks_per_row = (uint32_t)(cols / 8);
+  pro.ld_first = (uint32_t)(ld / 8);
+  const int64_t padded = (rows + 31) / 32 * 32;
+  const int lds = (int)(kTileRows * cols * 2);
+  int status = 0;
+  auto go = [&](auto kernel) {
+    static LdsLimitOnce limit;
+    if ((status = limit.ensure((const void*)kernel, (int)(kTileRows * kTileKernelMaxCols * 2))) != 0) return;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(padded / kTileRows)), dim3(64 * kTileRows), lds, stream, (const uint4*)x, (uint8_t*)codes,
+                       (uint8_t*)scales, (uint32_t)rows, norm, (float)cols, eps, inv_rms, gsp, pro);
+    status = (int)hipGetLastError();
+  };
+#define FPQ_LAUNCH_TILE_Z(GG, RR, ZZ)                                                       \
+  {                                                                                         \
+    if (cols <= 4096) go(rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 8>);                 \
+    else if (cols <= 8192) go(rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 16>);           \
+    else go(rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 32>);                             \
+    return status;                                                                          \
+  }
+#define FPQ_LAUNCH_TILE(GG, RR)                                                             \
+  {                                                                                         \
+    if (zero_policy == FPQ_ZERO_REFERENCE) FPQ_LAUNCH_TILE_Z(GG, RR, kZeroReference);       \
+    FPQ_LAUNCH_TILE_Z(GG, RR, kZeroSigned);                                                 \
+  }
+  if (rot_kind == FPQ_ROT_IDENTITY) FPQ_LAUNCH_TILE(32, FPQ_ROT_IDENTITY);
+  switch (g) {
+    case 16: FPQ_LAUNCH_TILE(16, FPQ_ROT_HADAMARD);
+    case 32: FPQ_LAUNCH_TILE(32, FPQ_ROT_HADAMARD);
+    case 64: FPQ_LAUNCH_TILE(64, FPQ_ROT_HADAMARD);
+    case 128: FPQ_LAUNCH_TILE(128, FPQ_ROT_HADAMARD);
+  }
+#undef FPQ_LAUNCH_TILE
+#undef FPQ_LAUNCH_TILE_Z
+  return FPQ_E_ROTATION;
+}
 }  // namespace fpq
 
 extern "C" int64_t fpq_rmsnorm_rows_max_rows(void) { return fpq::kPackedFewRows; }
@@ -1788,6 +2011,23 @@ extern "C" int fpq_rmsnorm_rows_quantize_nv_packed(const void* x, int64_t ld, co
                                                    void* packed_codes, void* packed_scales, int zero_policy,
                                                    void* stream) {
   return fpq::dispatch_rmsnorm_rows<fpq::kFmtNv>(x, ld, weight, rows, cols, eps, rot_kind, g, norm, inv_rms, normed,
+                                                 packed_codes, packed_scales, zero_policy, stream, global_scale);
+}
+
+extern "C" int fpq_rmsnorm_tile_quantize_mx_packed(const void* x, int64_t ld, const void* weight, int64_t rows,
+                                                   int64_t cols, float eps, int rot_kind, int g, float norm,
+                                                   float* inv_rms, void* normed, void* packed_codes,
+                                                   void* packed_scales, int zero_policy, void* stream) {
+  return fpq::dispatch_rmsnorm_tile<fpq::kFmtMx>(x, ld, weight, rows, cols, eps, rot_kind, g, norm, inv_rms, normed,
+                                                 packed_codes, packed_scales, zero_policy, stream);
+}
+
+extern "C" int fpq_rmsnorm_tile_quantize_nv_packed(const void* x, int64_t ld, const void* weight, int64_t rows,
+                                                   int64_t cols, float eps, int rot_kind, int g, float norm,
+                                                   const float* global_scale, float* inv_rms, void* normed,
+                                                   void* packed_codes, void* packed_scales, int zero_policy,
+                                                   void* stream) {
+  return fpq::dispatch_rmsnorm_tile<fpq::kFmtNv>(x, ld, weight, rows, cols, eps, rot_kind, g, norm, inv_rms, normed,
                                                  packed_codes, packed_scales, zero_policy, stream, global_scale);
 }
 

@@ -769,7 +769,8 @@ def _fused_quantize(entry: str, head: tuple, rows: int, cols: int, h: torch.Tens
     return qa
 
 
-_ROWS_KERNEL_MAX_ROWS = 64   # fpq_rmsnorm_rows_max_rows()
+_ROWS_KERNEL_MAX_ROWS = 64     # fpq_rmsnorm_rows_max_rows()
+_ONE_LAUNCH_MAX_COLS = 16384   # of fpq_rmsnorm_rows_quantize_* and fpq_rmsnorm_tile_quantize_*
 
 
 def rmsnorm_quantize(x: torch.Tensor, weight: torch.Tensor, eps: float, hadamard_matrix: torch.Tensor,
@@ -795,26 +796,27 @@ def rmsnorm_quantize(x: torch.Tensor, weight: torch.Tensor, eps: float, hadamard
         y = torch.empty_like(x_flat)
         w = weight.contiguous()
         qa = None
-        if (rows <= _ROWS_KERNEL_MAX_ROWS and cols % 256 == 0 and cols <= 16384
+        if (cols % 256 == 0 and cols <= _ONE_LAUNCH_MAX_COLS
                 and (nv_packed_eligible(rows, 32, cols, fused_linear=True) if nvfp4
                      else packed_linear_eligible(rows, cols, "abs_max"))):
-            # a decode step's few rows: statistic, normalisation and quantization in one launch
+            # statistic, normalisation and quantization in one launch: a decode step's few rows spread over many
+            # lanes each, more rows a wave each
+            kernel = "rows" if rows <= _ROWS_KERNEL_MAX_ROWS else "tile"
             pc = torch.empty(lib.fpq_packed_codes_bytes(rows, cols), dtype=torch.uint8, device=dev)
             qa = QuantizedActivations(rows, cols, nvfp4)
+            head = (x_flat.data_ptr(), cols, w.data_ptr(), rows, cols, eps, kind, h.shape[0], norm)
             if nvfp4:
                 ps = torch.empty(lib.fpq_packed_scales_bytes_nv(rows, cols), dtype=torch.uint8, device=dev)
                 gs = as_f32_scalar(act_global_scale)
-                st = lib.fpq_rmsnorm_rows_quantize_nv_packed(x_flat.data_ptr(), cols, w.data_ptr(), rows, cols, eps,
-                                                             kind, h.shape[0], norm, gs.data_ptr(), None, y.data_ptr(),
-                                                             pc.data_ptr(), ps.data_ptr(), ZERO_NIBBLE_POLICY, stream)
+                st = getattr(lib, f"fpq_rmsnorm_{kernel}_quantize_nv_packed")(
+                    *head, gs.data_ptr(), None, y.data_ptr(), pc.data_ptr(), ps.data_ptr(), ZERO_NIBBLE_POLICY, stream)
                 qa.nv_packed = (pc, ps)
             else:
                 ps = torch.empty(lib.fpq_packed_scales_bytes(rows, cols), dtype=torch.uint8, device=dev)
-                st = lib.fpq_rmsnorm_rows_quantize_mx_packed(x_flat.data_ptr(), cols, w.data_ptr(), rows, cols, eps,
-                                                             kind, h.shape[0], norm, None, y.data_ptr(), pc.data_ptr(),
-                                                             ps.data_ptr(), ZERO_NIBBLE_POLICY, stream)
+                st = getattr(lib, f"fpq_rmsnorm_{kernel}_quantize_mx_packed")(
+                    *head, None, y.data_ptr(), pc.data_ptr(), ps.data_ptr(), ZERO_NIBBLE_POLICY, stream)
                 qa.mx_packed = (pc, ps)
-            _engine.check(st, "fpq_rmsnorm_rows_quantize_packed")
+            _engine.check(st, "fpq_rmsnorm_quantize_packed")
         if qa is None:
             inv = torch.empty(rows, dtype=torch.float32, device=dev)
             _engine.check(lib.fpq_row_inv_rms(x_flat.data_ptr(), cols, rows, cols, eps, inv.data_ptr(), stream),

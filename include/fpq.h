@@ -255,6 +255,18 @@ int fpq_rmsnorm_rows_quantize_nv_packed(const void* x, int64_t ld, const void* w
                                         const float* global_scale, float* inv_rms, void* normed,
                                         void* packed_codes, void* packed_scales, int zero_policy, void* stream);
 /*
+ * The same for any number of rows: one pass over x, whose rows stay in registers and LDS between the statistic and
+ * the quantization.  cols % 256 == 0, cols <= 16384 (FPQ_E_LIMIT beyond); arguments, rotations and bits as above.
+ */
+int fpq_rmsnorm_tile_quantize_mx_packed(const void* x, int64_t ld, const void* weight, int64_t rows,
+                                        int64_t cols, float eps, int rot_kind, int g, float norm,
+                                        float* inv_rms, void* normed, void* packed_codes,
+                                        void* packed_scales, int zero_policy, void* stream);
+int fpq_rmsnorm_tile_quantize_nv_packed(const void* x, int64_t ld, const void* weight, int64_t rows,
+                                        int64_t cols, float eps, int rot_kind, int g, float norm,
+                                        const float* global_scale, float* inv_rms, void* normed,
+                                        void* packed_codes, void* packed_scales, int zero_policy, void* stream);
+/*
  * The NVFP4 fused producers writing the packed operand layout of fpq_gemm_nvf4_packed (cols % 256 == 0, as for
  * fpq_quantize_nv_packed).  Arguments as fpq_rmsnorm_quantize_nv / fpq_silu_mul_quantize_nv.
  */

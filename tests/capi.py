@@ -374,9 +374,10 @@ def fused_quantize_packed(kind, a, b, g=128, rot="hadamard", norm=None, eps=1e-5
 
 
 def rmsnorm_rows_quantize_packed(x, w, g=128, rot="hadamard", norm=None, eps=1e-5, want_out=True, want_inv=True,
-                                 ld=None, zero_policy=_engine.ZERO_REFERENCE, fill=0xCD, global_scale=None):
-    """fpq_rmsnorm_rows_quantize_{mx,nv}_packed (row statistic + RMSNorm + rotate + quantize of a few rows in
-    one launch; NVFP4 when `global_scale` is given).  Returns CPU (packed codes, packed scales, normed or None,
+                                 ld=None, zero_policy=_engine.ZERO_REFERENCE, fill=0xCD, global_scale=None,
+                                 entry="rows"):
+    """fpq_rmsnorm_{rows,tile}_quantize_{mx,nv}_packed (row statistic + RMSNorm + rotate + quantize in one launch,
+    of a few rows or of any number; NVFP4 when `global_scale` is given).  Returns CPU (packed codes, packed scales, normed or None,
     inv_rms or None)."""
     lib = _engine.lib()
     rows, cols = x.shape
@@ -397,9 +398,9 @@ def rmsnorm_rows_quantize_packed(x, w, g=128, rot="hadamard", norm=None, eps=1e-
     tail = (inv.data_ptr() if inv is not None else None, out.data_ptr() if out is not None else None, pc.data_ptr(),
             ps.data_ptr(), zero_policy, torch.cuda.current_stream().cuda_stream)
     if global_scale is not None:
-        st = lib.fpq_rmsnorm_rows_quantize_nv_packed(*head, gs.data_ptr(), *tail)
+        st = getattr(lib, f"fpq_rmsnorm_{entry}_quantize_nv_packed")(*head, gs.data_ptr(), *tail)
     else:
-        st = lib.fpq_rmsnorm_rows_quantize_mx_packed(*head, *tail)
+        st = getattr(lib, f"fpq_rmsnorm_{entry}_quantize_mx_packed")(*head, *tail)
     _engine.check(st, "fpq_rmsnorm_rows_quantize_packed")
     torch.cuda.synchronize()
     return pc.cpu(), ps.cpu(), (out.cpu() if out is not None else None), (inv.cpu() if inv is not None else None)
