@@ -8,6 +8,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "../../include/fpq.h"
 #include "fpq_device.h"
@@ -100,7 +101,7 @@ __device__ __forceinline__ float exp_det(float t) {
 // bf16(silu(g)) for every bf16 bit pattern g, filled once per device by silu_table_kernel: the
 // activation costs one 2-byte lookup per element (the hot part of the table stays in the L1)
 // instead of ~50 VALU operations, which would make the fused kernel compute-bound.
-__device__ uint16_t g_silu_table[65536];
+__device__ __attribute__((aligned(16))) uint16_t g_silu_table[65536];
 
 __global__ __launch_bounds__(256) void silu_table_kernel() {
   const uint32_t bits = blockIdx.x * 256u + threadIdx.x;
@@ -440,14 +441,43 @@ __device__ __forceinline__ uint32_t fix_zero_nibbles(uint32_t w) {
   return w;
 }
 
+// v[i] += sign * (v[i] of the lane that the quad permutation CTRL names), one instruction each.  Written as assembly
+// because the compiler keeps the lane move apart; a DPP operand may be read two wait states after it was written,
+// which the leading s_nop grants whatever comes before.
+template <int CTRL>
+__device__ __forceinline__ void fma_exchange8(float (&v)[8], float sign) {
+#define FPQ_FMAC_DPP(QP)                                                                                            \
+  asm volatile("s_nop 1\n\t"                                                                                        \
+               "v_fmac_f32_dpp %0, %0, %8 " QP "\n\tv_fmac_f32_dpp %1, %1, %8 " QP "\n\t"                           \
+               "v_fmac_f32_dpp %2, %2, %8 " QP "\n\tv_fmac_f32_dpp %3, %3, %8 " QP "\n\t"                           \
+               "v_fmac_f32_dpp %4, %4, %8 " QP "\n\tv_fmac_f32_dpp %5, %5, %8 " QP "\n\t"                           \
+               "v_fmac_f32_dpp %6, %6, %8 " QP "\n\tv_fmac_f32_dpp %7, %7, %8 " QP                                  \
+               : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])     \
+               : "v"(sign))
+  static_assert(CTRL == 0xB1 || CTRL == 0x4E, "lane ^ 1 or lane ^ 2");
+  if (CTRL == 0xB1) FPQ_FMAC_DPP("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf");
+  else FPQ_FMAC_DPP("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf");
+#undef FPQ_FMAC_DPP
+}
+
 // One lane's chunk of EPL consecutive elements, rotated in place: the butterflies with stride < EPL stay in the
 // lane's registers, a wider rotation takes one or two exchanges with the neighbouring lanes that hold the rest
 // of the block (lane % (G / EPL) is the chunk's place in it).
-template <int EPL, int G, int ROT>
+//
+// An exchange gives the lower lane a + b and the upper one a - b.  With KEEP_ZERO_SIGN the upper lane negates its own
+// value and both add (two instructions and a wait between them); otherwise a lane holds its values negated through
+// the stages before an exchange in which it is the upper one (the norm's sign: a rotation of negated values is the
+// negated rotation), and the exchange is ONE fused multiply-add with +-1, own + sign * other, whose product is exact.
+// The only difference is the sign of a zero, which the reference's zero policy does not look at.
+template <int EPL, int G, int ROT, bool KEEP_ZERO_SIGN>
 __device__ __forceinline__ void rotate_chunk(float (&v)[EPL], float norm, uint32_t lane) {
   if (ROT == FPQ_ROT_HADAMARD || ROT == FPQ_ROT_GSR) {
+    static_assert(G <= 4 * EPL, "at most two exchanges between lanes");
+    constexpr bool kNegate = !KEEP_ZERO_SIGN && G > EPL;
+    const uint32_t upper1 = (lane & 1u) << 31, upper2 = G > 2 * EPL ? (lane & 2u) << 30 : 0u;
+    const float n = kNegate ? __uint_as_float(__float_as_uint(norm) ^ upper1 ^ upper2) : norm;
 #pragma unroll
-    for (int i = 0; i < EPL; ++i) v[i] *= norm;
+    for (int i = 0; i < EPL; ++i) v[i] *= n;
 #pragma unroll
     for (int s = 1; s < (G < EPL ? G : EPL); s *= 2) {
       __builtin_amdgcn_sched_barrier(0);  // keep the stages in place: EPL live values, no more
@@ -460,31 +490,26 @@ __device__ __forceinline__ void rotate_chunk(float (&v)[EPL], float norm, uint32
         }
       }
     }
-    if (G > EPL) {
-      // stride EPL: the two halves of a rotation block sit in lanes 2u and 2u + 1.  The even
-      // lane needs a + b, the odd one a - b = (value of the even lane) + (-own value).
+    auto exchange = [&](auto ctrl, uint32_t upper) __attribute__((always_inline)) {
+      constexpr int kCtrl = decltype(ctrl)::value;
       __builtin_amdgcn_sched_barrier(0);
-      const uint32_t flip = (lane & 1u) << 31;
+      const float sign = __uint_as_float(0xbf800000u ^ upper);   // lower lane -1 (its partner holds -b), upper lane +1
+      if (kNegate) {
 #pragma unroll
-      for (int i = 0; i < EPL; ++i) {
-        const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(
-            (int)__float_as_uint(v[i]), 0xB1 /* quad_perm [1,0,3,2] */, 0xF, 0xF, true));
-        v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ flip);
-      }
-      if (G > 2 * EPL) {
-        // stride 2 EPL (a 128-wide rotation with EPL = 32): the quarters of a block sit in lanes
-        // 4u .. 4u + 3 and the partner is lane ^ 2
-        static_assert(G <= 4 * EPL, "at most two exchanges between lanes");
-        __builtin_amdgcn_sched_barrier(0);
-        const uint32_t flip2 = (lane & 2u) << 30;
+        for (int i = 0; i < EPL; i += 8) fma_exchange8<kCtrl>(*(float (*)[8])&v[i], sign);
+      } else {
 #pragma unroll
         for (int i = 0; i < EPL; ++i) {
-          const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp(
-              (int)__float_as_uint(v[i]), 0x4E /* quad_perm [2,3,0,1] */, 0xF, 0xF, true));
-          v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ flip2);
+          const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v[i]), kCtrl, 0xF,
+                                                                                 0xF, true));
+          v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ upper);
         }
       }
-    }
+    };
+    // stride EPL: the two halves of a rotation block sit in lanes 2u and 2u + 1; stride 2 EPL (a 128-wide rotation
+    // with EPL = 32): the quarters sit in lanes 4u .. 4u + 3 and the partner is lane ^ 2
+    if (G > EPL) exchange(std::integral_constant<int, 0xB1 /* quad_perm [1,0,3,2] */>{}, upper1);
+    if (G > 2 * EPL) exchange(std::integral_constant<int, 0x4E /* quad_perm [2,3,0,1] */>{}, upper2);
     __builtin_amdgcn_sched_barrier(0);
   }
   if (ROT == FPQ_ROT_GSR) {
@@ -630,15 +655,10 @@ __device__ __forceinline__ void quantize_chunk_slow(const float (&u)[EPL], float
 // exactly one lane slot of a packed kilobyte block, so codes are stored straight from registers in two
 // 512-byte runs per store.
 //
-// PRO != kProNone (PACKED only) applies a producer's arithmetic to the values as they leave LDS (see
-// Prologue): kProRmsNorm scales by the row's 1/rms and the column's weight (16-byte loads that hit
-// the L1: a wave touches two 128-byte pieces of the weight) and can write the bf16 result;
-// kProSiluMul streams a second tile (the multiplier) through LDS next to the first and looks the
-// activation up in an LDS copy of the silu table's busy part (|g| in [2^-14, 128)), the rest in the
-// global table.
-constexpr uint32_t kSiluLdsFirst = 113u << 7;         // bf16 magnitude bits of 2^-14
-constexpr uint32_t kSiluLdsCount = 21u * 128u;        // magnitudes up to (not including) 2^7
-
+// PRO == kProRmsNorm (PACKED only) applies the norm to the values as they leave LDS (see Prologue): the row's
+// 1/rms and the column's weight (16-byte loads that hit the L1: a wave touches two 128-byte pieces of the weight);
+// it can write the bf16 result.
+//
 // QUEST (MXFP4, no prologue): the scale of a group comes from its standard deviation instead of its
 // maximum (the rule and its fixed fp32 summation order are stated at lane8_process); a lane holds whole
 // groups, so the statistic needs no cross-lane step, the scale is a power of two, and the conversion
@@ -650,7 +670,7 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
     uint32_t scale_stride, float norm, const float* __restrict__ global_scale, Prologue pro) {
   static_assert(!PACKED || EPL == 64 || (EPL == 32 && PRO == kProNone),
                 "packed output: 64-element chunks; 32-element chunks without a prologue");
-  static_assert(PRO == kProNone || PACKED, "prologues exist for the packed output only");
+  static_assert(PRO == kProNone || (PRO == kProRmsNorm && PACKED), "the norm's prologue, with packed output, only");
   static_assert(!QUEST || (FMT == kFmtMx && PRO == kProNone), "the quest rule exists for plain MXFP4 only");
   constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
   constexpr int NG = EPL / GROUP;        // groups (= scale bytes) per chunk
@@ -661,30 +681,15 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
   constexpr int CW = EPL / 8;            // code dwords per chunk
   constexpr int CQ = CW / 4;             // 16-byte code pieces per chunk
   __shared__ __attribute__((aligned(128))) uint8_t smem[4][TILE];
-  // kProSiluMul: the second tile of every wave and the table copy live in dynamic LDS (together
-  // with the static part they exceed the 64 KB a kernel gets without asking); kProRmsNorm: a tile
-  // per wave for regrouping the by-product
+  // kProRmsNorm: a tile per wave for regrouping the by-product
   extern __shared__ __attribute__((aligned(128))) uint8_t dyn_lds[];
-  uint16_t* silu_lds = (uint16_t*)(dyn_lds + 4 * TILE);
-  // lookups go through a pointer that names the LDS address space, so that they are LDS reads and
-  // not flat loads (which take the texture path)
-  typedef __attribute__((address_space(3))) const uint16_t lds_u16;
-  lds_u16* silu_tab = (lds_u16*)silu_lds;
   __shared__ float2 lut[128];
-  if (PRO == kProSiluMul) {
-    for (uint32_t i = threadIdx.x; i < 2u * kSiluLdsCount; i += 256u) {
-      const uint32_t sgn = i >= kSiluLdsCount ? 1u : 0u;
-      silu_lds[i] = g_silu_table[(sgn << 15) | (kSiluLdsFirst + i - sgn * kSiluLdsCount)];
-    }
-    __syncthreads();
-  }
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t lane = threadIdx.x & 63u;
   uint8_t* my = smem[wave];
   const uint32_t my_base = (uint32_t)(uintptr_t)my;
   uint8_t* my2 = dyn_lds + (PRO != kProNone ? wave : 0) * TILE;
-  const uint32_t my2_base = (uint32_t)(uintptr_t)my2;
 
   float gs = 1.0f, rg = 1.0f;
   bool nv_fast = true;
@@ -717,7 +722,6 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
   constexpr int NV_OFF = PIECES == 8 ? 2 : 4;  // distinct swizzle phases over the instruction index
   // bytes from one row to the next (a prologue's inputs may sit in wider buffers)
   const uint32_t row_bytes = PRO == kProNone ? chunks_per_row * CB : pro.ld_first * 16u;
-  const uint32_t row_bytes2 = PRO == kProSiluMul ? pro.ld_second * 16u : 0u;
   // PACKED: chunk b of the tile is row b / CPR of the tile, chunk b % CPR of its columns.  With 64-element
   // chunks a tile is the 32 rows of a row tile x 2 chunks; with 32-element chunks it is 16 rows (half a row
   // tile) x 4 chunks, so that the 128 columns of the widest rotation still sit in neighbouring lanes.
@@ -725,12 +729,9 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
   constexpr uint32_t CPR = P32 ? 4u : 2u;     // chunks per row of a packed tile
   constexpr uint32_t RPI = CPI / CPR;         // rows filled by one DMA instruction
   const uint32_t b_off = PACKED ? (b_lo / CPR) * row_bytes + (b_lo % CPR) * CB : b_lo * CB;
-  uint32_t voff[NV_OFF], voff2[PRO == kProSiluMul ? NV_OFF : 1];
+  uint32_t voff[NV_OFF];
 #pragma unroll
-  for (int m = 0; m < NV_OFF; ++m) {
-    voff[m] = b_off + ((j_lo ^ sw(CPI * m + b_lo)) * 16u);
-    if (PRO == kProSiluMul) voff2[m] = voff[m] - (b_lo >> 1) * row_bytes + (b_lo >> 1) * row_bytes2;
-  }
+  for (int m = 0; m < NV_OFF; ++m) voff[m] = b_off + ((j_lo ^ sw(CPI * m + b_lo)) * 16u);
   const uint32_t rd_base = lane * CB, l_sw = sw(lane);
 
   const uint32_t pairs = chunks_per_row / CPR;  // PACKED: tiles side by side in a row (half) tile
@@ -758,9 +759,6 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
     }
     const uint8_t* src = PACKED ? x + ((size_t)rt * 32u + 16u * hh) * row_bytes + (size_t)(CPR * pr) * CB
                                 : x + (size_t)tile * TILE;
-    const uint8_t* src2 = PRO == kProSiluMul
-                              ? (const uint8_t*)pro.second + (size_t)rt * 32u * row_bytes2 + (size_t)(2u * pr) * CB
-                              : nullptr;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       // The lane offset is an unsigned 32-bit addend to a scalar base, so it must never be
@@ -770,13 +768,8 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
       if (PACKED) {
         const bool instr_valid = (uint32_t)(RPI * i) < valid;              // wave-uniform
         const uint8_t* base_i = instr_valid ? src + (size_t)(RPI * i) * row_bytes : src;
-        const bool past = RPI * i + b_lo / CPR >= valid;
-        if (past) off = (b_lo % CPR) * CB + j_lo * 16u;
+        if (RPI * i + b_lo / CPR >= valid) off = (b_lo % CPR) * CB + j_lo * 16u;
         lds_dma16_nt(base_i, off, my_base + i * 1024u);
-        if (PRO == kProSiluMul) {
-          const uint8_t* base2_i = instr_valid ? src2 + (size_t)(RPI * i) * row_bytes2 : src2;
-          lds_dma16_nt(base2_i, past ? off : voff2[i % NV_OFF], my2_base + i * 1024u);
-        }
       } else {
         const bool instr_valid = (uint32_t)(CPI * i) < valid;                // wave-uniform
         const uint8_t* base_i = instr_valid ? src + i * 1024 : src;          // scalar address arithmetic
@@ -792,7 +785,6 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
     const uint32_t p_row = PRO == kProNone ? 0u : min(rt * 32u + (lane >> 1), rows - 1u);
     const uint32_t p_cc = PRO == kProNone ? 0u : (2u * pr + (lane & 1u)) * (uint32_t)PIECES;
     const float p_rs = PRO == kProRmsNorm ? pro.row_scale[p_row] : 0.0f;
-    const bool p_store = PRO != kProNone && pro.out != nullptr && (lane >> 1) < valid;
     auto load_rotate = [&](float (&v)[EPL]) {
 #pragma unroll
     for (int k = 0; k < PIECES; ++k) {
@@ -801,39 +793,18 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
       unpack8(raw, e);
       if (PRO != kProNone) {
         float q[8];
-        if (PRO == kProRmsNorm) {
-          unpack8(pro.col_scale[p_cc + k], q);
+        unpack8(pro.col_scale[p_cc + k], q);
 #pragma unroll
-          for (int i = 0; i < 8; ++i) e[i] = bf16_rne(e[i] * p_rs);
-        } else {
-          unpack8(*(const uint4*)(my2 + rd_base + ((k ^ l_sw) * 16u)), q);
-          const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const uint32_t bits = (i & 1) ? (w[i >> 1] >> 16) : (w[i >> 1] & 0xffffu);
-            // the LDS read is unconditional (index clamped) and the rare global read separate, so that
-            // neither turns into a flat load through a pointer that could be either
-            const uint32_t idx = (bits & 0x7fffu) - kSiluLdsFirst;
-            const bool in_lds = idx < kSiluLdsCount;
-            uint32_t t = silu_tab[(bits >> 15) * kSiluLdsCount + (in_lds ? idx : 0u)];
-            if (!in_lds) t = g_silu_table[bits];
-            e[i] = __uint_as_float(t << 16);
-          }
-        }
+        for (int i = 0; i < 8; ++i) e[i] = bf16_rne(e[i] * p_rs);
 #pragma unroll
         for (int i = 0; i < 8; ++i) e[i] = bf16_rne(e[i] * q[i]);
-        if (PRO == kProRmsNorm ? pro.out != nullptr : p_store) {
-          const uint4 packed8 =
+        if (pro.out != nullptr) {
+          // parked in the wave's second LDS tile at the input's (swizzled) place, stored below
+          *(uint4*)(my2 + rd_base + ((k ^ l_sw) * 16u)) =
               make_uint4((__float_as_uint(e[0]) >> 16) | (__float_as_uint(e[1]) & 0xffff0000u),
                          (__float_as_uint(e[2]) >> 16) | (__float_as_uint(e[3]) & 0xffff0000u),
                          (__float_as_uint(e[4]) >> 16) | (__float_as_uint(e[5]) & 0xffff0000u),
                          (__float_as_uint(e[6]) >> 16) | (__float_as_uint(e[7]) & 0xffff0000u));
-          if (PRO == kProRmsNorm) {
-            // parked in the wave's second LDS tile at the input's (swizzled) place, stored below
-            *(uint4*)(my2 + rd_base + ((k ^ l_sw) * 16u)) = packed8;
-          } else {
-            pro.out[(size_t)p_row * chunks_per_row * PIECES + p_cc + k] = packed8;
-          }
         }
       }
 #pragma unroll
@@ -852,7 +823,7 @@ __global__ __launch_bounds__(256, 2) void quantize_stream_kernel(
         }
       }
     }
-    rotate_chunk<EPL, G, ROT>(v, norm, lane);
+    rotate_chunk<EPL, G, ROT, ZERO == kZeroSigned>(v, norm, lane);
     };
     float v[EPL];
     load_rotate(v);
@@ -1017,22 +988,19 @@ static int launch_stream_sized(const void* x, int64_t rows, int64_t cols, float 
                                                     scale_stride, zero_policy, stream);
 }
 
-constexpr int kSiluDynLds = 4 * 64 * 128 + 2 * (int)kSiluLdsCount * 2;  // second tiles + table copy
-
 template <int G, int ROT, int PRO = kProNone, int FMT = kFmtMx, bool QUEST = false, int EPL = 64>
 static int launch_stream_packed(const void* x, int64_t rows, int64_t cols, float norm, void* codes,
                                 void* scales, int zero_policy, hipStream_t stream,
                                 const Prologue& pro = Prologue{}, const float* gsp = nullptr) {
   const int64_t n_tiles = ((rows + 31) / 32) * (cols / 128) * (EPL == 32 ? 2 : 1);
   int64_t blocks = (n_tiles + 3) / 4;
-  // Waves stride over the tiles of a capped grid.  The SiLU*up prologue (two workgroups fit a CU, each
-  // copies the table's busy part into LDS first) is best with one resident round; the RMSNorm prologue
-  // measured 2 % better with a grid twice the plain kernel's (8192 x 4096 and 8192 x 14336 inputs).
-  constexpr int64_t kCap = PRO == kProSiluMul ? 512 : PRO == kProRmsNorm ? 2048 : 1024;
+  // Waves stride over the tiles of a capped grid; the RMSNorm prologue measured 2 % better with a grid twice
+  // the plain kernel's (8192 x 4096 and 8192 x 14336 inputs).
+  constexpr int64_t kCap = PRO == kProRmsNorm ? 2048 : 1024;
   if (blocks > kCap) blocks = kCap;
   const dim3 grid((unsigned)blocks), block(256);
   // kProRmsNorm: one more tile per wave, in which the bf16 by-product is regrouped into row segments
-  constexpr int kDyn = PRO == kProSiluMul ? kSiluDynLds : PRO == kProRmsNorm ? 4 * 64 * 128 : 0;
+  constexpr int kDyn = PRO == kProRmsNorm ? 4 * 64 * 128 : 0;
   int status = 0;
   auto go = [&](auto kernel) {
     if (kDyn) {
@@ -1063,6 +1031,175 @@ static int launch_stream_packed_sized(const void* x, int64_t rows, int64_t cols,
   }
   return launch_stream_packed<G, ROT, kProNone, FMT, QUEST>(x, rows, cols, norm, codes, scales, zero_policy, stream,
                                                             Prologue{}, gsp);
+}
+
+// SiLU*up + rotate + quantize of many rows into the packed operand layout.  A wave tile is 8 rows x 256 columns (one
+// scale block of 8 rows): gate and up are loaded 16 bytes per lane in 512-byte row segments, the next tile's while
+// this one is worked on; the lane that loaded them forms bf16(bf16(silu(gate)) * up), which goes through LDS (4 KB
+// per wave, swizzled so that the reads are conflict-free) to the lanes that own 32-element chunks: 8 rows x 8 chunks.
+// The activation is a lookup in an LDS copy of the silu table's busy part, |g| in [2^-14, 128), held as fp32; the two
+// table offsets of a pair of gates are formed with packed 16-bit arithmetic.  Smaller magnitudes are g / 2 exactly
+// (the relative deviation, |g| / 2, is below half a bf16 step) and larger ones come from the global table: a wave
+// that holds any redoes those lanes.
+// Memory and VALU bound it about equally: 532 MB at 8192 x 14336 in 103.8 us (5.1 TB/s; 121 us between GEMMs that have
+// taken the clock down).  The streaming kernel that did this before (tiles of both inputs through LDS by direct loads,
+// 16-bit table, an 8 KB wave tile that nothing overlapped) took 114.6 (145) us; 2048 rows 34.5 -> 28.2, 512 rows 13.1
+// -> 12.3, 128 rows 9.7 -> 6.5.  A first tile asked for only after the table copy cost 2 us at 512 rows.
+constexpr uint32_t kSiluLdsFirst = 113u << 7;         // bf16 magnitude bits of 2^-14
+constexpr uint32_t kSiluLdsCount = 21u * 128u;        // magnitudes up to (not including) 2^7
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+template <int G, int FMT, int ROT, int ZERO>
+__global__ __launch_bounds__(256, 4) void silu_mul_tile_quantize_kernel(
+    const uint4* __restrict__ gate, const uint4* __restrict__ up, uint8_t* __restrict__ codes,
+    uint8_t* __restrict__ scales, uint32_t rows, uint32_t n_tiles, float norm, const float* __restrict__ global_scale,
+    Prologue pro) {
+  constexpr int EPL = 32;
+  typedef __attribute__((address_space(3))) const float lds_f32;
+  __shared__ __attribute__((aligned(16))) float silu_lds[2 * kSiluLdsCount];
+  __shared__ __attribute__((aligned(128))) uint8_t stage[4][4096];
+  __shared__ float2 lut[FMT == kFmtNv ? 128 : 1];
+  const uint32_t lane = threadIdx.x & 63u;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint8_t* const my = stage[wave];
+  const uint32_t cpr = pro.chunks_per_row, blocks_per_row = cpr / 32u, units = cpr / 8u;
+  const uint32_t l_row = lane >> 5, l_oct = lane & 31u;      // loads: instruction i holds rows 2 i and 2 i + 1
+  const uint32_t r = lane >> 3, c = lane & 7u;               // chunks
+  auto place = [](uint32_t rr, uint32_t b, uint32_t piece) -> uint32_t {
+    return rr * 512u + b * 64u + ((piece ^ (((b >> 2) & 1u) | ((rr & 1u) << 1))) * 16u);
+  };
+  uint4 ga[4], ua[4];
+  auto load = [&](uint32_t tile, uint4 (&g)[4], uint4 (&u)[4]) __attribute__((always_inline)) {
+    const uint32_t rg8 = tile / blocks_per_row, kb = tile - rg8 * blocks_per_row;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t row = min(rg8 * 8u + 2u * i + l_row, rows - 1u), o = kb * 32u + l_oct;
+      g[i] = gate[(size_t)row * pro.ld_first + o];
+      u[i] = up[(size_t)row * pro.ld_second + o];
+    }
+  };
+  const uint32_t step = gridDim.x * 4u;
+  uint32_t tile = blockIdx.x * 4u + wave;
+  load(min(tile, n_tiles - 1u), ga, ua);   // on their way while the table is copied
+  for (uint32_t i = threadIdx.x; i < 2u * kSiluLdsCount / 4u; i += 256u) {
+    const uint32_t first = 4u * i, sgn = first >= kSiluLdsCount ? 1u : 0u;
+    const uint2 e = *(const uint2*)&g_silu_table[(sgn << 15) | (kSiluLdsFirst + first - sgn * kSiluLdsCount)];
+    *(v4f*)&silu_lds[first] = v4f{bf16_lo(e.x), bf16_hi(e.x), bf16_lo(e.y), bf16_hi(e.y)};
+  }
+  float gs = 1.0f, rg = 1.0f;
+  bool nv_fast = true;
+  if (FMT == kFmtNv) {
+    gs = *global_scale;
+    rg = gs == 0.0f ? 0.0f : 1.0f / gs;
+    nv_fast = gs >= 8.673617379884035e-19f && gs <= 1.152921504606847e18f;   // as quantize_stream_kernel
+    if (threadIdx.x < 128) {
+      const float s = e4m3_decode(threadIdx.x) * rg;
+      float2 e = make_float2(0.0f, 0.0f);
+      if (s != 0.0f && nv_fast) {
+        const float y = 1.0f / s;
+        e = make_float2(y, __builtin_fmaf(-s, y, 1.0f) / s);
+      }
+      lut[threadIdx.x] = e;
+    }
+  }
+  __syncthreads();
+  lds_f32* const table = (lds_f32*)silu_lds;
+
+  for (; tile < n_tiles; tile += step) {
+    const uint32_t rg8 = tile / blocks_per_row, kb = tile - rg8 * blocks_per_row;
+    uint4 gn[4], un[4];
+    load(min(tile + step, n_tiles - 1u), gn, un);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t w[4] = {ga[i].x, ga[i].y, ga[i].z, ga[i].w}, q[4] = {ua[i].x, ua[i].y, ua[i].z, ua[i].w};
+      float sv[8];
+      u16x2 most = u16x2{0, 0};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const u16x2 bits = __builtin_bit_cast(u16x2, w[k]);
+        const u16x2 idx = __builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu) - (unsigned short)kSiluLdsFirst;
+        most = __builtin_elementwise_max(most, idx);
+        const u16x2 in = __builtin_elementwise_min(idx, u16x2{kSiluLdsCount - 1, kSiluLdsCount - 1});
+        const u16x2 at = (bits >> (unsigned short)15) * (unsigned short)kSiluLdsCount + in;
+        sv[2 * k] = table[at.x];
+        sv[2 * k + 1] = table[at.y];
+      }
+      const bool outside = most.x >= kSiluLdsCount || most.y >= kSiluLdsCount;
+      if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t bits = (e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu, mag = bits & 0x7fffu;
+          if (mag < kSiluLdsFirst) sv[e] = bf16_rne(__uint_as_float(bits << 16) * 0.5f);
+          else if (mag >= kSiluLdsFirst + kSiluLdsCount) sv[e] = silu_bf16(bits);
+        }
+      }
+      uint32_t v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = pack_bf16x2(sv[2 * k] * bf16_lo(q[k]), sv[2 * k + 1] * bf16_hi(q[k]));
+      const uint4 pv = make_uint4(v[0], v[1], v[2], v[3]);
+      *(uint4*)(my + place(2u * i + l_row, l_oct >> 2, l_oct & 3u)) = pv;
+      if (pro.out) {
+        const uint32_t row = rg8 * 8u + 2u * i + l_row;
+        if (row < rows) store16_nt((uint8_t*)(pro.out + (size_t)row * cpr + kb * 32u + l_oct), pv);
+      }
+    }
+    asm volatile("" ::: "memory");
+
+    auto load_rotate = [&](float (&v)[EPL]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float e[8];
+        unpack8(*(const uint4*)(my + place(r, c, k)), e);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[8 * k + i] = e[i];
+      }
+      rotate_chunk<EPL, G, ROT, ZERO == kZeroSigned>(v, norm, lane);
+    };
+    float v[EPL];
+    load_rotate(v);
+    uint32_t cw[EPL / 8], sbytes = 0u, sb_lo = 0u;
+    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
+      float u[EPL];
+      load_rotate(u);
+      quantize_chunk_slow<EPL, FMT, ZERO>(u, gs, rg, cw, sbytes);
+    }
+    const uint32_t row = rg8 * 8u + r, rt = row >> 5;
+    if (row >= rows) {   // padding rows of the last row tile: zero codes, zero scale bytes
+      cw[0] = cw[1] = cw[2] = cw[3] = 0u;
+      sbytes = 0u;
+    }
+    const uint32_t unit = kb * 4u + (c >> 1), slot = (c & 1u) * 32u + (row & 31u);
+    store16_nt(codes + (((size_t)rt * units + unit) * 64u + slot) * 16u, make_uint4(cw[0], cw[1], cw[2], cw[3]));
+    if (FMT == kFmtMx) {
+      scales[((size_t)rt * blocks_per_row + kb) * 256u + slot * 4u + (c >> 1)] = (uint8_t)sbytes;
+    } else {
+      *(uint16_t*)(scales + ((size_t)rt * blocks_per_row + kb) * 512u + slot * 8u + 2u * (c >> 1)) = (uint16_t)sbytes;
+    }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ga[i] = gn[i];
+      ua[i] = un[i];
+    }
+  }
+}
+
+template <int G, int ROT, int FMT>
+static int launch_silu_tile(const void* gate, const void* up, int64_t rows, int64_t cols, float norm, void* codes,
+                            void* scales, int zero_policy, hipStream_t stream, const Prologue& pro, const float* gsp) {
+  const int64_t n_tiles = (rows + 31) / 32 * 4 * (cols / 256);
+  int64_t blocks = (n_tiles + 3) / 4;
+  // (four workgroups fit a CU; two rounds of them measured 103.8 us at 8192 x 14336 against 107.0 for one round and
+  // 109.3 for half of one, and the same within 1 % below 2048 rows)
+  if (blocks > 2048) blocks = 2048;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint4*)gate, (const uint4*)up,
+                       (uint8_t*)codes, (uint8_t*)scales, (uint32_t)rows, (uint32_t)n_tiles, norm, gsp, pro);
+  };
+  if (zero_policy == FPQ_ZERO_REFERENCE) go(silu_mul_tile_quantize_kernel<G, FMT, ROT, kZeroReference>);
+  else go(silu_mul_tile_quantize_kernel<G, FMT, ROT, kZeroSigned>);
+  return (int)hipGetLastError();
 }
 
 constexpr int64_t kPackedFewRows = 64;
@@ -1462,8 +1599,12 @@ static int dispatch_prologue_packed(const void* x, int64_t ld_first, const void*
     if (few)                                                                                                   \
       return launch_lane8_prologue<GG, FMT, RR, PRO>(x, rows, cols, norm, gsp, codes, scales, rows,            \
                                                      cols / (FMT == kFmtNv ? 16 : 32), zero_policy, stream, pro); \
-    return launch_stream_packed<GG, RR, PRO, FMT>(x, rows, cols, norm, codes, scales, zero_policy, stream,    \
-                                                  pro, gsp);                                                  \
+    if constexpr (PRO == kProSiluMul)                                                                          \
+      return launch_silu_tile<GG, RR, FMT>(x, second, rows, cols, norm, codes, scales, zero_policy, stream,   \
+                                           pro, gsp);                                                         \
+    else                                                                                                       \
+      return launch_stream_packed<GG, RR, PRO, FMT>(x, rows, cols, norm, codes, scales, zero_policy, stream,  \
+                                                    pro, gsp);                                                \
   }
   if (rot_kind == FPQ_ROT_IDENTITY) FPQ_LAUNCH_PRO_PACKED(32, FPQ_ROT_IDENTITY);
   switch (g) {
@@ -1661,7 +1802,7 @@ __global__ __launch_bounds__(64 * kTileRows) void rmsnorm_tile_quantize_kernel(
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[8 * k + i] = e[i];
       }
-      rotate_chunk<EPL, G, ROT>(v, norm, lane);
+      rotate_chunk<EPL, G, ROT, ZERO == kZeroSigned>(v, norm, lane);
     };
     float v[EPL];
     load_rotate(v);
