@@ -30,6 +30,7 @@ namespace fpq {
 // ---------------------------------------------------------------------------------------------
 // Row-major -> packed.  One workgroup re-tiles 32 rows x 256 K: reads are 128-byte row segments,
 // writes cover 4 KB of codes and 256 B of scales contiguously.
+// A K that is no multiple of 256 (but one of 32) is padded to whole blocks with zero codes and scale bytes.
 template <bool NV>
 __global__ __launch_bounds__(256) void pack_fp4_kernel(const uint8_t* __restrict__ codes,
                                                         const uint8_t* __restrict__ scales,
@@ -39,30 +40,33 @@ __global__ __launch_bounds__(256) void pack_fp4_kernel(const uint8_t* __restrict
   const int kb = blockIdx.x, rt = blockIdx.y;
   const int t = threadIdx.x;
   const int r = t >> 3, c = t & 7;  // row in the tile, 16-byte chunk of the 128-byte segment
-  const int row = rt * 32 + r;
+  const int row = rt * 32 + r, nkb = gridDim.x;
   uint4 v = make_uint4(0u, 0u, 0u, 0u);
-  if (row < rows) v = *(const uint4*)(codes + (size_t)row * (K >> 1) + kb * 128 + c * 16);
+  if (row < rows && kb * 256 + c * 32 < K) v = *(const uint4*)(codes + (size_t)row * (K >> 1) + kb * 128 + c * 16);
   const int ks = kb * 4 + (c >> 1), kh = c & 1;
-  *(uint4*)(pcodes + (((size_t)rt * (K >> 6) + ks) * 64 + kh * 32 + r) * 16) = v;
+  *(uint4*)(pcodes + (((size_t)rt * nkb * 4 + ks) * 64 + kh * 32 + r) * 16) = v;
   if (t < 64) {
     const int sr = t & 31, skh = t >> 5;
     const int srow = rt * 32 + sr;
     if (NV) {
       // 16 E4M3 bytes per row and 256 K; K step q, half kh uses bytes 4q + 2kh and 4q + 2kh + 1
-      uint32_t lo = 0u, hi = 0u;
+      uint32_t q[4] = {0u, 0u, 0u, 0u};
       if (srow < rows) {
         const uint8_t* sp = scales + (size_t)srow * scale_stride + kb * 16 + 2 * skh;
-        lo = (uint32_t)sp[0] | ((uint32_t)sp[1] << 8) | ((uint32_t)sp[4] << 16) | ((uint32_t)sp[5] << 24);
-        hi = (uint32_t)sp[8] | ((uint32_t)sp[9] << 8) | ((uint32_t)sp[12] << 16) | ((uint32_t)sp[13] << 24);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (kb * 256 + 64 * i + 32 * skh < K) q[i] = (uint32_t)sp[4 * i] | ((uint32_t)sp[4 * i + 1] << 8);
       }
-      *(uint2*)(pscales + (((size_t)rt * (K >> 8) + kb) * 64 + t) * 8) = make_uint2(lo, hi);
+      *(uint2*)(pscales + (((size_t)rt * nkb + kb) * 64 + t) * 8) = make_uint2(q[0] | (q[1] << 16), q[2] | (q[3] << 16));
     } else {
       uint32_t out = 0u;
       if (srow < rows) {
         const uint8_t* sp = scales + (size_t)srow * scale_stride + kb * 8 + skh;
-        out = (uint32_t)sp[0] | ((uint32_t)sp[2] << 8) | ((uint32_t)sp[4] << 16) | ((uint32_t)sp[6] << 24);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (kb * 256 + 64 * i + 32 * skh < K) out |= (uint32_t)sp[2 * i] << (8 * i);
       }
-      *(uint32_t*)(pscales + (((size_t)rt * (K >> 8) + kb) * 64 + t) * 4) = out;
+      *(uint32_t*)(pscales + (((size_t)rt * nkb + kb) * 64 + t) * 4) = out;
     }
   }
 }
@@ -79,32 +83,32 @@ __global__ __launch_bounds__(256) void unpack_fp4_kernel(const uint8_t* __restri
   const int r = t >> 3, c = t & 7;
   const int row = rt * 32 + r;
   const int ks = kb * 4 + (c >> 1), kh = c & 1;
-  const uint4 v = *(const uint4*)(pcodes + (((size_t)rt * (K >> 6) + ks) * 64 + kh * 32 + r) * 16);
-  if (row < rows) *(uint4*)(codes + (size_t)row * (K >> 1) + kb * 128 + c * 16) = v;
+  const int nkb = gridDim.x;
+  const uint4 v = *(const uint4*)(pcodes + (((size_t)rt * nkb * 4 + ks) * 64 + kh * 32 + r) * 16);
+  if (row < rows && kb * 256 + c * 32 < K) *(uint4*)(codes + (size_t)row * (K >> 1) + kb * 128 + c * 16) = v;
   if (t < 64) {
     const int sr = t & 31, skh = t >> 5;
     const int srow = rt * 32 + sr;
     if (NV) {
-      const uint2 in = *(const uint2*)(pscales + (((size_t)rt * (K >> 8) + kb) * 64 + t) * 8);
+      const uint2 in = *(const uint2*)(pscales + (((size_t)rt * nkb + kb) * 64 + t) * 8);
+      const uint32_t q[4] = {in.x & 0xffffu, in.x >> 16, in.y & 0xffffu, in.y >> 16};
       if (srow < rows) {
         uint8_t* sp = scales + (size_t)srow * scale_stride + kb * 16 + 2 * skh;
-        sp[0] = (uint8_t)in.x;
-        sp[1] = (uint8_t)(in.x >> 8);
-        sp[4] = (uint8_t)(in.x >> 16);
-        sp[5] = (uint8_t)(in.x >> 24);
-        sp[8] = (uint8_t)in.y;
-        sp[9] = (uint8_t)(in.y >> 8);
-        sp[12] = (uint8_t)(in.y >> 16);
-        sp[13] = (uint8_t)(in.y >> 24);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (kb * 256 + 64 * i + 32 * skh < K) {
+            sp[4 * i] = (uint8_t)q[i];
+            sp[4 * i + 1] = (uint8_t)(q[i] >> 8);
+          }
+        }
       }
     } else {
-      const uint32_t in = *(const uint32_t*)(pscales + (((size_t)rt * (K >> 8) + kb) * 64 + t) * 4);
+      const uint32_t in = *(const uint32_t*)(pscales + (((size_t)rt * nkb + kb) * 64 + t) * 4);
       if (srow < rows) {
         uint8_t* sp = scales + (size_t)srow * scale_stride + kb * 8 + skh;
-        sp[0] = (uint8_t)in;
-        sp[2] = (uint8_t)(in >> 8);
-        sp[4] = (uint8_t)(in >> 16);
-        sp[6] = (uint8_t)(in >> 24);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (kb * 256 + 64 * i + 32 * skh < K) sp[2 * i] = (uint8_t)(in >> (8 * i));
       }
     }
   }
@@ -776,16 +780,16 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
 
 template <bool NV>
 static int pack_operand(const void* codes, const void* scales, int64_t scale_stride, int64_t rows, int64_t K,
-                        void* packed_codes, void* packed_scales, void* stream) {
+                        void* packed_codes, void* packed_scales, void* stream, int64_t k_unit = 256) {
   constexpr int GROUP = NV ? 16 : 32;
   if (rows < 0 || K < 0) return FPQ_E_SHAPE;
   if (rows == 0) return FPQ_OK;
   if (!codes || !scales || !packed_codes || !packed_scales) return FPQ_E_NULL;
-  if (K == 0 || K % 256 != 0 || scale_stride < K / GROUP) return FPQ_E_SHAPE;
+  if (K == 0 || K % k_unit != 0 || scale_stride < K / GROUP) return FPQ_E_SHAPE;
   if (rows > (1 << 24) || K > (1 << 24)) return FPQ_E_SHAPE;
   if (((uintptr_t)codes & 15u) || ((uintptr_t)packed_codes & 15u) || ((uintptr_t)packed_scales & 7u))
     return FPQ_E_ALIGN;
-  const dim3 grid((unsigned)(K / 256), (unsigned)((rows + 31) / 32));
+  const dim3 grid((unsigned)((K + 255) / 256), (unsigned)((rows + 31) / 32));
   hipLaunchKernelGGL(pack_fp4_kernel<NV>, grid, dim3(256), 0, (hipStream_t)stream, (const uint8_t*)codes,
                      (const uint8_t*)scales, scale_stride, (int)rows, (int)K, (uint8_t*)packed_codes,
                      (uint8_t*)packed_scales);
@@ -906,15 +910,15 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
 }  // namespace fpq
 
 extern "C" int64_t fpq_packed_codes_bytes(int64_t rows, int64_t K) {
-  return ((rows + 31) / 32) * 32 * (K / 2);
+  return ((rows + 31) / 32) * 32 * ((K + 255) / 256 * 256 / 2);
 }
 
 extern "C" int64_t fpq_packed_scales_bytes(int64_t rows, int64_t K) {
-  return ((rows + 31) / 32) * 32 * (K / 32);
+  return ((rows + 31) / 32) * 32 * ((K + 255) / 256 * 256 / 32);
 }
 
 extern "C" int64_t fpq_packed_scales_bytes_nv(int64_t rows, int64_t K) {
-  return ((rows + 31) / 32) * 32 * (K / 16);
+  return ((rows + 31) / 32) * 32 * ((K + 255) / 256 * 256 / 16);
 }
 
 extern "C" int fpq_pack_mxf4(const void* codes, const void* scales, int64_t scale_stride, int64_t rows,
@@ -925,22 +929,34 @@ extern "C" int fpq_pack_mxf4(const void* codes, const void* scales, int64_t scal
 namespace fpq {
 template <bool NV>
 static int unpack_operand(const void* packed_codes, const void* packed_scales, int64_t rows, int64_t K, void* codes,
-                          void* scales, int64_t scale_stride, void* stream) {
+                          void* scales, int64_t scale_stride, void* stream, int64_t k_unit = 256) {
   constexpr int GROUP = NV ? 16 : 32;
   if (rows < 0 || K < 0) return FPQ_E_SHAPE;
   if (rows == 0) return FPQ_OK;
   if (!codes || !scales || !packed_codes || !packed_scales) return FPQ_E_NULL;
-  if (K == 0 || K % 256 != 0 || scale_stride < K / GROUP) return FPQ_E_SHAPE;
+  if (K == 0 || K % k_unit != 0 || scale_stride < K / GROUP) return FPQ_E_SHAPE;
   if (rows > (1 << 24) || K > (1 << 24)) return FPQ_E_SHAPE;
   if (((uintptr_t)codes & 15u) || ((uintptr_t)packed_codes & 15u) || ((uintptr_t)packed_scales & (NV ? 7u : 3u)))
     return FPQ_E_ALIGN;
-  const dim3 grid((unsigned)(K / 256), (unsigned)((rows + 31) / 32));
+  const dim3 grid((unsigned)((K + 255) / 256), (unsigned)((rows + 31) / 32));
   hipLaunchKernelGGL(unpack_fp4_kernel<NV>, grid, dim3(256), 0, (hipStream_t)stream, (const uint8_t*)packed_codes,
                      (const uint8_t*)packed_scales, (int)rows, (int)K, (uint8_t*)codes, (uint8_t*)scales,
                      scale_stride);
   return (int)hipGetLastError();
 }
 }  // namespace fpq
+
+extern "C" int fpq_pack_padded(int nv, const void* codes, const void* scales, int64_t scale_stride, int64_t rows,
+                               int64_t K, void* packed_codes, void* packed_scales, void* stream) {
+  return nv ? fpq::pack_operand<true>(codes, scales, scale_stride, rows, K, packed_codes, packed_scales, stream, 32)
+            : fpq::pack_operand<false>(codes, scales, scale_stride, rows, K, packed_codes, packed_scales, stream, 32);
+}
+
+extern "C" int fpq_unpack_padded(int nv, const void* packed_codes, const void* packed_scales, int64_t rows, int64_t K,
+                                 void* codes, void* scales, int64_t scale_stride, void* stream) {
+  return nv ? fpq::unpack_operand<true>(packed_codes, packed_scales, rows, K, codes, scales, scale_stride, stream, 32)
+            : fpq::unpack_operand<false>(packed_codes, packed_scales, rows, K, codes, scales, scale_stride, stream, 32);
+}
 
 extern "C" int fpq_unpack_mxf4(const void* packed_codes, const void* packed_scales, int64_t rows, int64_t K,
                                void* codes, void* scales, int64_t scale_stride, void* stream) {

@@ -55,6 +55,8 @@ struct Prologue {
   uint32_t packed_rows;     // generic kernel only: 0 = row-major codes and scales; otherwise the row count
                             // padded to a multiple of 32, and codes / scales are written in the packed
                             // operand layout of the GEMMs (padded rows: zero codes, zero scale bytes)
+  uint32_t packed_chunks;   // ... and the row width in 8-element chunks padded to a multiple of 256 columns (the
+                            // padding likewise zero)
 };
 
 // Packed operand layout, as 32-bit word / byte indices: the 4 code bytes of the 8-element chunk `cc`
@@ -243,7 +245,9 @@ __device__ __forceinline__ void lane8_process(const uint4* __restrict__ x, uint3
                                               uint32_t scale_stride, float norm, float gscale, float rg,
                                               float* __restrict__ stage, const uint16_t* __restrict__ hmat,
                                               uint8_t* __restrict__ mask = nullptr,
-                                              const Prologue& pro = Prologue{}, float row_scale = 0.0f) {
+                                              const Prologue& pro = Prologue{}, float row_scale = 0.0f,
+                                              uint32_t prow = 0u, uint32_t pcc = 0u) {
+  // (prow, pcc): the chunk's place in the packed output, when there is one
   static_assert(!QUEST || FMT == kFmtMx, "the quest rule exists for MXFP4 only");
   constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
   float p[8];
@@ -275,10 +279,9 @@ __device__ __forceinline__ void lane8_process(const uint4* __restrict__ x, uint3
       mbits |= (uint32_t)(__builtin_fabsf(q) < 6.0f) << i;
     }
     if (pro.packed_rows != 0u) {   // packed operand layout (no mask there); pad rows get zeros
-      if (chunk < pro.packed_rows * chunks_per_row) {
-        const uint32_t row = chunk / chunks_per_row, cc = chunk - row * chunks_per_row;
-        codes[packed_code_word(row, cc, chunks_per_row)] = active ? packed : 0u;
-        if ((cc & 3u) == 0u) scales[packed_scale_byte<FMT>(row, cc, chunks_per_row)] = active ? (uint8_t)ex : (uint8_t)0;
+      if (prow < pro.packed_rows) {
+        codes[packed_code_word(prow, pcc, pro.packed_chunks)] = active ? packed : 0u;
+        if ((pcc & 3u) == 0u) scales[packed_scale_byte<FMT>(prow, pcc, pro.packed_chunks)] = active ? (uint8_t)ex : (uint8_t)0;
       }
       return;
     }
@@ -317,11 +320,10 @@ __device__ __forceinline__ void lane8_process(const uint4* __restrict__ x, uint3
   }
 
   if (!QUEST && pro.packed_rows != 0u) {
-    if (chunk < pro.packed_rows * chunks_per_row) {
-      const uint32_t row = chunk / chunks_per_row, cc = chunk - row * chunks_per_row;
-      codes[packed_code_word(row, cc, chunks_per_row)] = active ? packed : 0u;
-      if ((cc & (GROUP / 8 - 1)) == 0u) {
-        scales[packed_scale_byte<FMT>(row, cc, chunks_per_row)] = active ? (uint8_t)gs.byte : (uint8_t)0;
+    if (prow < pro.packed_rows) {
+      codes[packed_code_word(prow, pcc, pro.packed_chunks)] = active ? packed : 0u;
+      if ((pcc & (GROUP / 8 - 1)) == 0u) {
+        scales[packed_scale_byte<FMT>(prow, pcc, pro.packed_chunks)] = active ? (uint8_t)gs.byte : (uint8_t)0;
       }
     }
     return;
@@ -365,16 +367,29 @@ __global__ __launch_bounds__(256) void quantize_lane8_kernel(
     for (int i = threadIdx.x; i < G * G; i += 256) hmat[i] = h[i];
     __syncthreads();
   }
-  const uint32_t chunk = blockIdx.x * 256u + threadIdx.x;
+  uint32_t chunk = blockIdx.x * 256u + threadIdx.x, prow = 0u, pcc = 0u;
+  bool active = chunk < n_chunks;
+  if (pro.packed_rows != 0u) {   // threads number the packed output, padding included
+    prow = chunk / pro.packed_chunks;
+    pcc = chunk - prow * pro.packed_chunks;
+    active = prow < rows && pcc < chunks_per_row;
+    chunk = prow * chunks_per_row + pcc;
+  }
   float g = 1.0f, rg = 1.0f;
   if (FMT == kFmtNv) {
     g = *global_scale;
     rg = g == 0.0f ? 0.0f : 1.0f / g;
   }
-  lane8_process<G, FMT, ROT, ZERO, QUEST, PRO>(x, codes, scales, chunk, chunk < n_chunks, threadIdx.x & 63u,
+  lane8_process<G, FMT, ROT, ZERO, QUEST, PRO>(x, codes, scales, chunk, active, threadIdx.x & 63u,
                                                chunks_per_row, scale_stride, norm, g, rg,
-                                               stage[kStage ? (threadIdx.x >> 6) : 0], hmat, mask, pro);
+                                               stage[kStage ? (threadIdx.x >> 6) : 0], hmat, mask, pro, 0.0f, prow, pcc);
   fill_scale_padding(scales, rows, chunks_per_row / (GROUP / 8), scale_rows, scale_stride);
+}
+
+// The packed output of a [rows, cols] tensor: rows padded to whole row tiles, columns to whole 256-K blocks.
+static void set_packed(Prologue& pro, int64_t rows, int64_t cols) {
+  pro.packed_rows = (uint32_t)((rows + 31) / 32 * 32);
+  pro.packed_chunks = (uint32_t)((cols + 255) / 256 * 32);
 }
 
 template <int G, int FMT, int ROT>
@@ -383,8 +398,8 @@ static int launch_lane8(const void* x, int64_t rows, int64_t cols, float norm, c
                         int zero_policy, hipStream_t stream, const void* h = nullptr, bool packed = false) {
   const int64_t n_chunks = rows * cols / 8;
   Prologue pro{};
-  pro.packed_rows = packed ? (uint32_t)((rows + 31) / 32 * 32) : 0u;
-  const int64_t threads = packed ? (int64_t)pro.packed_rows * (cols / 8) : n_chunks;
+  if (packed) set_packed(pro, rows, cols);
+  const int64_t threads = packed ? (int64_t)pro.packed_rows * pro.packed_chunks : n_chunks;
   const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
   auto args = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const uint4*)x, (uint32_t*)codes,
@@ -1033,10 +1048,13 @@ static int launch_stream_packed_sized(const void* x, int64_t rows, int64_t cols,
                                                             Prologue{}, gsp);
 }
 
-// SiLU*up + rotate + quantize of many rows into the packed operand layout.  A wave tile is 8 rows x 256 columns (one
-// scale block of 8 rows): gate and up are loaded 16 bytes per lane in 512-byte row segments, the next tile's while
-// this one is worked on; the lane that loaded them forms bf16(bf16(silu(gate)) * up), which goes through LDS (4 KB
-// per wave, swizzled so that the reads are conflict-free) to the lanes that own 32-element chunks: 8 rows x 8 chunks.
+// Rotate + quantize of many rows into the packed operand layout, optionally with SiLU*up in front.  A wave tile is 8
+// rows x 256 columns (one scale block of 8 rows): the inputs are loaded 16 bytes per lane in 512-byte row segments,
+// the next tile's while this one is worked on, and go through LDS (4 KB per wave, swizzled so that the reads are
+// conflict-free) to the lanes that own 32-element chunks: 8 rows x 8 chunks.  Columns past `cols` (the padding of the
+// last 256-K block, cols % 32 == 0) and rows past `rows` get zero codes and scale bytes.
+//
+// kProSiluMul: the lane that loaded gate and up forms bf16(bf16(silu(gate)) * up).
 // The activation is a lookup in an LDS copy of the silu table's busy part, |g| in [2^-14, 128), held as fp32; the two
 // table offsets of a pair of gates are formed with packed 16-bit arithmetic.  Smaller magnitudes are g / 2 exactly
 // (the relative deviation, |g| / 2, is below half a bf16 step) and larger ones come from the global table: a wave
@@ -1045,43 +1063,49 @@ static int launch_stream_packed_sized(const void* x, int64_t rows, int64_t cols,
 // taken the clock down).  The streaming kernel that did this before (tiles of both inputs through LDS by direct loads,
 // 16-bit table, an 8 KB wave tile that nothing overlapped) took 114.6 (145) us; 2048 rows 34.5 -> 28.2, 512 rows 13.1
 // -> 12.3, 128 rows 9.7 -> 6.5.  A first tile asked for only after the table copy cost 2 us at 512 rows.
+//
+// kProNone (also QUEST): inputs whose rows are no multiple of 256 columns, which the streaming kernel does not take.
 constexpr uint32_t kSiluLdsFirst = 113u << 7;         // bf16 magnitude bits of 2^-14
 constexpr uint32_t kSiluLdsCount = 21u * 128u;        // magnitudes up to (not including) 2^7
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
-template <int G, int FMT, int ROT, int ZERO>
-__global__ __launch_bounds__(256, 4) void silu_mul_tile_quantize_kernel(
-    const uint4* __restrict__ gate, const uint4* __restrict__ up, uint8_t* __restrict__ codes,
+template <int G, int FMT, int ROT, int ZERO, int PRO, bool QUEST = false>
+__global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
+    const uint4* __restrict__ x, const uint4* __restrict__ up, uint8_t* __restrict__ codes,
     uint8_t* __restrict__ scales, uint32_t rows, uint32_t n_tiles, float norm, const float* __restrict__ global_scale,
     Prologue pro) {
+  static_assert(PRO == kProNone || (PRO == kProSiluMul && !QUEST), "SiLU*up or nothing");
   constexpr int EPL = 32;
+  constexpr bool kSilu = PRO == kProSiluMul;
   typedef __attribute__((address_space(3))) const float lds_f32;
-  __shared__ __attribute__((aligned(16))) float silu_lds[2 * kSiluLdsCount];
+  __shared__ __attribute__((aligned(16))) float silu_lds[kSilu ? 2 * kSiluLdsCount : 4];
   __shared__ __attribute__((aligned(128))) uint8_t stage[4][4096];
   __shared__ float2 lut[FMT == kFmtNv ? 128 : 1];
   const uint32_t lane = threadIdx.x & 63u;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint8_t* const my = stage[wave];
-  const uint32_t cpr = pro.chunks_per_row, blocks_per_row = cpr / 32u, units = cpr / 8u;
+  const uint32_t cpr = pro.chunks_per_row, blocks_per_row = (cpr + 31u) / 32u, units = blocks_per_row * 4u;
   const uint32_t l_row = lane >> 5, l_oct = lane & 31u;      // loads: instruction i holds rows 2 i and 2 i + 1
   const uint32_t r = lane >> 3, c = lane & 7u;               // chunks
   auto place = [](uint32_t rr, uint32_t b, uint32_t piece) -> uint32_t {
     return rr * 512u + b * 64u + ((piece ^ (((b >> 2) & 1u) | ((rr & 1u) << 1))) * 16u);
   };
-  uint4 ga[4], ua[4];
-  auto load = [&](uint32_t tile, uint4 (&g)[4], uint4 (&u)[4]) __attribute__((always_inline)) {
+  constexpr int kUp = kSilu ? 4 : 1;
+  uint4 ga[4], ua[kUp];
+  // (rows and columns past the end re-read the last ones: what becomes of them is replaced by zeros before the stores)
+  auto load = [&](uint32_t tile, uint4 (&g)[4], uint4 (&u)[kUp]) __attribute__((always_inline)) {
     const uint32_t rg8 = tile / blocks_per_row, kb = tile - rg8 * blocks_per_row;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t row = min(rg8 * 8u + 2u * i + l_row, rows - 1u), o = kb * 32u + l_oct;
-      g[i] = gate[(size_t)row * pro.ld_first + o];
-      u[i] = up[(size_t)row * pro.ld_second + o];
+      const uint32_t row = min(rg8 * 8u + 2u * i + l_row, rows - 1u), o = min(kb * 32u + l_oct, cpr - 1u);
+      g[i] = x[(size_t)row * pro.ld_first + o];
+      if constexpr (kSilu) u[i] = up[(size_t)row * pro.ld_second + o];
     }
   };
   const uint32_t step = gridDim.x * 4u;
   uint32_t tile = blockIdx.x * 4u + wave;
   load(min(tile, n_tiles - 1u), ga, ua);   // on their way while the table is copied
-  for (uint32_t i = threadIdx.x; i < 2u * kSiluLdsCount / 4u; i += 256u) {
+  for (uint32_t i = threadIdx.x; kSilu && i < 2u * kSiluLdsCount / 4u; i += 256u) {
     const uint32_t first = 4u * i, sgn = first >= kSiluLdsCount ? 1u : 0u;
     const uint2 e = *(const uint2*)&g_silu_table[(sgn << 15) | (kSiluLdsFirst + first - sgn * kSiluLdsCount)];
     *(v4f*)&silu_lds[first] = v4f{bf16_lo(e.x), bf16_hi(e.x), bf16_lo(e.y), bf16_hi(e.y)};
@@ -1107,40 +1131,45 @@ __global__ __launch_bounds__(256, 4) void silu_mul_tile_quantize_kernel(
 
   for (; tile < n_tiles; tile += step) {
     const uint32_t rg8 = tile / blocks_per_row, kb = tile - rg8 * blocks_per_row;
-    uint4 gn[4], un[4];
+    uint4 gn[4], un[kUp];
     load(min(tile + step, n_tiles - 1u), gn, un);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t w[4] = {ga[i].x, ga[i].y, ga[i].z, ga[i].w}, q[4] = {ua[i].x, ua[i].y, ua[i].z, ua[i].w};
-      float sv[8];
-      u16x2 most = u16x2{0, 0};
+      uint8_t* const at_lds = my + place(2u * i + l_row, l_oct >> 2, l_oct & 3u);
+      if constexpr (kSilu) {
+        const uint32_t w[4] = {ga[i].x, ga[i].y, ga[i].z, ga[i].w}, q[4] = {ua[i].x, ua[i].y, ua[i].z, ua[i].w};
+        float sv[8];
+        u16x2 most = u16x2{0, 0};
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const u16x2 bits = __builtin_bit_cast(u16x2, w[k]);
-        const u16x2 idx = __builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu) - (unsigned short)kSiluLdsFirst;
-        most = __builtin_elementwise_max(most, idx);
-        const u16x2 in = __builtin_elementwise_min(idx, u16x2{kSiluLdsCount - 1, kSiluLdsCount - 1});
-        const u16x2 at = (bits >> (unsigned short)15) * (unsigned short)kSiluLdsCount + in;
-        sv[2 * k] = table[at.x];
-        sv[2 * k + 1] = table[at.y];
-      }
-      const bool outside = most.x >= kSiluLdsCount || most.y >= kSiluLdsCount;
-      if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t bits = (e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu, mag = bits & 0x7fffu;
-          if (mag < kSiluLdsFirst) sv[e] = bf16_rne(__uint_as_float(bits << 16) * 0.5f);
-          else if (mag >= kSiluLdsFirst + kSiluLdsCount) sv[e] = silu_bf16(bits);
+        for (int k = 0; k < 4; ++k) {
+          const u16x2 bits = __builtin_bit_cast(u16x2, w[k]);
+          const u16x2 idx = __builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu) - (unsigned short)kSiluLdsFirst;
+          most = __builtin_elementwise_max(most, idx);
+          const u16x2 in = __builtin_elementwise_min(idx, u16x2{kSiluLdsCount - 1, kSiluLdsCount - 1});
+          const u16x2 at = (bits >> (unsigned short)15) * (unsigned short)kSiluLdsCount + in;
+          sv[2 * k] = table[at.x];
+          sv[2 * k + 1] = table[at.y];
         }
-      }
-      uint32_t v[4];
+        const bool outside = most.x >= kSiluLdsCount || most.y >= kSiluLdsCount;
+        if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[k] = pack_bf16x2(sv[2 * k] * bf16_lo(q[k]), sv[2 * k + 1] * bf16_hi(q[k]));
-      const uint4 pv = make_uint4(v[0], v[1], v[2], v[3]);
-      *(uint4*)(my + place(2u * i + l_row, l_oct >> 2, l_oct & 3u)) = pv;
-      if (pro.out) {
-        const uint32_t row = rg8 * 8u + 2u * i + l_row;
-        if (row < rows) store16_nt((uint8_t*)(pro.out + (size_t)row * cpr + kb * 32u + l_oct), pv);
+          for (int e = 0; e < 8; ++e) {
+            const uint32_t bits = (e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu, mag = bits & 0x7fffu;
+            if (mag < kSiluLdsFirst) sv[e] = bf16_rne(__uint_as_float(bits << 16) * 0.5f);
+            else if (mag >= kSiluLdsFirst + kSiluLdsCount) sv[e] = silu_bf16(bits);
+          }
+        }
+        uint32_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = pack_bf16x2(sv[2 * k] * bf16_lo(q[k]), sv[2 * k + 1] * bf16_hi(q[k]));
+        const uint4 pv = make_uint4(v[0], v[1], v[2], v[3]);
+        *(uint4*)at_lds = pv;
+        if (pro.out) {
+          const uint32_t row = rg8 * 8u + 2u * i + l_row, o = kb * 32u + l_oct;
+          if (row < rows && o < cpr) store16_nt((uint8_t*)(pro.out + (size_t)row * cpr + o), pv);
+        }
+      } else {
+        *(uint4*)at_lds = ga[i];
       }
     }
     asm volatile("" ::: "memory");
@@ -1158,14 +1187,14 @@ __global__ __launch_bounds__(256, 4) void silu_mul_tile_quantize_kernel(
     float v[EPL];
     load_rotate(v);
     uint32_t cw[EPL / 8], sbytes = 0u, sb_lo = 0u;
-    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
-    if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
+    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    if (!QUEST && __builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
       float u[EPL];
       load_rotate(u);
       quantize_chunk_slow<EPL, FMT, ZERO>(u, gs, rg, cw, sbytes);
     }
     const uint32_t row = rg8 * 8u + r, rt = row >> 5;
-    if (row >= rows) {   // padding rows of the last row tile: zero codes, zero scale bytes
+    if (row >= rows || 4u * (kb * 8u + c) >= cpr) {   // padding: zero codes, zero scale bytes
       cw[0] = cw[1] = cw[2] = cw[3] = 0u;
       sbytes = 0u;
     }
@@ -1178,27 +1207,26 @@ __global__ __launch_bounds__(256, 4) void silu_mul_tile_quantize_kernel(
     }
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ga[i] = gn[i];
-      ua[i] = un[i];
-    }
+    for (int i = 0; i < 4; ++i) ga[i] = gn[i];
+#pragma unroll
+    for (int i = 0; i < kUp; ++i) ua[i] = un[i];
   }
 }
 
-template <int G, int ROT, int FMT>
-static int launch_silu_tile(const void* gate, const void* up, int64_t rows, int64_t cols, float norm, void* codes,
-                            void* scales, int zero_policy, hipStream_t stream, const Prologue& pro, const float* gsp) {
-  const int64_t n_tiles = (rows + 31) / 32 * 4 * (cols / 256);
+template <int G, int ROT, int FMT, int PRO, bool QUEST = false>
+static int launch_tile(const void* x, const void* up, int64_t rows, int64_t cols, float norm, void* codes, void* scales,
+                       int zero_policy, hipStream_t stream, const Prologue& pro, const float* gsp) {
+  const int64_t n_tiles = (rows + 31) / 32 * 4 * ((cols + 255) / 256);
   int64_t blocks = (n_tiles + 3) / 4;
   // (four workgroups fit a CU; two rounds of them measured 103.8 us at 8192 x 14336 against 107.0 for one round and
   // 109.3 for half of one, and the same within 1 % below 2048 rows)
   if (blocks > 2048) blocks = 2048;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint4*)gate, (const uint4*)up,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint4*)x, (const uint4*)up,
                        (uint8_t*)codes, (uint8_t*)scales, (uint32_t)rows, (uint32_t)n_tiles, norm, gsp, pro);
   };
-  if (zero_policy == FPQ_ZERO_REFERENCE) go(silu_mul_tile_quantize_kernel<G, FMT, ROT, kZeroReference>);
-  else go(silu_mul_tile_quantize_kernel<G, FMT, ROT, kZeroSigned>);
+  if (zero_policy == FPQ_ZERO_REFERENCE) go(tile_quantize_kernel<G, FMT, ROT, kZeroReference, PRO, QUEST>);
+  else go(tile_quantize_kernel<G, FMT, ROT, kZeroSigned, PRO, QUEST>);
   return (int)hipGetLastError();
 }
 
@@ -1258,8 +1286,8 @@ static int launch_lane8_quest(const void* x, int64_t rows, int64_t cols, float n
                               hipStream_t stream, const void* h, bool packed = false) {
   const int64_t n_chunks = rows * cols / 8;
   Prologue pro{};
-  pro.packed_rows = packed ? (uint32_t)((rows + 31) / 32 * 32) : 0u;
-  const int64_t threads = packed ? (int64_t)pro.packed_rows * (cols / 8) : n_chunks;
+  if (packed) set_packed(pro, rows, cols);
+  const int64_t threads = packed ? (int64_t)pro.packed_rows * pro.packed_chunks : n_chunks;
   const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
   auto args = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const uint4*)x, (uint32_t*)codes,
@@ -1384,6 +1412,68 @@ static int dispatch_quest_packed(const void* x, int64_t rows, int64_t cols, int 
   return FPQ_E_ROTATION;
 }
 
+// Any number of columns that the rotation divides (a multiple of 32), padded to whole 256-K blocks in the packed
+// output: a few rows on the generic kernel, more on the tile kernel (the streaming kernel takes whole 256-K blocks only,
+// and those are dispatched to it).
+template <int FMT, bool QUEST>
+static int dispatch_packed_padded(const void* x, int64_t rows, int64_t cols, int rot_kind, int g, float norm,
+                                  const float* gsp, void* codes, void* scales, int zero_policy, void* stream_) {
+  hipStream_t stream = (hipStream_t)stream_;
+  if (rows >= 0 && cols >= 0 && cols % 256 == 0) {
+    if constexpr (QUEST) return dispatch_quest_packed(x, rows, cols, rot_kind, g, norm, codes, scales, zero_policy, stream_);
+    else return dispatch_packed<FMT>(x, rows, cols, rot_kind, g, norm, gsp, codes, scales, zero_policy, stream_);
+  }
+  if (rows < 0 || cols < 0) return FPQ_E_SHAPE;
+  if (rows == 0) return FPQ_OK;
+  if (!x || !codes || !scales) return FPQ_E_NULL;
+  if (FMT == kFmtNv && !gsp) return FPQ_E_NULL;
+  if (zero_policy != FPQ_ZERO_REFERENCE && zero_policy != FPQ_ZERO_SIGNED) return FPQ_E_POLICY;
+  if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
+  if (g != 16 && g != 32 && g != 64 && g != 128) return FPQ_E_ROTATION;
+  if (cols % 32 != 0 || cols % g != 0) return FPQ_E_SHAPE;
+  if (rows * cols >= (int64_t)1 << 34) return FPQ_E_SHAPE;
+  if (((uintptr_t)x & 15u) || ((uintptr_t)codes & 15u) || ((uintptr_t)scales & 3u)) return FPQ_E_ALIGN;
+  const bool few = rows <= kPackedFewRows;
+  constexpr int64_t kGroupCols = FMT == kFmtMx ? 32 : 16;
+  Prologue pro{};
+  pro.chunks_per_row = pro.ld_first = (uint32_t)(cols / 8);
+#define FPQ_LAUNCH_PADDED(GG, RR)                                                                                  \
+  {                                                                                                                \
+    if constexpr (RR != FPQ_ROT_GSR || GG <= 32) {                                                                 \
+      if (!few)                                                                                                    \
+        return launch_tile<GG, RR, FMT, kProNone, QUEST>(x, nullptr, rows, cols, norm, codes, scales, zero_policy, \
+                                                         stream, pro, gsp);                                        \
+    }                                                                                                              \
+    if constexpr (QUEST)                                                                                           \
+      return launch_lane8_quest<GG, RR>(x, rows, cols, norm, codes, scales, rows, cols / 32, nullptr, zero_policy, \
+                                        stream, nullptr, true);                                                    \
+    else                                                                                                           \
+      return launch_lane8<GG, FMT, RR>(x, rows, cols, norm, gsp, codes, scales, rows, cols / kGroupCols,           \
+                                       zero_policy, stream, nullptr, true);                                        \
+  }
+  if (rot_kind == FPQ_ROT_IDENTITY) {
+    FPQ_LAUNCH_PADDED(32, FPQ_ROT_IDENTITY);
+  } else if (rot_kind == FPQ_ROT_HADAMARD) {
+    switch (g) {
+      case 16: FPQ_LAUNCH_PADDED(16, FPQ_ROT_HADAMARD);
+      case 32: FPQ_LAUNCH_PADDED(32, FPQ_ROT_HADAMARD);
+      case 64: FPQ_LAUNCH_PADDED(64, FPQ_ROT_HADAMARD);
+      case 128: FPQ_LAUNCH_PADDED(128, FPQ_ROT_HADAMARD);
+    }
+  } else if (rot_kind == FPQ_ROT_GSR) {
+    switch (g) {
+      case 16: FPQ_LAUNCH_PADDED(16, FPQ_ROT_GSR);
+      case 32: FPQ_LAUNCH_PADDED(32, FPQ_ROT_GSR);
+      case 64: FPQ_LAUNCH_PADDED(64, FPQ_ROT_GSR);
+    }
+    return FPQ_E_UNSUPPORTED;
+  } else if (rot_kind == FPQ_ROT_GENERAL) {
+    return FPQ_E_UNSUPPORTED;
+  }
+#undef FPQ_LAUNCH_PADDED
+  return FPQ_E_ROTATION;
+}
+
 template <int FMT>
 static int dispatch(const void* x, int64_t rows, int64_t cols, int rot_kind, int g, float norm,
                     const void* h, const float* gsp, void* codes, void* scales,
@@ -1451,7 +1541,7 @@ static int launch_lane8_prologue(const void* x, int64_t rows, int64_t cols, floa
                                  void* codes, void* scales, int64_t scale_rows, int64_t scale_stride,
                                  int zero_policy, hipStream_t stream, const Prologue& pro) {
   const int64_t n_chunks = rows * cols / 8;
-  const int64_t threads = pro.packed_rows ? (int64_t)pro.packed_rows * (cols / 8) : n_chunks;
+  const int64_t threads = pro.packed_rows ? (int64_t)pro.packed_rows * pro.packed_chunks : n_chunks;
   const dim3 grid((unsigned)((threads + 255) / 256)), block(256);
   auto args = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, (const uint4*)x, (uint32_t*)codes,
@@ -1549,7 +1639,8 @@ static int dispatch_prologue(const void* x, int64_t ld_first, const void* second
   return FPQ_E_ROTATION;
 }
 
-// The same with the packed operand layout as output (streaming kernel; cols % 256 == 0).
+// The same with the packed operand layout as output (kProRmsNorm: cols % 256 == 0; kProSiluMul: cols % 32 == 0, padded
+// to whole 256-K blocks).
 template <int PRO, int FMT = kFmtMx>
 static int dispatch_prologue_packed(const void* x, int64_t ld_first, const void* second, int64_t ld_second,
                                     const float* row_scale, const void* col_scale, void* out, int64_t rows,
@@ -1568,7 +1659,8 @@ static int dispatch_prologue_packed(const void* x, int64_t ld_first, const void*
     return (rot_kind == FPQ_ROT_GSR || rot_kind == FPQ_ROT_GENERAL) ? FPQ_E_UNSUPPORTED : FPQ_E_ROTATION;
   }
   if (g != 16 && g != 32 && g != 64 && g != 128) return FPQ_E_ROTATION;
-  if (cols % 256 != 0) return FPQ_E_SHAPE;
+  if (cols % 32 != 0 || cols % g != 0) return FPQ_E_SHAPE;
+  if (PRO == kProRmsNorm && cols % 256 != 0) return FPQ_E_SHAPE;
   if (ld_first < cols || ld_first % 8 != 0) return FPQ_E_SHAPE;
   if (PRO == kProSiluMul && (ld_second < cols || ld_second % 8 != 0)) return FPQ_E_SHAPE;
   // 32-bit byte offsets inside a row tile, 32-bit chunk counts
@@ -1593,14 +1685,14 @@ static int dispatch_prologue_packed(const void* x, int64_t ld_first, const void*
   pro.ld_second = (uint32_t)(ld_second / 8);
   pro.packed_rows = 0u;
   const bool few = rows <= kPackedFewRows;
-  if (few) pro.packed_rows = (uint32_t)((rows + 31) / 32 * 32);
+  if (few) set_packed(pro, rows, cols);
 #define FPQ_LAUNCH_PRO_PACKED(GG, RR)                                                                          \
   {                                                                                                            \
     if (few)                                                                                                   \
       return launch_lane8_prologue<GG, FMT, RR, PRO>(x, rows, cols, norm, gsp, codes, scales, rows,            \
                                                      cols / (FMT == kFmtNv ? 16 : 32), zero_policy, stream, pro); \
     if constexpr (PRO == kProSiluMul)                                                                          \
-      return launch_silu_tile<GG, RR, FMT>(x, second, rows, cols, norm, codes, scales, zero_policy, stream,   \
+      return launch_tile<GG, RR, FMT, PRO>(x, second, rows, cols, norm, codes, scales, zero_policy, stream,   \
                                            pro, gsp);                                                         \
     else                                                                                                       \
       return launch_stream_packed<GG, RR, PRO, FMT>(x, rows, cols, norm, codes, scales, zero_policy, stream,  \
@@ -1691,10 +1783,10 @@ __global__ __launch_bounds__(1024) void rmsnorm_rows_quantize_kernel(const uint4
   for (uint32_t c0 = 0; c0 < cpr; c0 += nthr) {   // the same trip count for every thread: lanes exchange values
     const uint32_t cc = c0 + threadIdx.x;
     const bool in = cc < cpr;
-    // a chunk index past the packed output makes the generic kernel skip the store
-    const uint32_t chunk = in ? row * cpr + cc : 0xffffffffu;
-    lane8_process<G, FMT, ROT, ZERO, false, kProRmsNorm>(x, codes, scales, chunk, real && in, lane, cpr, 0u, norm, gs,
-                                                         rg, nullptr, nullptr, nullptr, pro, rs);
+    // (a row past the packed output makes the generic kernel skip the store)
+    lane8_process<G, FMT, ROT, ZERO, false, kProRmsNorm>(x, codes, scales, row * cpr + (in ? cc : 0u), real && in, lane,
+                                                         cpr, 0u, norm, gs, rg, nullptr, nullptr, nullptr, pro, rs,
+                                                         in ? row : 0xffffffffu, cc);
   }
 }
 
@@ -1704,7 +1796,7 @@ __global__ __launch_bounds__(1024) void rmsnorm_rows_quantize_kernel(const uint4
 // row in LDS; then lanes own 32-element chunks (4 rows x 16 chunks per wave) and rotate, quantize and store them in
 // the packed operand layout as runs of 64 bytes.  The 16-byte pieces of a chunk sit in LDS XOR-swizzled by the
 // chunk so that the chunk reads hit every bank group once.  Rows past `rows` (the padding of the last 32-row tile)
-// get zero codes and scale bytes.
+// and columns past `cols` (the padding of the last 256-K block) get zero codes and scale bytes.
 // Memory bounds it: x in, by-product and codes out, 152 MB for 8192 x 4096 (30.2 us = 5.0 TB/s, a device copy's
 // rate; 23.9 us without the by-product).  The statistic in a launch of its own, with a second pass over x, took
 // 46.6 (39.1) us; 2048 rows 16.6 -> 9.6, 128 rows 9.3 -> 5.8, 8192 x 2048 25.0 -> 16.9, 3000 x 8192 37.7 -> 25.8.
@@ -1788,17 +1880,18 @@ __global__ __launch_bounds__(64 * kTileRows) void rmsnorm_tile_quantize_kernel(
   }
   __syncthreads();
 
-  const uint32_t r = lane / CPL, c = lane % CPL, chunks = cpr / 4u, units = cpr / 8u;
+  const uint32_t r = lane / CPL, c = lane % CPL, chunks = cpr / 4u;
+  const uint32_t padded = (cpr + 31u) / 32u * 8u, units = padded / 2u;   // chunks of whole 256-K blocks
   const uint32_t rt = row0 >> 5, rit = (row0 & 31u) + r;   // row tile, row inside it
   const bool row_ok = row0 + r < rows;
-  for (uint32_t c0 = wave * CPL; c0 < chunks; c0 += kTileRows * CPL) {
-    const bool in = c0 + c < chunks;                       // (whole quads of lanes: chunks % 8 == 0)
-    const uint32_t b = in ? c0 + c : c;
+  for (uint32_t c0 = wave * CPL; c0 < padded; c0 += kTileRows * CPL) {
+    // (lanes that exchange values are inside or outside together: cols % G == 0)
+    const uint32_t b = c0 + c, from = b < chunks ? b : c % (G > EPL ? G / EPL : 1);
     auto load_rotate = [&](float (&v)[EPL]) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         float e[8];
-        unpack8(*(const uint4*)(dyn_lds + place(r, 4u * b + k)), e);
+        unpack8(*(const uint4*)(dyn_lds + place(r, 4u * from + k)), e);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[8 * k + i] = e[i];
       }
@@ -1813,11 +1906,11 @@ __global__ __launch_bounds__(64 * kTileRows) void rmsnorm_tile_quantize_kernel(
       load_rotate(u);
       quantize_chunk_slow<EPL, FMT, ZERO>(u, gs, rg, cw, sbytes);
     }
-    if (!row_ok) {
+    if (!row_ok || b >= chunks) {
       cw[0] = cw[1] = cw[2] = cw[3] = 0u;
       sbytes = 0u;
     }
-    if (in) {
+    if (b < padded) {
       const uint32_t unit = b >> 1, slot = (b & 1u) * 32u + rit;
       store16_nt(codes + (((size_t)rt * units + unit) * 64u + slot) * 16u, make_uint4(cw[0], cw[1], cw[2], cw[3]));
       if (FMT == kFmtMx) {
@@ -1951,6 +2044,22 @@ extern "C" int fpq_quantize_nv_packed(const void* x, int64_t rows, int64_t cols,
                                            packed_scales, zero_policy, stream);
 }
 
+extern "C" int fpq_quantize_mx_packed_padded(const void* x, int64_t rows, int64_t cols, int quest, int rot_kind, int g,
+                                             float norm, void* packed_codes, void* packed_scales, int zero_policy,
+                                             void* stream) {
+  return quest ? fpq::dispatch_packed_padded<fpq::kFmtMx, true>(x, rows, cols, rot_kind, g, norm, nullptr, packed_codes,
+                                                                packed_scales, zero_policy, stream)
+               : fpq::dispatch_packed_padded<fpq::kFmtMx, false>(x, rows, cols, rot_kind, g, norm, nullptr, packed_codes,
+                                                                 packed_scales, zero_policy, stream);
+}
+
+extern "C" int fpq_quantize_nv_packed_padded(const void* x, int64_t rows, int64_t cols, int rot_kind, int g, float norm,
+                                             const float* global_scale, void* packed_codes, void* packed_scales,
+                                             int zero_policy, void* stream) {
+  return fpq::dispatch_packed_padded<fpq::kFmtNv, false>(x, rows, cols, rot_kind, g, norm, global_scale, packed_codes,
+                                                         packed_scales, zero_policy, stream);
+}
+
 extern "C" int fpq_quantize_nv(const void* x, int64_t rows, int64_t cols, int rot_kind, int g,
                                float norm, const void* h, const float* global_scale, void* codes,
                                void* scales, int64_t scale_rows, int64_t scale_stride,
@@ -2048,7 +2157,7 @@ static int dispatch_rmsnorm_rows(const void* x, int64_t ld, const void* weight, 
   pro.out = (uint4*)normed;
   pro.chunks_per_row = (uint32_t)(cols / 8);
   pro.ld_first = (uint32_t)(ld / 8);
-  pro.packed_rows = (uint32_t)((rows + 31) / 32 * 32);
+  set_packed(pro, rows, cols);
   // a row is one workgroup's work: wider rows get more waves (the row statistic does not depend on the count)
   const dim3 grid(pro.packed_rows), block(pro.chunks_per_row >= 1024u ? 1024 : pro.chunks_per_row >= 512u ? 512 : 256);
 #define FPQ_LAUNCH_ROWS(GG, RR)                                                                                 \
@@ -2089,7 +2198,7 @@ static int dispatch_rmsnorm_tile(const void* x, int64_t ld, const void* weight, 
     return (rot_kind == FPQ_ROT_GSR || rot_kind == FPQ_ROT_GENERAL) ? FPQ_E_UNSUPPORTED : FPQ_E_ROTATION;
   }
   if (g != 16 && g != 32 && g != 64 && g != 128) return FPQ_E_ROTATION;
-  if (cols % 256 != 0 || ld < cols || ld % 8 != 0 || ld >= (int64_t)1 << 24) return FPQ_E_SHAPE;
+  if (cols % 32 != 0 || cols % g != 0 || ld < cols || ld % 8 != 0 || ld >= (int64_t)1 << 24) return FPQ_E_SHAPE;
   if (rows * ld >= (int64_t)1 << 34) return FPQ_E_SHAPE;
   if (cols > kTileKernelMaxCols) return FPQ_E_LIMIT;
   if (((uintptr_t)x & 15u) || ((uintptr_t)weight & 15u) || ((uintptr_t)normed & 15u) || ((uintptr_t)inv_rms & 3u) ||

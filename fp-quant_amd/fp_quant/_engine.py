@@ -63,6 +63,10 @@ _SIGNATURES = {
     "fpq_rmsnorm_rows_max_rows": ([], _I64),
     "fpq_rmsnorm_rows_quantize_mx_packed": ([_P, _I64, _P, _I64, _I64, _F, _I, _I, _F, _P, _P, _P, _P, _I, _P], _I),
     "fpq_rmsnorm_rows_quantize_nv_packed": ([_P, _I64, _P, _I64, _I64, _F, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P], _I),
+    "fpq_pack_padded": ([_I, _P, _P, _I64, _I64, _I64, _P, _P, _P], _I),
+    "fpq_unpack_padded": ([_I, _P, _P, _I64, _I64, _P, _P, _I64, _P], _I),
+    "fpq_quantize_mx_packed_padded": ([_P, _I64, _I64, _I, _I, _I, _F, _P, _P, _I, _P], _I),
+    "fpq_quantize_nv_packed_padded": ([_P, _I64, _I64, _I, _I, _F, _P, _P, _P, _I, _P], _I),
     "fpq_rmsnorm_tile_quantize_mx_packed": ([_P, _I64, _P, _I64, _I64, _F, _I, _I, _F, _P, _P, _P, _P, _I, _P], _I),
     "fpq_rmsnorm_tile_quantize_nv_packed": ([_P, _I64, _P, _I64, _I64, _F, _I, _I, _F, _P, _P, _P, _P, _P, _I, _P], _I),
     "fpq_rmsnorm_quantize_nv_packed": ([_P, _I64, _P, _P, _I64, _I64, _I, _I, _F, _P, _P, _P, _P, _I, _P], _I),

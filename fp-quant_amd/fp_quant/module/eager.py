@@ -30,7 +30,9 @@ from .hip_ops import (
     packed_linear_eligible,
     packed_weight,
     packed_weight_ready,
+    packable_k,
     packed_weights_enabled,
+    padded_k,
     quantize_mx_packed,
     splitk_workspace,
     SPLIT_K_MAX_ROWS,
@@ -191,8 +193,8 @@ def quantize_activations(x_flat: torch.Tensor, h: torch.Tensor, kind: int, norm:
     if quest and want_packed:
         pc = torch.empty(lib.fpq_packed_codes_bytes(m, k), dtype=torch.uint8, device=dev)
         ps = torch.empty(lib.fpq_packed_scales_bytes(m, k), dtype=torch.uint8, device=dev)
-        st = lib.fpq_quantize_mx_quest_packed(x_flat.data_ptr(), m, k, kind, g, norm, pc.data_ptr(), ps.data_ptr(),
-                                              ZERO_NIBBLE_POLICY, stream)
+        st = lib.fpq_quantize_mx_packed_padded(x_flat.data_ptr(), m, k, 1, kind, g, norm, pc.data_ptr(), ps.data_ptr(),
+                                               ZERO_NIBBLE_POLICY, stream)
         if st != _engine.E_UNSUPPORTED:
             _engine.check(st, "fpq_quantize_mx_quest_packed")
             qa.mx_packed = (pc, ps)
@@ -209,8 +211,8 @@ def quantize_activations(x_flat: torch.Tensor, h: torch.Tensor, kind: int, norm:
     if want_packed and not nvfp4:
         pc = torch.empty(lib.fpq_packed_codes_bytes(m, k), dtype=torch.uint8, device=dev)
         ps = torch.empty(lib.fpq_packed_scales_bytes(m, k), dtype=torch.uint8, device=dev)
-        st = lib.fpq_quantize_mx_packed(x_flat.data_ptr(), m, k, kind, g, norm, pc.data_ptr(), ps.data_ptr(),
-                                        ZERO_NIBBLE_POLICY, stream)
+        st = lib.fpq_quantize_mx_packed_padded(x_flat.data_ptr(), m, k, 0, kind, g, norm, pc.data_ptr(), ps.data_ptr(),
+                                               ZERO_NIBBLE_POLICY, stream)
         if st == _engine.E_UNSUPPORTED:
             pc, ps = quantize_mx_packed(x_flat, h)
         else:
@@ -221,8 +223,8 @@ def quantize_activations(x_flat: torch.Tensor, h: torch.Tensor, kind: int, norm:
         pc = torch.empty(lib.fpq_packed_codes_bytes(m, k), dtype=torch.uint8, device=dev)
         ps = torch.empty(lib.fpq_packed_scales_bytes_nv(m, k), dtype=torch.uint8, device=dev)
         gs = as_f32_scalar(act_global_scale, remember)
-        st = lib.fpq_quantize_nv_packed(x_flat.data_ptr(), m, k, kind, g, norm, gs.data_ptr(), pc.data_ptr(),
-                                        ps.data_ptr(), ZERO_NIBBLE_POLICY, stream)
+        st = lib.fpq_quantize_nv_packed_padded(x_flat.data_ptr(), m, k, kind, g, norm, gs.data_ptr(), pc.data_ptr(),
+                                               ps.data_ptr(), ZERO_NIBBLE_POLICY, stream)
         if st != _engine.E_UNSUPPORTED:
             _engine.check(st, "fpq_quantize_nv_packed")
             qa.nv_packed = (pc, ps)
@@ -265,9 +267,10 @@ def linear_on(qa: QuantizedActivations, wq: torch.Tensor, ws: torch.Tensor, alph
     call may create and keep what the layer lacks (its split-K workspace)."""
     lib = _engine.lib()
     m, k = qa.m, qa.k
+    kp = padded_k(k)         # of the packed operands
     if packed is not None:   # packed MXFP4 weights of `n` rows handed in directly (a WeightGroup): wq, ws unused
         wp, wsp, n = packed
-        if wp.numel() * 2 != n * k:
+        if wp.numel() * 2 != n * kp:
             raise ValueError("packed weights need activations with the same inner dimension")
         use_packed = True
     elif is_packed_only(wq):   # a layer that holds its weight in the packed layout only
@@ -302,18 +305,18 @@ def linear_on(qa: QuantizedActivations, wq: torch.Tensor, ws: torch.Tensor, alph
                 st = lib.fpq_gemm_nvf4_packed_splitk(xp.data_ptr(), xsp.data_ptr(), wp.data_ptr(), wsp.data_ptr(),
                                                      alpha.data_ptr(), b_ptr,
                                                      residual.data_ptr() if residual is not None else None,
-                                                     y.data_ptr(), m, n, k, workspace.data_ptr(), workspace.numel(),
+                                                     y.data_ptr(), m, n, kp, workspace.data_ptr(), workspace.numel(),
                                                      stream)
                 _engine.check(st, "fpq_gemm_nvf4_packed_splitk")
                 return y
             if residual is not None:
                 st = lib.fpq_gemm_nvf4_packed_residual(xp.data_ptr(), xsp.data_ptr(), wp.data_ptr(), wsp.data_ptr(),
                                                        alpha.data_ptr(), b_ptr, residual.data_ptr(), y.data_ptr(),
-                                                       m, n, k, stream)
+                                                       m, n, kp, stream)
                 _engine.check(st, "fpq_gemm_nvf4_packed_residual")
                 return y
             st = lib.fpq_gemm_nvf4_packed(xp.data_ptr(), xsp.data_ptr(), wp.data_ptr(), wsp.data_ptr(),
-                                          alpha.data_ptr(), b_ptr, y.data_ptr(), m, n, k, stream)
+                                          alpha.data_ptr(), b_ptr, y.data_ptr(), m, n, kp, stream)
             _engine.check(st, "fpq_gemm_nvf4_packed")
         else:
             codes, scales = qa.rows()
@@ -333,14 +336,14 @@ def linear_on(qa: QuantizedActivations, wq: torch.Tensor, ws: torch.Tensor, alph
             st = lib.fpq_gemm_mxf4_packed_splitk(pc.data_ptr(), ps.data_ptr(), wp.data_ptr(), wsp.data_ptr(),
                                                  alpha.data_ptr(), b_ptr,
                                                  residual.data_ptr() if residual is not None else None, y.data_ptr(),
-                                                 m, n, k, workspace.data_ptr(), workspace.numel(), stream)
+                                                 m, n, kp, workspace.data_ptr(), workspace.numel(), stream)
         elif residual is not None:
             st = lib.fpq_gemm_mxf4_packed_residual(pc.data_ptr(), ps.data_ptr(), wp.data_ptr(), wsp.data_ptr(),
                                                    alpha.data_ptr(), b_ptr, residual.data_ptr(), y.data_ptr(),
-                                                   m, n, k, stream)
+                                                   m, n, kp, stream)
         else:
             st = lib.fpq_gemm_mxf4_packed(pc.data_ptr(), ps.data_ptr(), wp.data_ptr(), wsp.data_ptr(),
-                                          alpha.data_ptr(), b_ptr, y.data_ptr(), m, n, k, stream)
+                                          alpha.data_ptr(), b_ptr, y.data_ptr(), m, n, kp, stream)
         _engine.check(st, "fpq_gemm_mxf4_packed")
         return y
     codes, scales = qa.rows()
@@ -453,7 +456,7 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
     dev = first.device
     packed_only = is_packed_only(first)
     have_bias = [m[2] is not None for m in members]
-    if k < 256 or k % 256 != 0:
+    if not packable_k(k) or (packed_only and k % 256 != 0):
         return None
     for wq, ws, bias, k_in in members:
         if (wq.dtype != torch.uint8 or ws.dtype != torch.uint8 or not wq.is_cuda or wq.device != dev or k_in != k
@@ -475,7 +478,6 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
     group = WeightGroup()
     group.n, group.splits, group.k, group.nvfp4 = n, splits, k, nvfp4
     scales_bytes = lib.fpq_packed_scales_bytes_nv if nvfp4 else lib.fpq_packed_scales_bytes
-    pack = lib.fpq_pack_nvf4 if nvfp4 else lib.fpq_pack_mxf4
     reuse = previous
     if (reuse is not None and (reuse.nvfp4 != nvfp4 or reuse.k != k or reuse.splits != splits or reuse.wp.device != dev
                                or torch.cuda.is_current_stream_capturing())):
@@ -509,8 +511,9 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
                 if wq.data_ptr() != pc.data_ptr() or ws.data_ptr() != ps.data_ptr():
                     wq.data, ws.data = pc, ps
             else:
-                st = pack(wq.data_ptr(), ws.data_ptr(), ws.shape[1], rows, k, pc.data_ptr(), ps.data_ptr(), stream)
-                _engine.check(st, "fpq_pack")
+                st = lib.fpq_pack_padded(int(nvfp4), wq.data_ptr(), ws.data_ptr(), ws.shape[1], rows, k, pc.data_ptr(),
+                                         ps.data_ptr(), stream)
+                _engine.check(st, "fpq_pack_padded")
                 # the member's own packed copy: these views (same key as hip_ops.packed_weight uses)
                 wq._fpq_packed = ((wq.data_ptr(), _version(wq), ws.data_ptr(), _version(ws), tuple(wq.shape), nvfp4), pc, ps)
     group.key = tuple(_member_key(*m[:3]) for m in members)   # (packed-only members have just moved)
@@ -528,7 +531,7 @@ def linear_on_group(qa: QuantizedActivations, wp: torch.Tensor, wsp: torch.Tenso
     (`splits`: the layers' output features); returns the layers' outputs, bf16 [m, n_i] each.  Every
     layer gets a dense matrix of its own from the kernel when all n_i are multiples of 256; else the
     outputs are column ranges of one [m, sum n_i] matrix (rows keep the full stride)."""
-    m, k, n = qa.m, qa.k, sum(splits)
+    m, k, n = qa.m, padded_k(qa.k), sum(splits)
     if wp.numel() * 2 != n * k:
         raise ValueError("packed weights need activations with the same inner dimension")
     if len(splits) > 4 or any(s % 256 for s in splits):
@@ -740,7 +743,7 @@ def _fused_quantize(entry: str, head: tuple, rows: int, cols: int, h: torch.Tens
         qa = QuantizedActivations(rows, cols, nvfp4)
         qa.mx_packed = (pc, ps)
         return qa
-    if allow_packed and nvfp4 and cols % 256 == 0 and nv_packed_eligible(rows, 32, cols, fused_linear=True):
+    if allow_packed and nvfp4 and nv_packed_eligible(rows, 32, cols, fused_linear=True):
         # the row counts whose consumers run the packed NVFP4 GEMM: straight into its layout
         gs = as_f32_scalar(act_global_scale, remember)
         pc = torch.empty(lib.fpq_packed_codes_bytes(rows, cols), dtype=torch.uint8, device=dev)
@@ -796,12 +799,12 @@ def rmsnorm_quantize(x: torch.Tensor, weight: torch.Tensor, eps: float, hadamard
         y = torch.empty_like(x_flat)
         w = weight.contiguous()
         qa = None
-        if (cols % 256 == 0 and cols <= _ONE_LAUNCH_MAX_COLS
+        if (cols <= _ONE_LAUNCH_MAX_COLS
                 and (nv_packed_eligible(rows, 32, cols, fused_linear=True) if nvfp4
                      else packed_linear_eligible(rows, cols, "abs_max"))):
             # statistic, normalisation and quantization in one launch: a decode step's few rows spread over many
             # lanes each, more rows a wave each
-            kernel = "rows" if rows <= _ROWS_KERNEL_MAX_ROWS else "tile"
+            kernel = "rows" if rows <= _ROWS_KERNEL_MAX_ROWS and cols % 256 == 0 else "tile"
             pc = torch.empty(lib.fpq_packed_codes_bytes(rows, cols), dtype=torch.uint8, device=dev)
             qa = QuantizedActivations(rows, cols, nvfp4)
             head = (x_flat.data_ptr(), cols, w.data_ptr(), rows, cols, eps, kind, h.shape[0], norm)
@@ -822,7 +825,7 @@ def rmsnorm_quantize(x: torch.Tensor, weight: torch.Tensor, eps: float, hadamard
             _engine.check(lib.fpq_row_inv_rms(x_flat.data_ptr(), cols, rows, cols, eps, inv.data_ptr(), stream),
                           "fpq_row_inv_rms")
             qa = _fused_quantize("rmsnorm", (x_flat.data_ptr(), cols, inv.data_ptr(), w.data_ptr()), rows, cols, h, kind,
-                                 norm, act_global_scale, nvfp4, y, stream, dev)
+                                 norm, act_global_scale, nvfp4, y, stream, dev, allow_packed=cols % 256 == 0)
         if qa is None:
             return None
         y = y.view(x.shape)

@@ -99,7 +99,7 @@ def _padded(rows: int, groups: int) -> Tuple[int, int]:
 
 def quantize_mx_packed(x: torch.Tensor, hadamard_matrix: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
     """abs_max MXFP4 quantization of bf16 [rows, cols] straight into the packed GEMM layout
-    (cols % 256 == 0).  Rotations the packed quantizer has no kernel for go through the row-major
+    (cols % 32 == 0).  Rotations the packed quantizer has no kernel for go through the row-major
     quantizer and the re-tiling kernel."""
     lib = _engine.lib()
     rows, cols = x.shape
@@ -107,8 +107,8 @@ def quantize_mx_packed(x: torch.Tensor, hadamard_matrix: torch.Tensor) -> Tuple[
     g = hadamard_matrix.shape[0]
     pc = torch.empty(lib.fpq_packed_codes_bytes(rows, cols), dtype=torch.uint8, device=x.device)
     ps = torch.empty(lib.fpq_packed_scales_bytes(rows, cols), dtype=torch.uint8, device=x.device)
-    st = lib.fpq_quantize_mx_packed(x.data_ptr(), rows, cols, kind, g, norm, pc.data_ptr(), ps.data_ptr(),
-                                    ZERO_NIBBLE_POLICY, _stream(x))
+    st = lib.fpq_quantize_mx_packed_padded(x.data_ptr(), rows, cols, 0, kind, g, norm, pc.data_ptr(), ps.data_ptr(),
+                                           ZERO_NIBBLE_POLICY, _stream(x))
     if st == _engine.E_UNSUPPORTED:
         codes, scales, _ = fused_quantize_mx_op(x, hadamard_matrix, "abs_max", False)
         return pack_mxf4(codes, scales.view(torch.uint8), rows, cols)
@@ -116,8 +116,19 @@ def quantize_mx_packed(x: torch.Tensor, hadamard_matrix: torch.Tensor) -> Tuple[
     return pc, ps
 
 
+def padded_k(k: int) -> int:
+    """The K of packed operands: whole 256-K blocks (padded with zero codes and scale bytes)."""
+    return (k + 255) // 256 * 256
+
+
+def packable_k(k: int) -> bool:
+    """Whether operands with this K have a packed form.  A ragged K (3200, 2880) runs on the packed kernels too: the
+    row-major kernel that takes any K stages nothing through LDS (333 x 8640 x 3200: 40 us against 15)."""
+    return k >= 256 and k % 32 == 0
+
+
 def packed_linear_eligible(rows: int, k: int, forward_method: str) -> bool:
-    return forward_method == "abs_max" and rows >= PACKED_LINEAR_MIN_M and k % 256 == 0 and packed_weights_enabled()
+    return forward_method == "abs_max" and rows >= PACKED_LINEAR_MIN_M and packable_k(k) and packed_weights_enabled()
 
 
 @torch.library.custom_op("fp_quant::linear_alpha_op", mutates_args=())
@@ -166,7 +177,7 @@ def linear_mxf4_packed_op(
         wp, wsp = packed_weight(wq, ws_b)
         st = _engine.lib().fpq_gemm_mxf4_packed(
             xp.data_ptr(), xsp.data_ptr(), wp.data_ptr(), wsp.data_ptr(), a.data_ptr(), b_ptr,
-            y.data_ptr(), m, n, k, _stream(x))
+            y.data_ptr(), m, n, padded_k(k), _stream(x))
     _engine.check(st, "fpq_gemm_mxf4_packed")
     return y
 
@@ -321,12 +332,12 @@ def _pack_buffers(into, codes_bytes: int, scales_bytes: int, device) -> Tuple[to
 
 def pack_mxf4(codes: torch.Tensor, scales: torch.Tensor, rows: int, k: int, into=None) -> Tuple[torch.Tensor, torch.Tensor]:
     """Row-major codes [rows, k/2] and E8M0 scales [>=rows, >=k/32] -> the packed layout of
-    fpq_gemm_mxf4_packed (rows padded to a multiple of 32)."""
+    fpq_gemm_mxf4_packed (rows padded to a multiple of 32, k to one of 256)."""
     lib = _engine.lib()
     pc, ps = _pack_buffers(into, lib.fpq_packed_codes_bytes(rows, k), lib.fpq_packed_scales_bytes(rows, k), codes.device)
-    st = lib.fpq_pack_mxf4(codes.data_ptr(), scales.data_ptr(), scales.shape[1], rows, k,
-                           pc.data_ptr(), ps.data_ptr(), _stream(codes))
-    _engine.check(st, "fpq_pack_mxf4")
+    st = lib.fpq_pack_padded(0, codes.data_ptr(), scales.data_ptr(), scales.shape[1], rows, k,
+                             pc.data_ptr(), ps.data_ptr(), _stream(codes))
+    _engine.check(st, "fpq_pack_padded")
     return pc, ps
 
 
@@ -336,9 +347,9 @@ def pack_nvf4(codes: torch.Tensor, scales: torch.Tensor, rows: int, k: int, into
     lib = _engine.lib()
     pc, ps = _pack_buffers(into, lib.fpq_packed_codes_bytes(rows, k), lib.fpq_packed_scales_bytes_nv(rows, k),
                            codes.device)
-    st = lib.fpq_pack_nvf4(codes.data_ptr(), scales.data_ptr(), scales.shape[1], rows, k,
-                           pc.data_ptr(), ps.data_ptr(), _stream(codes))
-    _engine.check(st, "fpq_pack_nvf4")
+    st = lib.fpq_pack_padded(1, codes.data_ptr(), scales.data_ptr(), scales.shape[1], rows, k,
+                             pc.data_ptr(), ps.data_ptr(), _stream(codes))
+    _engine.check(st, "fpq_pack_padded")
     return pc, ps
 
 
@@ -346,7 +357,7 @@ def nv_packed_eligible(m: int, n: int, k: int, fused_linear: bool = False) -> bo
     """NVFP4: the packed kernels at every row count from the smallest they take (the weight-streaming kernel,
     the tile kernels, whose large tiles convert the operands of the next K step behind the matrix instructions
     of the current one and are 6-7 % faster than the row-major kernel: 4096 x 24576 x 4096 570 against 610 us)."""
-    return ((NV_PACKED_LINEAR_MIN_M if fused_linear else NV_PACKED_MIN_M) <= m and k % 256 == 0
+    return ((NV_PACKED_LINEAR_MIN_M if fused_linear else NV_PACKED_MIN_M) <= m and packable_k(k)
             and packed_weights_enabled())
 
 
@@ -357,10 +368,10 @@ def unpack_fp4(pc: torch.Tensor, ps: torch.Tensor, rows: int, k: int, nvfp4: boo
     group = 16 if nvfp4 else 32
     codes = torch.empty(rows, k // 2, dtype=torch.uint8, device=pc.device)
     scales = torch.empty(rows, k // group, dtype=torch.uint8, device=pc.device)
-    entry = lib.fpq_unpack_nvf4 if nvfp4 else lib.fpq_unpack_mxf4
     with on_device(pc.device):
-        st = entry(pc.data_ptr(), ps.data_ptr(), rows, k, codes.data_ptr(), scales.data_ptr(), k // group, _stream(pc))
-    _engine.check(st, "fpq_unpack_nvf4" if nvfp4 else "fpq_unpack_mxf4")
+        st = lib.fpq_unpack_padded(int(nvfp4), pc.data_ptr(), ps.data_ptr(), rows, k, codes.data_ptr(), scales.data_ptr(),
+                                   k // group, _stream(pc))
+    _engine.check(st, "fpq_unpack_padded")
     return codes, scales
 
 
@@ -470,6 +481,7 @@ def splitk_workspace(wq: torch.Tensor, n: int, k: int, create: bool, stream: Opt
     Either way the layer takes the same kernel and gives the same bits."""
     if not SPLIT_K:
         return None
+    k = padded_k(k)
     need = _splitk_need.get((n, k, nvfp4))
     if need is None:
         lib = _engine.lib()
@@ -529,13 +541,13 @@ def _gemm(entry: str, x, w, xs, ws, alpha, bias: Optional[torch.Tensor], group: 
         bias = bias.contiguous()
         b_ptr = bias.data_ptr()
     a = alpha.contiguous()
-    if entry == "fpq_gemm_mxf4" and (packed_only or (m >= PACKED_MIN_M and k % 256 == 0 and packed_weights_enabled())):
+    if entry == "fpq_gemm_mxf4" and (packed_only or (m >= PACKED_MIN_M and packable_k(k) and packed_weights_enabled())):
         with on_device(x.device):
             wp, wsp = packed_weight(wq, ws_b)
             xp, xsp = pack_mxf4(xq, xs_b, m, k)
             st = _engine.lib().fpq_gemm_mxf4_packed(
                 xp.data_ptr(), xsp.data_ptr(), wp.data_ptr(), wsp.data_ptr(), a.data_ptr(), b_ptr,
-                y.data_ptr(), m, n, k, _stream(x))
+                y.data_ptr(), m, n, padded_k(k), _stream(x))
         _engine.check(st, "fpq_gemm_mxf4_packed")
         return y
     if entry == "fpq_gemm_nvf4" and (packed_only or nv_packed_eligible(m, n, k)):
@@ -544,7 +556,7 @@ def _gemm(entry: str, x, w, xs, ws, alpha, bias: Optional[torch.Tensor], group: 
             xp, xsp = pack_nvf4(xq, xs_b, m, k)
             st = _engine.lib().fpq_gemm_nvf4_packed(
                 xp.data_ptr(), xsp.data_ptr(), wp.data_ptr(), wsp.data_ptr(), a.data_ptr(), b_ptr,
-                y.data_ptr(), m, n, k, _stream(x))
+                y.data_ptr(), m, n, padded_k(k), _stream(x))
         _engine.check(st, "fpq_gemm_nvf4_packed")
         return y
     with on_device(x.device):

@@ -173,7 +173,7 @@ class FPQuantLinear(nn.Module):
         qweight = getattr(self, "qweight", None)
         if (isinstance(qweight, torch.Tensor) and qweight.is_cuda and hip_ops.packed_weights_enabled()
                 and self.config.forward_dtype in (FPQuantDtype.MXFP4, FPQuantDtype.NVFP4)
-                and self.in_features % 256 == 0):
+                and hip_ops.packable_k(self.in_features)):
             hip_ops.splitk_workspace(qweight, self.out_features, self.in_features, True,
                                      nvfp4=self.config.forward_dtype == FPQuantDtype.NVFP4)
 

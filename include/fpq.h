@@ -152,7 +152,9 @@ int fpq_gemm_nvf4(const void* xq, const void* xs, int64_t xs_stride, const void*
 /*
  * Packed MXFP4 operands: the codes and scales of a [rows, K] operand re-tiled into the order the
  * 32x32x64 block-scaled matrix instruction consumes them, so that one operand of one instruction
- * is one contiguous kilobyte (K % 256 == 0; rows padded to a multiple of 32 with zero codes):
+ * is one contiguous kilobyte (rows padded to a multiple of 32 with zero codes; a K that is a multiple of 32
+ * but not of 256 padded to one with zero codes and scale bytes: below, K stands for the padded one, and the
+ * GEMMs are called with it; fpq_packed_*_bytes and the *_padded entries take the tensor's own):
  *   codes   block (rt, ks) = rows [32 rt, +32) x K [64 ks, +64) at byte (rt * K/64 + ks) * 1024;
  *           16 bytes at (32 kh + r) * 16 inside it = row 32 rt + r, K [64 ks + 32 kh, +32)
  *   scales  block (rt, kb) = the same rows x K [256 kb, +256) at byte (rt * K/256 + kb) * 256;
@@ -256,7 +258,8 @@ int fpq_rmsnorm_rows_quantize_nv_packed(const void* x, int64_t ld, const void* w
                                         void* packed_codes, void* packed_scales, int zero_policy, void* stream);
 /*
  * The same for any number of rows: one pass over x, whose rows stay in registers and LDS between the statistic and
- * the quantization.  cols % 256 == 0, cols <= 16384 (FPQ_E_LIMIT beyond); arguments, rotations and bits as above.
+ * the quantization.  cols <= 16384 (FPQ_E_LIMIT beyond), a multiple of 32 and of the rotation's size (padded to
+ * whole 256-K blocks); arguments, rotations and bits as above.
  */
 int fpq_rmsnorm_tile_quantize_mx_packed(const void* x, int64_t ld, const void* weight, int64_t rows,
                                         int64_t cols, float eps, int rot_kind, int g, float norm,
@@ -267,8 +270,8 @@ int fpq_rmsnorm_tile_quantize_nv_packed(const void* x, int64_t ld, const void* w
                                         const float* global_scale, float* inv_rms, void* normed,
                                         void* packed_codes, void* packed_scales, int zero_policy, void* stream);
 /*
- * The NVFP4 fused producers writing the packed operand layout of fpq_gemm_nvf4_packed (cols % 256 == 0, as for
- * fpq_quantize_nv_packed).  Arguments as fpq_rmsnorm_quantize_nv / fpq_silu_mul_quantize_nv.
+ * The NVFP4 fused producers writing the packed operand layout of fpq_gemm_nvf4_packed (cols % 256 == 0; SiLU*up of
+ * either format: a multiple of 32 and of the rotation's size, padded).  Arguments as fpq_rmsnorm_quantize_nv / fpq_silu_mul_quantize_nv.
  */
 int fpq_rmsnorm_quantize_nv_packed(const void* x, int64_t ld, const float* inv_rms, const void* weight,
                                    int64_t rows, int64_t cols, int rot_kind, int g, float norm,
@@ -413,6 +416,14 @@ int fpq_pack_nvf4(const void* codes, const void* scales, int64_t scale_stride, i
 /* The inverse of fpq_pack_nvf4 for the first `rows` rows (E4M3 scales, entry [row, k/16], scale_stride >= K/16). */
 int fpq_unpack_nvf4(const void* packed_codes, const void* packed_scales, int64_t rows, int64_t K,
                     void* codes, void* scales, int64_t scale_stride, void* stream);
+/*
+ * fpq_pack_mxf4 / fpq_pack_nvf4 and their inverses (nv: NVFP4) for a K that is any multiple of 32, padded to whole 256-K
+ * blocks of the packed layout with zero codes and scale bytes.
+ */
+int fpq_pack_padded(int nv, const void* codes, const void* scales, int64_t scale_stride, int64_t rows,
+                    int64_t K, void* packed_codes, void* packed_scales, void* stream);
+int fpq_unpack_padded(int nv, const void* packed_codes, const void* packed_scales, int64_t rows, int64_t K,
+                      void* codes, void* scales, int64_t scale_stride, void* stream);
 int fpq_gemm_nvf4_packed(const void* xq_packed, const void* xs_packed, const void* wq_packed,
                          const void* ws_packed, const float* alpha, const void* bias, void* y,
                          int64_t M, int64_t N, int64_t K, void* stream);
@@ -430,6 +441,18 @@ int fpq_gemm_nvf4_packed_residual(const void* xq_packed, const void* xs_packed, 
 int fpq_quantize_nv_packed(const void* x, int64_t rows, int64_t cols, int rot_kind, int g, float norm,
                            const float* global_scale, void* packed_codes, void* packed_scales,
                            int zero_policy, void* stream);
+/*
+ * fpq_quantize_mx_packed (quest != 0: fpq_quantize_mx_quest_packed) and fpq_quantize_nv_packed for any number of
+ * columns that the rotation divides (a multiple of 32), padded to whole 256-K blocks of the packed layout with zero
+ * codes and scale bytes.  Rotations the packed quantizers do not take return FPQ_E_UNSUPPORTED; with padding, so do
+ * sequency-ordered ones of 64 beyond 64 rows.
+ */
+int fpq_quantize_mx_packed_padded(const void* x, int64_t rows, int64_t cols, int quest, int rot_kind, int g,
+                                  float norm, void* packed_codes, void* packed_scales, int zero_policy,
+                                  void* stream);
+int fpq_quantize_nv_packed_padded(const void* x, int64_t rows, int64_t cols, int rot_kind, int g, float norm,
+                                  const float* global_scale, void* packed_codes, void* packed_scales,
+                                  int zero_policy, void* stream);
 
 /*
  * Measurement hook: `blocks` workgroups of four waves run `iters` x 16 FP4 32x32x64 block-scaled

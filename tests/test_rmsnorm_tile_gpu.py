@@ -6,16 +6,16 @@ import torch
 from oracle import fpq_oracle as O
 from tests import capi
 from tests.conftest import make_student_t
-from tests.test_packed_gpu import pack_by_definition, pack_nv_by_definition
+from tests.test_ragged_k_gpu import _padded_pack
 
 pytestmark = pytest.mark.gpu
 
 
 # one row tile and its neighbours, a last row tile with a part of a workgroup's four rows; one 256-column block, rows
-# that end inside a wave's last octet, and both sides of the 4096 and 8192 columns at which a lane holds more octets
+# that end inside a wave's last octet or inside a 256-K block, and both sides of the 4096 and 8192 columns at which a lane holds more octets
 @pytest.mark.parametrize("fmt,rot,g", [("mxfp4", "hadamard", 128), ("mxfp4", "hadamard", 32), ("mxfp4", "identity", 32),
                                        ("nvfp4", "hadamard", 16), ("nvfp4", "hadamard", 128)])
-@pytest.mark.parametrize("rows,cols", [(1, 256), (65, 768), (98, 4096), (35, 4352), (34, 8192), (5, 8448), (33, 16384)])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (65, 768), (98, 4096), (35, 4352), (34, 8192), (5, 8448), (33, 16384), (70, 384), (37, 896)])
 def test_rmsnorm_of_many_rows_in_one_pass_bit_exact(fmt, rot, g, rows, cols):
     x = make_student_t(rows, cols, seed=rows + g) * 2
     gen = torch.Generator().manual_seed(cols)
@@ -31,10 +31,9 @@ def test_rmsnorm_of_many_rows_in_one_pass_bit_exact(fmt, rot, g, rows, cols):
     gs = None if fmt == "mxfp4" else 777.0
     if fmt == "mxfp4":
         wc, ws, _ = O.quantize_mx(want_v, okind, g, norm)
-        want_c, want_s = pack_by_definition(wc, ws, cols)
     else:
         wc, ws, _ = O.quantize_nv(want_v, gs, okind, g, norm)
-        want_c, want_s = pack_nv_by_definition(wc, ws, cols)
+    want_c, want_s = _padded_pack(wc, ws, cols, fmt == "nvfp4")
     ld = cols + 64 if rows in (5, 33, 98) else None
     pc, ps, out, inv = capi.rmsnorm_rows_quantize_packed(x, w, g=g, rot=rot, ld=ld, global_scale=gs, entry="tile")
     assert torch.equal(inv, O.row_inv_rms(x, 1e-5))

@@ -5,7 +5,7 @@ import torch
 
 from oracle import fpq_oracle as O
 from tests import capi
-from tests.test_packed_gpu import pack_by_definition, pack_nv_by_definition
+from tests.test_ragged_k_gpu import _padded_pack
 
 pytestmark = pytest.mark.gpu
 
@@ -21,9 +21,10 @@ def test_every_gate_value():
     assert torch.equal(out.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
 
 
-# eight rows a wave, the last row tile with part of them; one 256-column block per row and several
+# eight rows a wave, the last row tile with part of them; one 256-column block per row, several, and
+# a part of one (20 rows: the generic kernel)
 @pytest.mark.parametrize("gs,g", [(None, 128), (None, 32), (777.0, 16), (777.0, 128)])
-@pytest.mark.parametrize("rows,cols", [(65, 256), (97, 768), (300, 2304)])
+@pytest.mark.parametrize("rows,cols", [(65, 256), (97, 768), (300, 2304), (70, 384), (20, 896)])
 def test_packed_codes_bit_exact(gs, g, rows, cols):
     gen = torch.Generator().manual_seed(rows + g)
     gate = (torch.randn(rows, cols, generator=gen) * 2).to(torch.bfloat16)
@@ -35,10 +36,9 @@ def test_packed_codes_bit_exact(gs, g, rows, cols):
     norm = float(O.hadamard_matrix(g)[0, 0])
     if gs is None:
         c, s, _ = O.quantize_mx(want_v, O.ROT_HADAMARD, g, norm)
-        want = pack_by_definition(c, s, cols)
     else:
         c, s, _ = O.quantize_nv(want_v, gs, O.ROT_HADAMARD, g, norm)
-        want = pack_nv_by_definition(c, s, cols)
+    want = _padded_pack(c, s, cols, gs is not None)
     pc, ps, out = capi.fused_quantize_packed("silu_mul", gate, up, g=g, ld_a=cols + 64, ld_b=2 * cols, global_scale=gs)
     assert torch.equal(out.view(torch.int16), want_v.view(torch.int16))
     assert torch.equal(pc, want[0]) and torch.equal(ps, want[1])
