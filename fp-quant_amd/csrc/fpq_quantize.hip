@@ -1064,7 +1064,8 @@ static int launch_stream_packed_sized(const void* x, int64_t rows, int64_t cols,
 // 16-bit table, an 8 KB wave tile that nothing overlapped) took 114.6 (145) us; 2048 rows 34.5 -> 28.2, 512 rows 13.1
 // -> 12.3, 128 rows 9.7 -> 6.5.  A first tile asked for only after the table copy cost 2 us at 512 rows.
 //
-// kProNone (also QUEST): inputs whose rows are no multiple of 256 columns, which the streaming kernel does not take.
+// kProNone (also QUEST): inputs whose rows are no multiple of 256 columns, which the streaming kernel does not take, and
+// NVFP4 inputs of few elements (dispatch_packed).
 constexpr uint32_t kSiluLdsFirst = 113u << 7;         // bf16 magnitude bits of 2^-14
 constexpr uint32_t kSiluLdsCount = 21u * 128u;        // magnitudes up to (not including) 2^7
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
@@ -1132,7 +1133,9 @@ __global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
   for (; tile < n_tiles; tile += step) {
     const uint32_t rg8 = tile / blocks_per_row, kb = tile - rg8 * blocks_per_row;
     uint4 gn[4], un[kUp];
-    load(min(tile + step, n_tiles - 1u), gn, un);
+    // (nothing is loaded past the last tile: with the index clamped to it, every wave asked for the same 4 KB in its
+    // last turn, and 2048 x 4096 took 21 us instead of 6)
+    if (tile + step < n_tiles) load(tile + step, gn, un);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint8_t* const at_lds = my + place(2u * i + l_row, l_oct >> 2, l_oct & 3u);
@@ -1169,7 +1172,8 @@ __global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
           if (row < rows && o < cpr) store16_nt((uint8_t*)(pro.out + (size_t)row * cpr + o), pv);
         }
       } else {
-        *(uint4*)at_lds = ga[i];
+        // (element by element: a copy of the struct keeps the array in scratch memory)
+        *(uint4*)at_lds = make_uint4(ga[i].x, ga[i].y, ga[i].z, ga[i].w);
       }
     }
     asm volatile("" ::: "memory");
@@ -1207,9 +1211,10 @@ __global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
     }
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ga[i] = gn[i];
-#pragma unroll
-    for (int i = 0; i < kUp; ++i) ua[i] = un[i];
+    for (int i = 0; i < 4; ++i) {
+      ga[i] = make_uint4(gn[i].x, gn[i].y, gn[i].z, gn[i].w);
+      if constexpr (kSilu) ua[i] = make_uint4(un[i].x, un[i].y, un[i].z, un[i].w);
+    }
   }
 }
 
@@ -1250,11 +1255,22 @@ static int dispatch_packed(const void* x, int64_t rows, int64_t cols, int rot_ki
   // streaming kernel, whose wave tile is 32 rows deep; it writes the same packed bytes.
   const bool few = rows <= kPackedFewRows;
   constexpr int64_t kGroupCols = FMT == kFmtMx ? 32 : 16;
+  // NVFP4 below 2^23 elements: the tile kernel, whose loads need no round trip through LDS before its scale table is
+  // built (us, Hadamard 16: 128 x 4096 3.8 -> 3.5, 512 x 4096 4.4 -> 3.8, 1024 x 4096 5.4 -> 4.6, 256 x 12288 5.0 -> 4.4,
+  // 512 x 12288 6.2 -> 5.7; 1024 x 12288 9.6 / 9.5, 2048 x 12288 13.3 / 16.6; MXFP4 +-5 % up to 2^22, slower beyond).
+  const bool tile = FMT == kFmtNv && rows * cols < (int64_t)1 << 23;
+  Prologue pro{};
+  pro.chunks_per_row = pro.ld_first = (uint32_t)(cols / 8);
 #define FPQ_LAUNCH_PACKED(GG, RR)                                                                                 \
   {                                                                                                               \
     if (few)                                                                                                      \
       return launch_lane8<GG, FMT, RR>(x, rows, cols, norm, gsp, codes, scales, rows, cols / kGroupCols,          \
                                        zero_policy, stream, nullptr, true);                                       \
+    if constexpr (FMT == kFmtNv && (RR != FPQ_ROT_GSR || GG <= 32)) {                                             \
+      if (tile)                                                                                                   \
+        return launch_tile<GG, RR, FMT, kProNone>(x, nullptr, rows, cols, norm, codes, scales, zero_policy,       \
+                                                  stream, pro, gsp);                                              \
+    }                                                                                                             \
     return launch_stream_packed_sized<GG, RR, FMT>(x, rows, cols, norm, codes, scales, zero_policy, stream, gsp); \
   }
   if (rot_kind == FPQ_ROT_IDENTITY) {
