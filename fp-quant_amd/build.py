@@ -1,4 +1,4 @@
-"""Builds libfpq_hip.so (the C-ABI HIP library) for gfx950 with hipcc, in-tree.
+"""Builds libfpq_hip.so (the C-ABI HIP library, gfx950, hipcc) and _fpq_host.so (host code, g++), in-tree.
 
 Usage: python fp-quant_amd/build.py [--force]
 """
@@ -10,6 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "fp_quant", "_lib")
 LIB = os.path.join(OUT_DIR, "libfpq_hip.so")
+HOST = os.path.join(OUT_DIR, "_fpq_host.so")   # the native host path of the eager layers (an extension module)
 SOURCES = ["fpq_capi.hip", "fpq_quantize.hip", "fpq_gemm.hip", "fpq_gemm_packed.hip", "fpq_gemm_stream.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
@@ -20,10 +21,25 @@ FLAGS = [
 ]
 
 
+def host_command():
+    """Host code only: g++ against the headers and libraries of the installed PyTorch."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    includes = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM=1", *(f for d in includes for f in ("-isystem", d)), os.path.join(CSRC, "fpq_host.cpp"), "-o", HOST,
+            "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+
+
 def build(force: bool = True, verbose: bool = True) -> str:
     os.makedirs(OUT_DIR, exist_ok=True)
     deps = [os.path.join(CSRC, f) for f in os.listdir(CSRC)] + [os.path.join(HERE, "..", "include", "fpq.h")]
-    if not force and os.path.exists(LIB) and all(os.path.getmtime(d) <= os.path.getmtime(LIB) for d in deps):
+    if not force and all(os.path.exists(out) and all(os.path.getmtime(d) <= os.path.getmtime(out) for d in deps)
+                         for out in (LIB, HOST)):
         return LIB
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     objs = []
@@ -35,9 +51,13 @@ def build(force: bool = True, verbose: bool = True) -> str:
         if verbose:
             print(" ".join(cmd), flush=True)
         procs.append((cmd, subprocess.Popen(cmd)))
+    host_cmd = host_command()
+    if verbose:
+        print(" ".join(host_cmd), flush=True)
+    procs.append((host_cmd, subprocess.Popen(host_cmd)))
     for cmd, p in procs:
         if p.wait() != 0:
-            raise RuntimeError("hipcc failed: " + " ".join(cmd))
+            raise RuntimeError("compiler failed: " + " ".join(cmd))
     link = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", LIB]
     if verbose:
         print(" ".join(link), flush=True)

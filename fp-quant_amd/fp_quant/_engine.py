@@ -91,6 +91,7 @@ def available() -> bool:
     """True if the HIP library is present and loads (says nothing about a GPU being there)."""
     try:
         lib()
+        host()
         return True
     except FPQEngineError:
         return False
@@ -117,6 +118,31 @@ def lib():
                 fn.restype = restype
             _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The extension module with the native host path of the eager layers (csrc/fpq_host.cpp)."""
+    global _host
+    if _host is None:
+        import importlib.util
+
+        import torch  # noqa: F401  (its libraries have to be there first)
+        path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "_fpq_host.so")
+        with _lock:
+            if _host is None:
+                if not os.path.exists(path):
+                    raise FPQEngineError(f"{path} is missing: build it with `python fp-quant_amd/build.py`")
+                try:
+                    spec = importlib.util.spec_from_file_location("fp_quant._lib._fpq_host", path)
+                    module = importlib.util.module_from_spec(spec)
+                    spec.loader.exec_module(module)
+                except ImportError as exc:
+                    raise FPQEngineError(f"cannot load {path}: {exc}") from exc
+                _host = module
+    return _host
 
 
 def check(status: int, what: str) -> None:

@@ -42,6 +42,10 @@ from .hip_ops import (
 )
 
 
+# the native host path (csrc/fpq_host.cpp); None where nothing is built, and every engine call raises
+_host = _engine.host() if _engine.available() else None
+
+
 def cached_on(t: torch.Tensor, slot: str, key, make, remember: bool = True, refresh: bool = False):
     """`make()` remembered on tensor `t` under attribute `slot` while `key` stays the same.
     `remember=False` uses what is remembered but stores nothing new: for callers that may be running
@@ -100,10 +104,17 @@ def as_f32_scalar(t: torch.Tensor, remember: bool = True, refresh: bool = False)
 SHARE_ACT_QUANT = os.environ.get("FPQ_SHARE_ACT_QUANT", "1") != "0"
 
 
-class QuantizedActivations:
+if _host is not None:
+    _ActivationFields = _host.Activations
+else:
+    class _ActivationFields:
+        __slots__ = ("m", "k", "nvfp4", "ref", "version", "key", "keep", "mx_packed", "row_major", "nv_packed")
+
+
+class QuantizedActivations(_ActivationFields):
     """Rotated and quantized activations of one [m, k] tensor, in whichever operand layouts have
     been asked for so far (row-major codes/scales, packed MXFP4, packed NVFP4)."""
-    __slots__ = ("m", "k", "nvfp4", "ref", "version", "key", "keep", "mx_packed", "row_major", "nv_packed")
+    __slots__ = ()
 
     def __init__(self, m: int, k: int, nvfp4: bool):
         self.m, self.k, self.nvfp4 = m, k, nvfp4
@@ -425,7 +436,7 @@ def linear_w4a4_op(x_flat: torch.Tensor, hadamard_matrix: torch.Tensor, wq: torc
 # are column slices of it.  The layers' own packed copies become views into the concatenated buffers, so
 # no 4-bit weight is held a further time.  MXFP4 and NVFP4 (one format per group).
 class WeightGroup:
-    __slots__ = ("key", "wp", "wsp", "bias", "n", "splits", "k", "nvfp4")
+    __slots__ = ("key", "wp", "wsp", "bias", "n", "splits", "k", "nvfp4", "plan", "plan_key")   # (the plan: module/host.py)
 
 
 def _member_key(wq: torch.Tensor, ws: torch.Tensor, bias: Optional[torch.Tensor]):
@@ -476,6 +487,7 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
     splits = [weight_rows(m[0], k) for m in members]
     n = sum(splits)
     group = WeightGroup()
+    group.plan = group.plan_key = None
     group.n, group.splits, group.k, group.nvfp4 = n, splits, k, nvfp4
     scales_bytes = lib.fpq_packed_scales_bytes_nv if nvfp4 else lib.fpq_packed_scales_bytes
     reuse = previous
@@ -516,6 +528,7 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
                 _engine.check(st, "fpq_pack_padded")
                 # the member's own packed copy: these views (same key as hip_ops.packed_weight uses)
                 wq._fpq_packed = ((wq.data_ptr(), _version(wq), ws.data_ptr(), _version(ws), tuple(wq.shape), nvfp4), pc, ps)
+                vars(wq).pop("_fpq_plan", None)   # (it would hold the copy that these views replace)
     group.key = tuple(_member_key(*m[:3]) for m in members)   # (packed-only members have just moved)
     group.bias = torch.cat([m[2] for m in members]).contiguous() if all(have_bias) else None
     try:
@@ -859,3 +872,10 @@ def silu_mul_quantize(gate: torch.Tensor, up: torch.Tensor, hadamard_matrix: tor
             return None
         return _fused_quantize("silu_mul", (gate.data_ptr(), ld_g, up.data_ptr(), ld_u), rows, cols, h, kind, norm,
                                act_global_scale, nvfp4, None, stream, dev, remember, allow_packed)
+
+
+if _host is not None:
+    from .hip_ops import NV_PACKED_MIN_M, PACKED_MIN_M, _stream_workspaces
+
+    _host.configure(_engine.library_path(), vars(_engine.lib()), _shared_activations, _stream_workspaces, globals(),
+                    QuantizedActivations, ZERO_NIBBLE_POLICY, PACKED_MIN_M, NV_PACKED_MIN_M)

@@ -34,7 +34,7 @@ def _version(t: torch.Tensor):
 
 
 _TENSOR_CACHES = ("_fpq_rotation", "_fpq_bf16", "_fpq_packed", "_fpq_group", "_fpq_alpha", "_fpq_f32", "_fpq_host",
-                  "_fpq_splitk")
+                  "_fpq_splitk", "_fpq_plan", "_fpq_qplan")
 
 
 def drop_tensor_caches(*tensors, keep=()) -> None:
@@ -92,6 +92,26 @@ def _require_cuda(*tensors: torch.Tensor) -> None:
 
 def _padded(rows: int, groups: int) -> Tuple[int, int]:
     return (rows + 127) // 128 * 128, (groups + 3) // 4 * 4
+
+
+def _direct(op, native_name: str):
+    """`op` (a custom operator) with plain eager calls answered by the native host path, which runs the operator's body
+    without the dispatch around it; every other call -- traced, under a mode, with gradients, keywords -- and every
+    one that it declines goes through the dispatcher as before."""
+    if not HAS_HIP_ENGINE:
+        return op
+    native = getattr(_engine.host(), native_name)
+
+    class Direct(type(op)):
+        def __call__(self, *args, **kwargs):
+            if not kwargs and not torch.compiler.is_compiling():
+                out = native(*args)
+                if out is not None:
+                    return out
+            return super().__call__(*args, **kwargs)
+
+    op.__class__ = Direct
+    return op
 
 
 ### Forward quantization
@@ -465,6 +485,20 @@ def _stream_workspace(device: torch.device, stream: int, need: int) -> torch.Ten
     return workspace
 
 
+def splitk_need(n: int, k: int, nvfp4: bool) -> int:
+    """Workspace bytes with which the packed GEMM of a layer [n, k] splits K at every row count at which it can."""
+    if not SPLIT_K:
+        return 0
+    k = padded_k(k)
+    need = _splitk_need.get((n, k, nvfp4))
+    if need is None:
+        lib = _engine.lib()
+        size = lib.fpq_gemm_nvf4_packed_workspace_bytes if nvfp4 else lib.fpq_gemm_mxf4_packed_workspace_bytes
+        rows = _SPLIT_K_PROBE_ROWS if nvfp4 else _SPLIT_K_PROBE_ROWS[:4]
+        need = _splitk_need[(n, k, nvfp4)] = max(int(size(m, n, k)) for m in rows)
+    return need
+
+
 def splitk_workspace(wq: torch.Tensor, n: int, k: int, create: bool, stream: Optional[int] = None,
                      nvfp4: bool = False) -> Optional[torch.Tensor]:
     """The workspace with which the packed GEMM of a layer [n, k] (either format) splits K across workgroups at
@@ -479,15 +513,7 @@ def splitk_workspace(wq: torch.Tensor, n: int, k: int, create: bool, stream: Opt
       same layer must not be replayed at the same time on different streams.
 
     Either way the layer takes the same kernel and gives the same bits."""
-    if not SPLIT_K:
-        return None
-    k = padded_k(k)
-    need = _splitk_need.get((n, k, nvfp4))
-    if need is None:
-        lib = _engine.lib()
-        size = lib.fpq_gemm_nvf4_packed_workspace_bytes if nvfp4 else lib.fpq_gemm_mxf4_packed_workspace_bytes
-        rows = _SPLIT_K_PROBE_ROWS if nvfp4 else _SPLIT_K_PROBE_ROWS[:4]
-        need = _splitk_need[(n, k, nvfp4)] = max(int(size(m, n, k)) for m in rows)
+    need = splitk_need(n, k, nvfp4)
     if need == 0:
         return None
     capturing = torch.cuda.is_current_stream_capturing()
@@ -632,3 +658,10 @@ def matmul_nvf4_bf16_tn_bias_op(
 @matmul_nvf4_bf16_tn_bias_op.register_fake
 def _(x, w, xs, ws, alpha, bias):
     return x.new_empty(*x.shape[:-1], weight_rows(w, x.shape[-1] * 2), dtype=torch.bfloat16)
+
+
+for _op, _name in ((fused_quantize_mx_op, "quantize_mx"), (fused_quantize_nv_op, "quantize_nv"),
+                   (matmul_mxf4_bf16_tn_op, "matmul_mx"), (matmul_ada_mxf4_bf16_tn_op, "matmul_mx"),
+                   (matmul_nvf4_bf16_tn_op, "matmul_nv"), (matmul_mxf4_bf16_tn_bias_op, "matmul_mx"),
+                   (matmul_nvf4_bf16_tn_bias_op, "matmul_nv")):
+    _direct(_op, _name)

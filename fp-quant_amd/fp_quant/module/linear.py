@@ -13,7 +13,7 @@ import torch
 from torch import nn
 
 from ..utils import FPQuantConfig, FPQuantDtype, validate_config
-from . import eager, hip_ops
+from . import eager, hip_ops, host
 from .linear_fns import FPQuant4x16NoMasterFn, forward_quantize
 
 def _sylvester_signs(n: int) -> torch.Tensor:
@@ -41,6 +41,8 @@ def get_gsr_matrix(group_size: int, dtype: torch.dtype, device: torch.device):
     order = torch.argsort(torch.diff(had, dim=0).ne(0).sum(dim=0))
     return had[:, order].contiguous()
 
+
+_native = host.native   # the native host path: None for every call that is not the plain eager one
 
 _TRANSFORMS = {"hadamard": get_hadamard_matrix, "identity": get_identity_matrix, "gsr": get_gsr_matrix}
 
@@ -264,13 +266,26 @@ class FPQuantLinear(nn.Module):
             and not cfg.store_master_weights
             and not cfg.pseudoquantization
         ):
+            residual = self._fpq_residual
+            if residual is not None and (residual.requires_grad or residual.shape[:-1] != x.shape[:-1]
+                                         or residual.shape[-1] != self.out_features):
+                residual = None    # (not taken: it stays set)
+            native = not torch.compiler.is_compiling() and _native
+            if native:
+                nvfp4 = cfg.forward_dtype == FPQuantDtype.NVFP4
+                y = native.linear(self, x, residual, nvfp4, cfg.forward_method)
+                if y is False and host.learnable():   # no current plan: made now
+                    host.learn_linear(self)
+                    y = native.linear(self, x, residual, nvfp4, cfg.forward_method)
+                if y is not None and y is not False:
+                    if residual is not None:
+                        self.__dict__["_fpq_residual"] = None
+                    return y
             # no autograd graph to build (inference): call the forward directly
             fn = (FPQuant4x16NoMasterFn.apply if (torch.is_grad_enabled() and x.requires_grad)
                   else _no_master_forward)
             extra = ()
-            residual = self._fpq_residual
-            if (residual is not None and fn is _no_master_forward and not residual.requires_grad
-                    and residual.shape[:-1] == x.shape[:-1] and residual.shape[-1] == self.out_features):
+            if residual is not None and fn is _no_master_forward:
                 self._fpq_residual = None
                 extra = (residual,)
             return fn(

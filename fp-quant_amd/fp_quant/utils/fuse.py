@@ -53,6 +53,28 @@ def _eager():
     return _eager_module
 
 
+_host_module = _native_module = None
+
+
+def _host():
+    """fp_quant.module.host, likewise."""
+    global _host_module
+    if _host_module is None:
+        from ..module import host
+
+        _host_module = host
+    return _host_module
+
+
+def _native():
+    """The native host path: each of its functions gives None (False: for want of a plan) for a call that is not the
+    plain eager one."""
+    global _native_module
+    if _native_module is None:
+        _native_module = _host().native
+    return _native_module
+
+
 def _is_real_quant_linear(layer) -> bool:
     from ..module import FPQuantLinear
 
@@ -167,6 +189,14 @@ def fuse_rmsnorm(norm: nn.Module, consumer) -> bool:
 
     def forward(self, hidden_states):
         layer = peer[0]
+        if not torch.compiler.is_compiling():
+            nvfp4 = layer.config.forward_dtype == FPQuantDtype.NVFP4
+            y = _native().rmsnorm(self, layer, hidden_states, nvfp4)
+            if y is False and _host().learnable():
+                _host().learn_quant(layer.forward_hadamard_matrix, layer.act_global_scale, nvfp4)
+                y = _native().rmsnorm(self, layer, hidden_states, nvfp4)
+            if y is not None and y is not False:
+                return y
         if _fusable_call(hidden_states) and self.weight.dtype == torch.bfloat16:
             y = _eager().rmsnorm_quantize(hidden_states, self.weight, self.variance_epsilon,
                                             layer.forward_hadamard_matrix, layer.act_global_scale,
@@ -205,6 +235,19 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
 
     def forward(self, x, residual=None):
         """`residual`: added to the result (a fused decoder block passes its skip connection)."""
+        pair = None
+        if not torch.compiler.is_compiling():
+            modules = self._modules
+            pair = _native_group(self._fpq_weight_group, (modules.get("gate_proj"), modules.get("up_proj")), x)
+            if pair is not None:
+                down = modules["down_proj"]
+                nvfp4 = down.config.forward_dtype == FPQuantDtype.NVFP4
+                y = _native().gated_down(down, *pair, residual, nvfp4)
+                if y is False and _host().learnable():
+                    _host().learn_linear(down)
+                    y = _native().gated_down(down, *pair, residual, nvfp4)
+                if y is not None and y is not False:
+                    return y
         if traceable and _traceable_call(x):
             # two operators: gate and up from one quantization of x; SiLU*up quantized as it is
             # formed and multiplied by down's weight
@@ -218,7 +261,8 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
         if not _fusable_call(x) or (residual is not None and not _fusable_call(residual)):
             y = unfused(x)
             return y if residual is None else residual + y
-        pair = _eager_group_linear(self, (self.gate_proj, self.up_proj), x) if traceable else None
+        if pair is None and traceable:
+            pair = _eager_group_linear(self, (self.gate_proj, self.up_proj), x)
         if pair is not None:
             gate, up = pair            # both from one GEMM
         else:
@@ -334,12 +378,13 @@ def fuse_residual_adds(block: nn.Module) -> bool:
             return unfused(hidden_states, *args, **kwargs)
         out_proj = self.self_attn.o_proj
         normed = self.input_layernorm(hidden_states)
-        out_proj._fpq_residual = hidden_states
+        state = vars(out_proj)   # (a plain attribute: what Module.__setattr__ does with one, without its searches)
+        state["_fpq_residual"] = hidden_states
         try:
             attn_out, _ = self.self_attn(hidden_states=normed, **{**defaults, **kwargs})
         finally:
-            pending = out_proj._fpq_residual
-            out_proj._fpq_residual = None
+            pending = state["_fpq_residual"]
+            state["_fpq_residual"] = None
         if pending is not None:   # o_proj did not take it
             attn_out = hidden_states + attn_out
         return self.mlp(self.post_attention_layernorm(attn_out), residual=attn_out)
@@ -364,6 +409,17 @@ class _ProjectionCalls(ast.NodeTransformer):
             self.seen.append(f.attr)
             return ast.copy_location(ast.Name(id="__fpq_" + f.attr[0], ctx=ast.Load()), node)
         return node
+
+
+def _native_group(group, layers, x: torch.Tensor):
+    """The outputs of `layers` on `x` through the native host path, or None."""
+    if group is None or None in layers:
+        return None
+    outs = _native().group(group.plan, layers, x)
+    if outs is False and _host().learnable():
+        _host().learn_group(group, layers)
+        outs = _native().group(group.plan, layers, x)
+    return outs or None
 
 
 def _eager_group_linear(owner: nn.Module, layers, x: torch.Tensor):
@@ -394,6 +450,12 @@ def _qkv(attn, hidden_states):
     (which cannot see that the three layers quantize the same tensor); from one GEMM on the layers'
     concatenated packed weights in eager calls that have them; else three ordinary calls (which
     share the quantization by themselves)."""
+    if not torch.compiler.is_compiling() and attn._fpq_qkv_alike:
+        modules = attn._modules
+        outs = _native_group(attn._fpq_weight_group, (modules.get("q_proj"), modules.get("k_proj"), modules.get("v_proj")),
+                             hidden_states)
+        if outs is not None:
+            return outs
     layers = (attn.q_proj, attn.k_proj, attn.v_proj)
     if attn._fpq_qkv_alike and _traceable_call(hidden_states):
         return _group_linear(layers, hidden_states, attn._fpq_weight_group)

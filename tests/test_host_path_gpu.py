@@ -1,0 +1,281 @@
+"""The native host path (csrc/fpq_host.cpp) gives the Python path's bits on every form of call that it accepts, declines
+the others, and notices every change of what its plans were made from."""
+import copy
+import io
+import threading
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    import fp_quant
+    from fp_quant.module import eager, hip_ops, host
+    from fp_quant.module import linear as linear_module
+
+
+class _Declines:
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+class _Counts:
+    def __init__(self):
+        self.answered = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            out = getattr(host.native, name)(*args)
+            if out is not None and out is not False:
+                self.answered.append(name)
+            return out
+        return call
+
+
+@pytest.fixture
+def native(monkeypatch):
+    counts = _Counts()
+    monkeypatch.setattr(linear_module, "_native", counts)
+    return counts
+
+
+def _python(layer, x, residual=None):
+    """The layer's result through the Python path, without a shared quantization."""
+    saved, linear_module._native = linear_module._native, _Declines()
+    share, eager.SHARE_ACT_QUANT = eager.SHARE_ACT_QUANT, False
+    try:
+        layer.__dict__["_fpq_residual"] = residual
+        return layer(x)
+    finally:
+        linear_module._native, eager.SHARE_ACT_QUANT = saved, share
+
+
+def _layer(fmt="mxfp4", method="abs_max", init="hadamard", g=128, k=512, n=288, bias=False, seed=0):
+    dtype = fp_quant.FPQuantDtype.MXFP4 if fmt == "mxfp4" else fp_quant.FPQuantDtype.NVFP4
+    cfg = fp_quant.FPQuantConfig(forward_dtype=dtype, forward_method=method, backward_dtype=fp_quant.FPQuantDtype.BF16,
+                                 hadamard_group_size=g, transform_init=init)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    layer = fp_quant.FPQuantLinear(k, n, cfg, bias=bias, device="cuda", dtype=torch.bfloat16)
+    layer.weight.data = torch.randn(n, k, generator=gen, device="cuda", dtype=torch.bfloat16)
+    if bias:
+        layer.bias.data = torch.randn(n, generator=gen, device="cuda", dtype=torch.bfloat16)
+    layer.pre_forward()
+    return layer
+
+
+FORMS = [("mxfp4", "abs_max", "hadamard", 128), ("mxfp4", "quest", "hadamard", 32), ("mxfp4", "abs_max", "identity", 64),
+         ("mxfp4", "abs_max", "gsr", 128), ("mxfp4", "quest", "gsr", 128), ("mxfp4", "abs_max", "general", 64),
+         ("nvfp4", "abs_max", "hadamard", 16), ("nvfp4", "abs_max", "gsr", 128), ("nvfp4", "abs_max", "general", 32)]
+
+
+@pytest.mark.parametrize("fmt,method,init,g", FORMS)
+@pytest.mark.parametrize("k", [512, 640])
+def test_linear_forms(fmt, method, init, g, k, native):
+    general = init == "general"
+    layer = _layer(fmt, method, "hadamard" if general else init, g, k, bias=True)
+    if general:
+        q, _ = torch.linalg.qr(torch.randn(g, g, generator=torch.Generator().manual_seed(1)))
+        layer.forward_hadamard_matrix = torch.nn.Buffer(q.to(torch.bfloat16).contiguous().cuda())
+    shapes = [(1, k), (33, k), (2, 3, k), (1, 1, 5, k), (130, k)]
+    with torch.no_grad():
+        layer(torch.randn(2, k, device="cuda", dtype=torch.bfloat16))   # the plans are made here
+        for i, shape in enumerate(shapes):
+            x = torch.randn(shape, device="cuda", dtype=torch.bfloat16)
+            res = torch.randn(*shape[:-1], 288, device="cuda", dtype=torch.bfloat16)
+            native.answered.clear()
+            got = layer(x)
+            assert native.answered == ["linear"] and layer._fpq_residual is None
+            assert torch.equal(got, _python(layer, x)) and torch.equal(layer(x), got)   # (the second: shared)
+            layer._fpq_residual = res
+            assert torch.equal(layer(x), _python(layer, x, res)) and layer._fpq_residual is None
+
+
+def test_declined_calls(native, monkeypatch):
+    layer = _layer(bias=True)
+    x = torch.randn(6, 512, device="cuda", dtype=torch.bfloat16)
+    layer(x)
+    strided = torch.randn(512, 6, device="cuda", dtype=torch.bfloat16).t()
+    for call in (x.float(), strided):
+        native.answered.clear()
+        assert torch.equal(layer(call), _python(layer, call)) and not native.answered
+    native.answered.clear()
+    xg = x.clone().requires_grad_()
+    assert layer(xg).requires_grad and not native.answered
+    with pytest.raises(Exception):
+        layer(x[:, :256].contiguous())
+    assert layer(x[:0]).shape == (0, 288)
+    with torch.inference_mode():
+        xi = x * 1.0
+        assert torch.equal(layer(xi), _python(layer, x)) and native.answered == ["linear"]
+        assert not eager._shared_activations or eager._shared_activations[0].ref() is not xi
+    native.answered.clear()
+    monkeypatch.setenv("FPQ_PACKED_WEIGHTS", "0")
+    assert torch.equal(layer(x), _python(layer, x)) and not native.answered
+
+
+def test_plans_notice_changes(native):
+    layer = _layer("nvfp4", g=16, k=512)
+    x = torch.randn(40, 512, device="cuda", dtype=torch.bfloat16)
+    layer(x), layer(x)
+    other = _layer("nvfp4", g=16, k=512, seed=3)
+
+    def check():
+        want = _python(layer, x)
+        for _ in range(3):
+            assert torch.equal(layer(x), want)
+        assert native.answered and native.answered[-1] == "linear"
+        native.answered.clear()
+
+    check()
+    with torch.no_grad():
+        layer.qweight.copy_(other.qweight)
+        check()
+        layer.scales.data = other.scales.data.clone()
+        check()
+        layer.act_global_scale.fill_(5.0)
+        check()
+        layer.weight_global_scale.fill_(20.0)
+        check()
+        layer.forward_hadamard_matrix.copy_(torch.eye(16))
+        check()
+        layer.bias = torch.nn.Parameter(torch.randn(288, device="cuda", dtype=torch.bfloat16))
+        check()
+        x.mul_(-2.0)
+        check()
+        layer.load_state_dict({**layer.state_dict(), "qweight": other.qweight.flip(0).contiguous()})
+        check()
+    assert layer.release_row_major()
+    check()
+    layer.restore_row_major()
+    check()
+    twin = copy.deepcopy(layer)
+    assert torch.equal(twin(x), layer(x)) and torch.equal(twin(x), layer(x))
+    buf = io.BytesIO()
+    torch.save(layer, buf)
+    buf.seek(0)
+    loaded = torch.load(buf, weights_only=False)   # (written above)
+    assert torch.equal(loaded(x), layer(x))
+
+
+@pytest.mark.parametrize("fmt,g", [("mxfp4", 64), ("nvfp4", 16)])
+def test_streams_and_threads(fmt, g, native):
+    """One layer that splits K (a workspace per stream) called from threads with a stream each."""
+    layer = _layer(fmt, g=g, k=14336, n=512)
+    xs = [torch.randn(8, 14336, device="cuda", dtype=torch.bfloat16) for _ in range(4)]
+    want = [_python(layer, x) for x in xs]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream), torch.no_grad():
+            for _ in range(20):
+                if not torch.equal(layer(xs[i]), want[i]):
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad and "linear" in native.answered
+
+
+def test_source_of_a_shared_quantization_dies(native):
+    layer = _layer()
+    x = torch.randn(6, 512, device="cuda", dtype=torch.bfloat16)
+    layer(x)
+    y = torch.randn(6, 512, device="cuda", dtype=torch.bfloat16)
+    native.answered.clear()
+    layer(y)
+    assert native.answered == ["linear"] and eager._shared_activations[0].ref() is y
+    del y
+    assert 0 not in eager._shared_activations
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [("mxfp4", 1, 72, 512), ("mxfp4", 47, 264, 288), ("mxfp4", 48, 264, 288),
+                                       ("mxfp4", 200, 256, 512), ("nvfp4", 1, 72, 512), ("nvfp4", 64, 264, 288),
+                                       ("nvfp4", 65, 264, 288), ("nvfp4", 200, 256, 512)])
+def test_operators(fmt, m, n, k):
+    """Operators called plainly and through the dispatcher (torch.ops): the same tensors."""
+    mx = fmt == "mxfp4"
+    w = torch.randn(n, k, device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
+    gs = torch.full((1,), 3.0, device="cuda")
+    alpha = torch.full((1,), 0.3, device="cuda")
+    bias = torch.randn(n, device="cuda", dtype=torch.bfloat16)
+    ops = torch.ops.fp_quant
+    h = linear_module.get_hadamard_matrix(32, torch.bfloat16, torch.device("cuda"))
+
+    def same(a, b):
+        assert len(a) == len(b)
+        for p, q in zip(a, b):
+            assert (p is None and q is None) or (p.dtype == q.dtype and p.shape == q.shape
+                                                 and torch.equal(p.view(torch.uint8), q.view(torch.uint8)))
+
+    name = "mxf4" if mx else "nvf4"
+    for _ in range(2):   # (the first call classifies the rotation and packs the weight)
+        if mx:
+            for method in ("abs_max", "quest"):
+                same(hip_ops.fused_quantize_mx_op(x, h, method, False), ops.fused_quantize_mx_op(x, h, method, False))
+            (qx, sx, _), (qw, sw, _) = (ops.fused_quantize_mx_op(t, h, "abs_max", False) for t in (x, w))
+        else:
+            same(hip_ops.fused_quantize_nv_op(x, h, gs), ops.fused_quantize_nv_op(x, h, gs))
+            x3 = x.view(1, m, k)
+            same(hip_ops.fused_quantize_nv_op(x3, h, gs), ops.fused_quantize_nv_op(x3, h, gs))
+            (qx, sx), (qw, sw) = (ops.fused_quantize_nv_op(t, h, gs) for t in (x, w))
+    for _ in range(2):
+        same([getattr(hip_ops, f"matmul_{name}_bf16_tn_op")(qx, qw, sx, sw, alpha)],
+             [getattr(ops, f"matmul_{name}_bf16_tn_op")(qx, qw, sx, sw, alpha)])
+        same([getattr(hip_ops, f"matmul_{name}_bf16_tn_bias_op")(qx[None], qw, sx, sw, alpha, bias)],
+             [getattr(ops, f"matmul_{name}_bf16_tn_bias_op")(qx[None], qw, sx, sw, alpha, bias)])
+    with pytest.raises(ValueError):
+        getattr(hip_ops, f"matmul_{name}_bf16_tn_op")(qx, qw[:, : k // 4], sx, sw, alpha)
+    with pytest.raises(ValueError):
+        (hip_ops.fused_quantize_mx_op(x.float(), h, "abs_max", False) if mx else
+         hip_ops.fused_quantize_nv_op(x.float(), h, gs))
+
+
+def test_fused_block_after_a_weight_changes():
+    """The grouped projections of a fused block: a member that is written to, and a rotation that is replaced."""
+    from perf.cases import Block
+    from fp_quant.utils import fuse_producers
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    case = dict(fmt="mxfp4", g=64, hidden=512, kv=256, inter=768)
+    block = Block(case, gen)
+    assert fuse_producers(block)
+    x = torch.randn(1, 5, 512, device="cuda", dtype=torch.bfloat16)
+
+    def run(native_path):
+        saved = fuse._native_module, linear_module._native
+        if not native_path:
+            fuse._native_module = linear_module._native = _Declines()
+            eager._shared_activations.clear()
+        try:
+            cache = []
+            return [block(x, cache=cache), *cache[0]]
+        finally:
+            fuse._native_module, linear_module._native = saved
+
+    import fp_quant.utils.fuse as fuse
+
+    def check():
+        for _ in range(2):
+            got = run(True)
+        for a, b in zip(got, run(False)):
+            assert torch.equal(a, b)
+
+    with torch.no_grad():
+        check()
+        block.self_attn.v_proj.qweight.bitwise_xor_(7)
+        check()
+        block.mlp.up_proj.scales.add_(1)
+        check()
+        block.mlp.down_proj.qweight.bitwise_xor_(3)
+        check()
+        for layer in (block.self_attn.q_proj, block.self_attn.k_proj, block.self_attn.v_proj):
+            layer.forward_hadamard_matrix.copy_(linear_module.get_identity_matrix(64, torch.bfloat16, x.device))
+        check()
+        block.self_attn.q_proj.weight_global_scale.mul_(2)
+        check()
+        block.input_layernorm.weight.mul_(0.5)
+        check()
