@@ -56,7 +56,7 @@ int device_cus() {
   return cus;
 }
 
-int ensure_silu_table(hipStream_t stream);   // fpq_quantize.hip
+int silu_table_address(hipStream_t stream, const uint16_t** out);   // fpq_quantize.hip; fills the table
 int scratch_address(void** out);             // fpq_gemm_stream.hip
 }  // namespace fpq
 
@@ -67,7 +67,8 @@ extern "C" int fpq_prepare_device(void* stream) {
   const hipError_t err = hipStreamIsCapturing((hipStream_t)stream, &cap);
   if (err != hipSuccess) return (int)err;
   if (cap != hipStreamCaptureStatusNone) return FPQ_E_UNSUPPORTED;   // it has to run, not be recorded
-  if (const int st = fpq::ensure_silu_table((hipStream_t)stream)) return st;
+  const uint16_t* table = nullptr;
+  if (const int st = fpq::silu_table_address((hipStream_t)stream, &table)) return st;
   void* scratch = nullptr;
   return fpq::scratch_address(&scratch);
 }

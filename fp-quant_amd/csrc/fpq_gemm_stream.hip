@@ -28,6 +28,7 @@
 #include "../../include/fpq.h"
 #include "fpq_device.h"
 #include "fpq_gemm_epilogue.h"
+#include "fpq_quantize_chunk.h"
 
 namespace fpq {
 
@@ -49,12 +50,32 @@ constexpr int stream_dynamic_lds(int nt, int mt) {
 // NV: NVFP4 operands (two E4M3 scale bytes per lane and K step, 512-byte scale blocks): a lane's dword s
 // of a 64-K unit, times its group's scale, is its fp16 operand of the s-th 32x32x16 matrix instruction
 // of the unit on both sides, so the K order is permuted consistently and the sum is complete.
-template <int NT, int MT, int DB, int NW, bool NV = false>
+//
+// IN = FewRows: the activations come as bf16 rows (few of them) and every wave rotates and quantizes the 256-K blocks it
+// multiplies, while its weights are on their way.  See few_rows_plan.
+struct Packed {};
+struct FewRows {
+  const uint4* x;            // bf16 [M, xk]; SiLU*up: gate
+  const uint4* up;           // SiLU*up: the multiplier
+  const uint16_t* silu;      // ... and the table of bf16(silu(g))
+  const float* gs;           // NVFP4: the activations' global scale
+  uint8_t *codes, *scales;   // optional: the quantized rows, in the packed layout (rows past M are not written)
+  float norm;
+  int xk;                    // a multiple of 32 and of the rotation's size; K is padded to whole blocks
+};
+// 32-element chunks a wave quantizes at most: one per lane and pass
+constexpr int few_rows_passes(bool silu) { return silu ? 1 : 2; }
+constexpr int few_rows_chunks(bool silu) { return 64 * few_rows_passes(silu); }
+
+template <int NT, int MT, int DB, int NW, bool NV = false, class IN = Packed, int XG = 32, int XROT = FPQ_ROT_IDENTITY,
+          bool XSILU = false>
 __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm_fp4_stream_kernel(
     const uint8_t* __restrict__ xq_all, const uint8_t* __restrict__ xs_all, const uint8_t* __restrict__ wq,
     const uint8_t* __restrict__ ws, const float* __restrict__ alpha_p, const uint16_t* __restrict__ bias,
     const uint16_t* residual_all, uint16_t* y, int M_all, int N, int K, int bps, int ksplit,
-    float* partial, unsigned* counters, const OutSegments seg) {
+    float* partial, unsigned* counters, const OutSegments seg, const IN in) {
+  constexpr bool kFew = std::is_same_v<IN, FewRows>;
+  static_assert(!kFew || (NT == 1 && MT == 1), "few rows: one tile");
   static_assert(NW == 4, "a wave owns a quarter of every tile");
   // More than 32 MT activation rows: blockIdx.z numbers slabs of 32 MT rows, each a product of its own
   // (the last may have fewer rows, even fewer row tiles).
@@ -104,6 +125,7 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   const uint8_t* xscale[MT];
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
+    if constexpr (kFew) break;
     const int l = (lane & 31) < M - 32 * j ? lane : (lane & 32);
     const int jt = min(j, (M - 1) >> 5);
     xcode[j] = xq + (size_t)jt * nu * 1024 + l * 16;
@@ -139,6 +161,7 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
     }
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
+      if constexpr (kFew) break;
 #pragma unroll
       for (int u = 0; u < 4; ++u) b[s][u][j] = *(const uint4*)(xcode[j] + (size_t)(kb * 4 + u) * 1024);
       if constexpr (NV) sb[s][j] = *(const uint2*)(xscale[j] + (size_t)kb * kSB);
@@ -251,7 +274,20 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
       }
     }
   };
-  auto run_block = [&](auto slot) __attribute__((always_inline)) {
+  // Few rows: the wave's quantized chunks, 16 bytes of codes each, and their scale bytes in the order the matrix
+  // instruction takes them: [block][K half][K step].  Lanes past the last row read row 0's, as above.
+  __shared__ __attribute__((aligned(16))) uint8_t few_codes[kFew ? 4 : 1][kFew ? few_rows_chunks(XSILU) * 16 : 16];
+  __shared__ __attribute__((aligned(16))) uint8_t few_scales[kFew ? 4 : 1][kFew ? few_rows_chunks(XSILU) * (NV ? 2 : 1) : 16];
+  const int few_row = (lane & 31) < M ? (lane & 31) * nblk : 0;   // first block of the lane's row
+  auto run_block = [&](auto slot, int t) __attribute__((always_inline)) {
+    if constexpr (kFew) {
+      constexpr int s = decltype(slot)::value;
+      const int blk = few_row + t, kh = lane >> 5;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) b[s][u][0] = *(const uint4*)&few_codes[wave][(blk * 8 + 2 * u + kh) * 16];
+      if constexpr (NV) sb[s][0] = *(const uint2*)&few_scales[wave][blk * 16 + kh * 8];
+      else sb[s][0].x = *(const uint32_t*)&few_scales[wave][blk * 8 + kh * 4];
+    }
     if constexpr (kPipelined) compute_block_nv(slot);
     else compute_block(slot);
   };
@@ -271,10 +307,107 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // more).  With three or four activation row tiles the effect is within +-4 % either way; only four tiles
   // of NVFP4 gain throughout (128 rows, N = 4096: 15.1 -> 14.6 us).  One block in flight has nothing to order.
   constexpr bool kOrdered = NT == 1 && DB >= 2 && (MT <= 2 || (NV && MT == 4));
+  // Few rows: the wave's chunks in lane order, row by row (the eight chunks of a block are neighbours, so the lanes of
+  // a rotation block are); asked for before the weights, since loads complete in order.
+  constexpr int kFewPasses = kFew ? few_rows_passes(XSILU) : 1;
+  const int few_chunks = kFew ? M * nblk * 8 : 0;
+  uint4 xr[kFewPasses][4], ur[XSILU ? kFewPasses : 1][4];
+  int few_col[kFewPasses], few_at[kFewPasses];
+  if constexpr (kFew) {
+#pragma unroll
+    for (int p = 0; p < kFewPasses; ++p) {
+      const int ci = min(p * 64 + lane, max(few_chunks - 1, 0)), blk = ci >> 3, row = nblk > 0 ? blk / nblk : 0;
+      const int kb = nblk > 0 ? first + NW * (blk - row * nblk) : 0;
+      few_col[p] = kb * 256 + (ci & 7) * 32;
+      few_at[p] = row * 0x10000 + kb;
+      // (a chunk in the padding of the last block reads the row's start and is replaced by zeros)
+      const size_t at = ((size_t)row * in.xk + (few_col[p] < in.xk ? few_col[p] : 0)) >> 3;
+      if (p == 0 || few_chunks > 64) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          xr[p][i] = in.x[at + i];
+          if constexpr (XSILU) ur[p][i] = in.up[at + i];
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   for_slots([&](auto slot) {
     load_block(slot, decltype(slot)::value);
-    if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kOrdered || kFew) __builtin_amdgcn_sched_barrier(0);
   });
+  if constexpr (kFew) {
+    constexpr int FMT = NV ? kFmtNv : kFmtMx;
+    __shared__ float2 lut[NV ? 128 : 1];
+    float gs = 1.0f, rg = 1.0f;
+    bool nv_fast = true;
+    if constexpr (NV) {
+      gs = *in.gs;
+      rg = gs == 0.0f ? 0.0f : 1.0f / gs;
+      nv_fast = nv_global_scale_fast(gs);
+      if (threadIdx.x < 128) lut[threadIdx.x] = nv_division(threadIdx.x, rg, nv_fast);
+      __syncthreads();
+    }
+#pragma unroll
+    for (int p = 0; p < kFewPasses; ++p) {
+      if (p * 64 < few_chunks) {   // (wave-uniform)
+        auto load_rotate = [&](float (&v)[32]) __attribute__((always_inline)) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float e[8];
+            unpack8(xr[p][i], e);
+            if constexpr (XSILU) {
+              float q[8];
+              unpack8(ur[p][i], q);
+              const uint32_t w[4] = {xr[p][i].x, xr[p][i].y, xr[p][i].z, xr[p][i].w};
+#pragma unroll
+              for (int k = 0; k < 8; ++k) {
+                const uint32_t bits = (k & 1) ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu;
+                e[k] = __uint_as_float((uint32_t)in.silu[bits] << 16);
+              }
+#pragma unroll
+              for (int k = 0; k < 8; k += 2) {
+                const uint32_t pr = pack_bf16x2(e[k] * q[k], e[k + 1] * q[k + 1]);
+                e[k] = bf16_lo(pr);
+                e[k + 1] = bf16_hi(pr);
+              }
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[8 * i + k] = e[k];
+          }
+          rotate_chunk<32, XG, XROT, false>(v, in.norm, lane);
+        };
+        float v[32];
+        load_rotate(v);
+        uint32_t cw[4], sbytes = 0u, sb_lo = 0u;
+        const bool need_slow = quantize_chunk<32, FMT, kZeroReference, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+        if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
+          float u[32];
+          load_rotate(u);
+          quantize_chunk_slow<32, FMT, kZeroReference>(u, gs, rg, cw, sbytes);
+        }
+        if (few_col[p] >= in.xk) {
+          cw[0] = cw[1] = cw[2] = cw[3] = 0u;
+          sbytes = 0u;
+        }
+        const int ci = p * 64 + lane, g8 = ci & 7;
+        if (ci < few_chunks) {
+          const uint4 c4 = make_uint4(cw[0], cw[1], cw[2], cw[3]);
+          *(uint4*)&few_codes[wave][ci * 16] = c4;
+          const int sc = (ci & ~7) + (g8 & 1) * 4 + (g8 >> 1);
+          if constexpr (NV) *(uint16_t*)&few_scales[wave][sc * 2] = (uint16_t)sbytes;
+          else few_scales[wave][sc] = (uint8_t)sbytes;
+          if (in.codes && blockIdx.x == 0) {   // the first weight tile's workgroups hand the rows on
+            const int row = few_at[p] >> 16, kb = few_at[p] & 0xffff, slot = (g8 & 1) * 32 + row;
+            *(uint4*)(in.codes + ((size_t)(kb * 4 + (g8 >> 1)) * 64 + slot) * 16) = c4;
+            if constexpr (NV) *(uint16_t*)(in.scales + (size_t)kb * 512 + slot * 8 + 2 * (g8 >> 1)) = (uint16_t)sbytes;
+            else in.scales[(size_t)kb * 256 + slot * 4 + (g8 >> 1)] = (uint8_t)sbytes;
+          }
+        }
+      }
+    }
+    asm volatile("" ::: "memory");   // (a wave's LDS accesses complete in order: its chunks are there when it reads them)
+  }
   // Where the epilogue will store, worked out while the first loads are in flight (after the reduction
   // every instruction delays the workgroup's end).  The epilogue's lane layout: 8 consecutive columns
   // (16 bytes) of row lane / 4 and of that row + 16.  16-byte accesses need the whole tile inside N and
@@ -300,20 +433,20 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   int t0 = 0;
   for (; t0 + 2 * DB <= nblk; t0 += DB) {   // steady state: the block DB ahead exists
     for_slots([&](auto slot) {
-      run_block(slot);
+      run_block(slot, t0 + decltype(slot)::value);
       if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
       load_block(slot, t0 + DB + decltype(slot)::value);
       if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
     });
   }
   for_slots([&](auto slot) {                // the ring's last full or partial content
-    if (t0 + decltype(slot)::value < nblk) run_block(slot);
+    if (t0 + decltype(slot)::value < nblk) run_block(slot, t0 + decltype(slot)::value);
     if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
   });
   if (nblk - t0 > DB) {                     // up to DB - 1 blocks more
     for_slots([&](auto slot) { load_block(slot, t0 + DB + decltype(slot)::value); });
     for_slots([&](auto slot) {
-      if (t0 + DB + decltype(slot)::value < nblk) run_block(slot);
+      if (t0 + DB + decltype(slot)::value < nblk) run_block(slot, t0 + DB + decltype(slot)::value);
     });
   }
 
@@ -543,7 +676,7 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
   hipLaunchKernelGGL((gemm_fp4_stream_kernel<NTT, MTT, DBB, 4, NV>), grid, dim3(256), 0, stream,        \
                      (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws, alpha, \
                      (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N,    \
-                     (int)K, plan.bps, plan.ksplit, partial, counters, seg)
+                     (int)K, plan.bps, plan.ksplit, partial, counters, seg, Packed{})
   const int mt = (int)((rows + 31) / 32);
 #define FPQ_STREAM_BIG(NTT, MTT, DBB)                                                                   \
   {                                                                                                     \
@@ -553,7 +686,7 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
     hipLaunchKernelGGL((gemm_fp4_stream_kernel<NTT, MTT, DBB, 4, NV>), grid, dim3(256), kLds, stream,   \
                        (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws, alpha, \
                        (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N,  \
-                       (int)K, plan.bps, plan.ksplit, partial, counters, seg);                          \
+                       (int)K, plan.bps, plan.ksplit, partial, counters, seg, Packed{});                          \
     return (int)hipGetLastError();                                                                      \
   }
   if constexpr (NV) {
@@ -602,6 +735,80 @@ int gemm_fp4_stream_slabs(bool nv, const void* xq, const void* xs, const void* w
             : launch_stream<false>(xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, nullptr, 0, seg, stream, slab_rows);
 }
 
+
+// Few activation rows quantized by the GEMM itself.  A layer of one token is two kernels of about 4 us each, of which
+// most is the start and the end of a kernel, and two launches of 3.3 us host time; here every workgroup repeats the
+// quantization of the blocks it multiplies (each wave its own, no exchange between them) behind the loads of its
+// weights, in the same arithmetic and with the same order of sums: the same bits as the two kernels.
+//
+// The vector work grows with rows x K and is repeated per weight tile, so it is taken for one or two passes of a
+// wave's lanes over its 32-element chunks (rows x 256-K blocks of a wave <= 8 or 16) and, since it does not hide
+// behind the loads once the workgroups fill the CUs over and over, up to a number of weight tiles.  Measured (us, two
+// kernels / one; graph replays, weights in the last-level cache):
+//   MXFP4 1 row:  4096 x 4096 7.1 / 4.8, N = 14336 10.2 / 6.3, N = 28672 14.8 / 12.2, N = 128256 44.4 / 42.1;
+//                 K = 14336, N = 4096 11.6 / 9.2; 8192 x 8192 10.7 / 6.8
+//   MXFP4 4 rows (two passes):  4096 x 4096 7.2 / 5.7, N = 14336 10.2 / 8.1, N = 28672 14.9 / 14.5, N = 128256 45.5 / 49.0
+//   NVFP4 1 row:  4096 x 4096 9.4 / 7.2, N = 14336 12.6 / 9.8, N = 28672 19.6 / 17.9, N = 128256 59.8 / 65.3
+//   NVFP4 4 rows: 4096 x 4096 9.4 / 8.2, N = 14336 12.5 / 11.5, N = 28672 19.5 / 19.9
+// SiLU*up (two more gathers per element) gains in one pass only: MXFP4, K = 14336, N = 4096: 1 row 12.1 / 11.0, 2 rows
+// 12.2 / 13.2; 4096 x 4096: 1 row 7.5 / 5.9, 4 rows 7.8 / 9.3.
+static bool few_rows_plan(const StreamPlan& plan, bool nv, bool silu, int64_t M, int64_t N, int64_t K, int64_t xk) {
+  const int64_t chunks = M * ((plan.bps + 3) / 4) * 8;   // of the wave with the most
+  if (!plan.use || plan.nt != 1 || M > 32 || chunks > few_rows_chunks(silu) || K >= ((int64_t)1 << 22) || xk > K) return false;
+  const int64_t tiles = (N + 31) / 32, cus = device_cus();
+  return chunks <= 64 ? !nv || tiles <= 4 * cus : tiles <= (nv ? 2 : 4) * cus;
+}
+
+int silu_table_address(hipStream_t stream, const uint16_t** out);   // fpq_quantize.hip
+
+template <bool NV>
+static int linear_rows(const FewRows& in, int rot_kind, int g, const void* wq, const void* ws, const float* alpha,
+                       const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t xk, void* workspace,
+                       int64_t workspace_bytes, int zero_policy, hipStream_t stream) {
+  const int64_t K = (xk + 255) / 256 * 256;
+  if (M < 1 || N < 1 || xk < 256 || workspace_bytes < 0) return FPQ_E_SHAPE;
+  if (!in.x || !wq || !ws || !alpha || !y || (NV && !in.gs)) return FPQ_E_NULL;
+  if (xk % 32 != 0 || N > (1 << 24) || xk > (1 << 24)) return FPQ_E_SHAPE;
+  if (((uintptr_t)wq & 15u) || ((uintptr_t)ws & 15u) || ((uintptr_t)y & 15u) || ((uintptr_t)residual & 15u) ||
+      ((uintptr_t)workspace & 255u) || ((uintptr_t)in.codes & 15u) || ((uintptr_t)in.scales & 15u))
+    return FPQ_E_ALIGN;
+  if (((uintptr_t)in.x & 15u) || ((uintptr_t)in.up & 15u) || zero_policy != FPQ_ZERO_REFERENCE) return FPQ_E_UNSUPPORTED;
+  if (!workspace) workspace_bytes = 0;
+  // The plan that fpq_gemm_*_packed_splitk follows for these rows: the same parts of K, the same sums.
+  const StreamPlan plan = stream_plan(M, N, K, workspace_bytes, NV);
+  if (!few_rows_plan(plan, NV, in.up != nullptr, M, N, K, xk)) return FPQ_E_UNSUPPORTED;
+  if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
+  else if (rot_kind != FPQ_ROT_HADAMARD || xk % g != 0) return FPQ_E_UNSUPPORTED;
+  const dim3 grid((unsigned)((N + 31) / 32), (unsigned)plan.ksplit);
+  const bool many = (int64_t)grid.x * grid.y >= 3 * device_cus() / 2;   // (as launch_stream)
+  unsigned* counters = (unsigned*)workspace;
+  float* partial = workspace ? (float*)((uint8_t*)workspace + kStreamCounterBytes) : nullptr;
+  auto go = [&](auto rows_g, auto rows_rot, auto silu) {
+    constexpr int G = decltype(rows_g)::value, ROT = decltype(rows_rot)::value;
+    constexpr bool S = decltype(silu)::value;
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, nullptr, nullptr, (const uint8_t*)wq, (const uint8_t*)ws, alpha,
+                         (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, plan.bps,
+                         plan.ksplit, partial, counters, OutSegments{}, in);
+    };
+    if (many) launch(gemm_fp4_stream_kernel<1, 1, 2, 4, NV, FewRows, G, ROT, S>);
+    else launch(gemm_fp4_stream_kernel<1, 1, 4, 4, NV, FewRows, G, ROT, S>);
+    return (int)hipGetLastError();
+  };
+  auto by_rotation = [&](auto silu) {
+    typedef std::integral_constant<int, FPQ_ROT_HADAMARD> Had;
+    if (rot_kind == FPQ_ROT_IDENTITY)
+      return go(std::integral_constant<int, 32>{}, std::integral_constant<int, FPQ_ROT_IDENTITY>{}, silu);
+    if constexpr (NV) {
+      if (g == 16) return go(std::integral_constant<int, 16>{}, Had{}, silu);
+    }
+    if (g == 32) return go(std::integral_constant<int, 32>{}, Had{}, silu);
+    if (g == 64) return go(std::integral_constant<int, 64>{}, Had{}, silu);
+    if (g == 128) return go(std::integral_constant<int, 128>{}, Had{}, silu);
+    return (int)FPQ_E_UNSUPPORTED;
+  };
+  return in.up ? by_rotation(std::true_type{}) : by_rotation(std::false_type{});
+}
 
 // ---- the entry point that allocates nothing -------------------------------------------------------
 // Counters and partial tiles of a split K live in this file-scope array instead of a caller-provided
@@ -666,4 +873,22 @@ extern "C" int fpq_test_noalloc_counters(void* out, int64_t bytes, void* stream)
   if (st != FPQ_OK) return st;
   if (bytes == 0) return FPQ_OK;
   return (int)hipMemcpyAsync(out, ptr, (size_t)bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream);
+}
+
+extern "C" int fpq_linear_rows(int nv, const void* x, const void* up, int64_t M, int64_t K, int rot_kind, int g, float norm,
+                               const float* global_scale, const void* wq, const void* ws, const float* alpha,
+                               const void* bias, const void* residual, void* y, int64_t N, void* packed_codes,
+                               void* packed_scales, void* workspace, int64_t workspace_bytes, int zero_policy,
+                               void* stream) {
+  fpq::FewRows in{(const uint4*)x, (const uint4*)up, nullptr, global_scale, (uint8_t*)packed_codes,
+                  (uint8_t*)packed_scales, norm, (int)K};
+  if (!packed_codes != !packed_scales) return FPQ_E_NULL;
+  if (K < 0 || K > (1 << 24)) return FPQ_E_SHAPE;
+  if (up) {
+    if (const int st = fpq::silu_table_address((hipStream_t)stream, &in.silu)) return st;
+  }
+  return nv ? fpq::linear_rows<true>(in, rot_kind, g, wq, ws, alpha, bias, residual, y, M, N, K, workspace,
+                                     workspace_bytes, zero_policy, (hipStream_t)stream)
+            : fpq::linear_rows<false>(in, rot_kind, g, wq, ws, alpha, bias, residual, y, M, N, K, workspace,
+                                      workspace_bytes, zero_policy, (hipStream_t)stream);
 }

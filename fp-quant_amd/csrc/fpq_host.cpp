@@ -14,7 +14,7 @@
 //
 // A plan states the tensors it was made from (object, address, modification counter), and every call compares them.
 // Every function here returns None (False where a plan is missing or outdated and may be made), having launched nothing that is not repeated, whenever a call is not the plain
-// one (tracing, a capture, gradients, tensor subclasses, modes, another device, strides): the caller then takes the Python path, which is the definition of the result and makes the plans anew.
+// one (tracing, gradients, tensor subclasses, modes, another device, strides): the caller then takes the Python path, which is the definition of the result and makes the plans anew.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
@@ -39,7 +39,7 @@ namespace {
 // ---- the library: the entry points of the build that the ctypes binding has loaded
 #define FPQ_ENTRIES(X)                                                                                       \
   X(fpq_stream_capture_id) X(fpq_quantize_mx) X(fpq_quantize_mx_quest) X(fpq_quantize_nv) X(fpq_pack_padded)          \
-  X(fpq_gemm_mxf4) X(fpq_gemm_nvf4)                                                                          \
+  X(fpq_gemm_mxf4) X(fpq_gemm_nvf4) X(fpq_linear_rows)                                                                          \
   X(fpq_quantize_mx_packed_padded) X(fpq_quantize_nv_packed_padded)                 \
   X(fpq_gemm_mxf4_packed) X(fpq_gemm_mxf4_packed_residual) X(fpq_gemm_mxf4_packed_splitk)                    \
   X(fpq_gemm_mxf4_packed_multi) X(fpq_gemm_nvf4_packed) X(fpq_gemm_nvf4_packed_residual)                     \
@@ -73,7 +73,7 @@ PyTypeObject* g_activations;  // eager.QuantizedActivations
 int g_policy, g_packed_rows_mx, g_packed_rows_nv;
 
 PyObject *s_qweight, *s_scales, *s_wgs, *s_ags, *s_h, *s_bias, *s_plan, *s_qplan, *s_alpha, *s_packed, *s_share,
-    *s_parameters, *s_buffers, *s_weight, *s_eps, *s_rotation;
+    *s_parameters, *s_buffers, *s_weight, *s_eps, *s_rotation, *s_splitk;
 
 // ---- tensors
 const at::Tensor* tensor_of(PyObject* o) { return o && THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
@@ -230,6 +230,7 @@ PyMethodDef source_died_def = {"source_died", source_died, METH_O, nullptr};
 struct Call {   // where a call runs
   c10::DeviceIndex dev;
   hipStream_t stream;
+  unsigned long long capture;   // of the graph being recorded, 0: none
 };
 
 // Whether `x` is an input that the plain path takes; fills `call`.
@@ -241,10 +242,8 @@ bool plain_call(const at::Tensor& x, Call& call, at::ScalarType type = at::kBFlo
   call.dev = x.device().index();
   if (c10::hip::current_device() != call.dev) return false;
   call.stream = c10::hip::getCurrentHIPStream(call.dev).stream();
-  unsigned long long capture = 0;
-  if (!plain_entry(E_fpq_stream_capture_id) || FPQ_CALL(fpq_stream_capture_id)(call.stream, &capture) != 0 || capture != 0)
-    return false;
-  return true;
+  call.capture = 0;
+  return plain_entry(E_fpq_stream_capture_id) && FPQ_CALL(fpq_stream_capture_id)(call.stream, &call.capture) == 0;
 }
 
 QuantPlan::Body* quant_plan(PyObject* h, PyObject* ags, bool nvfp4) {   // whatever is current, usable or not
@@ -256,8 +255,8 @@ QuantPlan::Body* quant_plan(PyObject* h, PyObject* ags, bool nvfp4) {   // whate
 
 // What two calls must agree on to share quantized activations, as eager._sharing_key states it; null: error.
 PyObject* sharing_key(const QuantPlan::Body& q, int64_t m, int64_t k, const Call& call, bool quest) {
-  return Py_BuildValue("(OOKi(LL)O)", q.rot, q.nvfp4 ? q.gs_host : Py_None, (unsigned long long)(uintptr_t)call.stream, 0,
-                       (long long)m, (long long)k, quest ? Py_True : Py_False);
+  return Py_BuildValue("(OOKK(LL)O)", q.rot, q.nvfp4 ? q.gs_host : Py_None, (unsigned long long)(uintptr_t)call.stream,
+                       call.capture, (long long)m, (long long)k, quest ? Py_True : Py_False);
 }
 bool sharing_enabled(const QuantPlan::Body& q, bool& declined) {
   PyObject* on = PyDict_GetItem(g_eager_globals, s_share);
@@ -294,6 +293,7 @@ bool publish(PyObject* src, const at::Tensor& t, PyObject* key, PyObject* keep, 
   return ok;
 }
 
+// The quantized buffers that publish() hands on hold rows of a whole 32-row tile.
 Packed packed_buffers(int64_t m, int64_t k, bool nvfp4, c10::DeviceIndex dev) {
   const int64_t rows = (m + 31) / 32 * 32, kp = (k + 255) / 256 * 256;
   const c10::Device d(c10::kCUDA, dev);
@@ -305,11 +305,12 @@ struct NoGil {
   ~NoGil() { PyEval_RestoreThread(s); }
 };
 
-// 1: done, 0: not the plain path, -1: Python error
-int activations(QuantPlan::Body& q, PyObject* src, const at::Tensor& x, PyObject* h, int64_t m, int64_t k, bool quest,
-                const Call& call, Packed& out) {
+// The quantized form of `src` that an earlier call left: 1 found, 2 none (`key`, if set: what to publish one under),
+// 0 not the plain path, -1 Python error
+int shared_activations(QuantPlan::Body& q, PyObject* src, const at::Tensor& x, int64_t m, int64_t k, bool quest,
+                       const Call& call, Packed& out, PyObject*& key) {
   bool declined = false;
-  PyObject* key = nullptr;
+  key = nullptr;
   if (sharing_enabled(q, declined)) {
     if (declined) return 0;
     key = sharing_key(q, m, k, call, quest);
@@ -322,10 +323,10 @@ int activations(QuantPlan::Body& q, PyObject* src, const at::Tensor& x, PyObject
       if (a->ref && PyWeakref_CheckRef(a->ref) && PyWeakref_GET_OBJECT(a->ref) == src && a->version && a->key &&
           PyLong_Check(a->version) && PyLong_AsUnsignedLong(a->version) == (unsigned long)x._version()) {
         const int same = PyObject_RichCompareBool(a->key, key, Py_EQ);
-        if (same < 0) { Py_DECREF(key); return -1; }
+        if (same < 0) { Py_CLEAR(key); return -1; }
         if (same) {
           PyObject* form = q.nvfp4 ? a->nv_packed : a->mx_packed;
-          Py_DECREF(key);
+          Py_CLEAR(key);
           if (!form || !PyTuple_Check(form) || PyTuple_GET_SIZE(form) != 2) return 0;   // (row-major: re-tiled there)
           const at::Tensor *c = tensor_of(PyTuple_GET_ITEM(form, 0)), *s = tensor_of(PyTuple_GET_ITEM(form, 1));
           if (!c || !s) return 0;
@@ -336,6 +337,12 @@ int activations(QuantPlan::Body& q, PyObject* src, const at::Tensor& x, PyObject
       if (PyErr_Occurred()) PyErr_Clear();
     }
   }
+  return 2;
+}
+
+// Steals `key`.  1: done, 0: not the plain path, -1: Python error
+int quantize(QuantPlan::Body& q, PyObject* src, const at::Tensor& x, PyObject* h, int64_t m, int64_t k, bool quest,
+             const Call& call, Packed& out, PyObject* key) {
   if (!plain_entry(E_fpq_quantize_nv_packed_padded) || !plain_entry(E_fpq_quantize_mx_packed_padded) || (quest && q.nvfp4)) {
     Py_XDECREF(key);
     return 0;
@@ -372,6 +379,13 @@ int activations(QuantPlan::Body& q, PyObject* src, const at::Tensor& x, PyObject
   if (st != FPQ_OK) { Py_XDECREF(key); return 0; }
   if (key && !publish(src, x, key, h, out, m, k, nv, call)) return -1;
   return 1;
+}
+
+int activations(QuantPlan::Body& q, PyObject* src, const at::Tensor& x, PyObject* h, int64_t m, int64_t k, bool quest,
+                const Call& call, Packed& out) {
+  PyObject* key;
+  const int rc = shared_activations(q, src, x, m, k, quest, call, out, key);
+  return rc == 2 ? quantize(q, src, x, h, m, k, quest, call, out, key) : rc;
 }
 
 bool packed_weights_enabled() {
@@ -439,21 +453,58 @@ bool residual_of(PyObject* o, int64_t m, int64_t n, const Call& call, const at::
   return true;
 }
 
+// The split-K workspace of a call, left undefined where none is used: the stream's own, which the Python path makes on
+// the stream's first call that needs it, or, in a capture, the layer's.  False: not there.
+bool splitk_workspace(const LinearPlan::Body& p, PyObject* qweight, int64_t m, const Call& call, at::Tensor& workspace) {
+  if (p.need == 0 || m > p.split_rows) return true;
+  const at::Tensor* w = nullptr;
+  if (call.capture) {
+    w = tensor_of(attribute(qweight, s_splitk));
+  } else {
+    PyObject* dev = PyLong_FromLong(call.dev);
+    PyObject* stream = PyLong_FromUnsignedLongLong((unsigned long long)(uintptr_t)call.stream);
+    PyObject* per = dev ? PyDict_GetItem(g_workspaces, dev) : nullptr;
+    w = per && stream && PyDict_Check(per) ? tensor_of(PyDict_GetItem(per, stream)) : nullptr;
+    Py_XDECREF(dev);
+    Py_XDECREF(stream);
+  }
+  if (!w || !w->is_cuda() || w->device().index() != call.dev || w->numel() < p.need) return false;
+  workspace = *w;
+  return true;
+}
+
+// A few rows in one launch, quantization included (fpq_linear_rows); `out`, if its tensors are there, receives the
+// quantized rows.  1: launched, 0: the kernel does not take them
+int linear_rows(const LinearPlan::Body& p, const QuantPlan::Body& q, const LayerTensors& t, const at::Tensor& x,
+                const at::Tensor* up, const at::Tensor* residual, const Packed& out, at::Tensor& y, int64_t m,
+                const Call& call) {
+  if (m > 16 || q.kind > 1 || !plain_entry(E_fpq_linear_rows)) return 0;
+  for (int e : {E_fpq_gemm_mxf4_packed, E_fpq_gemm_nvf4_packed, E_fpq_gemm_mxf4_packed_splitk, E_fpq_gemm_nvf4_packed_splitk,
+                E_fpq_gemm_mxf4_packed_residual, E_fpq_gemm_nvf4_packed_residual})
+    if (!plain_entry(e)) return 0;   // (whoever instruments the GEMMs sees every one of them)
+  at::Tensor workspace;
+  if (!splitk_workspace(p, t.qweight, m, call, workspace)) return 0;
+  const at::Tensor wp = p.packed_only ? *tensor_of(t.qweight) : p.wp, wsp = p.packed_only ? *tensor_of(t.scales) : p.wsp;
+  const at::Tensor alpha = p.alpha, bias = p.bias.held, gs = q.gs;
+  const int64_t n = p.n, k = p.k;
+  const int kind = q.kind, g = q.g;
+  const float norm = q.norm;
+  const bool nv = p.nvfp4;
+  NoGil nogil;
+  auto data = [](const at::Tensor& v) -> void* { return v.defined() ? v.data_ptr() : nullptr; };
+  return FPQ_CALL(fpq_linear_rows)(nv, x.const_data_ptr(), up ? up->const_data_ptr() : nullptr, m, k, kind, g, norm,
+                                   (const float*)data(gs), wp.const_data_ptr(), wsp.const_data_ptr(),
+                                   (const float*)alpha.const_data_ptr(), data(bias),
+                                   residual ? residual->const_data_ptr() : nullptr, y.mutable_data_ptr(), n, data(out.codes),
+                                   data(out.scales), data(workspace), workspace.defined() ? workspace.numel() : 0, g_policy,
+                                   call.stream) == FPQ_OK;
+}
+
 // 1: launched, 0: not the plain path
 int gemm(const LinearPlan::Body& p, const LayerTensors& t, const Packed& x, const at::Tensor* residual, at::Tensor& y,
          int64_t m, const Call& call) {
   at::Tensor workspace;
-  if (p.need > 0 && m <= p.split_rows) {
-    // the stream's own workspace, made by the Python path on the stream's first call that needs it
-    PyObject* dev = PyLong_FromLong(call.dev);
-    PyObject* stream = PyLong_FromUnsignedLongLong((unsigned long long)(uintptr_t)call.stream);
-    PyObject* per = dev ? PyDict_GetItem(g_workspaces, dev) : nullptr;
-    const at::Tensor* w = per && stream && PyDict_Check(per) ? tensor_of(PyDict_GetItem(per, stream)) : nullptr;
-    if (w && w->numel() >= p.need) workspace = *w;
-    Py_XDECREF(dev);
-    Py_XDECREF(stream);
-    if (!workspace.defined()) return 0;
-  }
+  if (!splitk_workspace(p, t.qweight, m, call, workspace)) return 0;
   const bool nv = p.nvfp4, split = workspace.defined();
   const int entry = split ? (nv ? E_fpq_gemm_nvf4_packed_splitk : E_fpq_gemm_mxf4_packed_splitk)
                     : residual ? (nv ? E_fpq_gemm_nvf4_packed_residual : E_fpq_gemm_mxf4_packed_residual)
@@ -518,10 +569,23 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   const THPObjectPtr hold_p(Py_NewRef(attribute(t.qweight, s_plan))), hold_q(Py_NewRef(attribute(t.h, s_qplan)));
   const THPObjectPtr hold_w(Py_NewRef(t.qweight)), hold_s(Py_NewRef(t.scales)), hold_h(Py_NewRef(t.h));
   Packed packed;
-  const int rc = activations(*q, args[1], x, t.h, m, k, quest, call, packed);
+  PyObject* key;
+  int rc = shared_activations(*q, args[1], x, m, k, quest, call, packed, key);
   if (rc < 0) return nullptr;
   if (rc == 0) Py_RETURN_NONE;
   at::Tensor y = output_like(x, p->n, call);
+  if (rc == 2) {
+    if (!quest && m <= 16 && q->kind <= 1) {
+      if (key) packed = packed_buffers(m, k, nvfp4, call.dev);
+      if (linear_rows(*p, *q, t, x, nullptr, residual, packed, y, m, call)) {
+        if (key && !publish(args[1], x, key, t.h, packed, m, k, nvfp4, call)) return nullptr;
+        return THPVariable_Wrap(std::move(y));
+      }
+    }
+    rc = quantize(*q, args[1], x, t.h, m, k, quest, call, packed, key);
+    if (rc < 0) return nullptr;
+    if (rc == 0) Py_RETURN_NONE;
+  }
   if (!gemm(*p, t, packed, residual, y, m, call)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
@@ -679,6 +743,8 @@ PyObject* host_gated_down(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (!plain_entry(entry)) Py_RETURN_NONE;
   const THPObjectPtr hold_p(Py_NewRef(attribute(t.qweight, s_plan))), hold_q(Py_NewRef(attribute(t.h, s_qplan)));
   const THPObjectPtr hold_w(Py_NewRef(t.qweight)), hold_s(Py_NewRef(t.scales));
+  at::Tensor y = output_like(gate, p->n, call);
+  if (linear_rows(*p, *q, t, gate, &u, residual, Packed{}, y, m, call)) return THPVariable_Wrap(std::move(y));
   Packed out = packed_buffers(m, k, nvfp4, call.dev);
   int st;
   {
@@ -694,7 +760,6 @@ PyObject* host_gated_down(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
                                                            nullptr, pc, ps, g_policy, call.stream);
   }
   if (st != FPQ_OK) Py_RETURN_NONE;
-  at::Tensor y = output_like(gate, p->n, call);
   if (!gemm(*p, t, out, residual, y, m, call)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
@@ -1048,7 +1113,8 @@ PyMODINIT_FUNC PyInit__fpq_host() {
                {&s_h, "forward_hadamard_matrix"}, {&s_bias, "bias"}, {&s_plan, "_fpq_plan"}, {&s_qplan, "_fpq_qplan"},
                {&s_alpha, "_fpq_alpha"}, {&s_packed, "_fpq_packed"}, {&s_share, "SHARE_ACT_QUANT"},
                {&s_parameters, "_parameters"}, {&s_buffers, "_buffers"}, {&s_weight, "weight"},
-               {&s_eps, "variance_epsilon"}, {&s_rotation, "_fpq_rotation"}};
+               {&s_eps, "variance_epsilon"}, {&s_rotation, "_fpq_rotation"},
+               {&s_splitk, "_fpq_splitk"}};
   for (auto& n : names)
     if (!(*n.slot = PyUnicode_InternFromString(n.text))) return nullptr;
   struct {

@@ -13,15 +13,13 @@
 #include "../../include/fpq.h"
 #include "fpq_device.h"
 #include "fpq_gemm_epilogue.h"  // LdsLimitOnce
+#include "fpq_quantize_chunk.h"
 
 namespace fpq {
 
 #ifndef FPQ_EPL
 #define FPQ_EPL 64  // elements owned by one lane in the streaming kernel (64 or 128)
 #endif
-
-constexpr int kFmtMx = 0;
-constexpr int kFmtNv = 1;
 
 // -------------------------------------------------------------------------------------------
 // Generic kernel: one lane owns 8 consecutive elements (one 16-byte load, 4 bytes of codes).
@@ -113,13 +111,6 @@ __global__ __launch_bounds__(256) void silu_table_kernel() {
 
 __device__ __forceinline__ float silu_bf16(uint32_t bits) {
   return __uint_as_float((uint32_t)g_silu_table[bits] << 16);
-}
-
-__device__ __forceinline__ void unpack8(const uint4& raw, float (&p)[8]) {
-  p[0] = bf16_lo(raw.x); p[1] = bf16_hi(raw.x);
-  p[2] = bf16_lo(raw.y); p[3] = bf16_hi(raw.y);
-  p[4] = bf16_lo(raw.z); p[5] = bf16_hi(raw.z);
-  p[6] = bf16_lo(raw.w); p[7] = bf16_hi(raw.w);
 }
 
 template <int G, int ROT, int PRO = kProNone>
@@ -428,238 +419,11 @@ static int launch_lane8(const void* x, int64_t rows, int64_t cols, float norm, c
 // XOR-swizzled by the lane number (through the choice of the piece each DMA lane fetches) so
 // those reads are bank-conflict free.  Codes return through the same LDS region so that global
 // stores are contiguous.
-constexpr float kKappa = -0x1.8p-26f;  // fma(x, 0.75, x * kKappa) rounds to the E2M1 code of x / fl(4/3)
-
-// Hadamard output index that sequency-ordered output k of a g-block takes: bitreverse(k ^ (k >> 1))
-__host__ __device__ constexpr int gsr_source(int k, int g) {
-  int gray = k ^ (k >> 1), r = 0;
-  for (int b = 1; b < g; b <<= 1) {
-    r = (r << 1) | (gray & 1);
-    gray >>= 1;
-  }
-  return r;
-}
-
 // 16-byte store that does not ask the L2 to keep the line: the streaming kernel's codes are written once
 // and read by a later kernel (2-3 % on the whole kernel against plain stores).
 __device__ __forceinline__ void store16_nt(uint8_t* p, uint4 v) {
   typedef unsigned v4u_nt __attribute__((ext_vector_type(4)));
   __builtin_nontemporal_store(v4u_nt{v.x, v.y, v.z, v.w}, (v4u_nt*)p);
-}
-
-template <int ZERO>
-__device__ __forceinline__ uint32_t fix_zero_nibbles(uint32_t w) {
-  if (ZERO == kZeroReference) {
-    const uint32_t nz = ((w & 0x77777777u) + 0x77777777u) & 0x88888888u;  // bit 3 set where magnitude != 0
-    w |= nz ^ 0x88888888u;
-  }
-  return w;
-}
-
-// v[i] += sign * (v[i] of the lane that the quad permutation CTRL names), one instruction each.  Written as assembly
-// because the compiler keeps the lane move apart; a DPP operand may be read two wait states after it was written,
-// which the leading s_nop grants whatever comes before.
-template <int CTRL>
-__device__ __forceinline__ void fma_exchange8(float (&v)[8], float sign) {
-#define FPQ_FMAC_DPP(QP)                                                                                            \
-  asm volatile("s_nop 1\n\t"                                                                                        \
-               "v_fmac_f32_dpp %0, %0, %8 " QP "\n\tv_fmac_f32_dpp %1, %1, %8 " QP "\n\t"                           \
-               "v_fmac_f32_dpp %2, %2, %8 " QP "\n\tv_fmac_f32_dpp %3, %3, %8 " QP "\n\t"                           \
-               "v_fmac_f32_dpp %4, %4, %8 " QP "\n\tv_fmac_f32_dpp %5, %5, %8 " QP "\n\t"                           \
-               "v_fmac_f32_dpp %6, %6, %8 " QP "\n\tv_fmac_f32_dpp %7, %7, %8 " QP                                  \
-               : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])     \
-               : "v"(sign))
-  static_assert(CTRL == 0xB1 || CTRL == 0x4E, "lane ^ 1 or lane ^ 2");
-  if (CTRL == 0xB1) FPQ_FMAC_DPP("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf");
-  else FPQ_FMAC_DPP("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf");
-#undef FPQ_FMAC_DPP
-}
-
-// One lane's chunk of EPL consecutive elements, rotated in place: the butterflies with stride < EPL stay in the
-// lane's registers, a wider rotation takes one or two exchanges with the neighbouring lanes that hold the rest
-// of the block (lane % (G / EPL) is the chunk's place in it).
-//
-// An exchange gives the lower lane a + b and the upper one a - b.  With KEEP_ZERO_SIGN the upper lane negates its own
-// value and both add (two instructions and a wait between them); otherwise a lane holds its values negated through
-// the stages before an exchange in which it is the upper one (the norm's sign: a rotation of negated values is the
-// negated rotation), and the exchange is ONE fused multiply-add with +-1, own + sign * other, whose product is exact.
-// The only difference is the sign of a zero, which the reference's zero policy does not look at.
-template <int EPL, int G, int ROT, bool KEEP_ZERO_SIGN>
-__device__ __forceinline__ void rotate_chunk(float (&v)[EPL], float norm, uint32_t lane) {
-  if (ROT == FPQ_ROT_HADAMARD || ROT == FPQ_ROT_GSR) {
-    static_assert(G <= 4 * EPL, "at most two exchanges between lanes");
-    constexpr bool kNegate = !KEEP_ZERO_SIGN && G > EPL;
-    const uint32_t upper1 = (lane & 1u) << 31, upper2 = G > 2 * EPL ? (lane & 2u) << 30 : 0u;
-    const float n = kNegate ? __uint_as_float(__float_as_uint(norm) ^ upper1 ^ upper2) : norm;
-#pragma unroll
-    for (int i = 0; i < EPL; ++i) v[i] *= n;
-#pragma unroll
-    for (int s = 1; s < (G < EPL ? G : EPL); s *= 2) {
-      __builtin_amdgcn_sched_barrier(0);  // keep the stages in place: EPL live values, no more
-#pragma unroll
-      for (int i = 0; i < EPL; ++i) {
-        if ((i & s) == 0) {
-          const float a = v[i], b = v[i + s];
-          v[i] = a + b;
-          v[i + s] = a - b;
-        }
-      }
-    }
-    auto exchange = [&](auto ctrl, uint32_t upper) __attribute__((always_inline)) {
-      constexpr int kCtrl = decltype(ctrl)::value;
-      __builtin_amdgcn_sched_barrier(0);
-      const float sign = __uint_as_float(0xbf800000u ^ upper);   // lower lane -1 (its partner holds -b), upper lane +1
-      if (kNegate) {
-#pragma unroll
-        for (int i = 0; i < EPL; i += 8) fma_exchange8<kCtrl>(*(float (*)[8])&v[i], sign);
-      } else {
-#pragma unroll
-        for (int i = 0; i < EPL; ++i) {
-          const float other = __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v[i]), kCtrl, 0xF,
-                                                                                 0xF, true));
-          v[i] = other + __uint_as_float(__float_as_uint(v[i]) ^ upper);
-        }
-      }
-    };
-    // stride EPL: the two halves of a rotation block sit in lanes 2u and 2u + 1; stride 2 EPL (a 128-wide rotation
-    // with EPL = 32): the quarters sit in lanes 4u .. 4u + 3 and the partner is lane ^ 2
-    if (G > EPL) exchange(std::integral_constant<int, 0xB1 /* quad_perm [1,0,3,2] */>{}, upper1);
-    if (G > 2 * EPL) exchange(std::integral_constant<int, 0x4E /* quad_perm [2,3,0,1] */>{}, upper2);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  if (ROT == FPQ_ROT_GSR) {
-    // sequency order inside every G-block (G <= EPL here): a compile-time renaming of registers
-    static_assert(ROT != FPQ_ROT_GSR || G <= EPL, "GSR blocks must fit in one lane");
-    float w[EPL];
-#pragma unroll
-    for (int k = 0; k < EPL; ++k) w[k] = v[(k & ~(G - 1)) | gsr_source(k & (G - 1), G)];
-#pragma unroll
-    for (int k = 0; k < EPL; ++k) v[k] = w[k];
-  }
-}
-
-// E2M1 codes and scale bytes of one lane's rotated chunk (cw: CW dwords of codes; sbytes: the scale bytes, with
-// eight of them the first four in sb_lo).  Returns whether a group left the range in which the two-operation
-// division is proven: the caller then redoes the chunk with quantize_chunk_slow.
-template <int EPL, int FMT, int ZERO, bool QUEST>
-__device__ __forceinline__ bool quantize_chunk(const float (&v)[EPL], float gs, bool nv_fast,
-                                               const float2* __restrict__ lut, uint32_t (&cw)[EPL / 8],
-                                               uint32_t& sbytes, uint32_t& sb_lo) {
-  constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
-  constexpr int NG = EPL / GROUP;
-  bool need_slow = false;
-#pragma unroll
-  for (int gi = 0; gi < NG; ++gi) {
-    float a = 0.0f;
-    if (!QUEST) {
-#pragma unroll
-      for (int i = 0; i < GROUP; ++i) a = __builtin_fmaxf(a, __builtin_fabsf(v[gi * GROUP + i]));
-    }
-    uint32_t byte;
-    bool fast;
-    float k1, k2, cvt_scale;
-    if (QUEST) {
-      float os[4], oq[4];
-#pragma unroll
-      for (int o = 0; o < 4; ++o) {
-        const float* p = &v[gi * GROUP + 8 * o];
-        float sum = p[0], sq = p[0] * p[0];
-#pragma unroll
-        for (int i = 1; i < 8; ++i) {
-          sum = sum + p[i];
-          sq = sq + p[i] * p[i];
-        }
-        os[o] = sum;
-        oq[o] = sq;
-      }
-      const float sum = (os[0] + os[1]) + (os[2] + os[3]), sq = (oq[0] + oq[1]) + (oq[2] + oq[3]);
-      const float mean = sum * 0.03125f, msq = sq * 0.03125f;
-      float var = msq - mean * mean;
-      var = var > 0.0f ? var : 0.0f;
-      const float sc = __builtin_sqrtf(var) * 0.48707976f + 1e-8f;   // fl32(2.92247856 / 6); >= 1e-8: normal
-      byte = (__float_as_uint(sc) >> 23) & 0xffu;
-      fast = true;
-      k1 = k2 = 0.0f;
-      cvt_scale = __uint_as_float(byte << 23);                         // s = 2^floor(log2(sc))
-    } else if (FMT == kFmtMx) {
-      const uint32_t bits = __float_as_uint(a);
-      byte = bits >> 23;
-      fast = (byte - 29u) <= 198u || bits == 0u;                       // -98 <= e <= 100, or all zero
-      k1 = 0.75f;
-      k2 = kKappa;
-      cvt_scale = __uint_as_float((bits & 0x7f800000u) - (2u << 23));  // 2^(e-2)
-      if (bits == 0u) {  // a zero group stores 2^-126 and zero codes
-        byte = 1u;
-        cvt_scale = 1.0f;
-      }
-    } else {
-      float t = div6_rn(a) * gs;
-      t = t > 448.0f ? 448.0f : t;
-      byte = e4m3_encode(t);
-      fast = nv_fast;
-      const float2 e = lut[byte & 0x7fu];
-      k1 = e.x;
-      k2 = e.y;
-      cvt_scale = 1.0f;
-    }
-    need_slow |= !fast;
-#pragma unroll
-    for (int d = 0; d < GROUP / 8; ++d) {
-      uint32_t w = 0u;
-#pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const float x0 = v[gi * GROUP + d * 8 + 2 * h], x1 = v[gi * GROUP + d * 8 + 2 * h + 1];
-        float q0 = QUEST ? x0 : __builtin_fmaf(x0, k1, x0 * k2);
-        float q1 = QUEST ? x1 : __builtin_fmaf(x1, k1, x1 * k2);
-        if (ZERO == kZeroSigned && !QUEST) {  // x / s keeps the sign of x, also for -0
-          q0 = __builtin_copysignf(q0, x0);
-          q1 = __builtin_copysignf(q1, x1);
-        }
-        if (h == 0) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 0);
-        if (h == 1) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 1);
-        if (h == 2) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 2);
-        if (h == 3) w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w, q0, q1, cvt_scale, 3);
-      }
-      if (FMT == kFmtNv && ZERO == kZeroSigned) w = byte == 0u ? 0u : w;  // zero scale: +0 codes
-      cw[gi * (GROUP / 8) + d] = fix_zero_nibbles<ZERO>(w);
-    }
-    sbytes |= (byte & 0xffu) << (8 * (gi & 3));
-    if (NG == 8 && gi == 3) {  // eight scale bytes per chunk: park the first four
-      sb_lo = sbytes;
-      sbytes = 0u;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  return need_slow;
-}
-
-template <int EPL, int FMT, int ZERO>
-__device__ __forceinline__ void quantize_chunk_slow(const float (&u)[EPL], float gs, float rg,
-                                                    uint32_t (&cw)[EPL / 8], uint32_t& sbytes) {
-  constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
-  constexpr int NG = EPL / GROUP;
-  sbytes = 0u;
-#pragma unroll 1
-  for (int gi = 0; gi < NG; ++gi) {
-    float a = 0.0f;
-#pragma unroll
-    for (int i = 0; i < GROUP; ++i) a = __builtin_fmaxf(a, __builtin_fabsf(u[gi * GROUP + i]));
-    const GroupScale g = FMT == kFmtMx ? mx_group_scale(a) : nv_group_scale(a, gs, rg);
-#pragma unroll
-    for (int d = 0; d < GROUP / 8; ++d) {
-      uint32_t w = 0u;
-#pragma unroll
-      for (int h = 0; h < 8; ++h) {
-        const float xv = u[gi * GROUP + d * 8 + h];
-        float q = scale_element(xv, g);
-        if (ZERO == kZeroSigned) q = __builtin_copysignf(q, xv);
-        if (FMT == kFmtNv) q = g.zero ? 0.0f : q;
-        w |= e2m1_code<ZERO>(q) << (4 * h);
-      }
-      cw[gi * (GROUP / 8) + d] = w;
-    }
-    sbytes |= (g.byte & 0xffu) << (8 * gi);
-  }
 }
 
 //
@@ -1576,7 +1340,7 @@ static int launch_lane8_prologue(const void* x, int64_t rows, int64_t cols, floa
 // Fills g_silu_table once per device.  The first call on a device builds the table on the caller's
 // stream and waits for it, so that calls on other streams can rely on it afterwards; while a stream
 // is being captured the build is recorded into the capture instead and nothing is remembered.
-int ensure_silu_table(hipStream_t stream) {   // also called by fpq_prepare_device (fpq_capi.hip)
+static int ensure_silu_table(hipStream_t stream) {
   static std::atomic<uint64_t> built{0};  // bit d: device d holds the table (devices >= 64 rebuild every call)
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -1594,6 +1358,26 @@ int ensure_silu_table(hipStream_t stream) {   // also called by fpq_prepare_devi
   if (e != hipSuccess) return (int)e;
   if (bit) built.fetch_or(bit, std::memory_order_release);
   return 0;
+}
+
+// Device address of the table on the current device, filled (looked up on the first call per device; two threads
+// racing on that first call store the same address).
+int silu_table_address(hipStream_t stream, const uint16_t** out) {   // for fpq_gemm_stream.hip, fpq_capi.hip
+  static std::atomic<const uint16_t*> address[64];
+  if (const int st = ensure_silu_table(stream)) return st;
+  int dev = -1;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return (int)e;
+  if (dev < 0 || dev >= 64) return FPQ_E_UNSUPPORTED;
+  *out = address[dev].load(std::memory_order_acquire);
+  if (!*out) {
+    void* ptr = nullptr;
+    e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_silu_table));
+    if (e != hipSuccess) return (int)e;
+    *out = (const uint16_t*)ptr;
+    address[dev].store(*out, std::memory_order_release);
+  }
+  return FPQ_OK;
 }
 
 // x: the prologue's first input with row stride ld_first elements (kProSiluMul: `second` with

@@ -361,6 +361,18 @@ int fpq_gemm_mxf4_packed_multi(const void* xq_packed, const void* xs_packed, con
                                const void* ws_packed, const float* alpha, const void* bias,
                                void* const* ys, const int64_t* ns, int64_t count, int64_t M, int64_t K,
                                void* stream);
+/*
+ * One linear on a few bf16 rows in one launch: what fpq_quantize_{mx,nv}_packed_padded (abs-max; with `up` non-null
+ * fpq_silu_mul_quantize_{mx,nv}_packed of gate = x and up) followed by fpq_gemm_{mxf4,nvf4}_packed_splitk computes, to
+ * the bit.  x (and up): [M, K] contiguous, 16-byte aligned, K a multiple of 32 and of g; weights packed with K padded to
+ * whole 256 blocks.  packed_codes / packed_scales (both or neither): receive the quantized rows in the packed layout;
+ * rows M .. 31 of it are not written.  FPQ_E_UNSUPPORTED, with nothing launched, where the two calls are the better
+ * way (more than a few rows) or the only one (GSR and general rotations, the signed zero policy).
+ */
+int fpq_linear_rows(int nv, const void* x, const void* up, int64_t M, int64_t K, int rot_kind, int g, float norm,
+                    const float* global_scale, const void* wq_packed, const void* ws_packed, const float* alpha,
+                    const void* bias, const void* residual, void* y, int64_t N, void* packed_codes, void* packed_scales,
+                    void* workspace, int64_t workspace_bytes, int zero_policy, void* stream);
 /* The same for packed NVFP4 operands (fpq_gemm_nvf4_packed). */
 int fpq_gemm_nvf4_packed_multi(const void* xq_packed, const void* xs_packed, const void* wq_packed,
                                const void* ws_packed, const float* alpha, const void* bias,
