@@ -132,20 +132,22 @@ constexpr int kScaleSlots = 4;
 constexpr int scale_block_bytes(bool nv) { return nv ? 512 : 256; }
 // (one kilobyte piece per load instruction, the same number of loads for each of the four waves: with six
 // pieces -- NVFP4, 256 x 128 tiles -- two each, the last two kilobytes copies that are never read)
-constexpr int scale_loads_per_wave(int blocks, bool nv) { return (blocks * scale_block_bytes(nv) / 1024 + 3) / 4; }
-constexpr int scale_slot_bytes(int blocks, bool nv) {
-  return (scale_loads_per_wave(blocks, nv) > 1 ? scale_loads_per_wave(blocks, nv) : 1) * 4096;
+constexpr int scale_loads_per_wave(int blocks, bool nv, int waves) {
+  return (blocks * scale_block_bytes(nv) / 1024 + waves - 1) / waves;
+}
+constexpr int scale_slot_bytes(int blocks, bool nv, int waves = 4) {
+  return (scale_loads_per_wave(blocks, nv, waves) > 1 ? scale_loads_per_wave(blocks, nv, waves) : 1) * waves * 1024;
 }
 constexpr int scale_slots(bool nv, int groups = 1) { return nv || groups > 1 ? 2 : kScaleSlots; }
-// LDS of a group of four waves whose unit holds `blocks` operand kilobytes (weight + activation row tiles)
-constexpr int packed_lds_bytes(int blocks, bool nv = false, int ring = kRing, int groups = 1) {
-  return ring * blocks * 1024 + scale_slots(nv, groups) * scale_slot_bytes(blocks, nv);
+// LDS of a group of waves whose unit holds `blocks` operand kilobytes (weight + activation row tiles)
+constexpr int packed_lds_bytes(int blocks, bool nv = false, int ring = kRing, int groups = 1, int waves = 4) {
+  return ring * blocks * 1024 + scale_slots(nv, groups) * scale_slot_bytes(blocks, nv, waves);
 }
-// ... and what is allocated: at least the epilogue's staging area (four waves, each WT_M rows of
+// ... and what is allocated: at least the epilogue's staging area (a group's waves, each WT_M rows of
 // WT_N bf16 + 16 bytes)
-constexpr int packed_lds_alloc(int blocks, bool nv, int ring, int wt_n, int wt_m, int groups = 1) {
-  const int rings = groups * packed_lds_bytes(blocks, nv, ring, groups), staging = 4 * wt_m * (wt_n * 2 + 16);
-  const int exchange = groups > 1 ? 4 * (wt_n / 32) * (wt_m / 32) * 4096 : 0;   // four waves' accumulators
+constexpr int packed_lds_alloc(int blocks, bool nv, int ring, int wt_n, int wt_m, int groups = 1, int waves = 4) {
+  const int rings = groups * packed_lds_bytes(blocks, nv, ring, groups, waves), staging = waves * wt_m * (wt_n * 2 + 16);
+  const int exchange = groups / 2 * waves * (wt_n / 32) * (wt_m / 32) * 4096;   // half of the groups' accumulators
   const int most = rings > staging ? rings : staging;
   return most > exchange ? most : exchange;
 }
@@ -195,8 +197,9 @@ __device__ __forceinline__ void barrier_lds_but() {
 // small tiles spends most of a unit waiting -- for its loads, for the barrier, for its two or four matrix
 // instructions to drain -- and alone on its SIMD nothing fills that time; with a second wave there, working
 // on the other half of K, something does, and each group's loop is half as long.
+// GR = 4 (NVFP4): four groups of two waves, a quarter of K each; see tile_plan.
 template <int NT, int KW, int MT, int WN, int WM, bool NV = false, int RING = kRing, int GR = 1>
-__global__ __launch_bounds__(256 * GR, (NT * MT <= 32 && GR == 1 ? 2 : 1)) void gemm_fp4_packed_kernel(
+__global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 1)) void gemm_fp4_packed_kernel(
     const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xs, const uint8_t* __restrict__ wq,
     const uint8_t* __restrict__ ws, const float* __restrict__ alpha_p,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int M, int N, int K, int tiles_m,
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(256 * GR, (NT * MT <= 32 && GR == 1 ? 2 : 1)) void 
     unsigned* counters) {
   constexpr int BN = NT * 32, BM = MT * 32;
   constexpr int NW = WN * WM;           // waves
-  static_assert(NW == 4 && NT <= KW && KW % 4 == 0 && MT % 4 == 0 && NT % WN == 0 && MT % WM == 0,
+  static_assert((NW == 4 || NW == 2) && NT <= KW && (KW + MT) % NW == 0 && KW % 2 == 0 && NT % WN == 0 && MT % WM == 0,
                 "unsupported tile / wave arrangement");
   constexpr int TN = NT / WN, TM = MT / WM;  // 32x32 MFMA tiles per wave along n and m
   constexpr int kBlocks = KW + MT;      // operand kilobytes per unit
@@ -213,19 +216,20 @@ __global__ __launch_bounds__(256 * GR, (NT * MT <= 32 && GR == 1 ? 2 : 1)) void 
   constexpr int kRpp = 1024 / kSB;                      // row tiles per 1 KB scale piece
   constexpr int kPieces = kBlocks / kRpp;               // scale pieces per 256-K block
   constexpr int kScLoads = kPieces >= NW ? (kPieces + NW - 1) / NW : 1;  // scale loads per wave per block
-  constexpr int kSlots = scale_slots(NV, GR), kSlotBytes = scale_slot_bytes(kBlocks, NV);
+  constexpr int kSlots = scale_slots(NV, GR), kSlotBytes = scale_slot_bytes(kBlocks, NV, NW);
   constexpr int kUnitBytes = kBlocks * 1024;
   static_assert(RING == 4 || RING == 8, "the ring holds one or two 256-K blocks");
-  constexpr int kPackedLds = packed_lds_bytes(kBlocks, NV, RING, GR);
+  constexpr int kPackedLds = packed_lds_bytes(kBlocks, NV, RING, GR, NW);
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_all[];
-  static_assert(GR == 1 || GR == 2, "one or two groups of four waves");
-  const int grp = GR > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  static_assert(GR == 1 || GR == 2 || GR == 4, "groups of waves");
+  static_assert((KW + MT) % kRpp == 0 && KW % kRpp == 0, "a scale piece holds weights or activations");
+  const int grp = GR > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * NW)) : 0;
   uint8_t* const smem = smem_all + grp * kPackedLds;   // this group's ring and scale slots
   const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
   constexpr int kScaleBase = RING * kUnitBytes;
   static_assert(kScaleBase + kSlots * kSlotBytes == kPackedLds, "LDS map does not match the allocation");
 
-  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3), lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & (NW - 1)), lane = threadIdx.x & 63;
   // (One workgroup per tile: a persistent variant that walked several tiles per CU measured slower, the
   // hardware's own dispatch balances the XCDs better.)
   int tile_m, tile_n;
@@ -554,31 +558,37 @@ __global__ __launch_bounds__(256 * GR, (NT * MT <= 32 && GR == 1 ? 2 : 1)) void 
 #undef FPQ_TAKE_SCALES_NOW
 #undef FPQ_TAKE_SCALES_AFTER
 
-  if constexpr (GR == 2) {
-    // The second group's accumulators go to the first through LDS (the rings are idle: every wave has waited
-    // for its last loads and read its last unit), added in a fixed order; then the second group only keeps
-    // the first company at the one barrier of the epilogue.  (Launched with K whole per workgroup: ksplit = 1.)
-    __syncthreads();
-    float* xch = (float*)smem_all + wave * (TN * TM * 16 * 64) + lane;
-    if (grp == 1) {
+  if constexpr (GR > 1) {
+    // The upper half of the groups hands its accumulators to the lower one through LDS (the rings are idle: every wave
+    // has waited for its last loads and read its last unit), and so on: a fixed order, (0 + 2) + (1 + 3).  Then the
+    // other groups only keep the first company at the one barrier of the epilogue.  (Launched with K whole per
+    // workgroup: ksplit = 1.)
 #pragma unroll
-      for (int i = 0; i < TN; ++i)
+    for (int half = GR / 2; half > 0; half /= 2) {
+      __syncthreads();
+      float* xch = (float*)smem_all + ((grp & (half - 1)) * NW + wave) * (TN * TM * 16 * 64) + lane;
+      if (grp >= half && grp < 2 * half) {
 #pragma unroll
-        for (int j = 0; j < TM; ++j)
+        for (int i = 0; i < TN; ++i)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) xch[((i * TM + j) * 16 + v) * 64] = acc[i][j][v];
+          for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) xch[((i * TM + j) * 16 + v) * 64] = acc[i][j][v];
+      }
+      __syncthreads();
+      if (grp < half) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] += xch[((i * TM + j) * 16 + v) * 64];
+      }
     }
-    __syncthreads();
-    if (grp == 1) {
+    if (grp > 0) {
       __syncthreads();
       return;
     }
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] += xch[((i * TM + j) * 16 + v) * 64];
   }
   if (GR == 1 && kCanSplit && ksplit > 1) {
     // The parts of a tile run on different XCDs, whose L2 caches are not coherent with each other for
@@ -624,7 +634,7 @@ __global__ __launch_bounds__(256 * GR, (NT * MT <= 32 && GR == 1 ? 2 : 1)) void 
   }
 
   const OutView out = out_view(seg, y, bias, n_blk + wn * TN * 32, N);
-  wave_tile_store<TN, TM, packed_lds_alloc(kBlocks, NV, RING, TN * 32, TM * 32, GR), NW>(
+  wave_tile_store<TN, TM, packed_lds_alloc(kBlocks, NV, RING, TN * 32, TM * 32, GR, NW), NW>(
       acc, smem_all, out.y, out.bias, alpha_p, out.n0, m_blk + wm * TM * 32, wave, lane, M, out.N, residual);
 }
 
@@ -657,18 +667,18 @@ static int launch_packed(const void* xq, const void* xs, const void* wq, const v
                          const void* bias, void* y, int64_t M, int64_t N, int64_t K, hipStream_t stream,
                          const void* residual, const OutSegments& seg, TileSplit split = TileSplit{},
                          void* workspace = nullptr) {
-  constexpr int kLds = packed_lds_alloc(KW + MT, NV, RING, NT / WN * 32, MT / WM * 32, GR);
+  constexpr int kLds = packed_lds_alloc(KW + MT, NV, RING, NT / WN * 32, MT / WM * 32, GR, WN * WM);
   static_assert(kLds <= 160 * 1024, "more LDS than a CU has");
   const int tiles_m = (int)((M + MT * 32 - 1) / (MT * 32)), tiles_n = (int)((N + NT * 32 - 1) / (NT * 32));
   if (split.ksplit <= 1 || !workspace || NT * MT > 16 || GR > 1) split = TileSplit{1, (int)(K / 256)};
-  if (GR > 1) {   // the two groups of a workgroup take one half of K each (the caller checked that K / 256 is even)
+  if (GR > 1) {   // the groups of a workgroup take equal parts of K (the caller checked that K / 256 divides)
     if ((K / 256) % GR != 0) return FPQ_E_UNSUPPORTED;
     split.bps = (int)(K / 256) / GR;
   }
   static LdsLimitOnce lds_limit;
   if (const int st = lds_limit.ensure((const void*)gemm_fp4_packed_kernel<NT, KW, MT, WN, WM, NV, RING, GR>, kLds)) return st;
   hipLaunchKernelGGL((gemm_fp4_packed_kernel<NT, KW, MT, WN, WM, NV, RING, GR>),
-                     dim3((unsigned)(tiles_m * tiles_n), (unsigned)split.ksplit), dim3(256 * GR), kLds, stream,
+                     dim3((unsigned)(tiles_m * tiles_n), (unsigned)split.ksplit), dim3(64 * WN * WM * GR), kLds, stream,
                      (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws, alpha,
                      (const uint16_t*)bias, (uint16_t*)y, (int)M, (int)N, (int)K, tiles_m,
                      (const uint16_t*)residual, seg, split.ksplit, split.bps,
@@ -707,7 +717,7 @@ struct TilePlan {
   int64_t tiles;
   int64_t part_bytes;
   TileSplit split;
-  int groups;        // 2: workgroups of eight waves, K halved inside the workgroup (no K split across workgroups then)
+  int groups;        // 2, 4: workgroups of eight waves, K in parts inside the workgroup (no K split across workgroups then)
 };
 template <bool NV>
 static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int cus) {
@@ -754,7 +764,14 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_byt
   // workgroups through the caller's workspace: 61.1 / 65.3).  MXFP4, whose waves wait on what the CU receives
   // from the L2, measured the same with 64 x 128 tiles and 8 % slower with 128 x 128: it keeps four waves.
   if (NV && plan.tiles <= cus && (K / 256) % 2 == 0 && K >= 2048) {
-    plan.groups = 2;
+    // Four groups of two waves, a quarter of K each, where K divides: the same eight waves with tiles of 64 x 64 (128 x 64)
+    // instead of 32 x 64 (64 x 64).  A wave converts TN + TM operand tiles for TN x TM matrix instructions, and the
+    // conversions bound these kernels (offsetting the two groups' barriers so that one converts while the other
+    // multiplies changed nothing): 1 instead of 1.5 per matrix instruction (0.75 instead of 1).  Weights from HBM, us:
+    // N = 4096: K = 12288, 512 / 384 rows 67.9 / 60.5 -> 53.0 / 46.9, K = 4096, 300 / 512 rows 22.4 / 22.8 -> 19.4 / 19.8;
+    // N = 8192, K = 8192, 256 rows 40.6 -> 33.9; 128 x 128 tiles: N = 8192, K = 6144, 512 rows 46.2 -> 43.3, N = 4096,
+    // K = 12288, 768 rows 80.0 -> 69.5.  No shape measured slower; two groups stay for a K that is no multiple of 1024.
+    plan.groups = (K / 256) % 4 == 0 ? 4 : 2;
     return plan;
   }
   // (NVFP4 beyond the 256 rows that two passes of the weight-streaming kernel serve better)
@@ -857,9 +874,10 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
     // kernels halve K inside their workgroups they take 23 us for K = 4096 at any of these row counts and the
     // two passes are ahead up to 192 rows only (weights from HBM; N = 6144: 144 rows 22.5 two passes / 25.8 us
     // tiles, 192 rows 23.7 / 23.6, 224 rows 26.7 / 23.5, 256 rows 28.7 / 22.9; N = 8192, K = 8192: 35.7 / 43.4,
-    // 39.5 / 42.6, 45.5 / 43.1, 49.7 / 42.8).
+    // 39.5 / 42.6, 45.5 / 43.1, 49.7 / 42.8); with K in quarters the tiles are ahead from 129 rows on (N = 6144 20.2 / 19.1,
+    // 192 rows 22.6 / 18.6; N = 8192, K = 8192 33.1 / 32.8, 39.0 / 32.8; N = 5120, K = 2048 12.5 / 11.7).
     const int64_t half = ((M + 1) / 2 + 31) / 32 * 32;   // rows of the first pass, whole 32-row tiles
-    const int64_t two_pass_rows = plan.groups == 2 ? 192 : 2 * FPQ_NV_STREAM_ROWS;
+    const int64_t two_pass_rows = plan.groups == 4 ? 0 : plan.groups == 2 ? 192 : 2 * FPQ_NV_STREAM_ROWS;
     if (!tile_splits && M > FPQ_NV_STREAM_ROWS && M <= two_pass_rows && (N + 31) / 32 <= cus &&
         stream_eligible(true, half, N, K)) {
       // (both passes may split K through the caller's workspace: they run one after the other on the stream)
@@ -880,6 +898,12 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
   // (K = 12288: 69 instead of 97 us) and 4-7 % less for MXFP4; with more tiles they measured 14 % slower.
   // Either of these two kernels splits K through the caller's workspace where that fills the CUs (tile_split_plan).
   if constexpr (NV) {
+    if (plan.groups == 4 && plan.kind == 0)
+      return launch_packed<2, 2, 4, 1, 2, true, 4, 4>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
+                                                      residual, seg);
+    if (plan.groups == 4 && plan.kind == 1)
+      return launch_packed<4, 4, 4, 1, 2, true, 4, 4>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
+                                                      residual, seg);
     if (plan.groups == 2 && plan.kind == 0)
       return launch_packed<2, 4, 4, 2, 2, true, kRing, 2>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
                                                           residual, seg);
