@@ -22,6 +22,7 @@
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/InferenceMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -239,6 +240,7 @@ bool plain_call(const at::Tensor& x, Call& call, at::ScalarType type = at::kBFlo
       x.requires_grad() || (x.is_inference() && !c10::InferenceMode::is_enabled()))
     return false;
   if (at::impl::PythonTorchFunctionTLS::stack_len() > 0 || c10::impl::TorchDispatchModeTLS::stack_len() > 0) return false;
+  if (c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::Tracer)) return false;   // (torch.jit.trace)
   call.dev = x.device().index();
   if (c10::hip::current_device() != call.dev) return false;
   call.stream = c10::hip::getCurrentHIPStream(call.dev).stream();

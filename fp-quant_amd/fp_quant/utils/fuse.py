@@ -66,12 +66,17 @@ def _host():
     return _host_module
 
 
+class _NotBuilt:
+    """Stands for the native host path where nothing is built: it answers no call."""
+    rmsnorm = group = gated_down = staticmethod(lambda *args: None)
+
+
 def _native():
     """The native host path: each of its functions gives None (False: for want of a plan) for a call that is not the
     plain eager one."""
     global _native_module
     if _native_module is None:
-        _native_module = _host().native
+        _native_module = _host().native or _NotBuilt
     return _native_module
 
 

@@ -279,3 +279,17 @@ def test_fused_block_after_a_weight_changes():
         check()
         block.input_layernorm.weight.mul_(0.5)
         check()
+
+
+def test_operators_are_recorded_by_a_jit_trace():
+    x, other = (torch.randn(64, 512, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    layer = _layer("nvfp4", g=16, k=512)
+    h, scale = layer.forward_hadamard_matrix, layer.act_global_scale.float()
+
+    def quantize(v):
+        return hip_ops.fused_quantize_nv_op(v, h, scale)
+
+    quantize(x)
+    traced = torch.jit.trace(quantize, (x,), check_trace=False)
+    for got, want in zip(traced(other), quantize(other)):
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))

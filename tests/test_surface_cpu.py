@@ -178,3 +178,29 @@ for what in ("loader", "module", "standin"):
     assert r.returncode == 0, r.stderr[-2000:]
     lines = dict(l.split(" ", 1) for l in r.stdout.strip().splitlines())
     assert lines == {"loader": "FPQEngineError", "module": "ValueError", "standin": "FPQEngineError"}, r.stdout
+
+
+def test_fused_norm_on_the_cpu_needs_no_library(monkeypatch):
+    from fp_quant.module import host
+    from fp_quant.utils import fuse
+
+    class LlamaRMSNorm(nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.weight = nn.Parameter(torch.ones(64))
+            self.variance_epsilon = 1e-6
+
+        def forward(self, hidden_states):
+            x = hidden_states.float()
+            return self.weight * (x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + self.variance_epsilon)).to(hidden_states.dtype)
+
+    layer = FPQuantLinear(64, 32, FPQuantConfig(forward_dtype=FPQuantDtype.MXFP4, forward_method="abs_max",
+                                                backward_dtype=FPQuantDtype.BF16), bias=False)
+    layer.qweight = nn.Parameter(torch.zeros(32, 32, dtype=torch.uint8), requires_grad=False)
+    layer.scales = nn.Parameter(torch.zeros(32, 2, dtype=torch.uint8), requires_grad=False)
+    norm, x = LlamaRMSNorm(), torch.randn(3, 64)
+    want = norm(x)
+    assert fuse.fuse_rmsnorm(norm, layer)
+    monkeypatch.setattr(host, "native", None)   # as where nothing is built
+    monkeypatch.setattr(fuse, "_native_module", None)
+    assert torch.equal(norm(x), want)
