@@ -546,9 +546,9 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int n = (rtg * NT + i) * 32 + 8 * wave + 4 * kh;   // bias is indexed by the product's column
-      float bv[4];
+      float bv[4];   // (columns past N are not stored: no branch around a load)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) bv[q] = n + q < N ? __uint_as_float((uint32_t)bias[n + q] << 16) : 0.f;
+      for (int q = 0; q < 4; ++q) bv[q] = __uint_as_float((uint32_t)bias[min(n + q, N - 1)] << 16);
 #pragma unroll
       for (int j = 0; j < MT; ++j) {
         const v4f& t = sum[i * MT + j];
