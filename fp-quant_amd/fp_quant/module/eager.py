@@ -450,7 +450,8 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
     """The WeightGroup of `members` = [(qweight, scales, bias or None, in_features), ...] (one format, same K,
     every N a multiple of 32, biases all absent or all contiguous bf16; weights row-major, or all in the packed
     layout only), remembered on the first member's qweight until a member is written to; built now if
-    `create`, else None when there is none.  A group built in place of an outdated one of the same shape
+    `create` and no graph is being captured (its buffers would hold nothing until a replay), else None when
+    there is none.  A group built in place of an outdated one of the same shape
     (`previous`, or the one remembered) is written into that one's buffers, so that the addresses a recorded
     graph holds stay those of the current weights."""
     first = members[0][0]
@@ -460,7 +461,7 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
         return hit
     if previous is None:
         previous = hit
-    if not create or not packed_weights_enabled():
+    if not create or not packed_weights_enabled() or torch.cuda.is_current_stream_capturing():
         return None
     k = members[0][3]
     sgroup = 16 if nvfp4 else 32
@@ -491,8 +492,8 @@ def weight_group(members, create: bool = False, nvfp4: bool = False,
     group.n, group.splits, group.k, group.nvfp4 = n, splits, k, nvfp4
     scales_bytes = lib.fpq_packed_scales_bytes_nv if nvfp4 else lib.fpq_packed_scales_bytes
     reuse = previous
-    if (reuse is not None and (reuse.nvfp4 != nvfp4 or reuse.k != k or reuse.splits != splits or reuse.wp.device != dev
-                               or torch.cuda.is_current_stream_capturing())):
+    if (reuse is not None
+            and (reuse.nvfp4 != nvfp4 or reuse.k != k or reuse.splits != splits or reuse.wp.device != dev)):
         reuse = None
     with on_device(dev):
         stream = _current_stream(dev.index)

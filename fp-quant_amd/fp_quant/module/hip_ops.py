@@ -428,16 +428,22 @@ def packed_weight(wq: torch.Tensor, ws: torch.Tensor, nvfp4: bool = False, into=
     """Packed copy of a weight, cached on the code tensor until either tensor is written to (a weight
     held in the packed layout only is its own packed copy).  A copy that has gone stale is re-packed into the
     buffers it already has, and a new one into `into` = (codes, scales) if those have the right sizes: the
-    addresses a recorded graph holds stay those of the layer's current weight."""
+    addresses a recorded graph holds stay those of the layer's current weight.
+
+    A copy made while a graph is being captured is the graph's own and not remembered: its buffers belong to the
+    graph's memory pool and hold nothing until the graph is replayed."""
     if wq.dim() == 1:
         return wq, ws
     key = _packed_weight_key(wq, ws, nvfp4)
     hit = getattr(wq, "_fpq_packed", None)
     if hit is not None and hit[0] == key:
         return hit[1], hit[2]
-    if hit is not None and into is None and not torch.cuda.is_current_stream_capturing():
+    pack = pack_nvf4 if nvfp4 else pack_mxf4
+    if torch.cuda.is_current_stream_capturing():
+        return pack(wq, ws, wq.shape[0], wq.shape[1] * 2)
+    if hit is not None and into is None:
         into = (hit[1], hit[2])
-    pc, ps = (pack_nvf4 if nvfp4 else pack_mxf4)(wq, ws, wq.shape[0], wq.shape[1] * 2, into)
+    pc, ps = pack(wq, ws, wq.shape[0], wq.shape[1] * 2, into)
     try:
         wq._fpq_packed = (key, pc, ps)
     except (AttributeError, RuntimeError):

@@ -430,12 +430,15 @@ def _native_group(group, layers, x: torch.Tensor):
 def _eager_group_linear(owner: nn.Module, layers, x: torch.Tensor):
     """Eager counterpart of _group_linear for layers with a WeightGroup: one GEMM (the quantized form of
     `x` is taken from, or left in, the sharing slot); None if there is no group.  The group kept on
-    `owner` is checked against the layers' tensors as they are now and rebuilt if they were written to."""
+    `owner` is checked against the layers' tensors as they are now and rebuilt if they were written to (not
+    while a graph is being captured: the layers are then called one by one)."""
     group = getattr(owner, "_fpq_weight_group", None)
     if group is None:
         return None
     first = layers[0]
     if group.key != tuple(_eager()._member_key(l.qweight, l.scales, l.bias) for l in layers):
+        if torch.cuda.is_current_stream_capturing():
+            return None
         group = owner._fpq_weight_group = _weight_group(layers, create=True, previous=group)
         if group is None:
             return None

@@ -293,3 +293,37 @@ def test_operators_are_recorded_by_a_jit_trace():
     traced = torch.jit.trace(quantize, (x,), check_trace=False)
     for got, want in zip(traced(other), quantize(other)):
         assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
+def test_group_of_a_rewritten_weight_is_not_rebuilt_inside_a_capture():
+    """A member written to, then the block recorded: calls outside the graph find no half-made group, and later ones
+    rebuild it."""
+    from perf.cases import Block
+    from fp_quant.utils import fuse_producers
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    block = Block(dict(fmt="mxfp4", g=64, hidden=512, kv=256, inter=768), gen)
+    assert fuse_producers(block)
+    x = torch.randn(1, 5, 512, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        block(x), block(x)
+        block.self_attn.k_proj.qweight.bitwise_xor_(7)
+        block.mlp.gate_proj.qweight.bitwise_xor_(5)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            cache = []
+            outs = [block(x, cache=cache), *cache[0]]
+        assert block.self_attn._fpq_weight_group is not None and block.mlp._fpq_weight_group is not None
+        for i in range(3):
+            cache = []
+            want = [block(x, cache=cache), *cache[0]]
+            if i:   # (the first call comes before any replay)
+                graph.replay()
+                torch.cuda.synchronize()
+                for a, b in zip(outs, want):
+                    assert torch.equal(a, b)
+        assert block.self_attn._fpq_weight_group.key == tuple(
+            eager._member_key(l.qweight, l.scales, l.bias)
+            for l in (block.self_attn.q_proj, block.self_attn.k_proj, block.self_attn.v_proj))
+    twin = copy.deepcopy(block.self_attn.k_proj)
+    assert torch.equal(twin(x), block.self_attn.k_proj(x))

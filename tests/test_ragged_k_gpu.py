@@ -5,7 +5,7 @@ import torch
 
 import fp_quant
 from fp_quant import _engine
-from fp_quant.module import hip_ops
+from fp_quant.module import eager, hip_ops
 from oracle import fpq_oracle as O
 from tests import capi
 from tests.conftest import make_student_t, needs_packed
@@ -112,3 +112,39 @@ def test_layer_matches_the_oracle(fmt, method, init, g, m, k, n):
     want = ref + bias.double()
     tol = 2.0 ** -8 * ref.abs() + 1e-5 * mag + 2.0 ** -8 * want.abs() + 1e-6
     assert ((y.cpu().double() - want).abs() <= tol).all()
+
+
+# (K = 512: a whole number of blocks)
+@needs_packed
+@pytest.mark.parametrize("fmt,g", [("mxfp4", 128), ("nvfp4", 16)])
+@pytest.mark.parametrize("k", [640, 512])
+def test_packed_weights_made_inside_a_capture_stay_there(fmt, g, k, monkeypatch):
+    """A layer whose first call is recorded into a graph: what the recording packs is not there before a replay, so
+    calls outside the graph pack for themselves; replays follow the row-major weight."""
+    monkeypatch.setattr(eager, "SHARE_ACT_QUANT", False)   # (NVFP4 reads the activation scale on the host to share)
+    cfg = fp_quant.FPQuantConfig(forward_dtype=fp_quant.FPQuantDtype(fmt), forward_method="abs_max",
+                                 backward_dtype=fp_quant.FPQuantDtype.BF16, hadamard_group_size=g)
+
+    def layer(seed):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        out = fp_quant.FPQuantLinear(k, 288, cfg, bias=False, device="cuda", dtype=torch.bfloat16)
+        out.weight.data = torch.randn(288, k, generator=gen, device="cuda", dtype=torch.bfloat16)
+        out.pre_forward()
+        return out
+
+    captured, x = layer(1), torch.randn(4, k, device="cuda", dtype=torch.bfloat16)
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad():
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            y = captured(x)
+        want = layer(1)(x)
+        assert torch.equal(captured(x), want)
+        for seed in (1, 2, 2):
+            if captured.qweight.dim() == 2:
+                captured.qweight.copy_(layer(seed).qweight)
+                captured.scales.copy_(layer(seed).scales)
+                want = layer(seed)(x)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want) and torch.equal(captured(x), want)
