@@ -8,11 +8,10 @@
 
 namespace fpq {
 
-// Raises a kernel's dynamic-LDS limit once per device (the attribute is per device; one
-// function-local static instance per kernel lives in the launcher).  Safe from any host thread: a
-// race only repeats the idempotent call.
 int device_cus();   // fpq_capi.hip: compute units of the current device (256 where none answers)
 
+// Raises a kernel's dynamic-LDS limit once per device (the attribute is per device; one static instance per kernel
+// lives in the launcher, or in raise_lds_limit).  Safe from any host thread: a race only repeats the idempotent call.
 struct LdsLimitOnce {
   std::atomic<uint64_t> done{0};  // bit d: set for device d (devices >= 64 set it on every call)
   int ensure(const void* kernel, int bytes) {
@@ -26,6 +25,18 @@ struct LdsLimitOnce {
     if (bit) done.fetch_or(bit, std::memory_order_release);
     return 0;
   }
+};
+
+// ... for a launcher that serves several kernels: the kernel is a template argument, since kernels with the same
+// parameters have one type, and a static keyed by that type would be raised for the first of them only.
+template <auto Kernel>
+int raise_lds_limit(int bytes) {
+  static LdsLimitOnce limit;
+  return limit.ensure((const void*)Kernel, bytes);
+}
+template <auto Kernel>
+struct KernelTag {
+  static constexpr auto kernel = Kernel;
 };
 
 // Which output tile a workgroup of a large-M kernel computes, and its number in the tile list (returned).

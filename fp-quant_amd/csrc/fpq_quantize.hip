@@ -781,19 +781,19 @@ static int launch_stream_packed(const void* x, int64_t rows, int64_t cols, float
   // kProRmsNorm: one more tile per wave, in which the bf16 by-product is regrouped into row segments
   constexpr int kDyn = PRO == kProRmsNorm ? 4 * 64 * 128 : 0;
   int status = 0;
-  auto go = [&](auto kernel) {
+  auto go = [&](auto tag) {
+    constexpr auto kernel = decltype(tag)::kernel;
     if (kDyn) {
-      static LdsLimitOnce limit;
-      if ((status = limit.ensure((const void*)kernel, kDyn)) != 0) return;
+      if ((status = raise_lds_limit<kernel>(kDyn)) != 0) return;
     }
     hipLaunchKernelGGL(kernel, grid, block, kDyn, stream, (const uint8_t*)x, (uint8_t*)codes,
                        (uint8_t*)scales, (uint32_t)(rows * cols / EPL), (uint32_t)(cols / EPL),
                        (uint32_t)rows, 0u, 0u, norm, gsp, pro);
   };
   if (zero_policy == FPQ_ZERO_REFERENCE) {
-    go(quantize_stream_kernel<EPL, G, FMT, ROT, kZeroReference, true, PRO, QUEST>);
+    go(KernelTag<quantize_stream_kernel<EPL, G, FMT, ROT, kZeroReference, true, PRO, QUEST>>{});
   } else {
-    go(quantize_stream_kernel<EPL, G, FMT, ROT, kZeroSigned, true, PRO, QUEST>);
+    go(KernelTag<quantize_stream_kernel<EPL, G, FMT, ROT, kZeroSigned, true, PRO, QUEST>>{});
   }
   if (status) return status;
   return (int)hipGetLastError();
@@ -2013,18 +2013,18 @@ static int dispatch_rmsnorm_tile(const void* x, int64_t ld, const void* weight, 
   const int64_t padded = (rows + 31) / 32 * 32;
   const int lds = (int)(kTileRows * cols * 2);
   int status = 0;
-  auto go = [&](auto kernel) {
-    static LdsLimitOnce limit;
-    if ((status = limit.ensure((const void*)kernel, (int)(kTileRows * kTileKernelMaxCols * 2))) != 0) return;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(padded / kTileRows)), dim3(64 * kTileRows), lds, stream, (const uint4*)x, (uint8_t*)codes,
-                       (uint8_t*)scales, (uint32_t)rows, norm, (float)cols, eps, inv_rms, gsp, pro);
+  auto go = [&](auto tag) {
+    constexpr auto kernel = decltype(tag)::kernel;
+    if ((status = raise_lds_limit<kernel>((int)(kTileRows * kTileKernelMaxCols * 2))) != 0) return;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(padded / kTileRows)), dim3(64 * kTileRows), lds, stream, (const uint4*)x,
+                       (uint8_t*)codes, (uint8_t*)scales, (uint32_t)rows, norm, (float)cols, eps, inv_rms, gsp, pro);
     status = (int)hipGetLastError();
   };
 #define FPQ_LAUNCH_TILE_Z(GG, RR, ZZ)                                                       \
   {                                                                                         \
-    if (cols <= 4096) go(rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 8>);                 \
-    else if (cols <= 8192) go(rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 16>);           \
-    else go(rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 32>);                             \
+    if (cols <= 4096) go(KernelTag<rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 8>>{});    \
+    else if (cols <= 8192) go(KernelTag<rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 16>>{}); \
+    else go(KernelTag<rmsnorm_tile_quantize_kernel<GG, FMT, RR, ZZ, 32>>{});                \
     return status;                                                                          \
   }
 #define FPQ_LAUNCH_TILE(GG, RR)                                                             \
