@@ -155,7 +155,7 @@ struct GroupPlan {
     PyObject* alpha_obj;
     at::Tensor wp, wsp, alpha, bias;
     int64_t k, kp;
-    bool nvfp4;
+    bool nvfp4, usable;
   }* b;
 };
 
@@ -679,12 +679,13 @@ PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     if (!module_tensors(layer, t)) Py_RETURN_NONE;
     if (!p->members[3 * i].is(t.qweight) || !p->members[3 * i + 1].is(t.scales) || !p->members[3 * i + 2].is(t.bias))
       Py_RETURN_FALSE;
-    if (i == 0) {
+    if (i == 0 && p->usable) {
       if (!p->wgs.is(t.wgs) || !p->ags.is(t.ags) || !is_alpha(t.wgs, p->alpha_obj)) Py_RETURN_FALSE;
       h = THPObjectPtr(Py_NewRef(t.h));
       first_ags = t.ags;
     }
   }
+  if (!p->usable) Py_RETURN_NONE;
   const at::Tensor x = *xp;
   const int64_t k = x.size(-1), m = x.numel() / k;
   QuantPlan::Body* q = quant_plan(h.get(), first_ags, p->nvfp4);
@@ -1008,14 +1009,15 @@ PyObject* host_linear_plan(PyObject*, PyObject* args) {
   return o.release();
   END_HANDLE_TH_ERRORS
 }
-// group_plan(members, splits, wgs, ags, alpha, wp, wsp, bias, k, nvfp4) -> plan or None
+// group_plan(members, splits, wgs, ags, alpha, wp, wsp, bias, k, nvfp4, usable) -> plan or None; not usable: a marker for
+// these members
 PyObject* host_group_plan(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
   PyObject *members, *splits, *wgs, *ags, *alpha, *wp, *wsp, *bias;
   long long k;
-  int nvfp4;
-  if (!PyArg_ParseTuple(args, "O!O!OOOOOOLp", &PyTuple_Type, &members, &PyTuple_Type, &splits, &wgs, &ags, &alpha, &wp, &wsp,
-                        &bias, &k, &nvfp4))
+  int nvfp4, usable;
+  if (!PyArg_ParseTuple(args, "O!O!OOOOOOLpp", &PyTuple_Type, &members, &PyTuple_Type, &splits, &wgs, &ags, &alpha, &wp, &wsp,
+                        &bias, &k, &nvfp4, &usable))
     return nullptr;
   THPObjectPtr o(plan_new<GroupPlan>(&GroupPlanType, nullptr, nullptr));
   if (!o) return nullptr;
@@ -1026,6 +1028,8 @@ PyObject* host_group_plan(PyObject*, PyObject* args) {
     b->members.emplace_back();
     if (!b->members.back().take(PyTuple_GET_ITEM(members, i), false)) Py_RETURN_NONE;
   }
+  b->usable = usable;
+  if (!usable) return o.release();
   int64_t n = 0;
   for (Py_ssize_t i = 0; i < count; ++i) {
     const long long s = PyLong_AsLongLong(PyTuple_GET_ITEM(splits, i));

@@ -2,7 +2,7 @@
 handed to native code that repeats the call without the interpreter.  A plan hangs on the tensor it describes
 (`_fpq_qplan` on a rotation, `_fpq_plan` on a layer's codes, `plan` of a WeightGroup), names the tensors it was made
 from, and is compared with them on every call.  Plans are made outside tracing and captures, by the first call that
-could have used them; a layer that the native path cannot serve gets a marker, so that it is not asked again."""
+could have used them; a layer or group that the native path cannot serve gets a marker, so that it is not asked again."""
 import torch
 
 from .. import _engine
@@ -87,9 +87,10 @@ def learn_group(group, layers) -> None:
     if group.plan_key == key:
         return
     group.plan = None
-    if len(layers) <= 4 and all(n % 256 == 0 for n in group.splits):
-        members = tuple(t for l in layers for t in (l.qweight, l.scales, l.bias))
-        if _plain(*(t for t in members if t is not None)):
-            group.plan = native.group_plan(members, tuple(group.splits), wgs, ags, alpha, group.wp, group.wsp, group.bias,
-                                           group.k, group.nvfp4)
+    members = tuple(t for l in layers for t in (l.qweight, l.scales, l.bias))
+    if len(layers) <= 4 and _plain(*(t for t in members if t is not None)):
+        # (a matrix of its own per layer needs whole 256-column tiles)
+        args = (members, tuple(group.splits), wgs, ags, alpha, group.wp, group.wsp, group.bias, group.k, group.nvfp4)
+        group.plan = (native.group_plan(*args, all(n % 256 == 0 for n in group.splits))
+                      or native.group_plan(*args, False))
     group.plan_key = key

@@ -327,3 +327,25 @@ def test_group_of_a_rewritten_weight_is_not_rebuilt_inside_a_capture():
             for l in (block.self_attn.q_proj, block.self_attn.k_proj, block.self_attn.v_proj))
     twin = copy.deepcopy(block.self_attn.k_proj)
     assert torch.equal(twin(x), block.self_attn.k_proj(x))
+
+
+@pytest.mark.parametrize("kv,fmt,g", [(128, "mxfp4", 64), (384, "mxfp4", 128), (128, "nvfp4", 16)])
+def test_a_group_that_native_code_cannot_serve_is_asked_about_once(kv, fmt, g, monkeypatch):
+    """Projections whose widths are no multiple of 256 share one output matrix, which only the Python path lays out."""
+    from perf.cases import Block
+    from fp_quant.utils import fuse_producers
+    block = Block(dict(fmt=fmt, g=g, hidden=512, kv=kv, inter=768), torch.Generator(device="cuda").manual_seed(7))
+    assert fuse_producers(block)
+    learned, learn = [], host.learn_group
+    monkeypatch.setattr(host, "learn_group", lambda group, layers: (learned.append(group), learn(group, layers)))
+    x = torch.randn(1, 5, 512, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        block(x)
+        for _ in range(4):
+            block(x)
+        qkv = block.self_attn._fpq_weight_group
+        assert qkv is not None and sum(g is qkv for g in learned) <= 1
+        block.self_attn.k_proj.qweight.bitwise_xor_(7)   # (another group now)
+        for _ in range(4):
+            block(x)
+        assert len(learned) <= 4
