@@ -426,6 +426,22 @@ bool module_tensors(PyObject* module, LayerTensors& t) {
   return module_dicts(module, &params, &buffers) && layer_tensors(params, buffers, t);
 }
 
+// What to answer for want of a plan: False (one may be made), or None where a tensor cannot be in one -- an inference
+// tensor has no modification counter, a subclass may be more than its data.
+bool may_be_planned(PyObject* o) {
+  const at::Tensor* t = tensor_of(o);
+  return t && plain_cuda(*t) && !t->is_inference();
+}
+PyObject* no_plan(const LayerTensors& t) {
+  for (PyObject* o : {t.qweight, t.scales, t.wgs, t.ags, t.h})
+    if (!may_be_planned(o)) Py_RETURN_NONE;
+  if (t.bias && t.bias != Py_None && !may_be_planned(t.bias)) Py_RETURN_NONE;
+  Py_RETURN_FALSE;
+}
+PyObject* no_quant_plan(PyObject* h, PyObject* ags) {
+  return Py_NewRef(may_be_planned(h) && may_be_planned(ags) ? Py_False : Py_None);
+}
+
 LinearPlan::Body* linear_plan(const LayerTensors& t) {   // whatever is current, usable or not
   PyObject* p = attribute(t.qweight, s_plan);
   if (!p || Py_TYPE(p) != &LinearPlanType) return nullptr;
@@ -563,7 +579,7 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   QuantPlan::Body* q = quant_plan(t.h, t.ags, nvfp4);
   const at::Tensor* residual;
   if (!p && !packed_weights_enabled()) Py_RETURN_NONE;
-  if (!p || !q) Py_RETURN_FALSE;
+  if (!p || !q) return no_plan(t);
   if (x.dim() < 2 || !serves(p, nvfp4, m, k) || !q->usable || tensor_of(t.qweight)->device().index() != call.dev ||
       !residual_of(args[2], m, p->n, call, &residual))
     Py_RETURN_NONE;
@@ -611,7 +627,7 @@ PyObject* host_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     Py_RETURN_NONE;
   QuantPlan::Body* q = quant_plan(t.h, t.ags, nvfp4);
   // (fused producers take Hadamard (0) and identity (1) rotations)
-  if (!q) Py_RETURN_FALSE;
+  if (!q) return no_quant_plan(t.h, t.ags);
   if (!q->usable || q->kind > 1 || cols % (q->g > 32 ? q->g : 32) != 0) Py_RETURN_NONE;
   const bool few = rows <= 64 && cols % 256 == 0;
   const int entry = few ? (nvfp4 ? E_fpq_rmsnorm_rows_quantize_nv_packed : E_fpq_rmsnorm_rows_quantize_mx_packed)
@@ -662,7 +678,15 @@ PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (Py_TYPE(args[0]) != &GroupPlanType) {   // no plan yet, if the call is a plain one
     const at::Tensor* t = tensor_of(args[2]);
     Call c;
-    return t && plain_call(*t, c) ? Py_NewRef(Py_False) : Py_NewRef(Py_None);
+    if (!t || !plain_call(*t, c)) Py_RETURN_NONE;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args[1]); ++i) {
+      LayerTensors l;
+      if (!module_tensors(PyTuple_GET_ITEM(args[1], i), l)) Py_RETURN_NONE;
+      PyObject* answer = no_plan(l);
+      if (answer == Py_None) return answer;
+      Py_DECREF(answer);
+    }
+    Py_RETURN_FALSE;
   }
   const THPObjectPtr hold(Py_NewRef(args[0]));
   auto* p = ((GroupPlan*)args[0])->b;
@@ -678,9 +702,9 @@ PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     LayerTensors t;
     if (!module_tensors(layer, t)) Py_RETURN_NONE;
     if (!p->members[3 * i].is(t.qweight) || !p->members[3 * i + 1].is(t.scales) || !p->members[3 * i + 2].is(t.bias))
-      Py_RETURN_FALSE;
+      return no_plan(t);
     if (i == 0 && p->usable) {
-      if (!p->wgs.is(t.wgs) || !p->ags.is(t.ags) || !is_alpha(t.wgs, p->alpha_obj)) Py_RETURN_FALSE;
+      if (!p->wgs.is(t.wgs) || !p->ags.is(t.ags) || !is_alpha(t.wgs, p->alpha_obj)) return no_plan(t);
       h = THPObjectPtr(Py_NewRef(t.h));
       first_ags = t.ags;
     }
@@ -690,7 +714,7 @@ PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   const int64_t k = x.size(-1), m = x.numel() / k;
   QuantPlan::Body* q = quant_plan(h.get(), first_ags, p->nvfp4);
   const int entry = p->nvfp4 ? E_fpq_gemm_nvf4_packed_multi : E_fpq_gemm_mxf4_packed_multi;
-  if (!q) Py_RETURN_FALSE;
+  if (!q) return no_quant_plan(h.get(), first_ags);
   if (!q->usable || k != p->k || x.dim() < 2 || p->wp.device().index() != call.dev || !plain_entry(entry)) Py_RETURN_NONE;
   const THPObjectPtr hold_q(Py_NewRef(attribute(h.get(), s_qplan)));
   Packed packed;
@@ -737,7 +761,7 @@ PyObject* host_gated_down(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   LinearPlan::Body* p = linear_plan(t);
   QuantPlan::Body* q = quant_plan(t.h, t.ags, nvfp4);
   const at::Tensor* residual;
-  if (!p || !q) Py_RETURN_FALSE;
+  if (!p || !q) return no_plan(t);
   if (!serves(p, nvfp4, m, k) || !q->usable || q->kind > 1 || k % (q->g > 32 ? q->g : 32) != 0 || !packed_weights_enabled() ||
       ((uintptr_t)gate.const_data_ptr() & 15) || ((uintptr_t)u.const_data_ptr() & 15) ||
       tensor_of(t.qweight)->device().index() != call.dev || !residual_of(args[3], m, p->n, call, &residual))

@@ -2,7 +2,8 @@
 handed to native code that repeats the call without the interpreter.  A plan hangs on the tensor it describes
 (`_fpq_qplan` on a rotation, `_fpq_plan` on a layer's codes, `plan` of a WeightGroup), names the tensors it was made
 from, and is compared with them on every call.  Plans are made outside tracing and captures, by the first call that
-could have used them; a layer or group that the native path cannot serve gets a marker, so that it is not asked again."""
+could have used them; a layer or group that the native path cannot serve gets a marker, so that it is not asked again.
+(Native code declines by itself where a tensor cannot be in a plan: inference tensors, tensor subclasses.)"""
 import torch
 
 from .. import _engine
@@ -37,7 +38,8 @@ def learn_quant(h, act_global_scale, nvfp4: bool) -> None:
             gs_host = cached_on(act_global_scale, "_fpq_host",
                                 (hip_ops._version(act_global_scale), act_global_scale.data_ptr()),
                                 lambda: float(act_global_scale))
-    h._fpq_qplan = native.quant_plan(h, act_global_scale, nvfp4, kind, norm, g, gs, rot, gs_host)
+    plan = native.quant_plan(h, act_global_scale, nvfp4, kind, norm, g, gs, rot, gs_host)
+    h._fpq_qplan = plan or native.quant_plan(h, act_global_scale, nvfp4, -1, norm, g, None, rot, None)
 
 
 def learn_linear(layer) -> None:
@@ -68,10 +70,10 @@ def learn_linear(layer) -> None:
             packed = q._fpq_packed
     alpha = linear_alpha(wgs, ags)
     need = hip_ops.splitk_need(n, k, nvfp4) if usable else 0
-    q._fpq_plan = native.linear_plan(
-        q, s, wgs, ags, bias, alpha, None if packed_only else packed, n, k, need,
-        hip_ops.SPLIT_K_MAX_ROWS if nvfp4 else hip_ops.SPLIT_K_ROWS,
-        hip_ops.NV_PACKED_LINEAR_MIN_M if nvfp4 else hip_ops.PACKED_LINEAR_MIN_M, nvfp4, packed_only, usable)
+    args = (q, s, wgs, ags, bias, alpha, None if packed_only else packed, n, k, need,
+            hip_ops.SPLIT_K_MAX_ROWS if nvfp4 else hip_ops.SPLIT_K_ROWS,
+            hip_ops.NV_PACKED_LINEAR_MIN_M if nvfp4 else hip_ops.PACKED_LINEAR_MIN_M, nvfp4, packed_only)
+    q._fpq_plan = native.linear_plan(*args, usable) or native.linear_plan(*args, False)
 
 
 def learn_group(group, layers) -> None:

@@ -349,3 +349,33 @@ def test_a_group_that_native_code_cannot_serve_is_asked_about_once(kv, fmt, g, m
         for _ in range(4):
             block(x)
         assert len(learned) <= 4
+
+
+def test_weights_that_cannot_be_in_a_plan_are_not_asked_about(native, monkeypatch):
+    """Layers built under inference mode: native code declines at once, and nobody tries to make a plan."""
+    from perf.cases import Block
+    from fp_quant.utils import fuse_producers
+    tried = []
+    for name in ("learn_linear", "learn_quant", "learn_group"):
+        monkeypatch.setattr(host, name, lambda *args, name=name: tried.append(name))
+    with torch.inference_mode():
+        for fmt, g in (("mxfp4", 128), ("nvfp4", 16)):
+            layer = _layer(fmt, g=g, bias=True)
+            for x in (torch.randn(6, 512, device="cuda", dtype=torch.bfloat16), torch.randn(6, 512).cuda().bfloat16()):
+                assert torch.equal(layer(x), _python(layer, x))
+            block = Block(dict(fmt=fmt, g=g, hidden=512, kv=256, inter=768), torch.Generator(device="cuda").manual_seed(8))
+            assert fuse_producers(block)
+            for _ in range(2):
+                block(torch.randn(1, 5, 512, device="cuda", dtype=torch.bfloat16))
+    assert not tried and not native.answered
+
+
+def test_a_layer_whose_plan_is_refused_gets_a_marker(native, monkeypatch):
+    layer = _layer()
+    x = torch.randn(6, 512, device="cuda", dtype=torch.bfloat16)
+    alpha, learned, learn = host.linear_alpha, [], host.learn_linear
+    monkeypatch.setattr(host, "linear_alpha", lambda *args: alpha(*args).expand(2))   # (no scalar: no plan takes it)
+    monkeypatch.setattr(host, "learn_linear", lambda layer: (learned.append(layer), learn(layer)))
+    for _ in range(4):
+        assert torch.equal(layer(x), _python(layer, x))
+    assert len(learned) == 1 and not native.answered
