@@ -71,7 +71,7 @@ PyObject* g_shared;           // device index -> the activations of the latest c
 PyObject* g_workspaces;       // device index -> {stream: workspace} (hip_ops._stream_workspaces)
 PyObject* g_eager_globals;    // eager.SHARE_ACT_QUANT is read from here on every call
 PyTypeObject* g_activations;  // eager.QuantizedActivations
-int g_policy, g_packed_rows_mx, g_packed_rows_nv;
+int g_policy, g_packed_rows_mx, g_packed_rows_nv, g_linear_rows_mx;
 
 PyObject *s_qweight, *s_scales, *s_wgs, *s_ags, *s_h, *s_bias, *s_plan, *s_qplan, *s_alpha, *s_packed, *s_share,
     *s_parameters, *s_buffers, *s_weight, *s_eps, *s_rotation, *s_splitk;
@@ -442,6 +442,12 @@ PyObject* no_quant_plan(PyObject* h, PyObject* ags) {
   return Py_NewRef(may_be_planned(h) && may_be_planned(ags) ? Py_False : Py_None);
 }
 
+// Whether a layer without a plan would run on packed weights, as every plan has it.
+bool may_pack(const LayerTensors& t, bool nvfp4, int64_t m) {
+  const at::Tensor* q = tensor_of(t.qweight);
+  return packed_weights_enabled() && (nvfp4 || m >= g_linear_rows_mx || (q && q->dim() == 1));
+}
+
 LinearPlan::Body* linear_plan(const LayerTensors& t) {   // whatever is current, usable or not
   PyObject* p = attribute(t.qweight, s_plan);
   if (!p || Py_TYPE(p) != &LinearPlanType) return nullptr;
@@ -578,7 +584,7 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   LinearPlan::Body* p = linear_plan(t);
   QuantPlan::Body* q = quant_plan(t.h, t.ags, nvfp4);
   const at::Tensor* residual;
-  if (!p && !packed_weights_enabled()) Py_RETURN_NONE;
+  if (!p && !may_pack(t, nvfp4, m)) Py_RETURN_NONE;
   if (!p || !q) return no_plan(t);
   if (x.dim() < 2 || !serves(p, nvfp4, m, k) || !q->usable || tensor_of(t.qweight)->device().index() != call.dev ||
       !residual_of(args[2], m, p->n, call, &residual))
@@ -761,6 +767,7 @@ PyObject* host_gated_down(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   LinearPlan::Body* p = linear_plan(t);
   QuantPlan::Body* q = quant_plan(t.h, t.ags, nvfp4);
   const at::Tensor* residual;
+  if (!p && !may_pack(t, nvfp4, m)) Py_RETURN_NONE;
   if (!p || !q) return no_plan(t);
   if (!serves(p, nvfp4, m, k) || !q->usable || q->kind > 1 || k % (q->g > 32 ? q->g : 32) != 0 || !packed_weights_enabled() ||
       ((uintptr_t)gate.const_data_ptr() & 15) || ((uintptr_t)u.const_data_ptr() & 15) ||
@@ -1078,13 +1085,15 @@ PyObject* host_group_plan(PyObject*, PyObject* args) {
 }
 
 // configure(library path, binding attributes, shared slot, workspaces, eager globals, QuantizedActivations, policy,
-// activation rows from which the MXFP4 and NVFP4 matmul operators re-tile their operands)
+// activation rows from which the MXFP4 and NVFP4 matmul operators re-tile their operands, and from which MXFP4 layers
+// run on packed weights)
 PyObject* host_configure(PyObject*, PyObject* args) {
   const char* path;
   PyObject *binding, *shared, *workspaces, *globals, *type;
   int policy;
-  if (!PyArg_ParseTuple(args, "sO!O!O!O!O!iii", &path, &PyDict_Type, &binding, &PyDict_Type, &shared, &PyDict_Type, &workspaces,
-                        &PyDict_Type, &globals, &PyType_Type, &type, &policy, &g_packed_rows_mx, &g_packed_rows_nv))
+  if (!PyArg_ParseTuple(args, "sO!O!O!O!O!iiii", &path, &PyDict_Type, &binding, &PyDict_Type, &shared, &PyDict_Type, &workspaces,
+                        &PyDict_Type, &globals, &PyType_Type, &type, &policy, &g_packed_rows_mx, &g_packed_rows_nv,
+                        &g_linear_rows_mx))
     return nullptr;
   if (!PyType_IsSubtype((PyTypeObject*)type, &ActivationsType)) {
     PyErr_SetString(PyExc_TypeError, "the activations type must derive from Activations");

@@ -876,7 +876,8 @@ def silu_mul_quantize(gate: torch.Tensor, up: torch.Tensor, hadamard_matrix: tor
 
 
 if _host is not None:
-    from .hip_ops import NV_PACKED_MIN_M, PACKED_MIN_M, _stream_workspaces
+    from .hip_ops import NV_PACKED_MIN_M, PACKED_LINEAR_MIN_M, PACKED_MIN_M, _stream_workspaces
 
     _host.configure(_engine.library_path(), vars(_engine.lib()), _shared_activations, _stream_workspaces, globals(),
-                    QuantizedActivations, ZERO_NIBBLE_POLICY, PACKED_MIN_M, NV_PACKED_MIN_M)
+                    QuantizedActivations, ZERO_NIBBLE_POLICY, PACKED_MIN_M, NV_PACKED_MIN_M,
+                    PACKED_LINEAR_MIN_M)

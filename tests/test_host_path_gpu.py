@@ -379,3 +379,37 @@ def test_a_layer_whose_plan_is_refused_gets_a_marker(native, monkeypatch):
     for _ in range(4):
         assert torch.equal(layer(x), _python(layer, x))
     assert len(learned) == 1 and not native.answered
+
+
+def test_calls_that_stay_on_the_row_major_weight_are_not_asked_about():
+    """Fewer rows than FPQ_PACKED_MIN_ROWS, or FPQ_PACKED_WEIGHTS=0: nobody tries to make a plan."""
+    import os
+    import subprocess
+    import sys
+    code = """
+import sys
+sys.path[:0] = ["fp-quant_amd", "."]
+import torch
+from tests.test_host_path_gpu import _layer, host
+from perf.cases import Block
+from fp_quant.utils import fuse_producers
+tried, learn = [], host.learn_linear
+host.learn_linear = lambda layer: (tried.append(layer), learn(layer))
+layer = _layer()
+block = Block(dict(fmt="mxfp4", g=64, hidden=512, kv=256, inter=768), torch.Generator(device="cuda").manual_seed(7))
+assert fuse_producers(block)
+with torch.no_grad():
+    for m in (4, 4, 4):
+        layer(torch.randn(m, 512, device="cuda", dtype=torch.bfloat16))
+        block(torch.randn(1, m, 512, device="cuda", dtype=torch.bfloat16))
+    assert not tried, len(tried)
+    if len(sys.argv) > 1:   # (rows that run on packed weights: planned after all)
+        x = torch.randn(40, 512, device="cuda", dtype=torch.bfloat16)
+        ys = [layer(x) for _ in range(4)]
+        assert tried and all(torch.equal(y, ys[0]) for y in ys) and host.native.linear_plan_current(layer)
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    for env, args in (({"FPQ_PACKED_MIN_ROWS": "32"}, ["rows"]), ({"FPQ_PACKED_WEIGHTS": "0"}, [])):
+        r = subprocess.run([sys.executable, "-c", code, *args], cwd=root, env={**os.environ, **env}, capture_output=True,
+                           text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
