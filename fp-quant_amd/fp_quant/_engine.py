@@ -93,7 +93,6 @@ def available() -> bool:
     """True if the HIP library is present and loads (says nothing about a GPU being there)."""
     try:
         lib()
-        host()
         return True
     except FPQEngineError:
         return False
@@ -122,29 +121,33 @@ def lib():
     return _lib
 
 
-_host = None
+_host = None   # (False: there is none)
 
 
 def host():
-    """The extension module with the native host path of the eager layers (csrc/fpq_host.cpp)."""
+    """The extension module with the native host path of the eager layers (csrc/fpq_host.cpp), or None, with one warning,
+    where none is built or the one there does not fit the installed PyTorch: the Python path then serves every call."""
     global _host
     if _host is None:
         import importlib.util
+        import warnings
 
         import torch  # noqa: F401  (its libraries have to be there first)
         path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "_fpq_host.so")
         with _lock:
             if _host is None:
-                if not os.path.exists(path):
-                    raise FPQEngineError(f"{path} is missing: build it with `python fp-quant_amd/build.py`")
                 try:
+                    if not os.path.exists(path):
+                        raise ImportError("it is missing")
                     spec = importlib.util.spec_from_file_location("fp_quant._lib._fpq_host", path)
                     module = importlib.util.module_from_spec(spec)
                     spec.loader.exec_module(module)
+                    _host = module
                 except ImportError as exc:
-                    raise FPQEngineError(f"cannot load {path}: {exc}") from exc
-                _host = module
-    return _host
+                    _host = False
+                    warnings.warn(f"{path}: {exc}; eager calls take the slower Python path until "
+                                  "`python fp-quant_amd/build.py` has built it for this PyTorch")
+    return _host or None
 
 
 def check(status: int, what: str) -> None:

@@ -42,7 +42,7 @@ from .hip_ops import (
 )
 
 
-# the native host path (csrc/fpq_host.cpp); None where nothing is built, and every engine call raises
+# the native host path (csrc/fpq_host.cpp); None where it is not built, or nothing is and every engine call raises
 _host = _engine.host() if _engine.available() else None
 
 

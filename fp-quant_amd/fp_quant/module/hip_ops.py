@@ -98,7 +98,7 @@ def _direct(op, native_name: str):
     """`op` (a custom operator) with plain eager calls answered by the native host path, which runs the operator's body
     without the dispatch around it; every other call -- traced, under a mode, with gradients, keywords -- and every
     one that it declines goes through the dispatcher as before."""
-    if not HAS_HIP_ENGINE:
+    if not HAS_HIP_ENGINE or _engine.host() is None:
         return op
     native = getattr(_engine.host(), native_name)
 

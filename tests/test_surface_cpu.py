@@ -180,6 +180,46 @@ for what in ("loader", "module", "standin"):
     assert lines == {"loader": "FPQEngineError", "module": "ValueError", "standin": "FPQEngineError"}, r.stdout
 
 
+@pytest.mark.parametrize("how", ["missing", "of another PyTorch"])
+def test_the_engine_is_there_without_the_native_host_path(how):
+    """The host path only shortens calls: where it is not built, or does not load, one warning says so and the Python path
+    serves the layers."""
+    import os
+    import subprocess
+    import sys
+    from fp_quant import _engine
+    if not os.path.exists(_engine.library_path()):
+        pytest.skip("the library is not built")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = r"""
+import importlib.util, os, sys, warnings
+sys.path.insert(0, sys.argv[1])
+if sys.argv[2] == "missing":
+    exists = os.path.exists
+    os.path.exists = lambda p: not str(p).endswith("_fpq_host.so") and exists(p)
+else:
+    spec = importlib.util.spec_from_file_location
+    def refused(name, *args, **kw):
+        if name.endswith("_fpq_host"):
+            raise ImportError("undefined symbol")
+        return spec(name, *args, **kw)
+    importlib.util.spec_from_file_location = refused
+with warnings.catch_warnings(record=True) as caught:
+    warnings.simplefilter("always")
+    import fp_quant
+    from fp_quant import _engine
+    from fp_quant.module import eager, hip_ops, linear
+assert _engine.available() and hip_ops.HAS_HIP_ENGINE
+assert eager._host is None and not linear._native and eager.QuantizedActivations(1, 32, False).m == 1
+assert sum("_fpq_host.so" in str(w.message) for w in caught) == 1
+fp_quant.FPQuantLinear(64, 32, fp_quant.FPQuantConfig(forward_method="abs_max",
+                       backward_dtype=fp_quant.FPQuantDtype.BF16), device="meta")
+"""
+    r = subprocess.run([sys.executable, "-c", code, os.path.join(root, "fp-quant_amd"), how], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_fused_norm_on_the_cpu_needs_no_library(monkeypatch):
     from fp_quant.module import host
     from fp_quant.utils import fuse
