@@ -395,6 +395,13 @@ bool packed_weights_enabled() {
   return !v || strcmp(v, "0") != 0;
 }
 
+// Whether operands with this K have a packed form (hip_ops.packable_k).
+bool packable_k(int64_t k) {
+  if (k < 256 || k % 32 != 0) return false;
+  const char* v = k % 256 != 0 ? getenv("FPQ_SINGLE_WEIGHT_COPY") : nullptr;
+  return !v || strcmp(v, "1") != 0;
+}
+
 bool is_alpha(PyObject* wgs, PyObject* alpha_obj) {   // what eager.linear_alpha holds for this layer is still that tensor
   PyObject* c = attribute(wgs, s_alpha);
   return c && PyTuple_Check(c) && PyTuple_GET_SIZE(c) == 2 && PyTuple_GET_ITEM(c, 1) == alpha_obj;
@@ -445,6 +452,7 @@ PyObject* no_quant_plan(PyObject* h, PyObject* ags) {
 // Whether a layer without a plan would run on packed weights, as every plan has it.
 bool may_pack(const LayerTensors& t, bool nvfp4, int64_t m) {
   const at::Tensor* q = tensor_of(t.qweight);
+  if (q && q->dim() == 2 && !packable_k(q->size(1) * 2)) return false;
   return packed_weights_enabled() && (nvfp4 || m >= g_linear_rows_mx || (q && q->dim() == 1));
 }
 
@@ -629,7 +637,7 @@ PyObject* host_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   const at::Tensor x = *xp, w = *wp;
   const int64_t cols = x.size(-1), rows = x.numel() / cols;
   if (w.scalar_type() != at::kBFloat16 || !w.is_contiguous() || w.numel() != cols || w.device().index() != call.dev ||
-      cols > 16384 || cols < 256 || cols % 32 != 0 || !packed_weights_enabled())
+      cols > 16384 || !packable_k(cols) || !packed_weights_enabled())
     Py_RETURN_NONE;
   QuantPlan::Body* q = quant_plan(t.h, t.ags, nvfp4);
   // (fused producers take Hadamard (0) and identity (1) rotations)
@@ -919,7 +927,7 @@ PyObject* host_matmul(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (w.size(1) != kb || n == 0 || xs.numel() / ldx < m || ldx < groups || ws.numel() / ldw < n || ldw < groups ||
       (bias.defined() && (bias.scalar_type() != at::kBFloat16 || bias.numel() != n)))
     Py_RETURN_NONE;
-  const bool packed = m >= (NV ? g_packed_rows_nv : g_packed_rows_mx) && k >= 256 && k % 32 == 0 && packed_weights_enabled();
+  const bool packed = m >= (NV ? g_packed_rows_nv : g_packed_rows_mx) && packable_k(k) && packed_weights_enabled();
   if (!plain_entry(E_fpq_gemm_mxf4) || !plain_entry(E_fpq_gemm_nvf4) || !plain_entry(E_fpq_gemm_mxf4_packed) ||
       !plain_entry(E_fpq_gemm_nvf4_packed) || !plain_entry(E_fpq_pack_padded))
     Py_RETURN_NONE;

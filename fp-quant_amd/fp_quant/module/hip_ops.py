@@ -141,10 +141,16 @@ def padded_k(k: int) -> int:
     return (k + 255) // 256 * 256
 
 
+def single_weight_copy() -> bool:
+    return os.environ.get("FPQ_SINGLE_WEIGHT_COPY", "0") == "1"
+
+
 def packable_k(k: int) -> bool:
     """Whether operands with this K have a packed form.  A ragged K (3200, 2880) runs on the packed kernels too: the
-    row-major kernel that takes any K stages nothing through LDS (333 x 8640 x 3200: 40 us against 15)."""
-    return k >= 256 and k % 32 == 0
+    row-major kernel that takes any K stages nothing through LDS (333 x 8640 x 3200: 40 us against 15).  Such a weight
+    cannot be held in the packed layout only (weight_rows reads the padding from K), so where weights are to be held once
+    it stays row-major and on that kernel."""
+    return k >= 256 and k % 32 == 0 and (k % 256 == 0 or not single_weight_copy())
 
 
 def packed_linear_eligible(rows: int, k: int, forward_method: str) -> bool:

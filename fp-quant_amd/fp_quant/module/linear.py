@@ -6,7 +6,6 @@ inference branch of `forward()` of the reference module
 the reference work unchanged.  Training branches (master weights, quantized backward) and
 pseudo-quantization are not part of this engine and raise.
 """
-import os
 from typing import Optional
 
 import torch
@@ -165,7 +164,7 @@ class FPQuantLinear(nn.Module):
                 and q.dtype == torch.uint8 and s.dtype == torch.uint8 and q.is_contiguous() and s.is_contiguous()
                 and hip_ops.packed_weights_enabled() and not torch.cuda.is_current_stream_capturing()):
             hip_ops.packed_weight(q, s, self.config.forward_dtype == FPQuantDtype.NVFP4, into=(stale[1], stale[2]))
-        if self._fpq_single_copy or os.environ.get("FPQ_SINGLE_WEIGHT_COPY", "0") == "1":
+        if self._fpq_single_copy or hip_ops.single_weight_copy():
             self.release_row_major()
         self._ensure_splitk_workspace()
 

@@ -148,3 +148,40 @@ def test_packed_weights_made_inside_a_capture_stay_there(fmt, g, k, monkeypatch)
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, want) and torch.equal(captured(x), want)
+
+
+@needs_packed
+@pytest.mark.parametrize("fmt,g", [("mxfp4", 128), ("nvfp4", 16)])
+def test_ragged_weights_are_held_once_where_asked_for(fmt, g, monkeypatch):
+    """FPQ_SINGLE_WEIGHT_COPY=1: a weight that cannot be held in the packed layout only gets no packed copy next to it,
+    in layers, fused blocks' groups and operators; its results are those of the row-major kernels."""
+    monkeypatch.setenv("FPQ_SINGLE_WEIGHT_COPY", "1")
+    monkeypatch.setattr(eager, "SHARE_ACT_QUANT", False)
+    nv = fmt == "nvfp4"
+    layers = []
+    for i in range(2):
+        cfg = fp_quant.FPQuantConfig(forward_dtype=fp_quant.FPQuantDtype(fmt), forward_method="abs_max",
+                                     backward_dtype=fp_quant.FPQuantDtype.BF16, hadamard_group_size=g)
+        gen = torch.Generator(device="cuda").manual_seed(i)
+        layers.append(fp_quant.FPQuantLinear(640, 96, cfg, bias=False, device="cuda", dtype=torch.bfloat16))
+        layers[-1].weight.data = torch.randn(96, 640, generator=gen, device="cuda", dtype=torch.bfloat16)
+        layers[-1].pre_forward()
+    assert eager.weight_group([(l.qweight, l.scales, None, 640) for l in layers], True, nv) is None
+    layer = layers[0]
+    alpha = (1.0 / (layer.weight_global_scale * layer.act_global_scale)).float()
+    for rows in (1, 70, 300):
+        x = torch.randn(rows, 640, device="cuda", dtype=torch.bfloat16)
+        with torch.no_grad():
+            y = layer(x)
+            if nv:
+                codes, scales = hip_ops.fused_quantize_nv_op(x, layer.forward_hadamard_matrix, layer.act_global_scale.float())
+                op = hip_ops.matmul_nvf4_bf16_tn_op
+            else:
+                codes, scales, _ = hip_ops.fused_quantize_mx_op(x, layer.forward_hadamard_matrix, "abs_max", False)
+                op = hip_ops.matmul_mxf4_bf16_tn_op
+            out = op(codes, layer.qweight, scales, layer.scales, alpha)
+            monkeypatch.setenv("FPQ_PACKED_WEIGHTS", "0")
+            want = op(codes, layer.qweight, scales, layer.scales, alpha)
+            monkeypatch.delenv("FPQ_PACKED_WEIGHTS")
+        assert torch.equal(y, want) and torch.equal(out, want)
+        assert not hasattr(layer.qweight, "_fpq_packed") and layer.qweight.dim() == 2
