@@ -280,6 +280,9 @@ class FPQuantLinear(nn.Module):
                     if residual is not None:
                         self.__dict__["_fpq_residual"] = None
                     return y
+            if x.shape[-1] != self.in_features and self.weights_packed_only:
+                # (a 1-D weight gives its rows for half the K as well: twice as many)
+                raise ValueError(f"inner dimensions differ: x has K={x.shape[-1]}, w has K={self.in_features}")
             # no autograd graph to build (inference): call the forward directly
             fn = (FPQuant4x16NoMasterFn.apply if (torch.is_grad_enabled() and x.requires_grad)
                   else _no_master_forward)

@@ -770,6 +770,17 @@ def test_release_row_major_keeps_results_and_the_reference_state_dict(bias, fmt,
             assert torch.equal(lin(x), w)
 
 
+@needs_packed
+@pytest.mark.parametrize("fmt,g", [("mxfp4", 64), ("nvfp4", 16)])
+def test_weights_held_once_refuse_another_inner_dimension(fmt, g):
+    lin = _quantized_linear(fmt, g, 512, 64, seed=4)
+    assert lin.release_row_major()
+    with torch.no_grad():
+        for k in (256, 1024, 480):
+            with pytest.raises(ValueError):
+                lin(torch.randn(3, k, device="cuda", dtype=torch.bfloat16))
+
+
 def test_release_row_major_declines_what_the_packed_layout_cannot_hold():
     nv = _quantized_linear("nvfp4", 16, 256, 48, seed=1)
     assert not nv.release_row_major() and nv.qweight.dim() == 2
