@@ -229,7 +229,7 @@ __device__ __forceinline__ void lane8_load_rotate(const uint4* __restrict__ x, u
 // (mxfp4.py:105-110, linear_fns.py:67-76).  fp32 evaluation order, fixed so that a CPU can
 // reproduce it: per octet of consecutive elements the sums of x and of fl(x*x) run left to right,
 // the four octet sums combine as (o0 + o1) + (o2 + o3); mean = sum/32, var = max(msq - fl(mean*mean), 0).
-template <int G, int FMT, int ROT, int ZERO, bool QUEST = false, int PRO = kProNone>
+template <int G, int FMT, int ROT, int ZERO, bool QUEST = false, int PRO = kProNone, bool PLACED = false>
 __device__ __forceinline__ void lane8_process(const uint4* __restrict__ x, uint32_t* __restrict__ codes,
                                               uint8_t* __restrict__ scales, uint32_t chunk, bool active,
                                               uint32_t lane, uint32_t chunks_per_row,
@@ -238,7 +238,8 @@ __device__ __forceinline__ void lane8_process(const uint4* __restrict__ x, uint3
                                               uint8_t* __restrict__ mask = nullptr,
                                               const Prologue& pro = Prologue{}, float row_scale = 0.0f,
                                               uint32_t prow = 0u, uint32_t pcc = 0u) {
-  // (prow, pcc): the chunk's place in the packed output, when there is one
+  // (prow, pcc): the chunk's place in the packed output, if there is one and it is PLACED; otherwise the chunk's number
+  // gives it, worked out behind the load (a division ahead of it costs 0.1 us: 32 x 14336 3.04 -> 3.11)
   static_assert(!QUEST || FMT == kFmtMx, "the quest rule exists for MXFP4 only");
   constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
   float p[8];
@@ -270,6 +271,10 @@ __device__ __forceinline__ void lane8_process(const uint4* __restrict__ x, uint3
       mbits |= (uint32_t)(__builtin_fabsf(q) < 6.0f) << i;
     }
     if (pro.packed_rows != 0u) {   // packed operand layout (no mask there); pad rows get zeros
+      if (!PLACED) {
+        prow = chunk / chunks_per_row;
+        pcc = chunk - prow * chunks_per_row;
+      }
       if (prow < pro.packed_rows) {
         codes[packed_code_word(prow, pcc, pro.packed_chunks)] = active ? packed : 0u;
         if ((pcc & 3u) == 0u) scales[packed_scale_byte<FMT>(prow, pcc, pro.packed_chunks)] = active ? (uint8_t)ex : (uint8_t)0;
@@ -311,6 +316,10 @@ __device__ __forceinline__ void lane8_process(const uint4* __restrict__ x, uint3
   }
 
   if (!QUEST && pro.packed_rows != 0u) {
+    if (!PLACED) {
+      prow = chunk / chunks_per_row;
+      pcc = chunk - prow * chunks_per_row;
+    }
     if (prow < pro.packed_rows) {
       codes[packed_code_word(prow, pcc, pro.packed_chunks)] = active ? packed : 0u;
       if ((pcc & (GROUP / 8 - 1)) == 0u) {
@@ -343,8 +352,9 @@ __device__ __forceinline__ void fill_scale_padding(uint8_t* __restrict__ scales,
   }
 }
 
-// Generic kernel: works for any cols % max(G, GROUP) == 0; one 8-element chunk per thread.
-template <int G, int FMT, int ROT, int ZERO, bool QUEST = false, int PRO = kProNone>
+// Generic kernel: works for any cols % max(G, GROUP) == 0; one 8-element chunk per thread.  RAGGED: packed output whose
+// rows are no whole 256-K blocks.
+template <int G, int FMT, int ROT, int ZERO, bool QUEST = false, int PRO = kProNone, bool RAGGED = false>
 __global__ __launch_bounds__(256) void quantize_lane8_kernel(
     const uint4* __restrict__ x, uint32_t* __restrict__ codes, uint8_t* __restrict__ scales,
     uint32_t n_chunks, uint32_t chunks_per_row, uint32_t rows, uint32_t scale_rows,
@@ -360,7 +370,7 @@ __global__ __launch_bounds__(256) void quantize_lane8_kernel(
   }
   uint32_t chunk = blockIdx.x * 256u + threadIdx.x, prow = 0u, pcc = 0u;
   bool active = chunk < n_chunks;
-  if (pro.packed_rows != 0u) {   // threads number the packed output, padding included
+  if (RAGGED) {   // threads number the packed output, padding included
     prow = chunk / pro.packed_chunks;
     pcc = chunk - prow * pro.packed_chunks;
     active = prow < rows && pcc < chunks_per_row;
@@ -371,9 +381,10 @@ __global__ __launch_bounds__(256) void quantize_lane8_kernel(
     g = *global_scale;
     rg = g == 0.0f ? 0.0f : 1.0f / g;
   }
-  lane8_process<G, FMT, ROT, ZERO, QUEST, PRO>(x, codes, scales, chunk, active, threadIdx.x & 63u,
-                                               chunks_per_row, scale_stride, norm, g, rg,
-                                               stage[kStage ? (threadIdx.x >> 6) : 0], hmat, mask, pro, 0.0f, prow, pcc);
+  lane8_process<G, FMT, ROT, ZERO, QUEST, PRO, RAGGED>(x, codes, scales, chunk, active, threadIdx.x & 63u,
+                                                       chunks_per_row, scale_stride, norm, g, rg,
+                                                       stage[kStage ? (threadIdx.x >> 6) : 0], hmat, mask, pro, 0.0f, prow,
+                                                       pcc);
   fill_scale_padding(scales, rows, chunks_per_row / (GROUP / 8), scale_rows, scale_stride);
 }
 
@@ -398,6 +409,13 @@ static int launch_lane8(const void* x, int64_t rows, int64_t cols, float norm, c
                        (uint32_t)scale_rows, (uint32_t)scale_stride, norm, gsp, (const uint16_t*)h,
                        (uint8_t*)nullptr, pro);
   };
+  if constexpr (ROT != FPQ_ROT_GENERAL) {   // (no packed output there)
+    if (packed && cols % 256 != 0) {
+      if (zero_policy == FPQ_ZERO_REFERENCE) args(quantize_lane8_kernel<G, FMT, ROT, kZeroReference, false, kProNone, true>);
+      else args(quantize_lane8_kernel<G, FMT, ROT, kZeroSigned, false, kProNone, true>);
+      return (int)hipGetLastError();
+    }
+  }
   if (zero_policy == FPQ_ZERO_REFERENCE) {
     args(quantize_lane8_kernel<G, FMT, ROT, kZeroReference>);
   } else {
@@ -1075,6 +1093,13 @@ static int launch_lane8_quest(const void* x, int64_t rows, int64_t cols, float n
                        (uint32_t)scale_rows, (uint32_t)scale_stride, norm, (const float*)nullptr,
                        (const uint16_t*)h, (uint8_t*)mask, pro);
   };
+  if constexpr (ROT != FPQ_ROT_GENERAL) {
+    if (packed && cols % 256 != 0) {
+      if (zero_policy == FPQ_ZERO_REFERENCE) args(quantize_lane8_kernel<G, kFmtMx, ROT, kZeroReference, true, kProNone, true>);
+      else args(quantize_lane8_kernel<G, kFmtMx, ROT, kZeroSigned, true, kProNone, true>);
+      return (int)hipGetLastError();
+    }
+  }
   if (zero_policy == FPQ_ZERO_REFERENCE) {
     args(quantize_lane8_kernel<G, kFmtMx, ROT, kZeroReference, true>);
   } else {
@@ -1329,6 +1354,11 @@ static int launch_lane8_prologue(const void* x, int64_t rows, int64_t cols, floa
                        (uint32_t)scale_rows, (uint32_t)scale_stride, norm, gsp, (const uint16_t*)nullptr,
                        (uint8_t*)nullptr, pro);
   };
+  if (pro.packed_rows != 0u && cols % 256 != 0) {
+    if (zero_policy == FPQ_ZERO_REFERENCE) args(quantize_lane8_kernel<G, FMT, ROT, kZeroReference, false, PRO, true>);
+    else args(quantize_lane8_kernel<G, FMT, ROT, kZeroSigned, false, PRO, true>);
+    return (int)hipGetLastError();
+  }
   if (zero_policy == FPQ_ZERO_REFERENCE) {
     args(quantize_lane8_kernel<G, FMT, ROT, kZeroReference, false, PRO>);
   } else {
@@ -1584,9 +1614,9 @@ __global__ __launch_bounds__(1024) void rmsnorm_rows_quantize_kernel(const uint4
     const uint32_t cc = c0 + threadIdx.x;
     const bool in = cc < cpr;
     // (a row past the packed output makes the generic kernel skip the store)
-    lane8_process<G, FMT, ROT, ZERO, false, kProRmsNorm>(x, codes, scales, row * cpr + (in ? cc : 0u), real && in, lane,
-                                                         cpr, 0u, norm, gs, rg, nullptr, nullptr, nullptr, pro, rs,
-                                                         in ? row : 0xffffffffu, cc);
+    lane8_process<G, FMT, ROT, ZERO, false, kProRmsNorm, true>(x, codes, scales, row * cpr + (in ? cc : 0u), real && in,
+                                                               lane, cpr, 0u, norm, gs, rg, nullptr, nullptr, nullptr,
+                                                               pro, rs, in ? row : 0xffffffffu, cc);
   }
 }
 
