@@ -1040,7 +1040,10 @@ static int dispatch_packed(const void* x, int64_t rows, int64_t cols, int rot_ki
   // NVFP4 below 2^23 elements: the tile kernel, whose loads need no round trip through LDS before its scale table is
   // built (us, Hadamard 16: 128 x 4096 3.8 -> 3.5, 512 x 4096 4.4 -> 3.8, 1024 x 4096 5.4 -> 4.6, 256 x 12288 5.0 -> 4.4,
   // 512 x 12288 6.2 -> 5.7; 1024 x 12288 9.6 / 9.5, 2048 x 12288 13.3 / 16.6; MXFP4 +-5 % up to 2^22, slower beyond).
-  const bool tile = FMT == kFmtNv && rows * cols < (int64_t)1 << 23;
+  // Up to 2^19 elements only with the rotations that the streaming kernel exchanges between lanes: the others fit its one
+  // un-overlapped round (streaming / tile: 128 x 1024 Hadamard 32 3.39 / 3.50, identity 3.04 / 3.11, Hadamard 64 3.6 / 3.4;
+  // 160 x 4096 Hadamard 16 3.70 / 3.43, 32 3.73 / 3.56, identity 3.40 / 3.20).
+  const bool tile = FMT == kFmtNv && rows * cols < (int64_t)1 << 23 && (g >= 64 || rows * cols > (int64_t)1 << 19);
   Prologue pro{};
   pro.chunks_per_row = pro.ld_first = (uint32_t)(cols / 8);
 #define FPQ_LAUNCH_PACKED(GG, RR)                                                                                 \
