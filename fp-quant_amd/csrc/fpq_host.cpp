@@ -644,6 +644,8 @@ PyObject* host_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (!q) return no_quant_plan(t.h, t.ags);
   if (!q->usable || q->kind > 1 || cols % (q->g > 32 ? q->g : 32) != 0) Py_RETURN_NONE;
   const bool few = rows <= 64 && cols % 256 == 0;
+  if (!few && rows <= 640 && cols > 8192 && cols % 256 == 0 && rows * cols <= (1 << 23))
+    Py_RETURN_NONE;   // (two launches: eager._norm_in_two_launches)
   const int entry = few ? (nvfp4 ? E_fpq_rmsnorm_rows_quantize_nv_packed : E_fpq_rmsnorm_rows_quantize_mx_packed)
                         : (nvfp4 ? E_fpq_rmsnorm_tile_quantize_nv_packed : E_fpq_rmsnorm_tile_quantize_mx_packed);
   bool declined = false;

@@ -790,6 +790,15 @@ _ROWS_KERNEL_MAX_ROWS = 64     # fpq_rmsnorm_rows_max_rows()
 _ONE_LAUNCH_MAX_COLS = 16384   # of fpq_rmsnorm_rows_quantize_* and fpq_rmsnorm_tile_quantize_*
 
 
+def _norm_in_two_launches(rows: int, cols: int) -> bool:
+    """More rows than the row-per-workgroup kernel takes, but too few wide ones to fill the CUs with the tile kernel's
+    four rows per workgroup: the statistic in a launch of its own, then the streaming quantizer, whose work is spread over
+    the columns too.  Two launches / tile kernel, us, MXFP4 with Hadamard 128: 65 x 14336 13.2 / 17.9, 256 x 8448
+    11.8 / 14.1, 384 x 12288 15.4 / 16.6, 640 x 12288 16.1 / 16.7, 640 x 8448 14.5 / 14.2, 640 x 14336 22.6 / 18.8,
+    256 x 8192 11.6 / 10.9."""
+    return (_ROWS_KERNEL_MAX_ROWS < rows <= 640 and cols > 8192 and cols % 256 == 0 and rows * cols <= 1 << 23)
+
+
 def rmsnorm_quantize(x: torch.Tensor, weight: torch.Tensor, eps: float, hadamard_matrix: torch.Tensor,
                      act_global_scale: Optional[torch.Tensor], nvfp4: bool) -> Optional[torch.Tensor]:
     """RMSNorm of bf16 `x` over its last dimension, y = bf16(weight * bf16(x / rms)), in one pass
@@ -813,7 +822,7 @@ def rmsnorm_quantize(x: torch.Tensor, weight: torch.Tensor, eps: float, hadamard
         y = torch.empty_like(x_flat)
         w = weight.contiguous()
         qa = None
-        if (cols <= _ONE_LAUNCH_MAX_COLS
+        if (cols <= _ONE_LAUNCH_MAX_COLS and not _norm_in_two_launches(rows, cols)
                 and (nv_packed_eligible(rows, 32, cols, fused_linear=True) if nvfp4
                      else packed_linear_eligible(rows, cols, "abs_max"))):
             # statistic, normalisation and quantization in one launch: a decode step's few rows spread over many

@@ -5,7 +5,7 @@ import torch
 
 from oracle import fpq_oracle as O
 from tests import capi
-from tests.conftest import make_student_t
+from tests.conftest import make_student_t, needs_packed
 from tests.test_ragged_k_gpu import _padded_pack
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +42,39 @@ def test_rmsnorm_of_many_rows_in_one_pass_bit_exact(fmt, rot, g, rows, cols):
     pc2, ps2, none, none2 = capi.rmsnorm_rows_quantize_packed(x, w, g=g, rot=rot, want_out=False, want_inv=False,
                                                               global_scale=gs, entry="tile")
     assert none is None and none2 is None and torch.equal(pc2, want_c) and torch.equal(ps2, want_s)
+
+
+# both sides of every line: 64 and 640 rows, 8192 columns, 2^23 elements, a row that is no whole number of blocks
+@needs_packed
+@pytest.mark.parametrize("fmt,g", [("mxfp4", 128), ("nvfp4", 16)])
+@pytest.mark.parametrize("rows,cols,two", [(64, 8448, False), (65, 8192, False), (65, 8448, True), (65, 8480, False),
+                                           (512, 16384, True), (513, 16384, False), (640, 8448, True), (641, 8448, False)])
+def test_wide_rows_take_the_statistic_in_a_launch_of_its_own(fmt, g, rows, cols, two, monkeypatch):
+    """The fused norm where its rows are wide and few: two launches, the tile kernel's bits."""
+    from fp_quant import _engine
+    from fp_quant.module import eager, hip_ops, linear
+    nv, cols = fmt == "nvfp4", cols + 96 if cols % g else cols
+    x = (make_student_t(rows, cols, seed=rows) * 2).cuda()
+    w = torch.randn(cols, device="cuda").to(torch.bfloat16)
+    h = linear.get_hadamard_matrix(g, torch.bfloat16, x.device)
+    gs = torch.full((1,), 3.0, device="cuda")
+    lib, calls = _engine.lib(), []
+    entry = lib.fpq_row_inv_rms
+    monkeypatch.setattr(lib, "fpq_row_inv_rms", lambda *args: (calls.append(args), entry(*args))[1])
+    y = eager.rmsnorm_quantize(x, w, 1e-5, h, gs, nv)
+    if not hip_ops.packable_k(cols):   # (weights held once: the row-major forms)
+        return
+    assert len(calls) == two
+    _, norm = hip_ops.classify_rotation(h)
+    pc = torch.empty(lib.fpq_packed_codes_bytes(rows, cols), dtype=torch.uint8, device="cuda")
+    ps = torch.empty((lib.fpq_packed_scales_bytes_nv if nv else lib.fpq_packed_scales_bytes)(rows, cols), dtype=torch.uint8,
+                     device="cuda")
+    out = torch.empty_like(x)
+    head = (x.data_ptr(), cols, w.data_ptr(), rows, cols, 1e-5, _engine.ROT_HADAMARD, g, norm)
+    tail = (None, out.data_ptr(), pc.data_ptr(), ps.data_ptr(), 0, hip_ops._current_stream(0))
+    _engine.check(lib.fpq_rmsnorm_tile_quantize_nv_packed(*head, gs.data_ptr(), *tail) if nv
+                  else lib.fpq_rmsnorm_tile_quantize_mx_packed(*head, *tail), "tile")
+    qa = eager._shared_activations[0]
+    assert torch.equal(y, out) and qa.ref() is y
+    for a, b in zip(qa.packed(), (pc, ps)):
+        assert torch.equal(a, b)
