@@ -380,7 +380,8 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
         float v[32];
         load_rotate(v);
         uint32_t cw[4], sbytes = 0u, sb_lo = 0u;
-        const bool need_slow = quantize_chunk<32, FMT, kZeroReference, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+        bool need_slow = chunk_not_finite<32>(v);
+        need_slow |= quantize_chunk<32, FMT, kZeroReference, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
         if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
           float u[32];
           load_rotate(u);

@@ -973,7 +973,17 @@ __global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
     float v[EPL];
     load_rotate(v);
     uint32_t cw[EPL / 8], sbytes = 0u, sb_lo = 0u;
-    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    bool need_slow = (cpr & 31u) != 0u && chunk_not_finite<EPL>(v);   // (ragged rows were the generic kernel's)
+    if (QUEST && __builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
+      quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+#pragma unroll
+      for (int i = 0; i < EPL; ++i) {
+        const uint32_t at = 4 * (i & 7);
+        if (v[i] != v[i]) cw[i >> 3] = (cw[i >> 3] & ~(0xfu << at)) | (e2m1_code<ZERO>(v[i]) << at);
+      }
+    } else {
+      need_slow |= quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    }
     if (!QUEST && __builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
       float u[EPL];
       load_rotate(u);
@@ -1733,7 +1743,8 @@ __global__ __launch_bounds__(64 * kTileRows) void rmsnorm_tile_quantize_kernel(
     float v[EPL];
     load_rotate(v);
     uint32_t cw[EPL / 8], sbytes = 0u, sb_lo = 0u;
-    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    bool need_slow = (cpr & 31u) != 0u && chunk_not_finite<EPL>(v);   // (ragged rows were the generic kernel's)
+    need_slow |= quantize_chunk<EPL, FMT, ZERO, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
     if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
       float u[EPL];
       load_rotate(u);

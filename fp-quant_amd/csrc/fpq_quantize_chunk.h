@@ -65,7 +65,7 @@ __device__ __forceinline__ void fma_exchange8(float (&v)[8], float sign) {
 // value and both add (two instructions and a wait between them); otherwise a lane holds its values negated through
 // the stages before an exchange in which it is the upper one (the norm's sign: a rotation of negated values is the
 // negated rotation), and the exchange is ONE fused multiply-add with +-1, own + sign * other, whose product is exact.
-// The only difference is the sign of a zero, which the reference's zero policy does not look at.
+// The only differences are the sign of a zero, which the reference's zero policy does not look at, and the sign of a NaN.
 template <int EPL, int G, int ROT, bool KEEP_ZERO_SIGN>
 __device__ __forceinline__ void rotate_chunk(float (&v)[EPL], float norm, uint32_t lane) {
   if (ROT == FPQ_ROT_HADAMARD || ROT == FPQ_ROT_GSR) {
@@ -118,6 +118,18 @@ __device__ __forceinline__ void rotate_chunk(float (&v)[EPL], float norm, uint32
 #pragma unroll
     for (int k = 0; k < EPL; ++k) v[k] = w[k];
   }
+}
+
+// Whether a rotated chunk holds a NaN or an infinity.  quantize_chunk gives a NaN element the code of its sign and the
+// largest magnitude, and an infinite NVFP4 group the scale byte of a NaN; quantize_chunk_slow, as the generic kernel, leaves
+// a NaN element out (code of zero) and clamps the group's scale.  Kernels that took calls over from the generic one send
+// such chunks there: one NaN in a decode row must not depend on how many rows are quantized with it.
+template <int EPL>
+__device__ __forceinline__ bool chunk_not_finite(const float (&v)[EPL]) {
+  float m = 0.0f;
+#pragma unroll
+  for (int i = 0; i < EPL; ++i) m = __builtin_elementwise_maximum(m, __builtin_fabsf(v[i]));   // (keeps a NaN)
+  return !(m <= 3.402823466e+38f);
 }
 
 // E2M1 codes and scale bytes of one lane's rotated chunk (cw: CW dwords of codes; sbytes: the scale bytes, with

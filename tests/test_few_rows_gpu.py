@@ -35,7 +35,6 @@ def _layer(fmt, init, g, k, n, bias):
                                         ("nvfp4", "identity", 64)])
 def test_same_bits_as_two_kernels(fmt, init, g, silu):
     lib, nv = _engine.lib(), fmt == "nvfp4"
-    taken = 0
     for m, k, n in SHAPES:
         if k % g:
             continue
@@ -48,6 +47,7 @@ def test_same_bits_as_two_kernels(fmt, init, g, silu):
         x[:, :32] = 0
         x[:, 64:96] *= 1e-34
         x[:, 128:160] *= 1e32
+        x[-1, 197], x[0, 227] = float("nan"), float("inf")
         x = x.to(torch.bfloat16)
         up = torch.randn(m, k, device="cuda", dtype=torch.bfloat16) if silu else None
         res = torch.randn(m, n, device="cuda", dtype=torch.bfloat16)
@@ -75,16 +75,16 @@ def test_same_bits_as_two_kernels(fmt, init, g, silu):
         st = lib.fpq_linear_rows(int(nv), x.data_ptr(), up.data_ptr() if silu else None, m, k, kind, g, norm, gs.data_ptr(),
                                  wp.data_ptr(), wsp.data_ptr(), alpha.data_ptr(), bias, res.data_ptr(), y2.data_ptr(), n,
                                  a2.data_ptr(), b2.data_ptr(), *tail[:2], 0, tail[2])
-        if st == _engine.E_UNSUPPORTED:
+        # chunks of the wave with the most, with the whole of K in one workgroup (a split leaves fewer): one pass of 64, or,
+        # but for SiLU*up, two
+        if m * -(-(-(-k // 256)) // 4) * 8 > (64 if silu else 128) and st == _engine.E_UNSUPPORTED:
             continue
-        assert st == 0
-        taken += 1
+        assert st == 0, (m, k, n)
         assert torch.equal(y.view(torch.int16), y2.view(torch.int16)), (m, k, n)
         for p, q in zip(hip_ops.unpack_fp4(a, b, m, k, nv), hip_ops.unpack_fp4(a2, b2, m, k, nv)):
             assert torch.equal(p, q), (m, k, n)
         if need:
             assert not ws[:16384].any()   # the counters are back at zero
-    assert taken >= 4
 
 
 def test_refused_calls():

@@ -6,7 +6,7 @@ import torch
 from oracle import fpq_oracle as O
 from fp_quant import _engine
 import capi
-from conftest import make_outlier_normal, needs_packed, needs_row_major_parameters, packed_copy
+from conftest import make_outlier_normal, make_student_t, needs_packed, needs_row_major_parameters, packed_copy
 
 pytestmark = pytest.mark.gpu
 
@@ -402,3 +402,36 @@ def test_nv_layers_end_to_end_get_their_own_outputs(m, splits, k, with_bias):
         assert o.shape == (m, s_)
         assert torch.equal(o.view(torch.int16), whole[:, col:col + s_].contiguous().view(torch.int16))
         col += s_
+
+
+# NaN and infinities.  Whole 256-K blocks: the scale bytes and codes of all other rotation blocks (up to 64 rows, of these
+# too).  Ragged rows, and the few that the GEMM quantizes itself, give all bytes of the row-major operator's generic kernel.
+@pytest.mark.parametrize("rows", [40, 70, 300])
+@pytest.mark.parametrize("kind,g,rot", [("mx", 32, "hadamard"), ("mx", 128, "hadamard"), ("mx", 32, "identity"),
+                                        ("quest", 128, "hadamard"), ("quest", 32, "identity"), ("nv", 16, "hadamard"),
+                                        ("nv", 128, "hadamard"), ("nv", 32, "identity")])
+@pytest.mark.parametrize("cols", [1024, 896])
+def test_non_finite_values(rows, kind, g, rot, cols):
+    from fp_quant.module import hip_ops, linear
+    from tests.test_ragged_k_gpu import _quantize_padded
+    nv, block = kind == "nv", g if rot == "hadamard" else 32
+    x = make_student_t(rows, cols, seed=rows + g)
+    for i, bad in enumerate((float("nan"), float("inf"), -float("inf"), -float("nan"))):
+        x[i::7, 100 * i + 3] = bad
+    x[5::7, 700], x[5::7, 701] = float("inf"), -float("inf")
+    make = linear.get_hadamard_matrix if rot == "hadamard" else linear.get_identity_matrix
+    h = make(g, torch.bfloat16, torch.device("cuda"))
+    gs = torch.full((1,), 777.0, device="cuda")
+    pc, ps = _quantize_padded(x, kind, rot, g, 777.0)
+    if nv:
+        codes, scales = hip_ops.fused_quantize_nv_op(x.cuda(), h, gs)
+    else:
+        codes, scales, _ = hip_ops.fused_quantize_mx_op(x.cuda(), h, "quest" if kind == "quest" else "abs_max", False)
+    got_c, got_s = hip_ops.unpack_fp4(pc.cuda(), ps.cuda(), rows, cols, nv)
+    got_c, codes = got_c.view(rows, -1, block // 2), codes.view(rows, -1, block // 2)
+    groups = cols // (16 if nv else 32)
+    got_s, scales = got_s.view(rows, cols // block, -1), scales.view(torch.uint8)[:rows, :groups].reshape(rows, cols // block, -1)
+    clean = torch.isfinite(x).view(rows, cols // block, block).all(-1).cuda()
+    if cols % 256 != 0 or rows <= 64:
+        clean |= True
+    assert clean.any() and torch.equal(got_c[clean], codes[clean]) and torch.equal(got_s[clean], scales[clean])
