@@ -7,6 +7,8 @@ import threading
 import pytest
 import torch
 
+from tests.conftest import SINGLE_WEIGHT_COPY, needs_packed, needs_row_major_parameters
+
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
@@ -69,8 +71,10 @@ FORMS = [("mxfp4", "abs_max", "hadamard", 128), ("mxfp4", "quest", "hadamard", 3
          ("nvfp4", "abs_max", "hadamard", 16), ("nvfp4", "abs_max", "gsr", 128), ("nvfp4", "abs_max", "general", 32)]
 
 
+# (K = 640 stays on the row-major weight where weights are held once: nothing for native code)
+@needs_packed
 @pytest.mark.parametrize("fmt,method,init,g", FORMS)
-@pytest.mark.parametrize("k", [512, 640])
+@pytest.mark.parametrize("k", [512] if SINGLE_WEIGHT_COPY else [512, 640])
 def test_linear_forms(fmt, method, init, g, k, native):
     general = init == "general"
     layer = _layer(fmt, method, "hadamard" if general else init, g, k, bias=True)
@@ -91,6 +95,7 @@ def test_linear_forms(fmt, method, init, g, k, native):
             assert torch.equal(layer(x), _python(layer, x, res)) and layer._fpq_residual is None
 
 
+@needs_packed
 def test_declined_calls(native, monkeypatch):
     layer = _layer(bias=True)
     x = torch.randn(6, 512, device="cuda", dtype=torch.bfloat16)
@@ -111,9 +116,12 @@ def test_declined_calls(native, monkeypatch):
         assert not eager._shared_activations or eager._shared_activations[0].ref() is not xi
     native.answered.clear()
     monkeypatch.setenv("FPQ_PACKED_WEIGHTS", "0")
-    assert torch.equal(layer(x), _python(layer, x)) and not native.answered
+    assert torch.equal(layer(x), _python(layer, x))
+    assert native.answered == (["linear"] if layer.weights_packed_only else [])
 
 
+@needs_packed
+@needs_row_major_parameters   # (another layer's are loaded)
 def test_plans_notice_changes(native):
     layer = _layer("nvfp4", g=16, k=512)
     x = torch.randn(40, 512, device="cuda", dtype=torch.bfloat16)
@@ -158,6 +166,7 @@ def test_plans_notice_changes(native):
     assert torch.equal(loaded(x), layer(x))
 
 
+@needs_packed
 @pytest.mark.parametrize("fmt,g", [("mxfp4", 64), ("nvfp4", 16)])
 def test_streams_and_threads(fmt, g, native):
     """One layer that splits K (a workspace per stream) called from threads with a stream each."""
@@ -180,6 +189,7 @@ def test_streams_and_threads(fmt, g, native):
     assert not bad and "linear" in native.answered
 
 
+@needs_packed
 def test_source_of_a_shared_quantization_dies(native):
     layer = _layer()
     x = torch.randn(6, 512, device="cuda", dtype=torch.bfloat16)
@@ -196,7 +206,7 @@ def test_source_of_a_shared_quantization_dies(native):
                                        ("mxfp4", 200, 256, 512), ("nvfp4", 1, 72, 512), ("nvfp4", 64, 264, 288),
                                        ("nvfp4", 65, 264, 288), ("nvfp4", 200, 256, 512)])
 def test_operators(fmt, m, n, k):
-    """Operators called plainly and through the dispatcher (torch.ops): the same tensors."""
+    """Operators called plainly and through the dispatcher (torch.ops): the same tensors; native code takes the plain calls."""
     mx = fmt == "mxfp4"
     w = torch.randn(n, k, device="cuda", dtype=torch.bfloat16)
     x = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
@@ -228,6 +238,10 @@ def test_operators(fmt, m, n, k):
              [getattr(ops, f"matmul_{name}_bf16_tn_op")(qx, qw, sx, sw, alpha)])
         same([getattr(hip_ops, f"matmul_{name}_bf16_tn_bias_op")(qx[None], qw, sx, sw, alpha, bias)],
              [getattr(ops, f"matmul_{name}_bf16_tn_bias_op")(qx[None], qw, sx, sw, alpha, bias)])
+    native = host.native
+    assert (native.quantize_mx(x, h, "abs_max", False) if mx else native.quantize_nv(x, h, gs)) is not None
+    matmul = native.matmul_mx if mx else native.matmul_nv
+    assert matmul(qx, qw, sx, sw, alpha) is not None and matmul(qx[None], qw, sx, sw, alpha, bias) is not None
     with pytest.raises(ValueError):
         getattr(hip_ops, f"matmul_{name}_bf16_tn_op")(qx, qw[:, : k // 4], sx, sw, alpha)
     with pytest.raises(ValueError):
@@ -235,12 +249,15 @@ def test_operators(fmt, m, n, k):
          hip_ops.fused_quantize_nv_op(x.float(), h, gs))
 
 
-def test_fused_block_after_a_weight_changes():
-    """The grouped projections of a fused block: a member that is written to, and a rotation that is replaced."""
+@needs_packed
+@pytest.mark.parametrize("fmt,g,kv", [("mxfp4", 64, 256), ("nvfp4", 64, 256), ("mxfp4", 64, 128)])
+def test_fused_block_after_a_weight_changes(fmt, g, kv, monkeypatch):
+    """The grouped projections of a fused block: a member that is written to, and a rotation that is replaced.  Native code
+    answers every norm, group (but for widths that are no multiples of 256) and MLP, and the output projection."""
     from perf.cases import Block
     from fp_quant.utils import fuse_producers
     gen = torch.Generator(device="cuda").manual_seed(5)
-    case = dict(fmt="mxfp4", g=64, hidden=512, kv=256, inter=768)
+    case = dict(fmt=fmt, g=g, hidden=512, kv=kv, inter=768)
     block = Block(case, gen)
     assert fuse_producers(block)
     x = torch.randn(1, 5, 512, device="cuda", dtype=torch.bfloat16)
@@ -258,9 +275,16 @@ def test_fused_block_after_a_weight_changes():
 
     import fp_quant.utils.fuse as fuse
 
+    counts = _Counts()
+    monkeypatch.setattr(fuse, "_native_module", counts)
+    monkeypatch.setattr(linear_module, "_native", counts)
+
     def check():
-        for _ in range(2):
-            got = run(True)
+        run(True)
+        counts.answered.clear()
+        got = run(True)
+        # (such widths are column ranges of one matrix: the output projection's input is strided too)
+        assert counts.answered == ["rmsnorm", *(["group", "linear"] if kv % 256 == 0 else []), "rmsnorm", "group", "gated_down"]
         for a, b in zip(got, run(False)):
             assert torch.equal(a, b)
 
@@ -295,6 +319,7 @@ def test_operators_are_recorded_by_a_jit_trace():
         assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
 
 
+@needs_packed
 def test_group_of_a_rewritten_weight_is_not_rebuilt_inside_a_capture():
     """A member written to, then the block recorded: calls outside the graph find no half-made group, and later ones
     rebuild it."""
@@ -329,6 +354,7 @@ def test_group_of_a_rewritten_weight_is_not_rebuilt_inside_a_capture():
     assert torch.equal(twin(x), block.self_attn.k_proj(x))
 
 
+@needs_packed
 @pytest.mark.parametrize("kv,fmt,g", [(128, "mxfp4", 64), (384, "mxfp4", 128), (128, "nvfp4", 16)])
 def test_a_group_that_native_code_cannot_serve_is_asked_about_once(kv, fmt, g, monkeypatch):
     """Projections whose widths are no multiple of 256 share one output matrix, which only the Python path lays out."""
@@ -370,6 +396,7 @@ def test_weights_that_cannot_be_in_a_plan_are_not_asked_about(native, monkeypatc
     assert not tried and not native.answered
 
 
+@needs_packed
 def test_a_layer_whose_plan_is_refused_gets_a_marker(native, monkeypatch):
     layer = _layer()
     x = torch.randn(6, 512, device="cuda", dtype=torch.bfloat16)
@@ -410,6 +437,7 @@ with torch.no_grad():
 """
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     for env, args in (({"FPQ_PACKED_MIN_ROWS": "32"}, ["rows"]), ({"FPQ_PACKED_WEIGHTS": "0"}, [])):
-        r = subprocess.run([sys.executable, "-c", code, *args], cwd=root, env={**os.environ, **env}, capture_output=True,
+        base = {k: v for k, v in os.environ.items() if k not in ("FPQ_PACKED_WEIGHTS", "FPQ_SINGLE_WEIGHT_COPY")}
+        r = subprocess.run([sys.executable, "-c", code, *args], cwd=root, env={**base, **env}, capture_output=True,
                            text=True, timeout=100)
         assert r.returncode == 0, r.stderr[-2000:]

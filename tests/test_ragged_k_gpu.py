@@ -8,7 +8,7 @@ from fp_quant import _engine
 from fp_quant.module import eager, hip_ops
 from oracle import fpq_oracle as O
 from tests import capi
-from tests.conftest import make_student_t, needs_packed
+from tests.conftest import SINGLE_WEIGHT_COPY, make_student_t, needs_packed
 from tests.test_packed_gpu import pack_by_definition, pack_nv_by_definition
 
 pytestmark = pytest.mark.gpu
@@ -96,7 +96,7 @@ def test_layer_matches_the_oracle(fmt, method, init, g, m, k, n):
     x = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
     with torch.no_grad():
         y = layer(x)
-    assert getattr(layer.qweight, "_fpq_packed", None) is not None
+    assert (getattr(layer.qweight, "_fpq_packed", None) is None) == SINGLE_WEIGHT_COPY
     okind = O.ROT_GSR if init == "gsr" else O.ROT_HADAMARD
     norm = float(O.hadamard_matrix(g)[0, 0])
     if fmt == "nvfp4":

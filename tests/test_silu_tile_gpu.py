@@ -3,6 +3,7 @@ lookup (the table's busy part, the small magnitudes beside it, the large ones, i
 import pytest
 import torch
 
+from fp_quant.module import hip_ops
 from oracle import fpq_oracle as O
 from tests import capi
 from tests.test_ragged_k_gpu import _padded_pack
@@ -14,11 +15,19 @@ def test_every_gate_value():
     gate = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).reshape(256, 256)
     gate = gate[torch.randperm(256, generator=torch.Generator().manual_seed(1))].contiguous()
     up = torch.ones(256, 256, dtype=torch.bfloat16)
-    _, _, out = capi.fused_quantize_packed("silu_mul", gate, up, g=128)
+    pc, ps, out = capi.fused_quantize_packed("silu_mul", gate, up, g=128)
     want = O.silu_mul(gate, up)
     nan = torch.isnan(want)
     assert torch.equal(torch.isnan(out), nan)
     assert torch.equal(out.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+    # and the codes and scales of every 128-wide block that is finite and overflows nowhere
+    quiet = torch.where(torch.isfinite(want) & (want.abs() < 1e36), want, torch.zeros_like(want))
+    clean = (quiet == want).view(256, 2, 128).all(-1)
+    assert clean.sum() > 100
+    c, s, _ = O.quantize_mx(quiet, O.ROT_HADAMARD, 128, float(O.hadamard_matrix(128)[0, 0]))
+    codes, scales = (t.cpu() for t in hip_ops.unpack_fp4(pc.cuda(), ps.cuda(), 256, 256))
+    assert torch.equal(codes.view(256, 2, 64)[clean], c.view(256, 2, 64)[clean])
+    assert torch.equal(scales.view(256, 2, 4)[clean], s[:256, :8].reshape(256, 2, 4)[clean])
 
 
 # eight rows a wave, the last row tile with part of them; one 256-column block per row, several, and
