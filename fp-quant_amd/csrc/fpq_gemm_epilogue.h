@@ -286,24 +286,18 @@ __device__ __forceinline__ void wave_tile_store(const v16f (&acc)[TN][TM], uint8
     }
     return;
   }
-  // The bias in one round trip ahead of the barrier, its columns clamped (what lies past N is not stored): fetched value
-  // by value behind a bounds check each, the eight or sixteen round trips of the last row or column of tiles made the whole
-  // kernel wait (us, with a bias: MXFP4 333 x 8640 x 3328 15.0 -> 12.4, 12.2 without one; 1000 x 14336 x 4096 41.2 -> 35.0,
-  // 2000 rows 69.4 -> 66.4; NVFP4 1500 x 6144 x 4096 83.0 -> 76.9, 500 x 4096 x 12288 52.1 -> 49.6).  (Asking for alpha
-  // at the kernel's start as well gained nothing.)
-  uint2 braw[TN * 4];
+  // The bias in one round trip ahead of the barrier, two columns per lane (clamped: what lies past N is not stored), from
+  // which the lanes that need them take them: fetched value by value behind a bounds check each, the eight or sixteen round
+  // trips of the last row or column of tiles made the whole kernel wait (us, with a bias: MXFP4 333 x 8640 x 3328
+  // 15.0 -> 12.4, 12.2 without one; 1000 x 14336 x 4096 41.2 -> 35.0, 2000 rows 69.4 -> 66.4; NVFP4 1500 x 6144 x 4096
+  // 83.0 -> 76.9, 500 x 4096 x 12288 52.1 -> 49.6).  Every lane holding all it needs takes registers that the 256 x 256
+  // tiles do not have: with 16 of them spilled, and scratch memory to set up, that kernel ran 0.7 % longer with or without
+  // a bias (NVFP4 4096 x 24576 x 4096 581.7 -> 585.5).
+  static_assert(WT_N <= 128, "two columns per lane");
+  uint32_t braw = 0u;
   if (bias) {
-    const bool quads = (N & 3) == 0 && ((uintptr_t)bias & 7u) == 0;
-#pragma unroll
-    for (int ig = 0; ig < TN * 4; ++ig) {
-      const int n = n0 + ig * 8 + 4 * kh;
-      if (quads) {
-        braw[ig] = *(const uint2*)(bias + min(n, N - 4));
-      } else {
-        braw[ig].x = (uint32_t)bias[min(n, N - 1)] | ((uint32_t)bias[min(n + 1, N - 1)] << 16);
-        braw[ig].y = (uint32_t)bias[min(n + 2, N - 1)] | ((uint32_t)bias[min(n + 3, N - 1)] << 16);
-      }
-    }
+    const int n = n0 + 2 * lane;
+    braw = (uint32_t)bias[min(n, N - 1)] | ((uint32_t)bias[min(n + 1, N - 1)] << 16);
   }
   __syncthreads();                                   // every wave is done reading operands
   uint8_t* stg = smem + wave * (WT_M * kStride);
@@ -312,12 +306,16 @@ __device__ __forceinline__ void wave_tile_store(const v16f (&acc)[TN][TM], uint8
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int nl = i * 32 + 8 * g + 4 * kh;
+      uint2 b = make_uint2(0u, 0u);
+      if (bias) {   // (uniform)
+        b.x = (uint32_t)__builtin_amdgcn_ds_bpermute(2 * nl, (int)braw);       // lane nl / 2 holds columns nl, nl + 1
+        b.y = (uint32_t)__builtin_amdgcn_ds_bpermute(2 * nl + 4, (int)braw);
+      }
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
         uint32_t lo = pack_bf16x2(acc[i][j][4 * g + 0] * alpha, acc[i][j][4 * g + 1] * alpha);
         uint32_t hi = pack_bf16x2(acc[i][j][4 * g + 2] * alpha, acc[i][j][4 * g + 3] * alpha);
         if (bias) {
-          const uint2 b = braw[i * 4 + g];
           lo = pack_bf16x2(__uint_as_float(lo << 16) + __uint_as_float(b.x << 16),
                            __uint_as_float(lo & 0xffff0000u) + __uint_as_float(b.x & 0xffff0000u));
           hi = pack_bf16x2(__uint_as_float(hi << 16) + __uint_as_float(b.y << 16),
