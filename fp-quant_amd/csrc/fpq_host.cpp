@@ -1,20 +1,22 @@
-// The eager calls of the quantized layers without the interpreter between their two or three launches.
+// The eager calls of the quantized layers without the interpreter between their one to three launches.
 //
 // What bounds a decode step is the host: one layer is 8 us of kernels behind 25 us of Python (attribute lookups on the
 // module, tensor constructors, two foreign calls of eleven to fourteen arguments, the checks of every cached constant),
 // a fused decoder block of one token 52 us of kernels behind 170, a quantize operator 6 us behind 18 (most of it
-// operator dispatch).  On this path they take 12, 55 and 7 us from call to call; what is left of a layer's 12 is two
-// launches of 3.3 us, three allocations and the module call around them.  Here the same sequence -- checks, allocations,
-// launches, the hand-over of quantized activations between layers that share an input -- runs as native code on
-// constants that the Python path has worked out once and left in plans (module/host.py):
+// operator dispatch).  On this path they take 8.7, 46 and 6.9 us from call to call: a layer of few rows is one launch
+// (fpq_linear_rows, 4.8 us), the rest of its time three allocations, what publish() makes and the module call around
+// them; with more rows it is two launches of 3.3 us (32 rows, 14336 -> 4096: 13.2 us).  Here the same sequence -- checks,
+// allocations, launches, the hand-over of quantized activations between layers that share an input -- runs as native code
+// on constants that the Python path has worked out once and left in plans (module/host.py):
 //
 //   QuantPlan   on a rotation matrix: its kind, norm and size, the activation scale as fp32
 //   LinearPlan  on a layer's code tensor: its packed operands, alpha, bias and split-K workspace size
 //   GroupPlan   on a WeightGroup: the same for layers whose packed weights lie end to end
 //
 // A plan states the tensors it was made from (object, address, modification counter), and every call compares them.
-// Every function here returns None (False where a plan is missing or outdated and may be made), having launched nothing that is not repeated, whenever a call is not the plain
-// one (tracing, gradients, tensor subclasses, modes, another device, strides): the caller then takes the Python path, which is the definition of the result and makes the plans anew.
+// Every function here returns None (False where a plan is missing or outdated and may be made), having launched nothing
+// that is not repeated, whenever a call is not the plain one (tracing, gradients, tensor subclasses, modes, another
+// device, strides): the caller then takes the Python path, which is the definition of the result and makes the plans anew.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
