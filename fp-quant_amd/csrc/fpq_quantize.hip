@@ -852,7 +852,9 @@ constexpr uint32_t kSiluLdsFirst = 113u << 7;         // bf16 magnitude bits of 
 constexpr uint32_t kSiluLdsCount = 21u * 128u;        // magnitudes up to (not including) 2^7
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
-template <int G, int FMT, int ROT, int ZERO, int PRO, bool QUEST = false>
+// RAGGED: rows that are no whole 256-K blocks, which the generic kernel took before; non-finite chunks get its bytes.  (A
+// kernel of its own: the check in the other one too took 19 registers more, and the NVFP4 slow path's array to scratch.)
+template <int G, int FMT, int ROT, int ZERO, int PRO, bool QUEST, bool RAGGED>
 __global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
     const uint4* __restrict__ x, const uint4* __restrict__ up, uint8_t* __restrict__ codes,
     uint8_t* __restrict__ scales, uint32_t rows, uint32_t n_tiles, float norm, const float* __restrict__ global_scale,
@@ -973,16 +975,17 @@ __global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
     float v[EPL];
     load_rotate(v);
     uint32_t cw[EPL / 8], sbytes = 0u, sb_lo = 0u;
-    bool need_slow = (cpr & 31u) != 0u && chunk_not_finite<EPL>(v);   // (ragged rows were the generic kernel's)
-    if (QUEST && __builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
-      quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    const bool not_finite = RAGGED && chunk_not_finite<EPL>(v);
+    bool need_slow = quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    if constexpr (RAGGED) {
+      need_slow |= not_finite;
+      if (QUEST && __builtin_amdgcn_ballot_w64(not_finite) != 0ull) {
 #pragma unroll
-      for (int i = 0; i < EPL; ++i) {
-        const uint32_t at = 4 * (i & 7);
-        if (v[i] != v[i]) cw[i >> 3] = (cw[i >> 3] & ~(0xfu << at)) | (e2m1_code<ZERO>(v[i]) << at);
+        for (int i = 0; i < EPL; ++i) {
+          const uint32_t at = 4 * (i & 7);
+          if (v[i] != v[i]) cw[i >> 3] = (cw[i >> 3] & ~(0xfu << at)) | (e2m1_code<ZERO>(v[i]) << at);
+        }
       }
-    } else {
-      need_slow |= quantize_chunk<EPL, FMT, ZERO, QUEST>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
     }
     if (!QUEST && __builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
       float u[EPL];
@@ -1022,8 +1025,16 @@ static int launch_tile(const void* x, const void* up, int64_t rows, int64_t cols
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint4*)x, (const uint4*)up,
                        (uint8_t*)codes, (uint8_t*)scales, (uint32_t)rows, (uint32_t)n_tiles, norm, gsp, pro);
   };
-  if (zero_policy == FPQ_ZERO_REFERENCE) go(tile_quantize_kernel<G, FMT, ROT, kZeroReference, PRO, QUEST>);
-  else go(tile_quantize_kernel<G, FMT, ROT, kZeroSigned, PRO, QUEST>);
+  auto by_width = [&](auto zero) {
+    constexpr int Z = decltype(zero)::value;
+    if (cols % 256 != 0) {
+      go(tile_quantize_kernel<G, FMT, ROT, Z, PRO, QUEST, true>);
+    } else if constexpr (FMT == kFmtNv || PRO == kProSiluMul) {   // (whole blocks of MXFP4: the streaming kernel)
+      go(tile_quantize_kernel<G, FMT, ROT, Z, PRO, QUEST, false>);
+    }
+  };
+  if (zero_policy == FPQ_ZERO_REFERENCE) by_width(std::integral_constant<int, kZeroReference>{});
+  else by_width(std::integral_constant<int, kZeroSigned>{});
   return (int)hipGetLastError();
 }
 
@@ -1743,8 +1754,7 @@ __global__ __launch_bounds__(64 * kTileRows) void rmsnorm_tile_quantize_kernel(
     float v[EPL];
     load_rotate(v);
     uint32_t cw[EPL / 8], sbytes = 0u, sb_lo = 0u;
-    bool need_slow = (cpr & 31u) != 0u && chunk_not_finite<EPL>(v);   // (ragged rows were the generic kernel's)
-    need_slow |= quantize_chunk<EPL, FMT, ZERO, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+    const bool need_slow = quantize_chunk<EPL, FMT, ZERO, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
     if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
       float u[EPL];
       load_rotate(u);

@@ -123,7 +123,9 @@ __device__ __forceinline__ void rotate_chunk(float (&v)[EPL], float norm, uint32
 // Whether a rotated chunk holds a NaN or an infinity.  quantize_chunk gives a NaN element the code of its sign and the
 // largest magnitude, and an infinite NVFP4 group the scale byte of a NaN; quantize_chunk_slow, as the generic kernel, leaves
 // a NaN element out (code of zero) and clamps the group's scale.  Kernels that took calls over from the generic one send
-// such chunks there: one NaN in a decode row must not depend on how many rows are quantized with it.
+// such chunks there: one NaN in a decode row must not depend on how many rows are quantized with it.  (Not the norm's tile
+// kernel, 2-5 % slower with the check: a NaN there is the whole block's, and meets a scale of 2^-126 or zero.)  It costs a
+// few rows' GEMM 0-1 % (4 x 4096 x 4096 5.87 -> 5.95 us) and ragged rows 1-4 % (2000 x 3200 4.63 -> 4.70, NVFP4 5.45 -> 5.66).
 template <int EPL>
 __device__ __forceinline__ bool chunk_not_finite(const float (&v)[EPL]) {
   float m = 0.0f;
