@@ -27,9 +27,6 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 #ifndef FPQ_GEMM_WM
 #define FPQ_GEMM_WM 2  // waves along m in the LDS-tiled MXFP4 kernel (2: 4 waves, 4: 8 waves)
 #endif
-#ifndef FPQ_SPLITK_MAX_M
-#define FPQ_SPLITK_MAX_M 64  // largest M served by the weight-streaming split-K kernel
-#endif
 
 __device__ __forceinline__ uint16_t bf16_bits_rne(float f) {
   uint32_t b = __float_as_uint(f);
@@ -152,226 +149,126 @@ __global__ __launch_bounds__(256) void gemm_mxf4_direct_kernel(
 }
 
 // -------------------------------------------------------------------------------------------
-// Weight-streaming kernel for small M (the reference's disabled small-M entry, linear_fns.py:55).
-// The time is the 31 MB weight read, so the job is to keep many loads in flight: a workgroup owns
-// 16 weight rows, its four waves each take a quarter of K and issue all of their loads before the
-// first MFMA; the four partial 16 x (16 TM) tiles are then summed through LDS by wave 0.
-template <int TN, int TM>
-__global__ __launch_bounds__(256) void gemm_mxf4_splitk_kernel(
-    const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xs, int xs_stride,
-    const uint8_t* __restrict__ wq, const uint8_t* __restrict__ ws, int ws_stride,
-    const float* __restrict__ alpha_p, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-    int M, int N, int K) {
-  __shared__ v4f part[3][TN][TM][64];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int r = lane & 15, kb = lane >> 4;
-  const int n0 = blockIdx.x * TN * 16, m0 = blockIdx.y * TM * 16;
-  const int kbytes = K >> 1;
-  const int kq = K >> 2;                       // K range of this wave: [wave * kq, wave * kq + kq)
-  const int steps = kq >> 7;                   // 128 per MFMA
-
-  const uint8_t* wp[TN];
-  const uint8_t* wsp[TN];
-#pragma unroll
-  for (int i = 0; i < TN; ++i) {
-    const int n = min(n0 + i * 16 + r, N - 1);
-    wp[i] = wq + (size_t)n * kbytes + ((wave * kq) >> 1) + kb * 16;
-    wsp[i] = ws + (size_t)n * ws_stride + ((wave * kq) >> 5);
-  }
-  const uint8_t* xp[TM];
-  const uint8_t* xsp[TM];
-#pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const int m = min(m0 + j * 16 + r, M - 1);
-    xp[j] = xq + (size_t)m * kbytes + ((wave * kq) >> 1) + kb * 16;
-    xsp[j] = xs + (size_t)m * xs_stride + ((wave * kq) >> 5);
-  }
-  v4f acc[TN][TM];
-#pragma unroll
-  for (int i = 0; i < TN; ++i)
-#pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  // Loads are issued in batches of 4 * Q K steps: per row tile and group of 4 steps four 16-byte
-  // code loads and ONE 16-byte scale load (the row's 16 scale bytes of those steps; byte 4 u + kb
-  // is this lane's scale in step u), all before the first MFMA of the batch.
-  constexpr int Q = (TN + TM <= 4) ? 2 : 1;
-  for (int s0 = 0; s0 < steps; s0 += 4 * Q) {
-    uint4 a[Q][4][TN], b[Q][4][TM], sa4[Q][TN], sb4[Q][TM];
-#pragma unroll
-    for (int h = 0; h < Q; ++h) {
-      const bool on = s0 + 4 * h < steps;  // steps is a multiple of 4
-#pragma unroll
-      for (int i = 0; i < TN; ++i) {
-        sa4[h][i] = make_uint4(0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu);
-        if (on) sa4[h][i] = *(const uint4*)(wsp[i] + (s0 + 4 * h) * 4);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          a[h][u][i] = make_uint4(0u, 0u, 0u, 0u);
-          if (on) {
-            const v4u ld = __builtin_nontemporal_load((const v4u*)(wp[i] + (s0 + 4 * h + u) * 64));
-            a[h][u][i] = make_uint4(ld.x, ld.y, ld.z, ld.w);
-          }
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        sb4[h][j] = make_uint4(0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu);
-        if (on) sb4[h][j] = *(const uint4*)(xsp[j] + (s0 + 4 * h) * 4);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          b[h][u][j] = make_uint4(0u, 0u, 0u, 0u);
-          if (on) b[h][u][j] = *(const uint4*)(xp[j] + (s0 + 4 * h + u) * 64);
-        }
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < Q; ++h) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-#pragma unroll
-        for (int j = 0; j < TM; ++j) {
-          const uint4 s4 = sb4[h][j];
-          const uint32_t sbw = u == 0 ? s4.x : u == 1 ? s4.y : u == 2 ? s4.z : s4.w;
-          const int sb = (int)((sbw >> (8 * kb)) & 0xffu);
-          const uint4 bq = b[h][u][j];
-          const v8i bv = v8i{(int)bq.x, (int)bq.y, (int)bq.z, (int)bq.w, 0, 0, 0, 0};
-#pragma unroll
-          for (int i = 0; i < TN; ++i) {
-            const uint4 t4 = sa4[h][i];
-            const uint32_t saw = u == 0 ? t4.x : u == 1 ? t4.y : u == 2 ? t4.z : t4.w;
-            const int sa = (int)((saw >> (8 * kb)) & 0xffu);
-            const uint4 aq = a[h][u][i];
-            const v8i av = v8i{(int)aq.x, (int)aq.y, (int)aq.z, (int)aq.w, 0, 0, 0, 0};
-            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc[i][j], 4, 4, 0, sa, 0, sb);
-          }
-        }
-      }
-    }
-  }
-  if (wave > 0) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) part[wave - 1][i][j][lane] = acc[i][j];
-  }
+// Weight-streaming kernels for ONE activation row (the reference's disabled small-M entry, linear_fns.py:55), K a multiple
+// of 2048.  A workgroup owns 16 weight rows, its four waves each take a quarter of K; the partial sums of 16 x 1 meet in
+// LDS.  Twice the workgroups of the 32-row kernel that serves up to 64 rows (gemm_fp4_rows), and loads that touch half as
+// many cache lines each, without its loads a block ahead: which of the two is faster is in gemm_dispatch.
+// Every wave's K quarter is a whole number of batches of four 128-K steps, whose scales a row has in one 16-byte load
+// (NVFP4: two).  All loads of two batches (NVFP4: of one) are issued before the first matrix instruction.
+__device__ __forceinline__ void one_row_store(v4f acc, v4f (&part)[3][64], uint16_t* y, const uint16_t* bias, float alpha,
+                                              int n0, int N, int wave, int lane) {
+  if (wave > 0) part[wave - 1][lane] = acc;
   __syncthreads();
   if (wave == 0) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j)
-        acc[i][j] = ((acc[i][j] + part[0][i][j][lane]) + part[1][i][j][lane]) + part[2][i][j][lane];
-    store_tile<TN, TM>(acc, y, bias, *alpha_p, n0, m0, M, N, r, kb);
+    v4f sum[1][1];
+    sum[0][0] = ((acc + part[0][lane]) + part[1][lane]) + part[2][lane];
+    store_tile<1, 1>(sum, y, bias, alpha, n0, 0, 1, N, lane & 15, lane >> 4);
   }
 }
 
-// The same weight-streaming scheme for NVFP4: a lane's 16 bytes of codes (32 K values) carry two
-// E4M3 scales; per batch of four 128-K steps a row's 32 scale bytes arrive as two 16-byte loads.
-// Dword s of every code load feeds fp16 MFMA s of the step on both operands (K order permuted
-// consistently), after exact in-register dequantization to fp16.
-template <int TN, int TM>
-__global__ __launch_bounds__(256) void gemm_nvf4_splitk_kernel(
-    const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xs, int xs_stride,
-    const uint8_t* __restrict__ wq, const uint8_t* __restrict__ ws, int ws_stride,
-    const float* __restrict__ alpha_p, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-    int M, int N, int K) {
-  __shared__ v4f part[3][TN][TM][64];
+__global__ __launch_bounds__(256) void gemm_mxf4_one_row_kernel(
+    const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xs, const uint8_t* __restrict__ wq,
+    const uint8_t* __restrict__ ws, int ws_stride, const float* __restrict__ alpha_p, const uint16_t* __restrict__ bias,
+    uint16_t* __restrict__ y, int N, int K) {
+  __shared__ v4f part[3][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, kb = lane >> 4;
-  const int n0 = blockIdx.x * TN * 16, m0 = blockIdx.y * TM * 16;
-  const int kbytes = K >> 1;
+  const int n0 = blockIdx.x * 16;
   const int kq = K >> 2;                       // K range of this wave: [wave * kq, wave * kq + kq)
-  const int steps = kq >> 7;                   // 128 K per step (four fp16 MFMAs)
-
-  const uint8_t* wp[TN];
-  const uint8_t* wsp[TN];
+  const int steps = kq >> 7;                   // 128 per matrix instruction
+  const int n = min(n0 + r, N - 1);
+  const uint8_t* wp = wq + (size_t)n * (K >> 1) + ((wave * kq) >> 1) + kb * 16;
+  const uint8_t* wsp = ws + (size_t)n * ws_stride + ((wave * kq) >> 5);
+  const uint8_t* xp = xq + ((wave * kq) >> 1) + kb * 16;
+  const uint8_t* xsp = xs + ((wave * kq) >> 5);
+  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < steps; s0 += 8) {
+    uint4 a[2][4], b[2][4], sa4[2], sb4[2];
 #pragma unroll
-  for (int i = 0; i < TN; ++i) {
-    const int n = min(n0 + i * 16 + r, N - 1);
-    wp[i] = wq + (size_t)n * kbytes + ((wave * kq) >> 1) + kb * 16;
-    wsp[i] = ws + (size_t)n * ws_stride + ((wave * kq) >> 4);
-  }
-  const uint8_t* xp[TM];
-  const uint8_t* xsp[TM];
-#pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const int m = min(m0 + j * 16 + r, M - 1);
-    xp[j] = xq + (size_t)m * kbytes + ((wave * kq) >> 1) + kb * 16;
-    xsp[j] = xs + (size_t)m * xs_stride + ((wave * kq) >> 4);
-  }
-  v4f acc[TN][TM];
-#pragma unroll
-  for (int i = 0; i < TN; ++i)
-#pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  for (int s0 = 0; s0 < steps; s0 += 4) {  // steps is a multiple of 4
-    uint4 a[4][TN], b[4][TM], sa8[2][TN], sb8[2][TM];
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-      sa8[0][i] = *(const uint4*)(wsp[i] + s0 * 8);
-      sa8[1][i] = *(const uint4*)(wsp[i] + s0 * 8 + 16);
+    for (int h = 0; h < 2; ++h) {
+      const bool on = s0 + 4 * h < steps;  // steps is a multiple of 4
+      sa4[h] = sb4[h] = make_uint4(0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu, 0x7f7f7f7fu);
+      if (on) sa4[h] = *(const uint4*)(wsp + (s0 + 4 * h) * 4);
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const v4u ld = __builtin_nontemporal_load((const v4u*)(wp[i] + (s0 + u) * 64));
-        a[u][i] = make_uint4(ld.x, ld.y, ld.z, ld.w);
+        a[h][u] = make_uint4(0u, 0u, 0u, 0u);
+        if (on) {
+          const v4u ld = __builtin_nontemporal_load((const v4u*)(wp + (s0 + 4 * h + u) * 64));
+          a[h][u] = make_uint4(ld.x, ld.y, ld.z, ld.w);
+        }
+      }
+      if (on) sb4[h] = *(const uint4*)(xsp + (s0 + 4 * h) * 4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        b[h][u] = make_uint4(0u, 0u, 0u, 0u);
+        if (on) b[h][u] = *(const uint4*)(xp + (s0 + 4 * h + u) * 64);
       }
     }
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      sb8[0][j] = *(const uint4*)(xsp[j] + s0 * 8);
-      sb8[1][j] = *(const uint4*)(xsp[j] + s0 * 8 + 16);
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t sbw[4] = {sb4[h].x, sb4[h].y, sb4[h].z, sb4[h].w}, saw[4] = {sa4[h].x, sa4[h].y, sa4[h].z, sa4[h].w};
 #pragma unroll
-      for (int u = 0; u < 4; ++u) b[u][j] = *(const uint4*)(xp[j] + (s0 + u) * 64);
+      for (int u = 0; u < 4; ++u) {   // byte kb of dword u is this lane's scale
+        const v8i av = v8i{(int)a[h][u].x, (int)a[h][u].y, (int)a[h][u].z, (int)a[h][u].w, 0, 0, 0, 0};
+        const v8i bv = v8i{(int)b[h][u].x, (int)b[h][u].y, (int)b[h][u].z, (int)b[h][u].w, 0, 0, 0, 0};
+        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, acc, 4, 4, 0, (int)((saw[u] >> (8 * kb)) & 0xffu), 0,
+                                                               (int)((sbw[u] >> (8 * kb)) & 0xffu));
+      }
     }
+  }
+  one_row_store(acc, part, y, bias, *alpha_p, n0, N, wave, lane);
+}
+
+// NVFP4: a lane's 16 bytes of codes (32 K values) carry two E4M3 scales; dword s of every code load feeds fp16 matrix
+// instruction s of the step on both operands (K order permuted consistently), after exact dequantization to fp16.
+__global__ __launch_bounds__(256) void gemm_nvf4_one_row_kernel(
+    const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xs, const uint8_t* __restrict__ wq,
+    const uint8_t* __restrict__ ws, int ws_stride, const float* __restrict__ alpha_p, const uint16_t* __restrict__ bias,
+    uint16_t* __restrict__ y, int N, int K) {
+  __shared__ v4f part[3][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r = lane & 15, kb = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const int kq = K >> 2;                       // K range of this wave: [wave * kq, wave * kq + kq)
+  const int steps = kq >> 7;                   // 128 K per step (four fp16 matrix instructions)
+  const int n = min(n0 + r, N - 1);
+  const uint8_t* wp = wq + (size_t)n * (K >> 1) + ((wave * kq) >> 1) + kb * 16;
+  const uint8_t* wsp = ws + (size_t)n * ws_stride + ((wave * kq) >> 4);
+  const uint8_t* xp = xq + ((wave * kq) >> 1) + kb * 16;
+  const uint8_t* xsp = xs + ((wave * kq) >> 4);
+  v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < steps; s0 += 4) {  // steps is a multiple of 4
+    uint4 a[4], b[4], sa8[2], sb8[2];
+    sa8[0] = *(const uint4*)(wsp + s0 * 8);
+    sa8[1] = *(const uint4*)(wsp + s0 * 8 + 16);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const v4u ld = __builtin_nontemporal_load((const v4u*)(wp + (s0 + u) * 64));
+      a[u] = make_uint4(ld.x, ld.y, ld.z, ld.w);
+    }
+    sb8[0] = *(const uint4*)(xsp + s0 * 8);
+    sb8[1] = *(const uint4*)(xsp + s0 * 8 + 16);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) b[u] = *(const uint4*)(xp + (s0 + u) * 64);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       // step u: scale bytes 8 (u % 2) + 2 kb and + 1 of 16-byte load u / 2
-      v8h bh[TM][4];
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        const uint4 s4 = sb8[u >> 1][j];
+      auto two = [&](const uint4& s4) {
         const uint32_t lo = (u & 1) ? s4.z : s4.x, hi = (u & 1) ? s4.w : s4.y;
-        const uint32_t two = ((kb & 2) ? hi : lo) >> (16 * (kb & 1));
-        const uint4 c = b[u][j];
-        bh[j][0] = dequant8_f16_s(c.x, e4m3_pair_f16(two));
-        bh[j][1] = dequant8_f16_s(c.y, e4m3_pair_f16(two));
-        bh[j][2] = dequant8_f16_s(c.z, e4m3_pair_f16(two >> 8));
-        bh[j][3] = dequant8_f16_s(c.w, e4m3_pair_f16(two >> 8));
-      }
+        return ((kb & 2) ? hi : lo) >> (16 * (kb & 1));
+      };
+      const uint32_t ta = two(sa8[u >> 1]), tb = two(sb8[u >> 1]);
+      const uint32_t aw[4] = {a[u].x, a[u].y, a[u].z, a[u].w}, bw[4] = {b[u].x, b[u].y, b[u].z, b[u].w};
+      v8h bh[4];   // (converted ahead of the matrix instructions: 8 % faster than in turn with the weights')
 #pragma unroll
-      for (int i = 0; i < TN; ++i) {
-        const uint4 s4 = sa8[u >> 1][i];
-        const uint32_t lo = (u & 1) ? s4.z : s4.x, hi = (u & 1) ? s4.w : s4.y;
-        const uint32_t two = ((kb & 2) ? hi : lo) >> (16 * (kb & 1));
-        const uint4 c = a[u][i];
-        const uint32_t cw[4] = {c.x, c.y, c.z, c.w};
+      for (int s = 0; s < 4; ++s) bh[s] = dequant8_f16_s(bw[s], e4m3_pair_f16(tb >> (8 * (s >> 1))));
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const v8h ah = dequant8_f16_s(cw[s], e4m3_pair_f16(two >> (8 * (s >> 1))));
-#pragma unroll
-          for (int j = 0; j < TM; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[j][s], acc[i][j], 0, 0, 0);
-        }
-      }
+      for (int s = 0; s < 4; ++s)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8_f16_s(aw[s], e4m3_pair_f16(ta >> (8 * (s >> 1)))), bh[s], acc,
+                                                     0, 0, 0);
     }
   }
-  if (wave > 0) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) part[wave - 1][i][j][lane] = acc[i][j];
-  }
-  __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j)
-        acc[i][j] = ((acc[i][j] + part[0][i][j][lane]) + part[1][i][j][lane]) + part[2][i][j][lane];
-    store_tile<TN, TM>(acc, y, bias, *alpha_p, n0, m0, M, N, r, kb);
-  }
+  one_row_store(acc, part, y, bias, *alpha_p, n0, N, wave, lane);
 }
 
 // -------------------------------------------------------------------------------------------
@@ -854,6 +751,11 @@ __global__ __launch_bounds__(256) void gemm_nvf4_lds_kernel(
   wave_quadrant_store<BN, BM, 2 * L::kStage>(acc, smem, y, bias, alpha_p, n_blk, m_blk, wn, wm, wave, lane, M, N);
 }
 
+// fpq_gemm_stream.hip: at most 64 activation rows
+int gemm_fp4_rows(bool nv, const void* xq, const void* xs, int64_t xs_stride, const void* wq, const void* ws,
+                  int64_t ws_stride, const float* alpha, const void* bias, void* y, int64_t M, int64_t N, int64_t K,
+                  hipStream_t stream);
+
 template <int FMT>
 static int gemm_dispatch(const void* xq, const void* xs, int64_t xs_stride, const void* wq,
                          const void* ws, int64_t ws_stride, const float* alpha, const void* bias,
@@ -885,6 +787,26 @@ static int gemm_dispatch(const void* xq, const void* xs, int64_t xs_stride, cons
     }                                                                                              \
   } while (0)
 
+  // At most 64 activation rows: gemm_fp4_rows, except where a kernel here is faster (us here / there, weights from HBM):
+  // * one row, K a multiple of 2048: 16 weight rows per workgroup.  MXFP4 always (N = 256 / 4096 / 28672: K = 4096 3.5 /
+  //   4.8, 4.3 / 5.4, 14.2 / 15.3; K = 14336, N = 4096 10.3 / 11.8); NVFP4 up to 1024 weight rows (N = 256, K = 8192 6.2 /
+  //   9.2), and below K = 8192 except between one and two 32-row tiles per CU (N = 4096 / 28672, K = 4096 5.5 / 6.4, 17.7 /
+  //   18.4; but N = 14336 12.0 / 10.8, and K = 14336, N = 6144 21.9 / 16.3);
+  // * up to 16 rows and K <= 512, where there is nothing to share between its four waves (MXFP4, one row, N = 4096: K = 96
+  //   2.2 / 2.8, K = 384 2.6 / 3.0; N = 16384, K = 512 3.8 / 3.9): the direct kernel.
+  const int64_t cus = device_cus();
+  const bool one_row = M == 1 && K % 2048 == 0 && ws_stride % 16 == 0 && !((uintptr_t)xs & 15u) && !((uintptr_t)ws & 15u) &&
+                       (FMT == 0 || N <= 1024 || (K < 8192 && (N <= 32 * cus || N > 64 * cus)));
+  if (one_row) {
+    hipLaunchKernelGGL(FMT == 0 ? gemm_mxf4_one_row_kernel : gemm_nvf4_one_row_kernel, dim3((unsigned)((N + 15) / 16)),
+                       dim3(256), 0, stream, (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws,
+                       (int)ws_stride, alpha, (const uint16_t*)bias, (uint16_t*)y, (int)N, (int)K);
+    return (int)hipGetLastError();
+  }
+  if (M > 16 || K > 512) {
+    const int st = gemm_fp4_rows(FMT == 1, xq, xs, xs_stride, wq, ws, ws_stride, alpha, bias, y, M, N, K, stream);
+    if (st != FPQ_E_UNSUPPORTED) return st;
+  }
   if (FMT == 1 && M > 64 && K % kKS == 0 && xs_stride % 16 == 0 && ws_stride % 16 == 0 &&
       !((uintptr_t)xs & 15u) && !((uintptr_t)ws & 15u) && N * (K / 2) < ((int64_t)1 << 32) &&
       M * (K / 2) < ((int64_t)1 << 32)) {
@@ -914,46 +836,6 @@ static int gemm_dispatch(const void* xq, const void* xs, int64_t xs_stride, cons
                        (const uint16_t*)bias, (uint16_t*)y, (int)M, (int)N, (int)K, tiles_m);
     return (int)hipGetLastError();
   }
-#define FPQ_SPLITK(TNN, TMM)                                                                       \
-  do {                                                                                             \
-    const dim3 grid((unsigned)((N + TNN * 16 - 1) / (TNN * 16)),                                   \
-                    (unsigned)((M + TMM * 16 - 1) / (TMM * 16)));                                  \
-    hipLaunchKernelGGL((gemm_mxf4_splitk_kernel<TNN, TMM>), grid, dim3(256), 0, stream,            \
-                       (const uint8_t*)xq, (const uint8_t*)xs, (int)xs_stride, (const uint8_t*)wq, \
-                       (const uint8_t*)ws, (int)ws_stride, alpha, (const uint16_t*)bias,           \
-                       (uint16_t*)y, (int)M, (int)N, (int)K);                                      \
-    return (int)hipGetLastError();                                                                 \
-  } while (0)
-  // K % 2048 == 0: every wave's K quarter is a whole number of 4-step batches and every 16-byte
-  // scale load is aligned (scale strides and bases must be 16-byte multiples too)
-#define FPQ_SPLITK_NV(TNN, TMM)                                                                    \
-  do {                                                                                             \
-    const dim3 grid((unsigned)((N + TNN * 16 - 1) / (TNN * 16)),                                   \
-                    (unsigned)((M + TMM * 16 - 1) / (TMM * 16)));                                  \
-    hipLaunchKernelGGL((gemm_nvf4_splitk_kernel<TNN, TMM>), grid, dim3(256), 0, stream,            \
-                       (const uint8_t*)xq, (const uint8_t*)xs, (int)xs_stride, (const uint8_t*)wq, \
-                       (const uint8_t*)ws, (int)ws_stride, alpha, (const uint16_t*)bias,           \
-                       (uint16_t*)y, (int)M, (int)N, (int)K);                                      \
-    return (int)hipGetLastError();                                                                 \
-  } while (0)
-  if (FMT == 1 && K % 2048 == 0 && M <= 64 && xs_stride % 16 == 0 && ws_stride % 16 == 0 &&
-      !((uintptr_t)xs & 15u) && !((uintptr_t)ws & 15u)) {
-    if (M == 1) FPQ_SPLITK_NV(1, 1);
-    if (M <= 16) FPQ_SPLITK_NV(2, 1);
-    if (M <= 32) FPQ_SPLITK_NV(2, 2);
-    FPQ_SPLITK_NV(2, 4);
-  }
-#undef FPQ_SPLITK_NV
-  if (FMT == 0 && K % 2048 == 0 && M <= FPQ_SPLITK_MAX_M && xs_stride % 16 == 0 && ws_stride % 16 == 0 &&
-      !((uintptr_t)xs & 15u) && !((uintptr_t)ws & 15u)) {
-    // 32 weight rows per workgroup once there is more than one activation row: halves the
-    // re-reading of the activations from L2 (measured best among 16 / 32 / 64 rows)
-    if (M == 1) FPQ_SPLITK(1, 1);
-    if (M <= 16) FPQ_SPLITK(2, 1);
-    if (M <= 32) FPQ_SPLITK(2, 2);
-    FPQ_SPLITK(2, 4);
-  }
-#undef FPQ_SPLITK
   if (M <= 16) {
     FPQ_GEMM(1, 1, 4, 1);
   } else if (M <= 32) {

@@ -110,6 +110,13 @@ __device__ __forceinline__ _Float16 e4m3_byte_f16(uint32_t d, int byte) {   // b
   const v2h h = (byte & 1) ? e4m3_odd_f16(d) : e4m3_even_f16(d);
   return (byte & 2) ? h.y : h.x;
 }
+// ... with the byte's sign (kernels on operands that no kernel of this library has re-tiled)
+__device__ __forceinline__ _Float16 e4m3_signed_f16(uint32_t d, int byte) {
+  uint32_t h = (byte & 1) ? ((d >> 1) & 0x3f803f80u) | (d & 0x80008000u) : ((d << 7) & 0x3f803f80u) | ((d << 8) & 0x80008000u);
+  asm("" : "+v"(h));
+  const v2h v = __builtin_bit_cast(v2h, h);
+  return (byte & 2) ? v.y : v.x;
+}
 __device__ __forceinline__ v8h dequant8_f16_h(uint32_t codes, _Float16 s) { return dequant8_f16_s(codes, v2h{s, s}); }
 // ... and one half of that: codes 4 part .. 4 part + 3
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));

@@ -63,6 +63,15 @@ struct FewRows {
   float norm;
   int xk;                    // a multiple of 32 and of the rotation's size; K is padded to whole blocks
 };
+// IN = RowMajor: both operands as the quantize operators write them, codes [rows, k / 2] and scales [rows, stride] with the
+// strides multiples of four.  A lane takes the same 16 bytes of codes of a row, and the same scale bytes, as from the
+// packed layout, so the sums are the same bit for bit; only the addresses differ.  See launch_rows.
+// RAGGED: k is no multiple of 256 (but one of 32).  The last block's groups past k read the row's start and are replaced.
+template <bool RAGGED>
+struct RowMajor {
+  int k;
+  uint32_t xs_stride, ws_stride;
+};
 // 32-element chunks a wave quantizes at most: one per lane and pass
 constexpr int few_rows_passes(bool silu) { return silu ? 1 : 2; }
 constexpr int few_rows_chunks(bool silu) { return 64 * few_rows_passes(silu); }
@@ -75,6 +84,7 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
     const uint16_t* residual_all, uint16_t* y, int M_all, int N, int K, int bps, int ksplit,
     float* partial, unsigned* counters, const OutSegments seg, const IN in) {
   constexpr bool kFew = std::is_same_v<IN, FewRows>;
+  constexpr bool kRagged = std::is_same_v<IN, RowMajor<true>>, kRow = kRagged || std::is_same_v<IN, RowMajor<false>>;
   static_assert(!kFew || (NT == 1 && MT == 1), "few rows: one tile");
   static_assert(NW == 4, "a wave owns a quarter of every tile");
   // More than 32 MT activation rows: blockIdx.z numbers slabs of 32 MT rows, each a product of its own
@@ -115,6 +125,12 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     const int rt = min(rtg * NT + i, rt_n - 1);
+    if constexpr (kRow) {
+      const int row = min(rt * 32 + (lane & 31), N - 1);
+      wcode[i] = wq + (size_t)row * (in.k >> 1) + (lane >> 5) * 16;
+      wscale[i] = ws + (size_t)row * in.ws_stride;
+      continue;
+    }
     wcode[i] = wq + (size_t)rt * nu * 1024 + lane * 16;
     wscale[i] = ws + (size_t)rt * nkb * kSB + lane * (kSB / 64);
   }
@@ -126,6 +142,12 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     if constexpr (kFew) break;
+    if constexpr (kRow) {
+      const int row = 32 * j + (lane & 31) < M ? 32 * j + (lane & 31) : 0;
+      xcode[j] = xq_all + (size_t)row * (in.k >> 1) + (lane >> 5) * 16;
+      xscale[j] = xs_all + (size_t)row * in.xs_stride;
+      continue;
+    }
     const int l = (lane & 31) < M - 32 * j ? lane : (lane & 32);
     const int jt = min(j, (M - 1) >> 5);
     xcode[j] = xq + (size_t)jt * nu * 1024 + l * 16;
@@ -143,12 +165,57 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // the compiler can no longer count which of them are still in flight and waits for all.
   uint4 a[DB][4][NT], b[DB][4][MT];
   uint2 sa[DB][NT], sb[DB][MT];   // MXFP4 uses .x only
+  // Row-major: a row's scale bytes of a block as they lie (MXFP4: .x and .y), of which run_block takes the lane's
+  uint4 sa_row[kRow ? DB : 1][NT], sb_row[kRow ? DB : 1][MT];
+  int tail_steps = 4;   // K steps of the last block in which this lane has a group
+  if constexpr (kRagged) tail_steps = ((in.k >> 5) - (nkb - 1) * 8 - (lane >> 5) + 1) >> 1;
+  auto row_scales = [&](const uint8_t* row, int kb, uint32_t stride) __attribute__((always_inline)) {
+    typedef uint32_t v2u_4 __attribute__((ext_vector_type(2), aligned(4)));
+    typedef uint32_t v4u_4 __attribute__((ext_vector_type(4), aligned(4)));
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if constexpr (kRagged) {   // dword by dword: the last ones of the block may lie past the row
+      const uint32_t last = stride - 4, at = (uint32_t)kb * (NV ? 16 : 8);
+      v.x = *(const uint32_t*)(row + min(at, last));
+      v.y = *(const uint32_t*)(row + min(at + 4, last));
+      if constexpr (NV) {
+        v.z = *(const uint32_t*)(row + min(at + 8, last));
+        v.w = *(const uint32_t*)(row + min(at + 12, last));
+      }
+    } else if constexpr (NV) {
+      const v4u_4 d = *(const v4u_4*)(row + (size_t)kb * 16);
+      v = make_uint4(d.x, d.y, d.z, d.w);
+    } else {
+      const v2u_4 d = *(const v2u_4*)(row + (size_t)kb * 8);
+      v.x = d.x;
+      v.y = d.y;
+    }
+    return v;
+  };
+  auto row_offset = [&](int kb, int u) __attribute__((always_inline)) {   // of the lane's codes of K step u
+    if constexpr (kRagged) return kb < nkb - 1 || u < tail_steps ? kb * 128 + u * 32 : -(lane >> 5) * 16;
+    else return kb * 128 + u * 32;
+  };
   const int t_last = nblk > 0 ? nblk - 1 : 0;
   // (the lambdas must be inlined whatever their size: a call would pin the register arrays they capture
   // to memory)
   auto load_block = [&](auto slot, int t) __attribute__((always_inline)) {
     constexpr int s = decltype(slot)::value;
     const int kb = min(first + NW * min(t, t_last), nkb - 1);
+    if constexpr (kRow) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[s][u][i] = *(const uint4*)(wcode[i] + row_offset(kb, u));
+        sa_row[s][i] = row_scales(wscale[i], kb, in.ws_stride);
+      }
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b[s][u][j] = *(const uint4*)(xcode[j] + row_offset(kb, u));
+        sb_row[s][j] = row_scales(xscale[j], kb, in.xs_stride);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
 #pragma unroll
@@ -171,6 +238,10 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // NVFP4: activation row tiles whose fp16 operands are held at a time (four tiles: two and two, the
   // weight operand is converted once more; all four at once left the register file)
   constexpr int kJB = (MT == 4) ? 2 : MT;
+  auto scale_f16 = [](uint32_t d, int byte) __attribute__((always_inline)) {
+    if constexpr (kRow) return e4m3_signed_f16(d, byte);
+    else return e4m3_byte_f16(d, byte);
+  };
   auto compute_block = [&](auto slot) __attribute__((always_inline)) {
     constexpr int s = decltype(slot)::value;
 #define FPQ_STREAM_STEP(U)                                                                              \
@@ -181,7 +252,7 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
         const uint4 bq = b[s][U][j0 + j];                                                               \
         const uint32_t bw[4] = {bq.x, bq.y, bq.z, bq.w};                                                \
         const uint32_t bsc = (U) < 2 ? sb[s][j0 + j].x : sb[s][j0 + j].y;                               \
-        const _Float16 bsh[2] = {e4m3_byte_f16(bsc, 2 * ((U) & 1)), e4m3_byte_f16(bsc, 2 * ((U) & 1) + 1)};   \
+        const _Float16 bsh[2] = {scale_f16(bsc, 2 * ((U) & 1)), scale_f16(bsc, 2 * ((U) & 1) + 1)};           \
         _Pragma("unroll") for (int s4 = 0; s4 < 4; ++s4)                                                \
           bh[j][s4] = dequant8_f16_h(bw[s4], bsh[s4 >> 1]);                                             \
       }                                                                                                 \
@@ -189,7 +260,7 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
         const uint4 aq = a[s][U][i];                                                                    \
         const uint32_t aw[4] = {aq.x, aq.y, aq.z, aq.w};                                                \
         const uint32_t asc = (U) < 2 ? sa[s][i].x : sa[s][i].y;                                         \
-        const _Float16 ash[2] = {e4m3_byte_f16(asc, 2 * ((U) & 1)), e4m3_byte_f16(asc, 2 * ((U) & 1) + 1)};   \
+        const _Float16 ash[2] = {scale_f16(asc, 2 * ((U) & 1)), scale_f16(asc, 2 * ((U) & 1) + 1)};           \
         _Pragma("unroll") for (int s4 = 0; s4 < 4; ++s4) {                                              \
           const v8h ah = dequant8_f16_h(aw[s4], ash[s4 >> 1]);                                          \
           _Pragma("unroll") for (int j = 0; j < kJB; ++j)                                               \
@@ -287,6 +358,33 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
       for (int u = 0; u < 4; ++u) b[s][u][0] = *(const uint4*)&few_codes[wave][(blk * 8 + 2 * u + kh) * 16];
       if constexpr (NV) sb[s][0] = *(const uint2*)&few_scales[wave][blk * 16 + kh * 8];
       else sb[s][0].x = *(const uint32_t*)&few_scales[wave][blk * 8 + kh * 4];
+    }
+    if constexpr (kRow) {
+      constexpr int s = decltype(slot)::value;
+      const int kh = lane >> 5;
+      const uint32_t sel = NV ? (kh ? 0x07060302u : 0x05040100u) : (kh ? 0x07050301u : 0x06040200u);
+      auto take = [&](const uint4& v) __attribute__((always_inline)) {
+        return make_uint2(__builtin_amdgcn_perm(v.y, v.x, sel), NV ? __builtin_amdgcn_perm(v.w, v.z, sel) : 0u);
+      };
+#pragma unroll
+      for (int i = 0; i < NT; ++i) sa[s][i] = take(sa_row[s][i]);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) sb[s][j] = take(sb_row[s][j]);
+      if (kRagged && first + NW * t == nkb - 1) {
+        // Past k: zero codes on the activations' side, and scale bytes that are no NaN on both (an E8M0 0xff beyond the
+        // end would make NaN of them; the E4M3 bytes are taken as finite whatever they are).
+        const uint32_t keep = tail_steps >= 4 ? 0xffffffffu : (1u << (8 * tail_steps)) - 1u;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+          if constexpr (!NV) sa[s][i].x &= keep;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          if constexpr (!NV) sb[s][j].x &= keep;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (u >= tail_steps) b[s][u][j] = make_uint4(0u, 0u, 0u, 0u);
+        }
+      }
     }
     if constexpr (kPipelined) compute_block_nv(slot);
     else compute_block(slot);
@@ -736,6 +834,48 @@ int gemm_fp4_stream_slabs(bool nv, const void* xq, const void* xs, const void* w
             : launch_stream<false>(xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, nullptr, 0, seg, stream, slab_rows);
 }
 
+
+// At most 64 activation rows, both operands row-major (the GEMM operators): the kernel above on rows instead of packed
+// blocks, without a K split across workgroups (there is no workspace).  An operand load touches the lines of 32 rows, 32
+// bytes each, where a packed one reads a kilobyte end to end, and the texture path bounds it (about 38 cycles per load;
+// NVFP4: the conversions, like the packed kernel's).  The kernels that it replaced took K in whole multiples of 2048 with
+// every load of a wave's quarter ahead of its matrix instructions but none across them, any other K a step at a time
+// (us, before / now, weights from HBM): NVFP4 64 x 6144 x 4096 15.7 / 11.1, 20 x 28672 x 14336 96 / 69, 4 x 23552 x 6656 62 /
+// 23, 40 x 2440 x 6784 94 / 18; MXFP4 64 x 6144 x 4096 13.3 / 9.7, 32 x 4096 x 14336 22.6 / 16.7, 1 x 10240 x 8704 42.7 /
+// 16.1, 64 x 4096 x 1280 12.9 / 4.9.  Two blocks in flight per wave; one where a wave has hardly two (below eight blocks:
+// 64 x 4096 x 1280 4.9 against 5.6, 14 x 28672 x 1024 6.1 against 9.1; at eight, 64 x 28672 x 2048 16.5 against 15.9).
+// Four, eight waves per workgroup, and two weight tiles per workgroup measured slower over most of the range.
+constexpr int64_t kRowMajorMaxRows = 64;
+template <bool NV>
+static int launch_rows(const void* xq, const void* xs, int64_t xs_stride, const void* wq, const void* ws, int64_t ws_stride,
+                       const float* alpha, const void* bias, void* y, int64_t M, int64_t N, int64_t K, hipStream_t stream) {
+  const int64_t nkb = (K + 255) / 256, tiles = (N + 31) / 32;
+  auto go = [&](auto ragged) {
+    typedef RowMajor<decltype(ragged)::value> In;
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(256), 0, stream, (const uint8_t*)xq, (const uint8_t*)xs,
+                         (const uint8_t*)wq, (const uint8_t*)ws, alpha, (const uint16_t*)bias, (const uint16_t*)nullptr,
+                         (uint16_t*)y, (int)M, (int)N, (int)(nkb * 256), (int)nkb, 1, (float*)nullptr, (unsigned*)nullptr,
+                         OutSegments{}, In{(int)K, (uint32_t)xs_stride, (uint32_t)ws_stride});
+    };
+    if (M > 32) nkb < 8 ? launch(gemm_fp4_stream_kernel<1, 2, 1, 4, NV, In>) : launch(gemm_fp4_stream_kernel<1, 2, 2, 4, NV, In>);
+    else nkb < 8 ? launch(gemm_fp4_stream_kernel<1, 1, 1, 4, NV, In>) : launch(gemm_fp4_stream_kernel<1, 1, 2, 4, NV, In>);
+    return (int)hipGetLastError();
+  };
+  return K % 256 != 0 ? go(std::true_type{}) : go(std::false_type{});
+}
+
+// Arguments are validated by the caller (fpq_gemm.hip); FPQ_E_UNSUPPORTED, with nothing launched: a shape or an alignment
+// that this kernel does not take.
+int gemm_fp4_rows(bool nv, const void* xq, const void* xs, int64_t xs_stride, const void* wq, const void* ws,
+                  int64_t ws_stride, const float* alpha, const void* bias, void* y, int64_t M, int64_t N, int64_t K,
+                  hipStream_t stream) {
+  if (M > kRowMajorMaxRows || K % 32 != 0 || ((xs_stride | ws_stride) & 3) || (((uintptr_t)xs | (uintptr_t)ws) & 3u) ||
+      xs_stride >= ((int64_t)1 << 31) || ws_stride >= ((int64_t)1 << 31))
+    return FPQ_E_UNSUPPORTED;
+  return nv ? launch_rows<true>(xq, xs, xs_stride, wq, ws, ws_stride, alpha, bias, y, M, N, K, stream)
+            : launch_rows<false>(xq, xs, xs_stride, wq, ws, ws_stride, alpha, bias, y, M, N, K, stream);
+}
 
 // Few activation rows quantized by the GEMM itself.  A layer of one token is two kernels of about 4 us each, of which
 // most is the start and the end of a kernel, and two launches of 3.3 us host time; here every workgroup repeats the
