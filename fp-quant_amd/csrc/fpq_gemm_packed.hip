@@ -24,6 +24,7 @@
 #include "../../include/fpq.h"
 #include "fpq_device.h"
 #include "fpq_gemm_epilogue.h"
+#include "fpq_quantize_chunk.h"
 
 namespace fpq {
 
@@ -170,6 +171,127 @@ __device__ __forceinline__ void barrier_lds_but() {
   asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// The epilogue of a GEMM whose weight rows are a gate and an up projection's, for the gated MLP's down projection:
+//   bf16(bf16(silu(gate)) * up), rotated and quantized into the packed layout of down's activations, to the bit what
+// writing gate and up and quantizing them afterwards gives.  A wave's TN tiles are TN / 2 of gate and the same TN / 2
+// of up, so the product is formed in its registers; it goes through LDS as bf16 [m][channel] (which two waves share)
+// to lanes that own 32 channels of a row, four lanes a row's 128.
+//
+// What it saves is memory traffic: at 8192 x 14336, K = 4096 the GEMM wrote 470 MB in 434 us and the SiLU*up quantizer
+// (108 us, 5 TB/s) read them back; with this epilogue the GEMM takes 477 us and writes 62 MB.  (Its vector work, about
+// 1500 instructions per wave, runs beside the other workgroup's matrix instructions on the same CU.)
+struct GatedOut {
+  uint8_t *codes, *scales;
+  const uint16_t* silu;     // table of bf16(silu(g))
+  const float* gs;          // NVFP4: the activations' global scale
+  float norm;
+  int rot, g, channels;     // channels: a multiple of 256
+};
+struct PlainOut {};
+constexpr int gated_lds_bytes(int channels, int rows) {
+  return 2 * (int)kSiluLdsCount * 4 + 1024 + rows * (channels * 2 + 16);
+}
+
+template <int TN, int TM, int WN, int WM, bool NV>
+__device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint8_t* smem, const GatedOut& out, float alpha,
+                                                 int tile_n, int m_blk, int wn, int wm, int wave, int lane, int M) {
+  constexpr int CN = TN / 2, kCols = WN * CN * 32, kRows = WM * TM * 32, kThreads = WN * WM * 64;
+  constexpr int kStride = kCols * 2 + 16, FMT = NV ? kFmtNv : kFmtMx;
+  static_assert(kCols == 128, "four lanes hold a row's channels");
+  float* const silu = (float*)smem;
+  float2* const lut = (float2*)(smem + 2 * kSiluLdsCount * 4);
+  uint8_t* const stage = smem + 2 * kSiluLdsCount * 4 + 1024;
+  __syncthreads();                                   // every wave is done reading operands
+  silu_table_to_lds<kThreads>(silu, out.silu);
+  float gs = 1.0f, rg = 1.0f;
+  bool nv_fast = true;
+  if constexpr (NV) {
+    gs = *out.gs;
+    rg = gs == 0.0f ? 0.0f : 1.0f / gs;
+    nv_fast = nv_global_scale_fast(gs);
+    if (threadIdx.x < 128) lut[threadIdx.x] = nv_division(threadIdx.x, rg, nv_fast);
+  }
+  __syncthreads();
+  const int r32 = lane & 31, kh = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < CN; ++i) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {   // eight values at a time
+        uint32_t gate[4], up[4];
+        float sv[8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int v = 8 * h + 2 * k;
+          gate[k] = pack_bf16x2(acc[i][j][v] * alpha, acc[i][j][v + 1] * alpha);
+          up[k] = pack_bf16x2(acc[i + CN][j][v] * alpha, acc[i + CN][j][v + 1] * alpha);
+        }
+        silu_lookup(gate, sv, (lds_f32*)silu, out.silu);
+        uint8_t* const at = stage + (wm * TM * 32 + j * 32 + r32) * kStride + (wn * CN * 32 + i * 32 + 16 * h + 4 * kh) * 2;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          *(uint2*)(at + 16 * g) = make_uint2(pack_bf16x2(sv[4 * g] * bf16_lo(up[2 * g]), sv[4 * g + 1] * bf16_hi(up[2 * g])),
+                                              pack_bf16x2(sv[4 * g + 2] * bf16_lo(up[2 * g + 1]), sv[4 * g + 3] * bf16_hi(up[2 * g + 1])));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  __syncthreads();
+  const int c = lane & 3, units = out.channels >> 6, unit = tile_n * 2 + (c >> 1);
+  const int padded = (M + 31) & ~31;
+  auto rows = [&](auto rot_g, auto rot) __attribute__((always_inline)) {
+    constexpr int G = decltype(rot_g)::value, ROT = decltype(rot)::value;
+#pragma unroll 1
+    for (int p = 0; p < kRows; p += kThreads / 4) {
+      const int row = p + wave * 16 + (lane >> 2), m = m_blk + row;
+      auto load_rotate = [&](float (&v)[32]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float e[8];
+          unpack8(*(const uint4*)(stage + row * kStride + c * 64 + k * 16), e);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) v[8 * k + q] = e[q];
+        }
+        rotate_chunk<32, G, ROT, false>(v, out.norm, lane);
+      };
+      float v[32];
+      load_rotate(v);
+      uint32_t cw[4], sbytes = 0u, sb_lo = 0u;
+      const bool need_slow = quantize_chunk<32, FMT, kZeroReference, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
+      if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
+        float u[32];
+        load_rotate(u);
+        quantize_chunk_slow<32, FMT, kZeroReference, true>(u, gs, rg, cw, sbytes);
+      }
+      if (m >= M) {   // padding: zero codes, zero scale bytes
+        cw[0] = cw[1] = cw[2] = cw[3] = 0u;
+        sbytes = 0u;
+      }
+      // (the scale bytes of both K steps of a K half lie side by side: lane c stores those of lane c + 2 too)
+      const uint32_t next = (uint32_t)__builtin_amdgcn_mov_dpp((int)sbytes, 0x4E /* quad_perm [2,3,0,1] */, 0xF, 0xF, true);
+      if (m < padded) {
+        typedef unsigned v4u_nt __attribute__((ext_vector_type(4)));
+        const size_t rt = (size_t)(m >> 5);
+        const int slot = (c & 1) * 32 + (m & 31);
+        __builtin_nontemporal_store(v4u_nt{cw[0], cw[1], cw[2], cw[3]},
+                                    (v4u_nt*)(out.codes + ((rt * units + unit) * 64 + slot) * 16));
+        if (c < 2) {
+          const size_t block = (rt * (units >> 2) + (tile_n >> 1)) * 64 + slot;
+          if constexpr (NV) *(uint32_t*)(out.scales + block * 8 + 4 * (tile_n & 1)) = sbytes | (next << 16);
+          else *(uint16_t*)(out.scales + block * 4 + 2 * (tile_n & 1)) = (uint16_t)(sbytes | (next << 8));
+        }
+      }
+    }
+  };
+  typedef std::integral_constant<int, FPQ_ROT_HADAMARD> Had;
+  if (out.rot == FPQ_ROT_IDENTITY) rows(std::integral_constant<int, 32>{}, std::integral_constant<int, FPQ_ROT_IDENTITY>{});
+  else if (out.g == 16) rows(std::integral_constant<int, 16>{}, Had{});
+  else if (out.g == 32) rows(std::integral_constant<int, 32>{}, Had{});
+  else if (out.g == 64) rows(std::integral_constant<int, 64>{}, Had{});
+  else rows(std::integral_constant<int, 128>{}, Had{});
+}
+
 // One workgroup of four waves (WN x WM) computes a tile of NT*32 weight rows (n) x MT*32 activation
 // rows (m); a wave owns TN x TM accumulator tiles of 32 x 32.  A unit holds KW >= NT weight and MT
 // activation operand blocks (KW, MT multiples of 4 so that loads and scale pieces split evenly).
@@ -201,13 +323,16 @@ __device__ __forceinline__ void barrier_lds_but() {
 // instructions to drain -- and alone on its SIMD nothing fills that time; with a second wave there, working
 // on the other half of K, something does, and each group's loop is half as long.
 // GR = 4 (NVFP4): four groups of two waves, a quarter of K each; see tile_plan.
-template <int NT, int KW, int MT, int WN, int WM, bool NV = false, int RING = kRing, int GR = 1>
+// OUT = GatedOut: the weight rows are a gate projection's and then an up projection's, and a workgroup's tile is NT / 2 row
+// tiles of each (gated_tile_store).
+template <int NT, int KW, int MT, int WN, int WM, bool NV = false, int RING = kRing, int GR = 1, class OUT = PlainOut>
 __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 1)) void gemm_fp4_packed_kernel(
     const uint8_t* __restrict__ xq, const uint8_t* __restrict__ xs, const uint8_t* __restrict__ wq,
     const uint8_t* __restrict__ ws, const float* __restrict__ alpha_p,
     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int M, int N, int K, int tiles_m,
     const uint16_t* __restrict__ residual, const OutSegments seg, int ksplit, int bps, float* partial,
-    unsigned* counters) {
+    unsigned* counters, const OUT out_to) {
+  constexpr bool kGated = std::is_same_v<OUT, GatedOut>;
   constexpr int BN = NT * 32, BM = MT * 32;
   constexpr int NW = WN * WM;           // waves
   static_assert((NW == 4 || NW == 2) && NT <= KW && (KW + MT) % NW == 0 && KW % 2 == 0 && NT % WN == 0 && MT % WM == 0,
@@ -256,12 +381,19 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
   // (weights from HBM: N = 14336, K = 4096, 128 rows 13.0 -> 12.0 us; N = 4096, K = 14336, 384 / 512 rows
   // 32.3 -> 28.7 / 29.1; N = 8192, K = 8192, 256 rows 21.6 -> 19.2).
   // Wave w loads operands w*kPer .. w*kPer + kPer - 1.
+  auto weight_tile = [&](int b) {   // row tile of weight operand b
+    if constexpr (kGated) {
+      const int w = b / TN, i = b % TN;
+      return tile_n * (NT / 2) + w * (TN / 2) + i % (TN / 2) + (i >= TN / 2 ? rt_n / 2 : 0);
+    }
+    return tile_n * NT + b % NT;
+  };
   const uint8_t* op_base[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     const int b = wave * kPer + j;
     if (b < KW) {
-      const int rt = min(tile_n * NT + b % NT, rt_n - 1);
+      const int rt = min(weight_tile(b), rt_n - 1);
       op_base[j] = wq + ((size_t)rt * nu + kb_begin * 4) * 1024;
     } else {
       const int rt = min(tile_m * MT + b - KW, rt_m - 1);
@@ -279,7 +411,7 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
     const int fb = ((wave * kScLoads + j) % kPieces) * kRpp;   // first operand block of the piece
     const bool is_w = fb < KW;
     constexpr int kLpr = 64 / kRpp;                            // lanes per row tile
-    const int rt = min(is_w ? tile_n * NT + (fb + (int)(lane / kLpr)) % NT : tile_m * MT + fb - KW + (int)(lane / kLpr),
+    const int rt = min(is_w ? weight_tile(fb + (int)(lane / kLpr)) : tile_m * MT + fb - KW + (int)(lane / kLpr),
                        (is_w ? rt_n : rt_m) - 1);
     sc_base[j] = (is_w ? ws : xs) + (size_t)kb_begin * kSB;
     sc_off[j] = (uint32_t)rt * (uint32_t)nkb_all * (uint32_t)kSB + (lane % kLpr) * 16;
@@ -636,6 +768,10 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
     if (threadIdx.x == 0) __hip_atomic_store(counters + logical, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
+  if constexpr (kGated) {
+    gated_tile_store<TN, TM, WN, WM, NV>(acc, smem_all, out_to, *alpha_p, tile_n, m_blk, wn, wm, wave, lane, M);
+    return;
+  }
   const OutView out = out_view(seg, y, bias, n_blk + wn * TN * 32, N);
   wave_tile_store<TN, TM, packed_lds_alloc(kBlocks, NV, RING, TN * 32, TM * 32, GR, NW), NW>(
       acc, smem_all, out.y, out.bias, alpha_p, out.n0, m_blk + wm * TM * 32, wave, lane, M, out.N, residual);
@@ -685,7 +821,24 @@ static int launch_packed(const void* xq, const void* xs, const void* wq, const v
                      (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws, alpha,
                      (const uint16_t*)bias, (uint16_t*)y, (int)M, (int)N, (int)K, tiles_m,
                      (const uint16_t*)residual, seg, split.ksplit, split.bps,
-                     workspace ? (float*)((uint8_t*)workspace + kTileCounterBytes) : nullptr, (unsigned*)workspace);
+                     workspace ? (float*)((uint8_t*)workspace + kTileCounterBytes) : nullptr, (unsigned*)workspace, PlainOut{});
+  return (int)hipGetLastError();
+}
+
+// The weights' rows are `out.channels` of a gate projection and as many of an up projection.
+template <int NT, int MT, bool NV, int RING>
+static int launch_gated(const void* xq, const void* xs, const void* wq, const void* ws, const float* alpha, int64_t M,
+                        int64_t K, hipStream_t stream, const GatedOut& out) {
+  constexpr int kRings = packed_lds_bytes(NT + MT, NV, RING), kOut = gated_lds_bytes(NT * 16, MT * 32);
+  constexpr int kLds = kRings > kOut ? kRings : kOut;
+  static_assert(kLds <= 160 * 1024, "more LDS than a CU has");
+  const int tiles_m = (int)((M + MT * 32 - 1) / (MT * 32)), tiles_n = out.channels / (NT * 16);
+  constexpr auto kernel = &gemm_fp4_packed_kernel<NT, NT, MT, 2, 2, NV, RING, 1, GatedOut>;
+  static LdsLimitOnce lds_limit;
+  if (const int st = lds_limit.ensure((const void*)kernel, kLds)) return st;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), kLds, stream, (const uint8_t*)xq,
+                     (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws, alpha, nullptr, nullptr, (int)M,
+                     2 * out.channels, (int)K, tiles_m, nullptr, OutSegments{}, 1, (int)(K / 256), nullptr, nullptr, out);
   return (int)hipGetLastError();
 }
 
@@ -1078,6 +1231,54 @@ static int gemm_packed_multi(const void* xq, const void* xs, const void* wq, con
   return gemm_packed<NV>(xq, xs, wq, ws, alpha, bias, ys[0], M, N, K, stream, nullptr, nullptr, 0, seg);
 }
 }  // namespace fpq
+
+namespace fpq {
+int silu_table_address(hipStream_t stream, const uint16_t** out);   // fpq_quantize.hip
+
+template <bool NV>
+static int gemm_packed_gated(const void* xq, const void* xs, const void* wq, const void* ws, const float* alpha, int64_t M,
+                             int64_t channels, int64_t K, GatedOut out, int zero_policy, hipStream_t stream) {
+  if (M < 0 || channels < 0 || K < 0) return FPQ_E_SHAPE;
+  if (M == 0 || channels == 0) return FPQ_OK;
+  if (!xq || !xs || !wq || !ws || !alpha || !out.codes || !out.scales || (NV && !out.gs)) return FPQ_E_NULL;
+  if (K == 0 || K % 256 != 0 || M > (1 << 24) || channels > (1 << 23) || K > (1 << 24)) return FPQ_E_SHAPE;
+  const int64_t N = 2 * channels, sdiv = NV ? 16 : 32;
+  if ((M + 31) / 32 * 32 * (K / sdiv) >= ((int64_t)1 << 32) || (N + 31) / 32 * 32 * (K / sdiv) >= ((int64_t)1 << 32))
+    return FPQ_E_SHAPE;
+  if (((uintptr_t)xq & 15u) || ((uintptr_t)wq & 15u) || ((uintptr_t)xs & 15u) || ((uintptr_t)ws & 15u) ||
+      ((uintptr_t)out.codes & 15u) || ((uintptr_t)out.scales & 15u))
+    return FPQ_E_ALIGN;
+  const bool rotation = out.rot == FPQ_ROT_IDENTITY ||
+                        (out.rot == FPQ_ROT_HADAMARD && (out.g == 16 || out.g == 32 || out.g == 64 || out.g == 128));
+  if (!rotation || channels % 256 != 0 || zero_policy != FPQ_ZERO_REFERENCE) return FPQ_E_UNSUPPORTED;
+  // Where the tiles hold 128 channels of both projections, one workgroup's share of a 128-wide rotation: the large ones.
+  // (us, the two calls / one: MXFP4 8192 x 14336 x 4096 583.6 / 476.7, 2048 rows 145.7 / 127.3, 1000 x 8448 x 2816 51.8 /
+  // 42.6, 333 x 17152 x 4352 43.9 / 40.8; NVFP4 8192 x 14336 x 4096 1422 / 1385, 1000 x 8448 x 2816 110.5 / 103.7)
+  const TilePlan plan = tile_plan<NV>(M, N, K, 0, device_cus());
+  if (plan.kind < 2) return FPQ_E_UNSUPPORTED;
+  if (const int st = silu_table_address(stream, &out.silu)) return st;
+  out.channels = (int)channels;
+  if constexpr (NV) {
+    if (plan.kind == 3) return launch_gated<8, 8, NV, kRing>(xq, xs, wq, ws, alpha, M, K, stream, out);
+  }
+  return launch_gated<8, 4, NV, 4>(xq, xs, wq, ws, alpha, M, K, stream, out);
+}
+}  // namespace fpq
+
+extern "C" int fpq_gemm_packed_gated_takes(int nv, int64_t M, int64_t channels, int64_t K) {
+  if (M < 1 || channels < 1 || channels % 256 != 0 || K < 256 || K % 256 != 0) return 0;
+  const int cus = fpq::device_cus();
+  return (nv ? fpq::tile_plan<true>(M, 2 * channels, K, 0, cus) : fpq::tile_plan<false>(M, 2 * channels, K, 0, cus)).kind >= 2;
+}
+
+extern "C" int fpq_gemm_packed_gated(int nv, const void* xq, const void* xs, const void* wq, const void* ws,
+                                     const float* alpha, int64_t M, int64_t channels, int64_t K, int rot_kind, int g,
+                                     float norm, const float* global_scale, void* packed_codes, void* packed_scales,
+                                     int zero_policy, void* stream) {
+  const fpq::GatedOut out{(uint8_t*)packed_codes, (uint8_t*)packed_scales, nullptr, global_scale, norm, rot_kind, g, 0};
+  return nv ? fpq::gemm_packed_gated<true>(xq, xs, wq, ws, alpha, M, channels, K, out, zero_policy, (hipStream_t)stream)
+            : fpq::gemm_packed_gated<false>(xq, xs, wq, ws, alpha, M, channels, K, out, zero_policy, (hipStream_t)stream);
+}
 
 extern "C" int fpq_gemm_mxf4_packed_multi(const void* xq, const void* xs, const void* wq, const void* ws,
                                           const float* alpha, const void* bias, void* const* ys,

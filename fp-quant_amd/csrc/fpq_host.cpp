@@ -48,7 +48,8 @@ namespace {
   X(fpq_gemm_mxf4_packed_multi) X(fpq_gemm_nvf4_packed) X(fpq_gemm_nvf4_packed_residual)                     \
   X(fpq_gemm_nvf4_packed_splitk) X(fpq_gemm_nvf4_packed_multi) X(fpq_rmsnorm_rows_quantize_mx_packed)        \
   X(fpq_rmsnorm_tile_quantize_mx_packed) X(fpq_rmsnorm_rows_quantize_nv_packed)                              \
-  X(fpq_rmsnorm_tile_quantize_nv_packed) X(fpq_silu_mul_quantize_mx_packed) X(fpq_silu_mul_quantize_nv_packed)
+  X(fpq_rmsnorm_tile_quantize_nv_packed) X(fpq_silu_mul_quantize_mx_packed) X(fpq_silu_mul_quantize_nv_packed) \
+  X(fpq_gemm_packed_gated) X(fpq_gemm_packed_gated_takes)
 enum Entry {
 #define X(name) E_##name,
   FPQ_ENTRIES(X)
@@ -689,6 +690,25 @@ PyObject* host_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
+// Whether the layers' tensors are those of a group's plan: null, with the first layer's rotation and activation scale, or
+// what to answer (None, False).
+PyObject* group_members(const GroupPlan::Body& p, PyObject* layers, THPObjectPtr& h, PyObject*& first_ags) {
+  const size_t count = PyTuple_GET_SIZE(layers);
+  if (count * 3 != p.members.size() || count > 4) Py_RETURN_NONE;
+  for (size_t i = 0; i < count; ++i) {
+    LayerTensors t;
+    if (!module_tensors(PyTuple_GET_ITEM(layers, i), t)) Py_RETURN_NONE;
+    if (!p.members[3 * i].is(t.qweight) || !p.members[3 * i + 1].is(t.scales) || !p.members[3 * i + 2].is(t.bias))
+      return no_plan(t);
+    if (i == 0 && p.usable) {
+      if (!p.wgs.is(t.wgs) || !p.ags.is(t.ags) || !is_alpha(t.wgs, p.alpha_obj)) return no_plan(t);
+      h = THPObjectPtr(Py_NewRef(t.h));
+      first_ags = t.ags;
+    }
+  }
+  return nullptr;
+}
+
 // group(plan, layers, x): the outputs of layers whose packed weights lie end to end (eager.linear_cat)
 PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
@@ -712,21 +732,9 @@ PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   Call call;
   if (!xp || !plain_call(*xp, call)) Py_RETURN_NONE;
   const size_t count = PyTuple_GET_SIZE(args[1]);
-  if (count * 3 != p->members.size() || count > 4) Py_RETURN_NONE;
   THPObjectPtr h;
   PyObject* first_ags = nullptr;
-  for (size_t i = 0; i < count; ++i) {
-    PyObject* layer = PyTuple_GET_ITEM(args[1], i);
-    LayerTensors t;
-    if (!module_tensors(layer, t)) Py_RETURN_NONE;
-    if (!p->members[3 * i].is(t.qweight) || !p->members[3 * i + 1].is(t.scales) || !p->members[3 * i + 2].is(t.bias))
-      return no_plan(t);
-    if (i == 0 && p->usable) {
-      if (!p->wgs.is(t.wgs) || !p->ags.is(t.ags) || !is_alpha(t.wgs, p->alpha_obj)) return no_plan(t);
-      h = THPObjectPtr(Py_NewRef(t.h));
-      first_ags = t.ags;
-    }
-  }
+  if (PyObject* answer = group_members(*p, args[1], h, first_ags)) return answer;
   if (!p->usable) Py_RETURN_NONE;
   const at::Tensor x = *xp;
   const int64_t k = x.size(-1), m = x.numel() / k;
@@ -807,6 +815,68 @@ PyObject* host_gated_down(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   }
   if (st != FPQ_OK) Py_RETURN_NONE;
   if (!gemm(*p, t, out, residual, y, m, call)) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// gated_mlp(plan, (gate, up), down, x, residual): group() and gated_down() of its outputs where one GEMM forms and
+// quantizes the product in its epilogue (fpq_gemm_packed_gated: many rows); None for any other call.
+PyObject* host_gated_mlp(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
+  HANDLE_TH_ERRORS
+  if (n_args != 5 || Py_TYPE(args[0]) != &GroupPlanType || !PyTuple_Check(args[1])) Py_RETURN_NONE;
+  const THPObjectPtr hold(Py_NewRef(args[0]));
+  auto* p = ((GroupPlan*)args[0])->b;
+  const at::Tensor* xp = tensor_of(args[3]);
+  Call call;
+  LayerTensors t;
+  if (!xp || !plain_call(*xp, call) || xp->dim() < 2 || !p->usable || p->splits.size() != 2 || p->splits[0] != p->splits[1] ||
+      p->bias.defined() || !module_tensors(args[2], t))
+    Py_RETURN_NONE;
+  const at::Tensor x = *xp;
+  const int64_t k = x.size(-1), m = x.numel() / k, inner = p->splits[0];
+  const bool nvfp4 = p->nvfp4;
+  if (k != p->k || p->wp.device().index() != call.dev ||
+      !FPQ_CALL(fpq_gemm_packed_gated_takes)(nvfp4, m, inner, p->kp))
+    Py_RETURN_NONE;
+  THPObjectPtr h;
+  PyObject* first_ags = nullptr;
+  if (PyObject* answer = group_members(*p, args[1], h, first_ags)) {
+    Py_DECREF(answer);
+    Py_RETURN_NONE;
+  }
+  QuantPlan::Body* q = quant_plan(h.get(), first_ags, nvfp4);
+  LinearPlan::Body* d = linear_plan(t);
+  QuantPlan::Body* dq = quant_plan(t.h, t.ags, nvfp4);
+  const at::Tensor* residual;
+  if (!q || !q->usable || !serves(d, nvfp4, m, inner) || !dq || !dq->usable || dq->kind > 1 || !packed_weights_enabled() ||
+      inner % (dq->g > 32 ? dq->g : 32) != 0 || tensor_of(t.qweight)->device().index() != call.dev ||
+      !residual_of(args[4], m, d->n, call, &residual))
+    Py_RETURN_NONE;
+  for (int e : {E_fpq_gemm_nvf4_packed_multi, E_fpq_gemm_mxf4_packed_multi, E_fpq_silu_mul_quantize_nv_packed,
+                E_fpq_silu_mul_quantize_mx_packed, E_fpq_gemm_packed_gated})
+    if (!plain_entry(e)) Py_RETURN_NONE;   // (whoever instruments either kernel sees both)
+  const THPObjectPtr hold_q(Py_NewRef(attribute(h.get(), s_qplan)));
+  const THPObjectPtr hold_d(Py_NewRef(attribute(t.qweight, s_plan))), hold_dq(Py_NewRef(attribute(t.h, s_qplan)));
+  const THPObjectPtr hold_w(Py_NewRef(t.qweight)), hold_s(Py_NewRef(t.scales));
+  Packed in;
+  const int rc = activations(*q, args[3], x, h.get(), m, k, false, call, in);
+  if (rc < 0) return nullptr;
+  if (rc == 0) Py_RETURN_NONE;
+  const Packed product = packed_buffers(m, inner, nvfp4, call.dev);
+  at::Tensor y = output_like(x, d->n, call);
+  int st;
+  {
+    const at::Tensor gs = dq->gs;
+    const int kind = dq->kind, g = dq->g;
+    const float norm = dq->norm;
+    NoGil nogil;   // (the plans, and with them every operand, are held)
+    st = FPQ_CALL(fpq_gemm_packed_gated)(nvfp4, in.codes.const_data_ptr(), in.scales.const_data_ptr(), p->wp.const_data_ptr(),
+                                         p->wsp.const_data_ptr(), (const float*)p->alpha.const_data_ptr(), m, inner, p->kp,
+                                         kind, g, norm, gs.defined() ? (const float*)gs.const_data_ptr() : nullptr,
+                                         product.codes.mutable_data_ptr(), product.scales.mutable_data_ptr(), g_policy,
+                                         call.stream);
+  }
+  if (st != FPQ_OK || !gemm(*d, t, product, residual, y, m, call)) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -1139,6 +1209,7 @@ PyMethodDef methods[] = {
     {"linear", (PyCFunction)(void (*)())host_linear, METH_FASTCALL, nullptr},
     {"rmsnorm", (PyCFunction)(void (*)())host_rmsnorm, METH_FASTCALL, nullptr},
     {"group", (PyCFunction)(void (*)())host_group, METH_FASTCALL, nullptr},
+    {"gated_mlp", (PyCFunction)(void (*)())host_gated_mlp, METH_FASTCALL, nullptr},
     {"gated_down", (PyCFunction)(void (*)())host_gated_down, METH_FASTCALL, nullptr},
     {"quantize_mx", (PyCFunction)(void (*)())host_quantize<false>, METH_FASTCALL, nullptr},
     {"quantize_nv", (PyCFunction)(void (*)())host_quantize<true>, METH_FASTCALL, nullptr},

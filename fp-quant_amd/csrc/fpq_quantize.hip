@@ -837,10 +837,7 @@ static int launch_stream_packed_sized(const void* x, int64_t rows, int64_t cols,
 // last 256-K block, cols % 32 == 0) and rows past `rows` get zero codes and scale bytes.
 //
 // kProSiluMul: the lane that loaded gate and up forms bf16(bf16(silu(gate)) * up).
-// The activation is a lookup in an LDS copy of the silu table's busy part, |g| in [2^-14, 128), held as fp32; the two
-// table offsets of a pair of gates are formed with packed 16-bit arithmetic.  Smaller magnitudes are g / 2 exactly
-// (the relative deviation, |g| / 2, is below half a bf16 step) and larger ones come from the global table: a wave
-// that holds any redoes those lanes.
+// The activation is silu_lookup's, written out here (through the function this kernel measured 1-5 % slower).
 // Memory and VALU bound it about equally: 532 MB at 8192 x 14336 in 103.8 us (5.1 TB/s; 121 us between GEMMs that have
 // taken the clock down).  The streaming kernel that did this before (tiles of both inputs through LDS by direct loads,
 // 16-bit table, an 8 KB wave tile that nothing overlapped) took 114.6 (145) us; 2048 rows 34.5 -> 28.2, 512 rows 13.1
@@ -848,9 +845,6 @@ static int launch_stream_packed_sized(const void* x, int64_t rows, int64_t cols,
 //
 // kProNone (also QUEST): inputs whose rows are no multiple of 256 columns, which the streaming kernel does not take, and
 // NVFP4 inputs of few elements (dispatch_packed).
-constexpr uint32_t kSiluLdsFirst = 113u << 7;         // bf16 magnitude bits of 2^-14
-constexpr uint32_t kSiluLdsCount = 21u * 128u;        // magnitudes up to (not including) 2^7
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // RAGGED: rows that are no whole 256-K blocks, which the generic kernel took before; non-finite chunks get its bytes.  (A
 // kernel of its own: the check in the other one too took 19 registers more, and the NVFP4 slow path's array to scratch.)
@@ -862,7 +856,6 @@ __global__ __launch_bounds__(256, 4) void tile_quantize_kernel(
   static_assert(PRO == kProNone || (PRO == kProSiluMul && !QUEST), "SiLU*up or nothing");
   constexpr int EPL = 32;
   constexpr bool kSilu = PRO == kProSiluMul;
-  typedef __attribute__((address_space(3))) const float lds_f32;
   __shared__ __attribute__((aligned(16))) float silu_lds[kSilu ? 2 * kSiluLdsCount : 4];
   __shared__ __attribute__((aligned(128))) uint8_t stage[4][4096];
   __shared__ float2 lut[FMT == kFmtNv ? 128 : 1];

@@ -19,6 +19,55 @@ __device__ __forceinline__ void unpack8(const uint4& raw, float (&p)[8]) {
 
 constexpr float kKappa = -0x1.8p-26f;  // fma(x, 0.75, x * kKappa) rounds to the E2M1 code of x / fl(4/3)
 
+// SiLU by lookup: an LDS copy of the busy part of a 65536-entry table of bf16(silu(g)), |g| in [2^-14, 128), held as fp32;
+// the two table offsets of a pair of gates are formed with packed 16-bit arithmetic.  Smaller magnitudes are g / 2 exactly
+// (the relative deviation, |g| / 2, is below half a bf16 step) and larger ones come from the global table: a wave that
+// holds any redoes those lanes.
+constexpr uint32_t kSiluLdsFirst = 113u << 7;         // bf16 magnitude bits of 2^-14
+constexpr uint32_t kSiluLdsCount = 21u * 128u;        // magnitudes up to (not including) 2^7
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) const float lds_f32;
+
+template <int THREADS>
+__device__ __forceinline__ void silu_table_to_lds(float* lds, const uint16_t* __restrict__ table) {
+  for (uint32_t i = threadIdx.x; i < 2u * kSiluLdsCount / 4u; i += THREADS) {
+    const uint32_t first = 4u * i, sgn = first >= kSiluLdsCount ? 1u : 0u;
+    const uint2 e = *(const uint2*)&table[(sgn << 15) | (kSiluLdsFirst + first - sgn * kSiluLdsCount)];
+    *(float4*)&lds[first] = make_float4(bf16_lo(e.x), bf16_hi(e.x), bf16_lo(e.y), bf16_hi(e.y));
+  }
+}
+
+// sv[i]: bf16(silu(.)) of the i-th of the bf16 values in `w`
+template <int N>
+__device__ __forceinline__ void silu_lookup(const uint32_t (&w)[N], float (&sv)[2 * N], lds_f32* table,
+                                            const uint16_t* __restrict__ global) {
+  u16x2 most = u16x2{0, 0};
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const u16x2 bits = __builtin_bit_cast(u16x2, w[k]);
+    const u16x2 idx = __builtin_bit_cast(u16x2, w[k] & 0x7fff7fffu) - (unsigned short)kSiluLdsFirst;
+    most = __builtin_elementwise_max(most, idx);
+    const u16x2 in = __builtin_elementwise_min(idx, u16x2{kSiluLdsCount - 1, kSiluLdsCount - 1});
+    const u16x2 at = (bits >> (unsigned short)15) * (unsigned short)kSiluLdsCount + in;
+    sv[2 * k] = table[at.x];
+    sv[2 * k + 1] = table[at.y];
+  }
+  const bool outside = most.x >= kSiluLdsCount || most.y >= kSiluLdsCount;
+  if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
+#pragma unroll
+    for (int e = 0; e < 2 * N; ++e) {
+      const uint32_t bits = (e & 1) ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu, mag = bits & 0x7fffu;
+      if (mag < kSiluLdsFirst) {
+        uint32_t b = __float_as_uint(__uint_as_float(bits << 16) * 0.5f);   // rounded to bf16, to nearest even
+        b += 0x7fffu + ((b >> 16) & 1u);
+        sv[e] = __uint_as_float(b & 0xffff0000u);
+      } else if (mag >= kSiluLdsFirst + kSiluLdsCount) {
+        sv[e] = __uint_as_float((uint32_t)global[bits] << 16);
+      }
+    }
+  }
+}
+
 // Hadamard output index that sequency-ordered output k of a g-block takes: bitreverse(k ^ (k >> 1))
 __host__ __device__ constexpr int gsr_source(int k, int g) {
   int gray = k ^ (k >> 1), r = 0;
@@ -229,13 +278,14 @@ __device__ __forceinline__ bool quantize_chunk(const float (&v)[EPL], float gs, 
   return need_slow;
 }
 
-template <int EPL, int FMT, int ZERO>
+// UNROLL: for kernels that may not have an array in scratch memory (cw, indexed by a loop's group)
+template <int EPL, int FMT, int ZERO, bool UNROLL = false>
 __device__ __forceinline__ void quantize_chunk_slow(const float (&u)[EPL], float gs, float rg,
                                                     uint32_t (&cw)[EPL / 8], uint32_t& sbytes) {
   constexpr int GROUP = FMT == kFmtMx ? 32 : 16;
   constexpr int NG = EPL / GROUP;
   sbytes = 0u;
-#pragma unroll 1
+#pragma unroll UNROLL ? NG : 1
   for (int gi = 0; gi < NG; ++gi) {
     float a = 0.0f;
 #pragma unroll

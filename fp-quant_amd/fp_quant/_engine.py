@@ -58,6 +58,8 @@ _SIGNATURES = {
     "fpq_gemm_nvf4_packed_residual": ([_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _I),
     "fpq_gemm_mxf4_packed_multi": ([_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _I),
     "fpq_gemm_nvf4_packed_multi": ([_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P], _I),
+    "fpq_gemm_packed_gated": ([_I, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _F, _P, _P, _P, _I, _P], _I),
+    "fpq_gemm_packed_gated_takes": ([_I, _I64, _I64, _I64], _I),
     "fpq_linear_rows": ([_I, _P, _P, _I64, _I64, _I, _I, _F, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _I64, _I, _P],
                         _I),
     "fpq_unpack_mxf4": ([_P, _P, _I64, _I64, _P, _P, _I64, _P], _I),

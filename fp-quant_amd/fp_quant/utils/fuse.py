@@ -68,7 +68,7 @@ def _host():
 
 class _NotBuilt:
     """Stands for the native host path where nothing is built: it answers no call."""
-    rmsnorm = group = gated_down = staticmethod(lambda *args: None)
+    rmsnorm = group = gated_mlp = gated_down = staticmethod(lambda *args: None)
 
 
 def _native():
@@ -243,7 +243,12 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
         pair = None
         if not torch.compiler.is_compiling():
             modules = self._modules
-            pair = _native_group(self._fpq_weight_group, (modules.get("gate_proj"), modules.get("up_proj")), x)
+            group, layers = self._fpq_weight_group, (modules.get("gate_proj"), modules.get("up_proj"))
+            if group is not None and None not in layers and x.numel() > 64 * x.shape[-1]:   # (never for fewer rows)
+                y = _native().gated_mlp(group.plan, layers, modules["down_proj"], x, residual)
+                if y is not None:
+                    return y
+            pair = _native_group(group, layers, x)
             if pair is not None:
                 down = modules["down_proj"]
                 nvfp4 = down.config.forward_dtype == FPQuantDtype.NVFP4

@@ -374,6 +374,20 @@ int fpq_linear_rows(int nv, const void* x, const void* up, int64_t M, int64_t K,
                     const float* global_scale, const void* wq_packed, const void* ws_packed, const float* alpha,
                     const void* bias, const void* residual, void* y, int64_t N, void* packed_codes, void* packed_scales,
                     void* workspace, int64_t workspace_bytes, int zero_policy, void* stream);
+/*
+ * A gated MLP's gate and up projections and what feeds its down projection in one launch: what
+ * fpq_gemm_{mxf4,nvf4}_packed_multi into gate and up [M, channels] followed by
+ * fpq_silu_mul_quantize_{mx,nv}_packed of the two computes, to the bit, without writing gate and up.
+ * Operands as fpq_gemm_{mxf4,nvf4}_packed with N = 2 * channels, gate's rows first; channels % 256 == 0; rotation,
+ * global scale and packed outputs as fpq_silu_mul_quantize_{mx,nv}_packed.  FPQ_E_UNSUPPORTED, with nothing launched,
+ * where the two calls are the better way (few rows) or the only one (a rotation or zero policy the kernel lacks).
+ */
+int fpq_gemm_packed_gated(int nv, const void* xq_packed, const void* xs_packed, const void* wq_packed,
+                          const void* ws_packed, const float* alpha, int64_t M, int64_t channels, int64_t K, int rot_kind,
+                          int g, float norm, const float* global_scale, void* packed_codes, void* packed_scales,
+                          int zero_policy, void* stream);
+/* Whether fpq_gemm_packed_gated takes these sizes (1) or answers FPQ_E_UNSUPPORTED (0). */
+int fpq_gemm_packed_gated_takes(int nv, int64_t M, int64_t channels, int64_t K);
 /* The same for packed NVFP4 operands (fpq_gemm_nvf4_packed). */
 int fpq_gemm_nvf4_packed_multi(const void* xq_packed, const void* xs_packed, const void* wq_packed,
                                const void* ws_packed, const float* alpha, const void* bias,
