@@ -56,13 +56,15 @@ constexpr int stream_dynamic_lds(int nt, int mt) {
 struct Packed {};
 struct FewRows {
   const uint4* x;            // bf16 [M, xk]; SiLU*up: gate
-  const uint4* up;           // SiLU*up: the multiplier
+  const uint4* up;           // SiLU*up: the multiplier; RMSNorm: the norm's weight [xk]
   const uint16_t* silu;      // ... and the table of bf16(silu(g))
   const float* gs;           // NVFP4: the activations' global scale
   uint8_t *codes, *scales;   // optional: the quantized rows, in the packed layout (rows past M are not written)
   float norm;
   int xk;                    // a multiple of 32 and of the rotation's size; K is padded to whole blocks
+  float eps;                 // RMSNorm
 };
+enum { kFewPlain = 0, kFewSilu = 1, kFewNorm = 2 };   // what a few rows' chunk goes through before it is rotated
 // IN = RowMajor: both operands as the quantize operators write them, codes [rows, k / 2] and scales [rows, stride] with the
 // strides multiples of four.  A lane takes the same 16 bytes of codes of a row, and the same scale bytes, as from the
 // packed layout, so the sums are the same bit for bit; only the addresses differ.  See launch_rows.
@@ -73,11 +75,12 @@ struct RowMajor {
   uint32_t xs_stride, ws_stride;
 };
 // 32-element chunks a wave quantizes at most: one per lane and pass
-constexpr int few_rows_passes(bool silu) { return silu ? 1 : 2; }
-constexpr int few_rows_chunks(bool silu) { return 64 * few_rows_passes(silu); }
+constexpr int few_rows_passes(int pro) { return pro == kFewPlain ? 2 : 1; }
+constexpr int few_rows_chunks(int pro) { return 64 * few_rows_passes(pro); }
+constexpr int kFewNormRows = 4;   // at most, with a norm (see norm_rows_multi)
 
 template <int NT, int MT, int DB, int NW, bool NV = false, class IN = Packed, int XG = 32, int XROT = FPQ_ROT_IDENTITY,
-          bool XSILU = false>
+          int XPRO = kFewPlain>
 __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm_fp4_stream_kernel(
     const uint8_t* __restrict__ xq_all, const uint8_t* __restrict__ xs_all, const uint8_t* __restrict__ wq,
     const uint8_t* __restrict__ ws, const float* __restrict__ alpha_p, const uint16_t* __restrict__ bias,
@@ -347,8 +350,8 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   };
   // Few rows: the wave's quantized chunks, 16 bytes of codes each, and their scale bytes in the order the matrix
   // instruction takes them: [block][K half][K step].  Lanes past the last row read row 0's, as above.
-  __shared__ __attribute__((aligned(16))) uint8_t few_codes[kFew ? 4 : 1][kFew ? few_rows_chunks(XSILU) * 16 : 16];
-  __shared__ __attribute__((aligned(16))) uint8_t few_scales[kFew ? 4 : 1][kFew ? few_rows_chunks(XSILU) * (NV ? 2 : 1) : 16];
+  __shared__ __attribute__((aligned(16))) uint8_t few_codes[kFew ? 4 : 1][kFew ? few_rows_chunks(XPRO) * 16 : 16];
+  __shared__ __attribute__((aligned(16))) uint8_t few_scales[kFew ? 4 : 1][kFew ? few_rows_chunks(XPRO) * (NV ? 2 : 1) : 16];
   const int few_row = (lane & 31) < M ? (lane & 31) * nblk : 0;   // first block of the lane's row
   auto run_block = [&](auto slot, int t) __attribute__((always_inline)) {
     if constexpr (kFew) {
@@ -407,9 +410,9 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   constexpr bool kOrdered = NT == 1 && DB >= 2 && (MT <= 2 || (NV && MT == 4));
   // Few rows: the wave's chunks in lane order, row by row (the eight chunks of a block are neighbours, so the lanes of
   // a rotation block are); asked for before the weights, since loads complete in order.
-  constexpr int kFewPasses = kFew ? few_rows_passes(XSILU) : 1;
+  constexpr int kFewPasses = kFew ? few_rows_passes(XPRO) : 1;
   const int few_chunks = kFew ? M * nblk * 8 : 0;
-  uint4 xr[kFewPasses][4], ur[XSILU ? kFewPasses : 1][4];
+  uint4 xr[kFewPasses][4], ur[XPRO != kFewPlain ? kFewPasses : 1][4];
   int few_col[kFewPasses], few_at[kFewPasses];
   if constexpr (kFew) {
 #pragma unroll
@@ -424,7 +427,8 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           xr[p][i] = in.x[at + i];
-          if constexpr (XSILU) ur[p][i] = in.up[at + i];
+          if constexpr (XPRO == kFewSilu) ur[p][i] = in.up[at + i];
+          if constexpr (XPRO == kFewNorm) ur[p][i] = in.up[few_col[p] / 8 + i];   // (xk is whole blocks there)
         }
       }
     }
@@ -444,17 +448,79 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
       rg = gs == 0.0f ? 0.0f : 1.0f / gs;
       nv_fast = nv_global_scale_fast(gs);
       if (threadIdx.x < 128) lut[threadIdx.x] = nv_division(threadIdx.x, rg, nv_fast);
-      __syncthreads();
+    }
+    // RMSNorm: the octets' sums of squares of all rows, added by every wave in row_inv_rms_kernel's order
+    constexpr int kOctets = few_rows_chunks(kFewNorm) * 4 * 4;   // of a workgroup's rows, at most
+    __shared__ __attribute__((aligned(16))) float octets[XPRO == kFewNorm ? kOctets : 4];
+    float row_rs[kFewNormRows] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (XPRO == kFewNorm) {
+#pragma unroll
+      for (int p = 0; p < kFewPasses; ++p) {
+        if (p * 64 + lane < few_chunks) {
+          float s[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float e[8];
+            unpack8(xr[p][i], e);
+            s[i] = e[0] * e[0];
+#pragma unroll
+            for (int k = 1; k < 8; ++k) s[i] = s[i] + e[k] * e[k];
+          }
+          *(v4f*)&octets[((few_at[p] >> 16) * in.xk + few_col[p]) / 8] = v4f{s[0], s[1], s[2], s[3]};
+        }
+      }
+    }
+    // (the weights' loads stay in flight: a barrier for LDS only)
+    if constexpr (NV || XPRO == kFewNorm) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (XPRO == kFewNorm) {
+      const int cpr = in.xk / 8;
+      const float cols_f = (float)in.xk;
+#pragma unroll
+      for (int r = 0; r < kFewNormRows; ++r) {
+        if (r >= M) break;   // (uniform)
+        float a = 0.0f;
+        for (int c0 = 0; c0 < cpr; c0 += 512) {   // eight reads at a time (adding zero is adding nothing: a >= 0)
+          float t[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) t[i] = c0 + 64 * i + lane < cpr ? octets[r * cpr + c0 + 64 * i + lane] : 0.0f;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) a = a + t[i];
+        }
+        // the butterfly a += a[lane ^ m], m = 1, 2, ..., 32 (mirrors are lane ^ 4 and ^ 8 once a quad's lanes agree)
+        auto dpp = [](float v, auto ctrl) __attribute__((always_inline)) {
+          return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), decltype(ctrl)::value, 0xF, 0xF, true));
+        };
+        a = a + dpp(a, std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
+        a = a + dpp(a, std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
+        a = a + dpp(a, std::integral_constant<int, 0x141>{});   // row_half_mirror
+        a = a + dpp(a, std::integral_constant<int, 0x140>{});   // row_mirror
+        a = a + __shfl_xor(a, 16, 64);
+        a = a + __shfl_xor(a, 32, 64);
+        row_rs[r] = 1.0f / __builtin_sqrtf(a / cols_f + in.eps);
+      }
     }
 #pragma unroll
     for (int p = 0; p < kFewPasses; ++p) {
       if (p * 64 < few_chunks) {   // (wave-uniform)
+        const int few_r = few_at[p] >> 16;
+        const float rs = few_r == 0 ? row_rs[0] : few_r == 1 ? row_rs[1] : few_r == 2 ? row_rs[2] : row_rs[3];
         auto load_rotate = [&](float (&v)[32]) __attribute__((always_inline)) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             float e[8];
             unpack8(xr[p][i], e);
-            if constexpr (XSILU) {
+            if constexpr (XPRO == kFewNorm) {
+              float q[8];
+              unpack8(ur[p][i], q);
+#pragma unroll
+              for (int k = 0; k < 8; k += 2) {
+                const uint32_t t = pack_bf16x2(e[k] * rs, e[k + 1] * rs);
+                const uint32_t pr = pack_bf16x2(bf16_lo(t) * q[k], bf16_hi(t) * q[k + 1]);
+                e[k] = bf16_lo(pr);
+                e[k + 1] = bf16_hi(pr);
+              }
+            }
+            if constexpr (XPRO == kFewSilu) {
               float q[8];
               unpack8(ur[p][i], q);
               const uint32_t w[4] = {xr[p][i].x, xr[p][i].y, xr[p][i].z, xr[p][i].w};
@@ -893,14 +959,48 @@ int gemm_fp4_rows(bool nv, const void* xq, const void* xs, int64_t xs_stride, co
 //   NVFP4 4 rows: 4096 x 4096 9.4 / 8.2, N = 14336 12.5 / 11.5, N = 28672 19.5 / 19.9
 // SiLU*up (two more gathers per element) gains in one pass only: MXFP4, K = 14336, N = 4096: 1 row 12.1 / 11.0, 2 rows
 // 12.2 / 13.2; 4096 x 4096: 1 row 7.5 / 5.9, 4 rows 7.8 / 9.3.
-static bool few_rows_plan(const StreamPlan& plan, bool nv, bool silu, int64_t M, int64_t N, int64_t K, int64_t xk) {
+static bool few_rows_plan(const StreamPlan& plan, bool nv, int pro, int64_t M, int64_t N, int64_t K, int64_t xk) {
   const int64_t chunks = M * ((plan.bps + 3) / 4) * 8;   // of the wave with the most
-  if (!plan.use || plan.nt != 1 || M > 32 || chunks > few_rows_chunks(silu) || K >= ((int64_t)1 << 22) || xk > K) return false;
+  if (!plan.use || plan.nt != 1 || M > 32 || chunks > few_rows_chunks(pro) || K >= ((int64_t)1 << 22) || xk > K) return false;
   const int64_t tiles = (N + 31) / 32, cus = device_cus();
   return chunks <= 64 ? !nv || tiles <= 4 * cus : tiles <= (nv ? 2 : 4) * cus;
 }
 
 int silu_table_address(hipStream_t stream, const uint16_t** out);   // fpq_quantize.hip
+
+// (`plan`, and what it takes, are the caller's)
+template <bool NV, int PRO>
+static int launch_few_rows(const FewRows& in, const StreamPlan& plan, int rot_kind, int g, const void* wq, const void* ws,
+                           const float* alpha, const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K,
+                           void* workspace, const OutSegments& seg, hipStream_t stream) {
+  if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
+  else if (rot_kind != FPQ_ROT_HADAMARD || in.xk % g != 0) return FPQ_E_UNSUPPORTED;
+  const dim3 grid((unsigned)((N + 31) / 32), (unsigned)plan.ksplit);
+  const bool many = (int64_t)grid.x * grid.y >= 3 * device_cus() / 2;   // (as launch_stream)
+  unsigned* counters = (unsigned*)workspace;
+  float* partial = workspace ? (float*)((uint8_t*)workspace + kStreamCounterBytes) : nullptr;
+  auto go = [&](auto rows_g, auto rows_rot) {
+    constexpr int G = decltype(rows_g)::value, ROT = decltype(rows_rot)::value;
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, nullptr, nullptr, (const uint8_t*)wq, (const uint8_t*)ws, alpha,
+                         (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, plan.bps,
+                         plan.ksplit, partial, counters, seg, in);
+    };
+    if (many) launch(gemm_fp4_stream_kernel<1, 1, 2, 4, NV, FewRows, G, ROT, PRO>);
+    else launch(gemm_fp4_stream_kernel<1, 1, 4, 4, NV, FewRows, G, ROT, PRO>);
+    return (int)hipGetLastError();
+  };
+  typedef std::integral_constant<int, FPQ_ROT_HADAMARD> Had;
+  if (rot_kind == FPQ_ROT_IDENTITY)
+    return go(std::integral_constant<int, 32>{}, std::integral_constant<int, FPQ_ROT_IDENTITY>{});
+  if constexpr (NV) {
+    if (g == 16) return go(std::integral_constant<int, 16>{}, Had{});
+  }
+  if (g == 32) return go(std::integral_constant<int, 32>{}, Had{});
+  if (g == 64) return go(std::integral_constant<int, 64>{}, Had{});
+  if (g == 128) return go(std::integral_constant<int, 128>{}, Had{});
+  return FPQ_E_UNSUPPORTED;
+}
 
 template <bool NV>
 static int linear_rows(const FewRows& in, int rot_kind, int g, const void* wq, const void* ws, const float* alpha,
@@ -917,38 +1017,35 @@ static int linear_rows(const FewRows& in, int rot_kind, int g, const void* wq, c
   if (!workspace) workspace_bytes = 0;
   // The plan that fpq_gemm_*_packed_splitk follows for these rows: the same parts of K, the same sums.
   const StreamPlan plan = stream_plan(M, N, K, workspace_bytes, NV);
-  if (!few_rows_plan(plan, NV, in.up != nullptr, M, N, K, xk)) return FPQ_E_UNSUPPORTED;
-  if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
-  else if (rot_kind != FPQ_ROT_HADAMARD || xk % g != 0) return FPQ_E_UNSUPPORTED;
-  const dim3 grid((unsigned)((N + 31) / 32), (unsigned)plan.ksplit);
-  const bool many = (int64_t)grid.x * grid.y >= 3 * device_cus() / 2;   // (as launch_stream)
-  unsigned* counters = (unsigned*)workspace;
-  float* partial = workspace ? (float*)((uint8_t*)workspace + kStreamCounterBytes) : nullptr;
-  auto go = [&](auto rows_g, auto rows_rot, auto silu) {
-    constexpr int G = decltype(rows_g)::value, ROT = decltype(rows_rot)::value;
-    constexpr bool S = decltype(silu)::value;
-    auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, nullptr, nullptr, (const uint8_t*)wq, (const uint8_t*)ws, alpha,
-                         (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, plan.bps,
-                         plan.ksplit, partial, counters, OutSegments{}, in);
-    };
-    if (many) launch(gemm_fp4_stream_kernel<1, 1, 2, 4, NV, FewRows, G, ROT, S>);
-    else launch(gemm_fp4_stream_kernel<1, 1, 4, 4, NV, FewRows, G, ROT, S>);
-    return (int)hipGetLastError();
-  };
-  auto by_rotation = [&](auto silu) {
-    typedef std::integral_constant<int, FPQ_ROT_HADAMARD> Had;
-    if (rot_kind == FPQ_ROT_IDENTITY)
-      return go(std::integral_constant<int, 32>{}, std::integral_constant<int, FPQ_ROT_IDENTITY>{}, silu);
-    if constexpr (NV) {
-      if (g == 16) return go(std::integral_constant<int, 16>{}, Had{}, silu);
-    }
-    if (g == 32) return go(std::integral_constant<int, 32>{}, Had{}, silu);
-    if (g == 64) return go(std::integral_constant<int, 64>{}, Had{}, silu);
-    if (g == 128) return go(std::integral_constant<int, 128>{}, Had{}, silu);
-    return (int)FPQ_E_UNSUPPORTED;
-  };
-  return in.up ? by_rotation(std::true_type{}) : by_rotation(std::false_type{});
+  if (!few_rows_plan(plan, NV, in.up ? kFewSilu : kFewPlain, M, N, K, xk)) return FPQ_E_UNSUPPORTED;
+  return in.up ? launch_few_rows<NV, kFewSilu>(in, plan, rot_kind, g, wq, ws, alpha, bias, residual, y, M, N, K, workspace,
+                                               OutSegments{}, stream)
+               : launch_few_rows<NV, kFewPlain>(in, plan, rot_kind, g, wq, ws, alpha, bias, residual, y, M, N, K, workspace,
+                                                OutSegments{}, stream);
+}
+
+// RMSNorm in front of a group of projections, for a token or a few: one launch instead of the norm's (a workgroup per row,
+// 4.7 us for any row) and the GEMM's.  Every workgroup has its rows' chunks in registers anyway; the octets' sums of squares
+// go through LDS, each wave adds them up in row_inv_rms_kernel's order, and the normalised bf16 values stay in registers.
+// (the by-product that the norm's own kernel writes is not written: for callers that need the projections only)
+// K is whole (no split across workgroups: a row has to be in one workgroup), as for these rows in
+// fpq_gemm_*_packed_multi: the same sums.
+//
+// Up to four rows, in one pass of a wave's lanes over its chunks (rows x 256-K blocks of a wave <= 8).  Measured (us, two
+// kernels / one; graph replays, weights from HBM), the launch that a caller saves besides not counted:
+//   MXFP4 1 row:  K = 4096, N = 6144 9.8 / 6.8, N = 28672 16.5 / 14.5; K = 1024, N = 1536 7.6 / 5.9
+//   MXFP4 2 rows: 9.5 / 7.2, 16.6 / 15.7; 4 rows: K = 2048, N = 2560 8.5 / 7.2, N = 14336 9.5 / 9.4
+//   NVFP4 1 row:  12.2 / 9.2, 21.8 / 20.6; 2 rows 11.8 / 9.7, 21.3 / 21.6; 4 rows: K = 2048 9.4 / 8.4
+// Two passes (twice the registers for rows and weight) took 10.7 and 24.9 for 4 MXFP4 rows of K = 4096 (9.8, 16.8 in two kernels).
+template <bool NV>
+static int norm_rows_multi(const FewRows& in, int rot_kind, int g, const void* wq, const void* ws, const float* alpha,
+                           const void* bias, const OutSegments& seg, int64_t M, int64_t N, int64_t K, int zero_policy,
+                           hipStream_t stream) {
+  if (M > kFewNormRows || K > (1 << 20) || zero_policy != FPQ_ZERO_REFERENCE) return FPQ_E_UNSUPPORTED;
+  const StreamPlan plan = stream_plan(M, N, K, 0, NV);
+  if (!few_rows_plan(plan, NV, kFewNorm, M, N, K, K)) return FPQ_E_UNSUPPORTED;
+  return launch_few_rows<NV, kFewNorm>(in, plan, rot_kind, g, wq, ws, alpha, bias, nullptr, seg.y[0], M, N, K, nullptr, seg,
+                                       stream);
 }
 
 // ---- the entry point that allocates nothing -------------------------------------------------------
@@ -1022,7 +1119,7 @@ extern "C" int fpq_linear_rows(int nv, const void* x, const void* up, int64_t M,
                                void* packed_scales, void* workspace, int64_t workspace_bytes, int zero_policy,
                                void* stream) {
   fpq::FewRows in{(const uint4*)x, (const uint4*)up, nullptr, global_scale, (uint8_t*)packed_codes,
-                  (uint8_t*)packed_scales, norm, (int)K};
+                  (uint8_t*)packed_scales, norm, (int)K, 0.0f};
   if (!packed_codes != !packed_scales) return FPQ_E_NULL;
   if (K < 0 || K > (1 << 24)) return FPQ_E_SHAPE;
   if (up) {
@@ -1032,4 +1129,29 @@ extern "C" int fpq_linear_rows(int nv, const void* x, const void* up, int64_t M,
                                      workspace_bytes, zero_policy, (hipStream_t)stream)
             : fpq::linear_rows<false>(in, rot_kind, g, wq, ws, alpha, bias, residual, y, M, N, K, workspace,
                                       workspace_bytes, zero_policy, (hipStream_t)stream);
+}
+
+extern "C" int fpq_norm_rows_multi(int nv, const void* x, const void* norm_weight, float eps, int64_t M, int64_t K,
+                                   int rot_kind, int g, float norm, const float* global_scale, const void* wq,
+                                   const void* ws, const float* alpha, const void* bias, void* const* ys,
+                                   const int64_t* ns, int64_t count, int zero_policy, void* stream) {
+  if (count < 1 || count > fpq::kMaxSegments || M < 0 || K < 256 || K % 256 != 0 || K > (1 << 24)) return FPQ_E_SHAPE;
+  if (M == 0) return FPQ_OK;
+  if (!x || !norm_weight || !wq || !ws || !alpha || !ys || !ns || (nv && !global_scale)) return FPQ_E_NULL;
+  if (((uintptr_t)x & 15u) || ((uintptr_t)norm_weight & 15u) || ((uintptr_t)wq & 15u) || ((uintptr_t)ws & 15u))
+    return FPQ_E_ALIGN;
+  fpq::OutSegments seg{};
+  int64_t N = 0;
+  for (int64_t i = 0; i < count; ++i) {   // (as fpq_gemm_*_packed_multi)
+    if (ns[i] < 1 || ns[i] % fpq::kSegmentAlign != 0 || N + ns[i] > (1 << 24)) return FPQ_E_SHAPE;
+    if (!ys[i]) return FPQ_E_NULL;
+    if ((uintptr_t)ys[i] & 15u) return FPQ_E_ALIGN;
+    N += ns[i];
+    seg.end[i] = (int)N;
+    seg.y[i] = (uint16_t*)ys[i];
+  }
+  seg.count = (int)count;
+  const fpq::FewRows in{(const uint4*)x, (const uint4*)norm_weight, nullptr, global_scale, nullptr, nullptr, norm, (int)K, eps};
+  return nv ? fpq::norm_rows_multi<true>(in, rot_kind, g, wq, ws, alpha, bias, seg, M, N, K, zero_policy, (hipStream_t)stream)
+            : fpq::norm_rows_multi<false>(in, rot_kind, g, wq, ws, alpha, bias, seg, M, N, K, zero_policy, (hipStream_t)stream);
 }

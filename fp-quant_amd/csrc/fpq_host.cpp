@@ -49,7 +49,7 @@ namespace {
   X(fpq_gemm_nvf4_packed_splitk) X(fpq_gemm_nvf4_packed_multi) X(fpq_rmsnorm_rows_quantize_mx_packed)        \
   X(fpq_rmsnorm_tile_quantize_mx_packed) X(fpq_rmsnorm_rows_quantize_nv_packed)                              \
   X(fpq_rmsnorm_tile_quantize_nv_packed) X(fpq_silu_mul_quantize_mx_packed) X(fpq_silu_mul_quantize_nv_packed) \
-  X(fpq_gemm_packed_gated) X(fpq_gemm_packed_gated_takes)
+  X(fpq_gemm_packed_gated) X(fpq_gemm_packed_gated_takes) X(fpq_norm_rows_multi)
 enum Entry {
 #define X(name) E_##name,
   FPQ_ENTRIES(X)
@@ -626,63 +626,82 @@ PyObject* host_linear(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
+// The weight and epsilon of an RMSNorm module over `cols` columns, if the fused kernels take them.
+bool norm_of(PyObject* norm, int64_t cols, const Call& call, at::Tensor& weight, float& eps) {
+  PyObject *params, *buffers;
+  if (!module_dicts(norm, &params, &buffers)) return false;
+  PyObject* eps_obj = PyDict_GetItem(*_PyObject_GetDictPtr(norm), s_eps);
+  const at::Tensor* w = tensor_of(member(params, buffers, s_weight));
+  if (!eps_obj || !PyFloat_Check(eps_obj) || !w || !plain_cuda(*w) || w->scalar_type() != at::kBFloat16 ||
+      !w->is_contiguous() || w->numel() != cols || w->device().index() != call.dev || cols > 16384 || !packable_k(cols) ||
+      !packed_weights_enabled())
+    return false;
+  weight = *w;
+  eps = (float)PyFloat_AS_DOUBLE(eps_obj);
+  return true;
+}
+// (fused producers take Hadamard (0) and identity (1) rotations)
+bool norm_rotation(const QuantPlan::Body& q, int64_t cols) {
+  return q.usable && q.kind <= 1 && cols % (q.g > 32 ? q.g : 32) == 0;
+}
+bool norm_few(int64_t rows, int64_t cols) { return rows <= 64 && cols % 256 == 0; }
+bool norm_in_two_launches(int64_t rows, int64_t cols) {   // (eager._norm_in_two_launches)
+  return !norm_few(rows, cols) && rows <= 640 && cols > 8192 && cols % 256 == 0 && rows * cols <= (1 << 23);
+}
+int norm_entry(int64_t rows, int64_t cols, bool nvfp4) {
+  return norm_few(rows, cols) ? (nvfp4 ? E_fpq_rmsnorm_rows_quantize_nv_packed : E_fpq_rmsnorm_rows_quantize_mx_packed)
+                              : (nvfp4 ? E_fpq_rmsnorm_tile_quantize_nv_packed : E_fpq_rmsnorm_tile_quantize_mx_packed);
+}
+// `y`: receives the norm's bf16 result, if it is wanted.  The status of the launch.
+int norm_quantize(const QuantPlan::Body& q, const at::Tensor& x, const at::Tensor& w, float eps, at::Tensor* y, Packed& out,
+                  int64_t rows, int64_t cols, bool nvfp4, const Call& call) {
+  const bool few = norm_few(rows, cols);
+  const at::Tensor gs = q.gs;
+  const int kind = q.kind, g = q.g;
+  const float norm = q.norm;
+  NoGil nogil;
+  const void *xd = x.const_data_ptr(), *wd = w.const_data_ptr();
+  void *yd = y ? y->mutable_data_ptr() : nullptr, *pc = out.codes.mutable_data_ptr(), *ps = out.scales.mutable_data_ptr();
+  if (nvfp4) {
+    const float* g_s = (const float*)gs.const_data_ptr();
+    return few ? FPQ_CALL(fpq_rmsnorm_rows_quantize_nv_packed)(xd, cols, wd, rows, cols, eps, kind, g, norm, g_s, nullptr, yd,
+                                                               pc, ps, g_policy, call.stream)
+               : FPQ_CALL(fpq_rmsnorm_tile_quantize_nv_packed)(xd, cols, wd, rows, cols, eps, kind, g, norm, g_s, nullptr, yd,
+                                                               pc, ps, g_policy, call.stream);
+  }
+  return few ? FPQ_CALL(fpq_rmsnorm_rows_quantize_mx_packed)(xd, cols, wd, rows, cols, eps, kind, g, norm, nullptr, yd, pc, ps,
+                                                             g_policy, call.stream)
+             : FPQ_CALL(fpq_rmsnorm_tile_quantize_mx_packed)(xd, cols, wd, rows, cols, eps, kind, g, norm, nullptr, yd, pc, ps,
+                                                             g_policy, call.stream);
+}
+
 // rmsnorm(norm, layer, x, nvfp4): eager.rmsnorm_quantize with the rotation and activation scale of `layer`
 PyObject* host_rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  PyObject *params, *buffers;
   LayerTensors t;
-  if (n_args != 4 || !module_tensors(args[1], t) || !module_dicts(args[0], &params, &buffers)) Py_RETURN_NONE;
-  PyObject* eps_obj = PyDict_GetItem(*_PyObject_GetDictPtr(args[0]), s_eps);
-  const at::Tensor *xp = tensor_of(args[2]), *wp = tensor_of(member(params, buffers, s_weight));
+  if (n_args != 4 || !module_tensors(args[1], t)) Py_RETURN_NONE;
+  const at::Tensor* xp = tensor_of(args[2]);
   Call call;
-  if (!eps_obj || !PyFloat_Check(eps_obj) || !xp || !wp || !plain_call(*xp, call) || !plain_cuda(*wp)) Py_RETURN_NONE;
+  if (!xp || !plain_call(*xp, call)) Py_RETURN_NONE;
   const bool nvfp4 = args[3] == Py_True;
-  const at::Tensor x = *xp, w = *wp;
+  const at::Tensor x = *xp;
+  at::Tensor w;
+  float eps;
   const int64_t cols = x.size(-1), rows = x.numel() / cols;
-  if (w.scalar_type() != at::kBFloat16 || !w.is_contiguous() || w.numel() != cols || w.device().index() != call.dev ||
-      cols > 16384 || !packable_k(cols) || !packed_weights_enabled())
-    Py_RETURN_NONE;
+  if (!norm_of(args[0], cols, call, w, eps)) Py_RETURN_NONE;
   QuantPlan::Body* q = quant_plan(t.h, t.ags, nvfp4);
-  // (fused producers take Hadamard (0) and identity (1) rotations)
   if (!q) return no_quant_plan(t.h, t.ags);
-  if (!q->usable || q->kind > 1 || cols % (q->g > 32 ? q->g : 32) != 0) Py_RETURN_NONE;
-  const bool few = rows <= 64 && cols % 256 == 0;
-  if (!few && rows <= 640 && cols > 8192 && cols % 256 == 0 && rows * cols <= (1 << 23))
-    Py_RETURN_NONE;   // (two launches: eager._norm_in_two_launches)
-  const int entry = few ? (nvfp4 ? E_fpq_rmsnorm_rows_quantize_nv_packed : E_fpq_rmsnorm_rows_quantize_mx_packed)
-                        : (nvfp4 ? E_fpq_rmsnorm_tile_quantize_nv_packed : E_fpq_rmsnorm_tile_quantize_mx_packed);
+  if (!norm_rotation(*q, cols) || norm_in_two_launches(rows, cols)) Py_RETURN_NONE;
   bool declined = false;
   const bool share = sharing_enabled(*q, declined);
-  if (!plain_entry(entry) || declined) Py_RETURN_NONE;
+  if (!plain_entry(norm_entry(rows, cols, nvfp4)) || declined) Py_RETURN_NONE;
   THPObjectPtr hold_h(Py_NewRef(t.h));
   const THPObjectPtr hold_q(Py_NewRef(attribute(t.h, s_qplan)));
   THPObjectPtr key(share ? sharing_key(*q, rows, cols, call, false) : nullptr);
   if (share && !key) return nullptr;
   at::Tensor y = output_like(x, cols, call);
   Packed out = packed_buffers(rows, cols, nvfp4, call.dev);
-  const double eps = PyFloat_AS_DOUBLE(eps_obj);
-  int st;
-  {
-    const at::Tensor gs = q->gs;
-    const int kind = q->kind, g = q->g;
-    const float norm = q->norm;
-    NoGil nogil;
-    const void *xd = x.const_data_ptr(), *wd = w.const_data_ptr();
-    void *yd = y.mutable_data_ptr(), *pc = out.codes.mutable_data_ptr(), *ps = out.scales.mutable_data_ptr();
-    if (nvfp4) {
-      const float* g_s = (const float*)gs.const_data_ptr();
-      st = few ? FPQ_CALL(fpq_rmsnorm_rows_quantize_nv_packed)(xd, cols, wd, rows, cols, (float)eps, kind, g, norm, g_s,
-                                                               nullptr, yd, pc, ps, g_policy, call.stream)
-               : FPQ_CALL(fpq_rmsnorm_tile_quantize_nv_packed)(xd, cols, wd, rows, cols, (float)eps, kind, g, norm, g_s,
-                                                               nullptr, yd, pc, ps, g_policy, call.stream);
-    } else {
-      st = few ? FPQ_CALL(fpq_rmsnorm_rows_quantize_mx_packed)(xd, cols, wd, rows, cols, (float)eps, kind, g, norm, nullptr,
-                                                               yd, pc, ps, g_policy, call.stream)
-               : FPQ_CALL(fpq_rmsnorm_tile_quantize_mx_packed)(xd, cols, wd, rows, cols, (float)eps, kind, g, norm, nullptr,
-                                                               yd, pc, ps, g_policy, call.stream);
-    }
-  }
-  if (st != FPQ_OK) Py_RETURN_NONE;
+  if (norm_quantize(*q, x, w, eps, &y, out, rows, cols, nvfp4, call) != FPQ_OK) Py_RETURN_NONE;
   THPObjectPtr result(THPVariable_Wrap(y));
   if (!result) return nullptr;
   if (share && !publish(result.get(), y, key.release(), hold_h.get(), out, rows, cols, nvfp4, call)) return nullptr;
@@ -709,10 +728,29 @@ PyObject* group_members(const GroupPlan::Body& p, PyObject* layers, THPObjectPtr
   return nullptr;
 }
 
+// What a norm in front of a group does to the group's call: rows that one launch takes together with the GEMM, rows whose
+// norm is a launch of its own but need not leave its bf16 result (8192 x 4096: 30.2 us with it, 23.9 without), or neither
+// (the caller runs the norm module first).
+constexpr int64_t kNormInGemmRows = 4, kNormAloneRows = 64;
+
+// The quantized output of `norm` on x where that is a launch of its own.  1: done, 0: not the plain path
+int norm_activations(const QuantPlan::Body& q, PyObject* norm, const at::Tensor& x, int64_t m, int64_t k, bool nvfp4,
+                     const Call& call, Packed& out) {
+  at::Tensor w;
+  float eps;
+  if (m <= kNormAloneRows || !norm_of(norm, k, call, w, eps) || !norm_rotation(q, k) || norm_in_two_launches(m, k) ||
+      !plain_entry(norm_entry(m, k, nvfp4)))
+    return 0;
+  out = packed_buffers(m, k, nvfp4, call.dev);
+  return norm_quantize(q, x, w, eps, nullptr, out, m, k, nvfp4, call) == FPQ_OK;
+}
+
 // group(plan, layers, x): the outputs of layers whose packed weights lie end to end (eager.linear_cat)
+// norm_group(plan, layers, x, norm): ... on norm(x)
 PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 3 || !PyTuple_Check(args[1])) Py_RETURN_NONE;
+  if ((n_args != 3 && n_args != 4) || !PyTuple_Check(args[1])) Py_RETURN_NONE;
+  PyObject* const norm = n_args == 4 ? args[3] : nullptr;
   if (Py_TYPE(args[0]) != &GroupPlanType) {   // no plan yet, if the call is a plain one
     const at::Tensor* t = tensor_of(args[2]);
     Call c;
@@ -743,10 +781,20 @@ PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   if (!q) return no_quant_plan(h.get(), first_ags);
   if (!q->usable || k != p->k || x.dim() < 2 || p->wp.device().index() != call.dev || !plain_entry(entry)) Py_RETURN_NONE;
   const THPObjectPtr hold_q(Py_NewRef(attribute(h.get(), s_qplan)));
+  const bool one_launch = norm && m <= kNormInGemmRows;
   Packed packed;
-  const int rc = activations(*q, args[2], x, h.get(), m, k, false, call, packed);
-  if (rc < 0) return nullptr;
-  if (rc == 0) Py_RETURN_NONE;
+  at::Tensor w;
+  float eps = 0.0f;
+  if (one_launch) {
+    if (!norm_of(norm, k, call, w, eps) || !norm_rotation(*q, k) || !plain_entry(norm_entry(m, k, p->nvfp4)) ||
+        !plain_entry(E_fpq_norm_rows_multi))
+      Py_RETURN_NONE;
+  } else {
+    const int rc = norm ? norm_activations(*q, norm, x, m, k, p->nvfp4, call, packed)
+                        : activations(*q, args[2], x, h.get(), m, k, false, call, packed);
+    if (rc < 0) return nullptr;
+    if (rc == 0) Py_RETURN_NONE;
+  }
   at::Tensor ys[4];
   void* y_ptr[4];
   for (size_t i = 0; i < count; ++i) {
@@ -754,7 +802,17 @@ PyObject* host_group(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
     y_ptr[i] = ys[i].mutable_data_ptr();
   }
   int st;
-  {
+  if (one_launch) {
+    const at::Tensor gs = q->gs;
+    const int kind = q->kind, g = q->g;
+    const float h_norm = q->norm;
+    NoGil nogil;
+    st = FPQ_CALL(fpq_norm_rows_multi)(p->nvfp4, x.const_data_ptr(), w.const_data_ptr(), eps, m, k, kind, g, h_norm,
+                                       gs.defined() ? (const float*)gs.const_data_ptr() : nullptr, p->wp.const_data_ptr(),
+                                       p->wsp.const_data_ptr(), (const float*)p->alpha.const_data_ptr(),
+                                       p->bias.defined() ? p->bias.const_data_ptr() : nullptr, y_ptr, p->splits.data(),
+                                       (int64_t)count, g_policy, call.stream);
+  } else {
     NoGil nogil;   // (the plan, and with it every operand, is held)
     auto fn = p->nvfp4 ? FPQ_CALL(fpq_gemm_nvf4_packed_multi) : FPQ_CALL(fpq_gemm_mxf4_packed_multi);
     st = fn(packed.codes.const_data_ptr(), packed.scales.const_data_ptr(), p->wp.const_data_ptr(), p->wsp.const_data_ptr(),
@@ -819,11 +877,12 @@ PyObject* host_gated_down(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
-// gated_mlp(plan, (gate, up), down, x, residual): group() and gated_down() of its outputs where one GEMM forms and
+// gated_mlp(plan, (gate, up), down, x, residual, norm): norm (unless it is None), group() and gated_down() of its outputs where one GEMM forms and
 // quantizes the product in its epilogue (fpq_gemm_packed_gated: many rows); None for any other call.
 PyObject* host_gated_mlp(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
-  if (n_args != 5 || Py_TYPE(args[0]) != &GroupPlanType || !PyTuple_Check(args[1])) Py_RETURN_NONE;
+  if ((n_args != 5 && n_args != 6) || Py_TYPE(args[0]) != &GroupPlanType || !PyTuple_Check(args[1])) Py_RETURN_NONE;
+  PyObject* const norm = n_args == 6 && args[5] != Py_None ? args[5] : nullptr;
   const THPObjectPtr hold(Py_NewRef(args[0]));
   auto* p = ((GroupPlan*)args[0])->b;
   const at::Tensor* xp = tensor_of(args[3]);
@@ -859,7 +918,8 @@ PyObject* host_gated_mlp(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   const THPObjectPtr hold_d(Py_NewRef(attribute(t.qweight, s_plan))), hold_dq(Py_NewRef(attribute(t.h, s_qplan)));
   const THPObjectPtr hold_w(Py_NewRef(t.qweight)), hold_s(Py_NewRef(t.scales));
   Packed in;
-  const int rc = activations(*q, args[3], x, h.get(), m, k, false, call, in);
+  const int rc = norm ? norm_activations(*q, norm, x, m, k, nvfp4, call, in)
+                      : activations(*q, args[3], x, h.get(), m, k, false, call, in);
   if (rc < 0) return nullptr;
   if (rc == 0) Py_RETURN_NONE;
   const Packed product = packed_buffers(m, inner, nvfp4, call.dev);
@@ -1209,6 +1269,7 @@ PyMethodDef methods[] = {
     {"linear", (PyCFunction)(void (*)())host_linear, METH_FASTCALL, nullptr},
     {"rmsnorm", (PyCFunction)(void (*)())host_rmsnorm, METH_FASTCALL, nullptr},
     {"group", (PyCFunction)(void (*)())host_group, METH_FASTCALL, nullptr},
+    {"norm_group", (PyCFunction)(void (*)())host_group, METH_FASTCALL, nullptr},
     {"gated_mlp", (PyCFunction)(void (*)())host_gated_mlp, METH_FASTCALL, nullptr},
     {"gated_down", (PyCFunction)(void (*)())host_gated_down, METH_FASTCALL, nullptr},
     {"quantize_mx", (PyCFunction)(void (*)())host_quantize<false>, METH_FASTCALL, nullptr},

@@ -7,7 +7,9 @@ keep one activation quantizer per such group).  With those projections being FPQ
 
 * each RMSNorm computes its bf16 output and the rotated, quantized form of it in one kernel; the
   projections that are then called with that output find the quantized form and go straight to
-  their GEMM;
+  their GEMM.  In a block whose forward is patched (below), a norm whose output nobody but those
+  projections reads is left to their call: for at most four rows it is part of the GEMM's launch,
+  for many its bf16 output is not written;
 * the MLP quantizes bf16(silu(gate)) * up directly from `gate` and `up`, without writing the product;
 * the two `residual + hidden_states` additions of the block happen in the epilogues of the `o_proj`
   and `down_proj` GEMMs (blocks whose forward is, statement for statement, the one of transformers'
@@ -68,7 +70,7 @@ def _host():
 
 class _NotBuilt:
     """Stands for the native host path where nothing is built: it answers no call."""
-    rmsnorm = group = gated_mlp = gated_down = staticmethod(lambda *args: None)
+    rmsnorm = group = norm_group = gated_mlp = gated_down = staticmethod(lambda *args: None)
 
 
 def _native():
@@ -211,8 +213,27 @@ def fuse_rmsnorm(norm: nn.Module, consumer) -> bool:
         return unfused(hidden_states)
 
     norm._fpq_unfused_forward = unfused
-    norm.forward = types.MethodType(forward, norm)
+    norm.forward = norm._fpq_fused_forward = types.MethodType(forward, norm)
     return True
+
+
+def _hands_on(norm: nn.Module, reader: nn.Module) -> bool:
+    """Whether `reader`, a module patched to take a norm (`norm=`), may be given `norm` and the norm's input in place of the
+    norm's output: nobody else sees that output -- `reader` reads it in its projections only, `norm` runs nothing but the
+    fused forward, and no hook is handed either's input or result."""
+    n, r = vars(norm), vars(reader)
+    hooks = nn.modules.module
+    return ("_fpq_fused_forward" in n and n.get("forward") is n["_fpq_fused_forward"]
+            and r.get("_fpq_takes_norm") is not None and r.get("forward") is r["_fpq_takes_norm"]
+            and not (n["_forward_hooks"] or n["_forward_pre_hooks"] or r["_forward_hooks"] or r["_forward_pre_hooks"]
+                     or hooks._global_forward_hooks or hooks._global_forward_pre_hooks))
+
+
+def _norm_joins(x: torch.Tensor) -> bool:
+    """Row counts at which the projections' call takes the norm: with so few rows it is part of the GEMM's launch; beyond 64
+    it is a launch that need not write the norm's output."""
+    rows = x.numel() // x.shape[-1]
+    return rows <= 4 or rows > 64
 
 
 def fuse_gated_mlp(mlp: nn.Module) -> bool:
@@ -238,17 +259,23 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
                      and (down_proj.bias is None or (down_proj.bias.dtype == torch.bfloat16
                                                      and down_proj.bias.is_contiguous())))
 
-    def forward(self, x, residual=None):
-        """`residual`: added to the result (a fused decoder block passes its skip connection)."""
+    def forward(self, x, residual=None, norm=None):
+        """`residual`: added to the result (a fused decoder block passes its skip connection).  `norm`: the input is
+        norm(x)."""
         pair = None
         if not torch.compiler.is_compiling():
             modules = self._modules
             group, layers = self._fpq_weight_group, (modules.get("gate_proj"), modules.get("up_proj"))
             if group is not None and None not in layers and x.numel() > 64 * x.shape[-1]:   # (never for fewer rows)
-                y = _native().gated_mlp(group.plan, layers, modules["down_proj"], x, residual)
+                y = _native().gated_mlp(group.plan, layers, modules["down_proj"], x, residual, norm)
                 if y is not None:
                     return y
-            pair = _native_group(group, layers, x)
+            if norm is not None:
+                pair = _native_group(group, layers, x, norm)
+                if pair is None:
+                    x, norm = norm(x), None
+            if pair is None:
+                pair = _native_group(group, layers, x)
             if pair is not None:
                 down = modules["down_proj"]
                 nvfp4 = down.config.forward_dtype == FPQuantDtype.NVFP4
@@ -258,6 +285,8 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
                     y = _native().gated_down(down, *pair, residual, nvfp4)
                 if y is not None and y is not False:
                     return y
+        if norm is not None:
+            x, norm = norm(x), None
         if traceable and _traceable_call(x):
             # two operators: gate and up from one quantization of x; SiLU*up quantized as it is
             # formed and multiplied by down's weight
@@ -292,7 +321,7 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
     if traceable:
         _attach_weight_group(mlp, ("gate_proj", "up_proj"))   # gate/up as one GEMM where the format allows
     mlp._fpq_unfused_forward = unfused
-    mlp.forward = types.MethodType(forward, mlp)
+    mlp.forward = mlp._fpq_takes_norm = types.MethodType(forward, mlp)
     return True
 
 
@@ -364,6 +393,9 @@ def _attention_call_defaults(block: nn.Module) -> Optional[Dict[str, object]]:
     return defaults
 
 
+_NOTHING: Dict[str, object] = {}
+
+
 def fuse_residual_adds(block: nn.Module) -> bool:
     """Move the two `residual + hidden_states` additions of a decoder block into the GEMMs of
     `self_attn.o_proj` and `mlp.down_proj`.  Needs the MLP patched by fuse_gated_mlp, `o_proj` an
@@ -386,18 +418,27 @@ def fuse_residual_adds(block: nn.Module) -> bool:
     def forward(self, hidden_states, *args, **kwargs):
         if args or not isinstance(hidden_states, torch.Tensor) or not _fusable_call(hidden_states):
             return unfused(hidden_states, *args, **kwargs)
-        out_proj = self.self_attn.o_proj
-        normed = self.input_layernorm(hidden_states)
+        attn = self.self_attn
+        out_proj = attn.o_proj
+        norm = self.input_layernorm
+        joins = _norm_joins(hidden_states)
+        if joins and _hands_on(norm, attn):
+            normed, extra = hidden_states, {"_fpq_norm": norm}
+        else:
+            normed, extra = norm(hidden_states), _NOTHING
         state = vars(out_proj)   # (a plain attribute: what Module.__setattr__ does with one, without its searches)
         state["_fpq_residual"] = hidden_states
         try:
-            attn_out, _ = self.self_attn(hidden_states=normed, **{**defaults, **kwargs})
+            attn_out, _ = attn(hidden_states=normed, **{**defaults, **kwargs, **extra})
         finally:
             pending = state["_fpq_residual"]
             state["_fpq_residual"] = None
         if pending is not None:   # o_proj did not take it
             attn_out = hidden_states + attn_out
-        return self.mlp(self.post_attention_layernorm(attn_out), residual=attn_out)
+        norm, mlp = self.post_attention_layernorm, self.mlp
+        if joins and _hands_on(norm, mlp):
+            return mlp(attn_out, residual=attn_out, norm=norm)
+        return mlp(norm(attn_out), residual=attn_out)
 
     block._fpq_unfused_forward = unfused
     block.forward = types.MethodType(forward, block)
@@ -421,14 +462,16 @@ class _ProjectionCalls(ast.NodeTransformer):
         return node
 
 
-def _native_group(group, layers, x: torch.Tensor):
-    """The outputs of `layers` on `x` through the native host path, or None."""
+def _native_group(group, layers, x: torch.Tensor, norm=None):
+    """The outputs of `layers` on `x`, or on norm(x), through the native host path, or None."""
     if group is None or None in layers:
         return None
-    outs = _native().group(group.plan, layers, x)
+    native = _native()
+    call, args = (native.group, (layers, x)) if norm is None else (native.norm_group, (layers, x, norm))
+    outs = call(group.plan, *args)
     if outs is False and _host().learnable():
         _host().learn_group(group, layers)
-        outs = _native().group(group.plan, layers, x)
+        outs = call(group.plan, *args)
     return outs or None
 
 
@@ -458,17 +501,24 @@ def _eager_group_linear(owner: nn.Module, layers, x: torch.Tensor):
     return [o.view(*lead, o.shape[-1]) for o in outs]
 
 
-def _qkv(attn, hidden_states):
-    """q, k and v projections of `hidden_states`: from one operator when a compiler is tracing
+def _qkv(attn, hidden_states, norm=None):
+    """q, k and v projections of `hidden_states` (`norm`: of norm(hidden_states)): from one operator when a compiler is tracing
     (which cannot see that the three layers quantize the same tensor); from one GEMM on the layers'
     concatenated packed weights in eager calls that have them; else three ordinary calls (which
     share the quantization by themselves)."""
     if not torch.compiler.is_compiling() and attn._fpq_qkv_alike:
         modules = attn._modules
-        outs = _native_group(attn._fpq_weight_group, (modules.get("q_proj"), modules.get("k_proj"), modules.get("v_proj")),
-                             hidden_states)
+        group, layers = attn._fpq_weight_group, (modules.get("q_proj"), modules.get("k_proj"), modules.get("v_proj"))
+        if norm is not None:
+            outs = _native_group(group, layers, hidden_states, norm)
+            if outs is not None:
+                return outs
+            hidden_states, norm = norm(hidden_states), None
+        outs = _native_group(group, layers, hidden_states)
         if outs is not None:
             return outs
+    if norm is not None:
+        hidden_states = norm(hidden_states)
     layers = (attn.q_proj, attn.k_proj, attn.v_proj)
     if attn._fpq_qkv_alike and _traceable_call(hidden_states):
         return _group_linear(layers, hidden_states, attn._fpq_weight_group)
@@ -509,9 +559,19 @@ def fuse_qkv(attn: nn.Module) -> bool:
     if ([h[1] for h in hits] != [["q_proj"], ["k_proj"], ["v_proj"]]
             or [h[0] for h in hits] != list(range(hits[0][0], hits[0][0] + 3))):
         return False
+    # The projections and the tensor's shape are all that the forward reads of its input: a norm in front of it may be left
+    # to the grouped call (`_fpq_norm`; the input is then the norm's own, of the same shape).
+    shapes = {id(n.value) for n in ast.walk(fdef) if isinstance(n, ast.Attribute) and n.attr == "shape"}
+    names = [n for n in ast.walk(fdef) if isinstance(n, ast.Name)]
+    takes_norm = (all(id(n) in shapes for n in names if n.id == "hidden_states")
+                  and not any(n.id in ("locals", "vars", "eval", "exec", "_fpq_norm") for n in names))
     # (the helper is reached through `self`: a name added to a copy of the module's globals would be
     # invisible to a tracer that resolves globals through the module itself)
-    grouped = ast.parse("__fpq_q, __fpq_k, __fpq_v = self._fpq_qkv(hidden_states)").body[0]
+    call = "self._fpq_qkv(hidden_states, _fpq_norm)" if takes_norm else "self._fpq_qkv(hidden_states)"
+    grouped = ast.parse(f"__fpq_q, __fpq_k, __fpq_v = {call}").body[0]
+    if takes_norm:
+        fdef.args.kwonlyargs.append(ast.arg(arg="_fpq_norm"))
+        fdef.args.kw_defaults.append(ast.Constant(value=None))
     fdef.body.insert(hits[0][0], grouped)
     fdef.name = "forward"
     ast.fix_missing_locations(tree)
@@ -527,6 +587,7 @@ def fuse_qkv(attn: nn.Module) -> bool:
     attn._fpq_qkv = types.MethodType(_qkv, attn)
     attn._fpq_unfused_forward = attn.forward
     attn.forward = types.MethodType(namespace["forward"], attn)
+    attn._fpq_takes_norm = attn.forward if takes_norm else None
     return True
 
 
@@ -557,6 +618,8 @@ def unfuse_producers(model: nn.Module) -> None:
             else:
                 module.forward = unfused
             module._fpq_unfused_forward = None
+            vars(module).pop("_fpq_fused_forward", None)
+            vars(module).pop("_fpq_takes_norm", None)
             hook = getattr(module, "_fpq_weight_group_hook", None)
             if hook is not None:
                 hook.remove()

@@ -375,6 +375,17 @@ int fpq_linear_rows(int nv, const void* x, const void* up, int64_t M, int64_t K,
                     const void* bias, const void* residual, void* y, int64_t N, void* packed_codes, void* packed_scales,
                     void* workspace, int64_t workspace_bytes, int zero_policy, void* stream);
 /*
+ * RMSNorm and the projections that read its output, for at most four rows, in one launch: what
+ * fpq_rmsnorm_rows_quantize_{mx,nv}_packed of x [M, K] (contiguous, 16-byte aligned) followed by
+ * fpq_gemm_{mxf4,nvf4}_packed_multi computes, to the bit, without the norm's bf16 result.  K % 256 == 0; ys, ns, count, bias
+ * as fpq_gemm_mxf4_packed_multi.  FPQ_E_UNSUPPORTED, with nothing launched, for more rows, a K that the kernel does not
+ * hold, and rotations and zero policies that fpq_linear_rows does not take.
+ */
+int fpq_norm_rows_multi(int nv, const void* x, const void* norm_weight, float eps, int64_t M, int64_t K, int rot_kind, int g,
+                        float norm, const float* global_scale, const void* wq_packed, const void* ws_packed,
+                        const float* alpha, const void* bias, void* const* ys, const int64_t* ns, int64_t count,
+                        int zero_policy, void* stream);
+/*
  * A gated MLP's gate and up projections and what feeds its down projection in one launch: what
  * fpq_gemm_{mxf4,nvf4}_packed_multi into gate and up [M, channels] followed by
  * fpq_silu_mul_quantize_{mx,nv}_packed of the two computes, to the bit, without writing gate and up.
