@@ -171,6 +171,9 @@ __device__ __forceinline__ void barrier_lds_but() {
   asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// This wave's LDS reads and writes are complete.
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // The epilogue of a GEMM whose weight rows are a gate and an up projection's, for the gated MLP's down projection:
 //   bf16(bf16(silu(gate)) * up), rotated and quantized into the packed layout of down's activations, to the bit what
 // writing gate and up and quantizing them afterwards gives.  A wave's TN tiles are TN / 2 of gate and the same TN / 2
@@ -323,6 +326,16 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
 // instructions to drain -- and alone on its SIMD nothing fills that time; with a second wave there, working
 // on the other half of K, something does, and each group's loop is half as long.
 // GR = 4 (NVFP4): four groups of two waves, a quarter of K each; see tile_plan.
+//
+// WN = WM = 1, GR = 8 (kSolo), 64 x 128 tiles: every wave multiplies the whole tile over an eighth of K, with a ring of its
+// own, and the eight parts are added through LDS.  What bounded these tiles was the waves' lockstep: at every unit's barrier
+// all of them converted operands or waited at the same time, so the matrix pipes had the other half of the time.  Without a
+// barrier in the loop the two waves of a SIMD drift apart and one's conversions (NVFP4: 0.75 operand tiles per matrix
+// instruction instead of 1) or waits run behind the other's matrix instructions; an operand is read from LDS by one wave
+// only.  Eight rings leave room for two units each, so a slot is refilled as soon as its unit has reached the registers.  It
+// pays with a longer tail (256 KB through LDS, 2 us).  us, weights from HBM, groups of two waves (MXFP4: one of four) / this:
+//   NVFP4 512 x 4096 x 12288 51.6 / 45.0 (1.15 PFLOP/s), 512 x 4096 x 4096 21.0 / 19.2, 300 x 4096 x 3328 21.3 / 16.1
+//   MXFP4 320 x 4096 x 14336 29.1 / 24.5, 512 x 4096 x 14336 30.5 / 27.8, 512 x 4096 x 4096 10.8 / 11.6
 // OUT = GatedOut: the weight rows are a gate projection's and then an up projection's, and a workgroup's tile is NT / 2 row
 // tiles of each (gated_tile_store).
 template <int NT, int KW, int MT, int WN, int WM, bool NV = false, int RING = kRing, int GR = 1, class OUT = PlainOut>
@@ -335,21 +348,23 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
   constexpr bool kGated = std::is_same_v<OUT, GatedOut>;
   constexpr int BN = NT * 32, BM = MT * 32;
   constexpr int NW = WN * WM;           // waves
-  static_assert((NW == 4 || NW == 2) && NT <= KW && (KW + MT) % NW == 0 && KW % 2 == 0 && NT % WN == 0 && MT % WM == 0,
+  constexpr bool kSolo = NW == 1;       // every wave has a part of K and a ring of its own
+  static_assert((NW == 4 || NW == 2 || (kSolo && GR == NT * MT)) && NT <= KW && (KW + MT) % NW == 0 && KW % 2 == 0 &&
+                    NT % WN == 0 && MT % WM == 0,
                 "unsupported tile / wave arrangement");
   constexpr int TN = NT / WN, TM = MT / WM;  // 32x32 MFMA tiles per wave along n and m
   constexpr int kBlocks = KW + MT;      // operand kilobytes per unit
-  constexpr int kPer = kBlocks / NW;    // code loads per wave per unit
+  constexpr int kPer = kSolo ? NT + MT : kBlocks / NW;    // code loads per wave per unit (kSolo: no copies)
   constexpr int kSB = scale_block_bytes(NV);            // scale bytes per row tile and 256-K block
   constexpr int kRpp = 1024 / kSB;                      // row tiles per 1 KB scale piece
   constexpr int kPieces = kBlocks / kRpp;               // scale pieces per 256-K block
   constexpr int kScLoads = kPieces >= NW ? (kPieces + NW - 1) / NW : 1;  // scale loads per wave per block
   constexpr int kSlots = scale_slots(NV, GR), kSlotBytes = scale_slot_bytes(kBlocks, NV, NW);
   constexpr int kUnitBytes = kBlocks * 1024;
-  static_assert(RING == 4 || RING == 8, "the ring holds one or two 256-K blocks");
+  static_assert(kSolo ? RING == 2 : RING == 4 || RING == 8, "the ring holds half a 256-K block, or one or two");
   constexpr int kPackedLds = packed_lds_bytes(kBlocks, NV, RING, GR, NW);
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_all[];
-  static_assert(GR == 1 || GR == 2 || GR == 4, "groups of waves");
+  static_assert(GR == 1 || GR == 2 || GR == 4 || (kSolo && GR == 8), "groups of waves");
   static_assert((KW + MT) % kRpp == 0 && KW % kRpp == 0, "a scale piece holds weights or activations");
   const int grp = GR > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * NW)) : 0;
   uint8_t* const smem = smem_all + grp * kPackedLds;   // this group's ring and scale slots
@@ -370,8 +385,10 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
   // Only the kernels for few tiles are ever launched that way (the large tiles have no register to spare).
   constexpr bool kCanSplit = NT * MT <= 16;
   static_assert(GR == 1 || kCanSplit, "groups split K");
-  const int kb_begin = kCanSplit ? (blockIdx.y * GR + grp) * bps : 0;   // (GR = 2: both halves hold bps blocks)
-  const int nkb = kCanSplit ? min(nkb_all - kb_begin, bps) : nkb_all;
+  // (GR = 2, 4: every group holds bps blocks; kSolo: bps of them and one more for the first waves, none has none)
+  const int solo_rest = kSolo ? nkb_all - bps * GR : 0;
+  const int kb_begin = kSolo ? grp * bps + min(grp, solo_rest) : kCanSplit ? (blockIdx.y * GR + grp) * bps : 0;
+  const int nkb = kSolo ? bps + (grp < solo_rest) : kCanSplit ? min(nkb_all - kb_begin, bps) : nkb_all;
   const int rt_n = (N + 31) >> 5, rt_m = (M + 31) >> 5;
 
   // ---- loads.  Operand b of a unit: b < KW weight row tile tile_n*NT + b % NT, else activation row tile
@@ -391,7 +408,7 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
   const uint8_t* op_base[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const int b = wave * kPer + j;
+    const int b = kSolo && j >= NT ? KW + j - NT : wave * kPer + j;
     if (b < KW) {
       const int rt = min(weight_tile(b), rt_n - 1);
       op_base[j] = wq + ((size_t)rt * nu + kb_begin * 4) * 1024;
@@ -430,7 +447,8 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
     }
     const uint32_t dst = smem_base + (u % RING) * kUnitBytes + wave * kPer * 1024;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) lds_dma16(op_base[j] + (size_t)u * 1024, lane16, dst + j * 1024);
+    for (int j = 0; j < kPer; ++j)
+      lds_dma16(op_base[j] + (size_t)u * 1024, lane16, dst + (kSolo && j >= NT ? KW + j - NT : j) * 1024);
   };
 
   v16f acc[TN][TM];
@@ -492,7 +510,7 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
   // younger units are outstanding (a wave issues kPer per unit, one more with scales).
   if (n_pro == RING) wait_vmem_le<(RING - (kDeep ? 2 : 1)) * kPer>();
   else wait_vmem();
-  barrier_lds();
+  if constexpr (!kSolo) barrier_lds();
   read_unit(0, 0);
   if constexpr (kDeep) read_unit(1, 1);   // (a K range holds at least four units)
   read_scales(0);
@@ -501,6 +519,13 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
     for (int i = 0; i < TN; ++i) sa[i] = sa_next[i];
 #pragma unroll
     for (int j = 0; j < TM; ++j) sb[j] = sb_next[j];
+  }
+
+  // kSolo: nobody else reads the wave's ring, so there is no barrier, and a slot is free once its unit has reached the
+  // registers: unit u + 3 is issued in the middle of unit u, into the slot that unit u + 1 has just been read from.
+  if constexpr (kSolo) {
+    wait_lds();
+    issue_unit(2, false);
   }
 
   // One 64-K unit: 16 MFMAs per wave.  After the first row of MFMAs comes the hand-over: every
@@ -545,7 +570,7 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
   constexpr int kHpr = kNvPipe ? 2 * TM / TN : 1;   // halves of activation tiles converted per row
   // conversion instructions behind each matrix instruction of a row (a row converts 9 + 4.5 kHpr for its TM; one
   // more or less measured 1-3 % slower)
-  constexpr int kPinValu = TN == 4 ? (TM == 4 ? 5 : 6) : 8;
+  constexpr int kPinValu = TN == 4 ? (TM == 4 ? 5 : 6) : TM == 4 ? 7 : 8;
   v8h ah_c[kNvPipe ? TN : 1], ah_n[kNvPipe ? TN : 1];
   v4h bh_c[kNvPipe ? TM : 1][2], bh_n[kNvPipe ? TM : 1][2];
   auto nv_scale = [&](const uint2& cur, const uint2& next, int qn, int sn, bool nxt) __attribute__((always_inline)) {
@@ -613,11 +638,20 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
       }                                                                                             \
       if (s4 == 0) {                                                                                \
         wait_vmem_le<(ALLOWED)>();                                                                  \
-        barrier_lds();                                                                              \
-        if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                               \
+        if constexpr (!kSolo) {                                                                     \
+          barrier_lds();                                                                            \
+          if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                             \
+        }                                                                                           \
         if (READ) read_unit((U) + 1, ((Q) + 1) & 1);                                                \
         if ((Q) == 3 && (NEXT_BLOCK)) read_scales(((U) + 1) >> 2);                                  \
         __builtin_amdgcn_sched_barrier(0);                                                          \
+      }                                                                                             \
+      if constexpr (kSolo) {                                                                        \
+        if (s4 == 2 && (ISSUE)) {                                                                   \
+          wait_lds();                                                                               \
+          issue_unit((U) + 3, (Q) == 1);                                                            \
+          __builtin_amdgcn_sched_barrier(0);                                                        \
+        }                                                                                           \
       }                                                                                             \
       _Pragma("unroll") for (int i = 0; i < TN; ++i) ah_c[i] = ah_n[i];                             \
       _Pragma("unroll") for (int j = 0; j < TM; ++j) {                                              \
@@ -629,12 +663,21 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
     FPQ_PREP_B(Q)                                                                                   \
     _Pragma("unroll") for (int i0 = 0; i0 < kHand; ++i0) FPQ_MFMA_ROW(Q, i0)                        \
     wait_vmem_le<(ALLOWED)>();                                                                      \
-    barrier_lds();                                                                                  \
-    if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                                   \
+    if constexpr (!kSolo) {                                                                         \
+      barrier_lds();                                                                                \
+      if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                                 \
+    }                                                                                               \
     if (READ) read_unit((U) + 1, ((Q) + 1) & 1);                                                    \
     if ((Q) == 3 && (NEXT_BLOCK)) read_scales(((U) + 1) >> 2);                                      \
     __builtin_amdgcn_sched_barrier(0);                                                              \
     _Pragma("unroll") for (int i1 = kHand; i1 < TN; ++i1) FPQ_MFMA_ROW(Q, i1)                       \
+    if constexpr (kSolo) {                                                                          \
+      if (ISSUE) {                                                                                  \
+        wait_lds();                                                                                 \
+        issue_unit((U) + 3, (Q) == 1);                                                              \
+        __builtin_amdgcn_sched_barrier(0);                                                          \
+      }                                                                                             \
+    }                                                                                               \
   }
 #define FPQ_TAKE_SCALES_NOW()                                                                       \
   {                                                                                                 \
@@ -657,7 +700,23 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
   // steady state: every unit of these blocks still has a unit RING ahead of it to issue
   constexpr int kDrain = RING / 4;   // blocks in the last ring of units
   const int kb_tail = max(nkb - kDrain, 0);
-  for (int kb = 0; kb < kb_tail; ++kb) {
+  if constexpr (kSolo) {   // (unit u + 2 may be outstanding while unit u + 1 is complete, with the scales it opens a block with)
+    for (int kb = 0; kb < nkb - 1; ++kb) {
+      const int u0 = kb * 4;
+      FPQ_TAKE_SCALES()
+      FPQ_UNIT(0, u0 + 0, kPer, true, true, true, true)
+      FPQ_UNIT(1, u0 + 1, kPer, true, true, true, true)
+      FPQ_UNIT(2, u0 + 2, kPer + kScLoads, true, true, true, true)
+      FPQ_UNIT(3, u0 + 3, kPer, true, true, true, true)
+    }
+    const int u0 = nkb * 4 - 4;
+    FPQ_TAKE_SCALES()
+    FPQ_UNIT(0, u0 + 0, kPer, true, true, false, true)
+    FPQ_UNIT(1, u0 + 1, kPer, false, true, false, true)
+    FPQ_UNIT(2, u0 + 2, 0, false, true, false, false)
+    FPQ_UNIT(3, u0 + 3, 0, false, false, false, false)
+  }
+  for (int kb = 0; !kSolo && kb < kb_tail; ++kb) {
     const int u0 = kb * 4;
     FPQ_TAKE_SCALES()
     FPQ_UNIT(0, u0 + 0, (RING - 2) * kPer, true, true, true, true)
@@ -693,6 +752,40 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
 #undef FPQ_TAKE_SCALES_NOW
 #undef FPQ_TAKE_SCALES_AFTER
 
+  if constexpr (kSolo) {
+    // As many waves as accumulator tiles: every wave adds up and stores one of them.  Half of the tiles at a time (LDS holds
+    // no more), 16 bytes per lane and access, the parts in a fixed order.
+    constexpr int kHalf = GR / 2;
+    v4f* const xch = (v4f*)smem_all + lane;
+    v16f sum[1][1];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      __syncthreads();   // (the rings, then the first half's tiles, are read)
+#pragma unroll
+      for (int t = h * kHalf; t < (h + 1) * kHalf; ++t) {
+        const v16f& a = acc[t / TM][t % TM];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          xch[((grp * kHalf + t - h * kHalf) * 4 + q) * 64] = v4f{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+      }
+      __syncthreads();
+      if (grp / kHalf == h) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v4f k[GR];
+#pragma unroll
+          for (int w = 0; w < GR; ++w) k[w] = xch[((w * kHalf + grp % kHalf) * 4 + q) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sum[0][0][4 * q + e] = ((k[0][e] + k[4][e]) + (k[2][e] + k[6][e])) + ((k[1][e] + k[5][e]) + (k[3][e] + k[7][e]));
+        }
+      }
+    }
+    const OutView out = out_view(seg, y, bias, n_blk, N);
+    wave_tile_store<1, 1, kPackedLds * GR, GR>(sum, smem_all, out.y, out.bias, alpha_p, out.n0 + grp / TM * 32,
+                                               m_blk + grp % TM * 32, grp, lane, M, out.N, residual);
+    return;
+  }
   if constexpr (GR > 1) {
     // The upper half of the groups hands its accumulators to the lower one through LDS (the rings are idle: every wave
     // has waited for its last loads and read its last unit), and so on: a fixed order, (0 + 2) + (1 + 3).  Then the
@@ -811,7 +904,7 @@ static int launch_packed(const void* xq, const void* xs, const void* wq, const v
   const int tiles_m = (int)((M + MT * 32 - 1) / (MT * 32)), tiles_n = (int)((N + NT * 32 - 1) / (NT * 32));
   if (split.ksplit <= 1 || !workspace || NT * MT > 16 || GR > 1) split = TileSplit{1, (int)(K / 256)};
   if (GR > 1) {   // the groups of a workgroup take equal parts of K (the caller checked that K / 256 divides)
-    if ((K / 256) % GR != 0) return FPQ_E_UNSUPPORTED;
+    if (WN * WM > 1 ? (K / 256) % GR != 0 : K / 256 < GR) return FPQ_E_UNSUPPORTED;
     split.bps = (int)(K / 256) / GR;
   }
   static LdsLimitOnce lds_limit;
@@ -873,7 +966,7 @@ struct TilePlan {
   int64_t tiles;
   int64_t part_bytes;
   TileSplit split;
-  int groups;        // 2, 4: workgroups of eight waves, K in parts inside the workgroup (no K split across workgroups then)
+  int groups;        // 2, 4, 8: workgroups of eight waves, K in parts inside the workgroup (no K split across workgroups then)
 };
 template <bool NV>
 static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_bytes, int cus) {
@@ -913,21 +1006,28 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_byt
     return plan;
   }
   plan.split = TileSplit{1, (int)(K / 256)};
-  // NVFP4 with at most one workgroup per CU: two groups of four waves per workgroup, one half of K each (the
-  // in-register conversions of one wave overlap the matrix instructions of the other on its SIMD, and the halves
-  // meet in LDS): 300-512 rows, N = 4096, K = 4096 25.9 -> 23.4 us; 640-1024 rows 34.9-37.3 -> 32.2-35.6;
-  // N = 12288, 129-256 rows 35.1 -> 32.9; K = 12288, 384 / 512 rows 69 / 70 -> 59.3 / 62.7 (a K split across two
-  // workgroups through the caller's workspace: 61.1 / 65.3).  MXFP4, whose waves wait on what the CU receives
-  // from the L2, measured the same with 64 x 128 tiles and 8 % slower with 128 x 128: it keeps four waves.
-  if (NV && plan.tiles <= cus && (K / 256) % 2 == 0 && K >= 2048) {
-    // Four groups of two waves, a quarter of K each, where K divides: the same eight waves with tiles of 64 x 64 (128 x 64)
-    // instead of 32 x 64 (64 x 64).  A wave converts TN + TM operand tiles for TN x TM matrix instructions, and the
-    // conversions bound these kernels (offsetting the two groups' barriers so that one converts while the other
-    // multiplies changed nothing): 1 instead of 1.5 per matrix instruction (0.75 instead of 1).  Weights from HBM, us:
-    // N = 4096: K = 12288, 512 / 384 rows 67.9 / 60.5 -> 53.0 / 46.9, K = 4096, 300 / 512 rows 22.4 / 22.8 -> 19.4 / 19.8;
-    // N = 8192, K = 8192, 256 rows 40.6 -> 33.9; 128 x 128 tiles: N = 8192, K = 6144, 512 rows 46.2 -> 43.3, N = 4096,
-    // K = 12288, 768 rows 80.0 -> 69.5.  No shape measured slower; two groups stay for a K that is no multiple of 1024.
-    plan.groups = (K / 256) % 4 == 0 ? 4 : 2;
+  // 64 x 128 tiles (at most one workgroup per CU): eight waves, an eighth of K each, without a barrier in the loop (kSolo
+  // above).  Against four groups of two waves (K a multiple of 1024; one group for an odd number of blocks), weights from
+  // HBM, us: NVFP4 N = 4096: K = 12288, 512 rows 51.6 -> 45.0, K = 14336, 384 rows 52.7 -> 44.5, K = 4096, 300 / 512 rows
+  // 20.3 / 21.0 -> 17.7 / 19.2, K = 3328, 300 rows 21.3 -> 16.1; N = 8192, K = 8192, 256 rows 37.3 -> 34.0; N = 6144, 144 / 200
+  // rows 19.8 / 19.7 -> 17.6 / 17.3; N = 14336, 128 rows 22.8 -> 21.3; K = 2048, N = 5120, 200 rows 12.5 -> 11.8.  An odd
+  // number of blocks long enough to be cut across workgroups still is: callers size their workspace for it.
+  // MXFP4, whose waves do not convert anything, has to earn the longer tail with a long K, and with weights that more than
+  // one row of tiles reads: N = 4096: K = 14336, 320 / 384 / 512 rows 29.1 / 27.8 / 30.5 -> 24.5 / 26.3 / 27.8, K = 8192, 512
+  // rows 18.8 -> 18.1; N = 3072, K = 10240, 400 rows 21.5 -> 18.2; N = 8192, K = 8192, 256 rows 19.6 -> 19.4.  Not K = 4096, N =
+  // 4096, 512 rows 10.8 -> 11.6; not one row of tiles, 128 rows, N = 14336: K = 4096 11.8 -> 13.4, K = 14336 32.2 -> 33.8.
+  const int64_t nkb = K / 256;
+  if (plan.kind == 0 && (NV ? nkb >= 8 && (nkb % 2 == 0 || nkb < 2 * kTileSplitMinBlocks) : nkb >= 32 && M > 128)) {
+    plan.groups = 8;
+    return plan;
+  }
+  // NVFP4, 128 x 128 tiles: four groups of two waves (wave tiles of 128 x 64), a quarter of K each, or two groups of four
+  // (64 x 64) for a K that is no multiple of 1024.  A wave converts TN + TM operand tiles for TN x TM matrix instructions and
+  // the conversions bound these kernels: 0.75 or 1 per matrix instruction.  One group -> two: 640-1024 rows, N = 4096, K =
+  // 4096 34.9-37.3 -> 32.2-35.6 us; N = 12288, 129-256 rows 35.1 -> 32.9.  Two -> four: N = 8192, K = 6144, 512 rows 46.2 ->
+  // 43.3, N = 4096, K = 12288, 768 rows 80.0 -> 69.5.  MXFP4 measured 8 % slower in two groups and keeps four waves.
+  if (NV && plan.kind == 1 && nkb % 2 == 0 && nkb >= 8) {
+    plan.groups = nkb % 4 == 0 ? 4 : 2;
     return plan;
   }
   // (NVFP4 beyond the 256 rows that two passes of the weight-streaming kernel serve better)
@@ -1030,10 +1130,10 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
     // kernels halve K inside their workgroups they take 23 us for K = 4096 at any of these row counts and the
     // two passes are ahead up to 192 rows only (weights from HBM; N = 6144: 144 rows 22.5 two passes / 25.8 us
     // tiles, 192 rows 23.7 / 23.6, 224 rows 26.7 / 23.5, 256 rows 28.7 / 22.9; N = 8192, K = 8192: 35.7 / 43.4,
-    // 39.5 / 42.6, 45.5 / 43.1, 49.7 / 42.8); with K in quarters the tiles are ahead from 129 rows on (N = 6144 20.2 / 19.1,
-    // 192 rows 22.6 / 18.6; N = 8192, K = 8192 33.1 / 32.8, 39.0 / 32.8; N = 5120, K = 2048 12.5 / 11.7).
+    // 39.5 / 42.6, 45.5 / 43.1, 49.7 / 42.8); with K in quarters or eighths the tiles are ahead from 129 rows on (N = 6144
+    // 20.2 / 17.6, 192 rows 22.6 / 17.3; N = 8192, K = 8192, 192 rows 39.0 / 32.8; N = 5120, K = 2048 12.5 / 11.7).
     const int64_t half = ((M + 1) / 2 + 31) / 32 * 32;   // rows of the first pass, whole 32-row tiles
-    const int64_t two_pass_rows = plan.groups == 4 ? 0 : plan.groups == 2 ? 192 : 2 * FPQ_NV_STREAM_ROWS;
+    const int64_t two_pass_rows = plan.groups >= 4 ? 0 : plan.groups == 2 ? 192 : 2 * FPQ_NV_STREAM_ROWS;
     if (!tile_splits && M > FPQ_NV_STREAM_ROWS && M <= two_pass_rows && (N + 31) / 32 <= cus &&
         stream_eligible(true, half, N, K)) {
       // (both passes may split K through the caller's workspace: they run one after the other on the stream)
@@ -1053,17 +1153,14 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
   // same accumulation order and bits) take 25 instead of 34.5 us for NVFP4 at 257-512 rows, N = 4096, K = 4096
   // (K = 12288: 69 instead of 97 us) and 4-7 % less for MXFP4; with more tiles they measured 14 % slower.
   // Either of these two kernels splits K through the caller's workspace where that fills the CUs (tile_split_plan).
+  if (plan.groups == 8)
+    return launch_packed<2, NV ? 2 : 4, 4, 1, 1, NV, 2, 8>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
+                                                           residual, seg);
   if constexpr (NV) {
-    if (plan.groups == 4 && plan.kind == 0)
-      return launch_packed<2, 2, 4, 1, 2, true, 4, 4>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
-                                                      residual, seg);
-    if (plan.groups == 4 && plan.kind == 1)
+    if (plan.groups == 4)
       return launch_packed<4, 4, 4, 1, 2, true, 4, 4>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
                                                       residual, seg);
-    if (plan.groups == 2 && plan.kind == 0)
-      return launch_packed<2, 4, 4, 2, 2, true, kRing, 2>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
-                                                          residual, seg);
-    if (plan.groups == 2 && plan.kind == 1)
+    if (plan.groups == 2)
       return launch_packed<4, 4, 4, 2, 2, true, kRing, 2>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
                                                           residual, seg);
   }
