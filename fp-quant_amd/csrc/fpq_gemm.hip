@@ -794,9 +794,11 @@ static int gemm_dispatch(const void* xq, const void* xs, int64_t xs_stride, cons
   //   18.4; but N = 14336 12.0 / 10.8, and K = 14336, N = 6144 21.9 / 16.3);
   // * up to 16 rows and K <= 512, where there is nothing to share between its four waves (MXFP4, one row, N = 4096: K = 96
   //   2.2 / 2.8, K = 384 2.6 / 3.0; N = 16384, K = 512 3.8 / 3.9): the direct kernel.
-  const int64_t cus = device_cus();
-  const bool one_row = M == 1 && K % 2048 == 0 && ws_stride % 16 == 0 && !((uintptr_t)xs & 15u) && !((uintptr_t)ws & 15u) &&
-                       (FMT == 0 || N <= 1024 || (K < 8192 && (N <= 32 * cus || N > 64 * cus)));
+  bool one_row = M == 1 && K % 2048 == 0 && ws_stride % 16 == 0 && !((uintptr_t)xs & 15u) && !((uintptr_t)ws & 15u);
+  if (one_row && FMT == 1 && N > 1024) {
+    const int64_t cus = device_cus();
+    one_row = K < 8192 && (N <= 32 * cus || N > 64 * cus);
+  }
   if (one_row) {
     hipLaunchKernelGGL(FMT == 0 ? gemm_mxf4_one_row_kernel : gemm_nvf4_one_row_kernel, dim3((unsigned)((N + 15) / 16)),
                        dim3(256), 0, stream, (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws,

@@ -229,11 +229,13 @@ def _hands_on(norm: nn.Module, reader: nn.Module) -> bool:
                      or hooks._global_forward_hooks or hooks._global_forward_pre_hooks))
 
 
-def _norm_joins(x: torch.Tensor) -> bool:
-    """Row counts at which the projections' call takes the norm: with so few rows it is part of the GEMM's launch; beyond 64
-    it is a launch that need not write the norm's output."""
-    rows = x.numel() // x.shape[-1]
-    return rows <= 4 or rows > 64
+def _norm_joins(elements: int, width: int) -> bool:
+    """Row counts at which the projections' call takes the norm: with at most four rows it is part of the GEMM's launch, as long
+    as a wave holds its share of them (64 chunks of 32 elements: 4 x 2048, 1 x 8192; a call that is declined costs 3 us of host
+    time, 4 x 5120: 60.7 us a block, 64.2 with it); beyond 64 it is a launch that need not write the norm's output."""
+    if elements <= 4 * width:
+        return width % 256 == 0 and elements // width * -(-width // 1024) <= 8
+    return elements > 64 * width
 
 
 def fuse_gated_mlp(mlp: nn.Module) -> bool:
@@ -247,7 +249,7 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
     if getattr(mlp, "_fpq_unfused_forward", None) is not None:
         return True
     unfused = mlp.forward
-    down_proj = parts[2]
+    few, down_proj = 64 * parts[0].in_features, parts[2]
     # what the traced form needs on top: gate/up quantize alike, a SiLU*up quantizer for down's rotation
     traceable = False
     if down_proj.forward_hadamard_matrix.is_cuda:
@@ -266,7 +268,7 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
         if not torch.compiler.is_compiling():
             modules = self._modules
             group, layers = self._fpq_weight_group, (modules.get("gate_proj"), modules.get("up_proj"))
-            if group is not None and None not in layers and x.numel() > 64 * x.shape[-1]:   # (never for fewer rows)
+            if group is not None and None not in layers and x.numel() > few:   # (never for fewer rows)
                 y = _native().gated_mlp(group.plan, layers, modules["down_proj"], x, residual, norm)
                 if y is not None:
                     return y
@@ -414,6 +416,7 @@ def fuse_residual_adds(block: nn.Module) -> bool:
     if defaults is None:
         return False
     unfused = block.forward
+    width = o_proj.out_features
 
     def forward(self, hidden_states, *args, **kwargs):
         if args or not isinstance(hidden_states, torch.Tensor) or not _fusable_call(hidden_states):
@@ -421,7 +424,7 @@ def fuse_residual_adds(block: nn.Module) -> bool:
         attn = self.self_attn
         out_proj = attn.o_proj
         norm = self.input_layernorm
-        joins = _norm_joins(hidden_states)
+        joins = _norm_joins(hidden_states.numel(), width)
         if joins and _hands_on(norm, attn):
             normed, extra = hidden_states, {"_fpq_norm": norm}
         else:

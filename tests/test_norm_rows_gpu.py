@@ -83,6 +83,17 @@ def test_refusals():
     assert call(m=0) == 0
 
 
+@pytest.mark.parametrize("m,k", [(1, 8192), (1, 8448), (2, 4096), (2, 4352), (3, 2048), (3, 2304), (4, 2048), (4, 2304), (4, 256), (1, 384)])
+def test_rule_offers_what_the_kernel_takes(m, k):
+    from fp_quant import _engine
+    from fp_quant.utils.fuse import _norm_joins
+    p = torch.zeros(4 << 20, dtype=torch.uint8, device="cuda").data_ptr()
+    st = _engine.lib().fpq_norm_rows_multi(0, p, p, 1e-5, m, k, 0, 32, 0.1, None, p, p, p, None, (ctypes.c_void_p * 1)(p + (2 << 20)),
+                                           (ctypes.c_int64 * 1)(256), 1, 0, None)
+    assert _norm_joins(m * k, k) == (st == 0)
+    assert not _norm_joins(5 * k, k) and not _norm_joins(64 * k, k) and _norm_joins(65 * k, k)
+
+
 @needs_packed
 @pytest.mark.parametrize("fmt,g", [("mxfp4", 128), ("nvfp4", 16)])
 @pytest.mark.parametrize("m,kv", [(1, 256), (4, 512), (65, 256), (600, 512), (2, 128), (70, 128)])
