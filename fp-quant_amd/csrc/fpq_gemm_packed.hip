@@ -1045,6 +1045,11 @@ int gemm_fp4_stream_slabs(bool nv, const void* xq, const void* xs, const void* w
                           const float* alpha, const void* bias, const void* residual, void* y, int64_t M, int64_t N,
                           int64_t K, int64_t slab_rows, const OutSegments& seg, hipStream_t stream);
 
+// Whether gemm_packed gives a shape that it does not cut into slabs to the weight-streaming kernel.
+static bool streams(bool nv, int64_t M, int64_t N, int64_t K) {
+  return stream_eligible(nv, M, N, K) && (!nv || M <= FPQ_NV_STREAM_ROWS);
+}
+
 template <bool NV>
 static int gemm_packed(const void* xq, const void* xs, const void* wq, const void* ws, const float* alpha,
                        const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* stream,
@@ -1117,7 +1122,7 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
       break;   // one slab, or a shape the kernel does not take: the paths below
     }
   }
-  if (stream_eligible(NV, M, N, K) && (!NV || M <= FPQ_NV_STREAM_ROWS))
+  if (streams(NV, M, N, K))
     return gemm_fp4_stream(NV, xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, workspace, workspace_bytes,
                            seg, (hipStream_t)stream);
   if constexpr (NV) {
@@ -1332,6 +1337,20 @@ static int gemm_packed_multi(const void* xq, const void* xs, const void* wq, con
 namespace fpq {
 int silu_table_address(hipStream_t stream, const uint16_t** out);   // fpq_quantize.hip
 
+// Whether one GEMM with the gated epilogue stands for the GEMM into gate and up and the quantizer behind it, and on which tiles.
+// Where those hold 128 channels of both projections, one workgroup's share of a 128-wide rotation: the large ones.
+// (us, the two calls / one: MXFP4 8192 x 14336 x 4096 583.6 / 476.7, 2048 rows 145.7 / 127.3, 1000 x 8448 x 2816 51.8 /
+// 42.6, 333 x 17152 x 4352 43.9 / 40.8; NVFP4 8192 x 14336 x 4096 1422 / 1385, 1000 x 8448 x 2816 110.5 / 103.7)
+// Not where that GEMM streams its weights, NVFP4's up to 96 rows of more than 16384 channels: large tiles hold mostly
+// padding there (65 x 17152 x 4352 49.3 / 57.4, 96 rows 48.6 / 52.5; but 96 x 28672 x 8192 116.9 / 111.0), and they sum in
+// another order, so the bytes would not be those of the two calls.  (Row slabs: never with this many tiles.)
+template <bool NV>
+static bool gated_plan(int64_t M, int64_t channels, int64_t K, TilePlan& plan) {
+  if (streams(NV, M, 2 * channels, K)) return false;
+  plan = tile_plan<NV>(M, 2 * channels, K, 0, device_cus());
+  return plan.kind >= 2;
+}
+
 template <bool NV>
 static int gemm_packed_gated(const void* xq, const void* xs, const void* wq, const void* ws, const float* alpha, int64_t M,
                              int64_t channels, int64_t K, GatedOut out, int zero_policy, hipStream_t stream) {
@@ -1348,11 +1367,8 @@ static int gemm_packed_gated(const void* xq, const void* xs, const void* wq, con
   const bool rotation = out.rot == FPQ_ROT_IDENTITY ||
                         (out.rot == FPQ_ROT_HADAMARD && (out.g == 16 || out.g == 32 || out.g == 64 || out.g == 128));
   if (!rotation || channels % 256 != 0 || zero_policy != FPQ_ZERO_REFERENCE) return FPQ_E_UNSUPPORTED;
-  // Where the tiles hold 128 channels of both projections, one workgroup's share of a 128-wide rotation: the large ones.
-  // (us, the two calls / one: MXFP4 8192 x 14336 x 4096 583.6 / 476.7, 2048 rows 145.7 / 127.3, 1000 x 8448 x 2816 51.8 /
-  // 42.6, 333 x 17152 x 4352 43.9 / 40.8; NVFP4 8192 x 14336 x 4096 1422 / 1385, 1000 x 8448 x 2816 110.5 / 103.7)
-  const TilePlan plan = tile_plan<NV>(M, N, K, 0, device_cus());
-  if (plan.kind < 2) return FPQ_E_UNSUPPORTED;
+  TilePlan plan;
+  if (!gated_plan<NV>(M, channels, K, plan)) return FPQ_E_UNSUPPORTED;
   if (const int st = silu_table_address(stream, &out.silu)) return st;
   out.channels = (int)channels;
   if constexpr (NV) {
@@ -1364,8 +1380,8 @@ static int gemm_packed_gated(const void* xq, const void* xs, const void* wq, con
 
 extern "C" int fpq_gemm_packed_gated_takes(int nv, int64_t M, int64_t channels, int64_t K) {
   if (M < 1 || channels < 1 || channels % 256 != 0 || K < 256 || K % 256 != 0) return 0;
-  const int cus = fpq::device_cus();
-  return (nv ? fpq::tile_plan<true>(M, 2 * channels, K, 0, cus) : fpq::tile_plan<false>(M, 2 * channels, K, 0, cus)).kind >= 2;
+  fpq::TilePlan plan;
+  return nv ? fpq::gated_plan<true>(M, channels, K, plan) : fpq::gated_plan<false>(M, channels, K, plan);
 }
 
 extern "C" int fpq_gemm_packed_gated(int nv, const void* xq, const void* xs, const void* wq, const void* ws,

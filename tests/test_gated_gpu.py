@@ -90,6 +90,22 @@ def test_refusals():
     assert call(k=100) == -2 and call(m=-1) == -2 and call(codes=None) == -1 and call(codes=p + 8) == -4 and call(m=0) == 0
 
 
+# More than 16384 channels: a single row tile is large tiles to the tile kernels, but up to 96 rows (MXFP4: 64) the GEMM that
+# would be replaced streams its weights, in another order of sums.
+@pytest.mark.parametrize("nv,m,channels,taken", [
+    (0, 1, 20480, 0), (0, 64, 16640, 0), (0, 65, 16640, 1), (0, 97, 16640, 1), (0, 128, 16640, 1),
+    (1, 1, 20480, 0), (1, 64, 16640, 0), (1, 65, 16640, 0), (1, 96, 20480, 0), (1, 97, 16640, 1), (1, 128, 16640, 1),
+])
+def test_few_rows_of_many_channels(nv, m, channels, taken):
+    from fp_quant import _engine
+    lib = _engine.lib()
+    assert lib.fpq_gemm_packed_gated_takes(nv, m, channels, 512) == taken
+    if taken:
+        return test_gated_bytes(nv, m, channels, 512, 0, 128, 0)
+    p = torch.zeros(1 << 10, dtype=torch.uint8, device="cuda").data_ptr()   # (nothing is launched)
+    assert lib.fpq_gemm_packed_gated(nv, p, p, p, p, p, m, channels, 512, 0, 128, 0.1, p, p, p, 0, None) == _engine.E_UNSUPPORTED
+
+
 @needs_packed
 @pytest.mark.parametrize("fmt,g,m", [("mxfp4", 128, 1037), ("mxfp4", 32, 2048), ("nvfp4", 16, 1037)])
 def test_fused_block_runs_the_gated_gemm(fmt, g, m, monkeypatch):
