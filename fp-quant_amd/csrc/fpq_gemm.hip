@@ -261,11 +261,10 @@ __global__ __launch_bounds__(256) void gemm_nvf4_one_row_kernel(
       const uint32_t aw[4] = {a[u].x, a[u].y, a[u].z, a[u].w}, bw[4] = {b[u].x, b[u].y, b[u].z, b[u].w};
       v8h bh[4];   // (converted ahead of the matrix instructions: 8 % faster than in turn with the weights')
 #pragma unroll
-      for (int s = 0; s < 4; ++s) bh[s] = dequant8_f16_s(bw[s], e4m3_pair_f16(tb >> (8 * (s >> 1))));
+      for (int s = 0; s < 4; ++s) bh[s] = dequant8_f16_h(bw[s], e4m3_signed_f16(tb, s >> 1));
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8_f16_s(aw[s], e4m3_pair_f16(ta >> (8 * (s >> 1)))), bh[s], acc,
-                                                     0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8_f16_h(aw[s], e4m3_signed_f16(ta, s >> 1)), bh[s], acc, 0, 0, 0);
     }
   }
   one_row_store(acc, part, y, bias, *alpha_p, n0, N, wave, lane);

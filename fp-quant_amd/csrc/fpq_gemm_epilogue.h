@@ -78,13 +78,8 @@ typedef const __attribute__((address_space(1))) void global_void;
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-// NVFP4 operands for the fp16 MFMA.  e4m3 byte (>= 0) -> the same value * 2^-8 as fp16, in both
-// halves of a dword (bits above the byte are ignored) ...
-__device__ __forceinline__ v2h e4m3_pair_f16(uint32_t byte) {
-  const uint32_t h = (byte << 7) & 0x3f80u;
-  return __builtin_bit_cast(v2h, h | (h << 16));
-}
-// ... and 8 E2M1 codes (one dword) times that scale -> 8 exact fp16 values (code * 2^8 * scale * 2^-8)
+// NVFP4 operands for the fp16 MFMA: 8 E2M1 codes (one dword) times an E4M3 scale that is held as value * 2^-8 in both halves
+// of a dword -> 8 exact fp16 values (code * 2^8 * scale * 2^-8)
 __device__ __forceinline__ v8h dequant8_f16_s(uint32_t codes, v2h s2) {
   const v2h p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 256.0f, 0) * s2;
   const v2h p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 256.0f, 1) * s2;

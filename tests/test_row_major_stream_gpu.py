@@ -57,3 +57,16 @@ def test_negative_e4m3_scales_keep_their_sign():
     pos = capi.gemm(xq, xs, wq, ws & 0x7F, 0.01, "nvfp4")
     y = capi.gemm(xq, xs, wq, ws, 0.01, "nvfp4")
     assert torch.equal(y[:, ::2], -pos[:, ::2]) and torch.equal(y[:, 1::2], pos[:, 1::2])
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 48, 2048), (2, 48, 2048), (1, 1100, 4096), (1, 33, 8192), (1, 48, 480), (64, 48, 2048)])
+def test_signed_e4m3_scales_match_the_oracle(m, n, k):
+    """Up to 64 rows every kernel, the one-row ones too, takes a scale byte's sign."""
+    import capi
+    gen = torch.Generator().manual_seed(m + n + k)
+    xq, wq = _codes(m, k, gen), _codes(n, k, gen)
+    xs, ws = (_scales(r, k, "nvfp4", gen, k // 16) for r in (m, n))
+    xs, ws = (s ^ (0x80 * torch.randint(0, 2, s.shape, dtype=torch.uint8, generator=gen)) for s in (xs, ws))
+    y = capi.gemm(xq, xs, wq, ws, 0.01, "nvfp4")
+    ref, mag = O.gemm_ref(xq, xs, wq, ws, 0.01, "nvfp4")
+    assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * mag).all()
