@@ -220,6 +220,12 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
   for (int i = 0; i < CN; ++i) {
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
+      // Padding rows have gates of zero, which are outside the table: row tiles of nothing else are left out, and a lane of
+      // padding does not send the others through the global table.  (It did, and the workgroups of the last rows ended last;
+      // decoder block, us, before / now: MXFP4 129 / 258 rows, 3072 -> 11008 77.8 / 74.5, 95.2 / 91.4, 317 rows, 2048 -> 6144
+      // 61.0 / 57.2; NVFP4 770 rows, 1536 -> 5120 119.9 / 110.4.)
+      const int m0 = m_blk + wm * TM * 32 + j * 32;
+      if (m0 >= M) break;   // (uniform)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {   // eight values at a time
         uint32_t gate[4], up[4];
@@ -230,7 +236,7 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
           gate[k] = pack_bf16x2(acc[i][j][v] * alpha, acc[i][j][v + 1] * alpha);
           up[k] = pack_bf16x2(acc[i + CN][j][v] * alpha, acc[i + CN][j][v + 1] * alpha);
         }
-        silu_lookup(gate, sv, (lds_f32*)silu, out.silu);
+        silu_lookup(gate, sv, (lds_f32*)silu, out.silu, m0 + r32 < M);
         uint8_t* const at = stage + (wm * TM * 32 + j * 32 + r32) * kStride + (wn * CN * 32 + i * 32 + 16 * h + 4 * kh) * 2;
 #pragma unroll
         for (int g = 0; g < 2; ++g)
@@ -248,6 +254,7 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
 #pragma unroll 1
     for (int p = 0; p < kRows; p += kThreads / 4) {
       const int row = p + wave * 16 + (lane >> 2), m = m_blk + row;
+      if (m_blk + p + wave * 16 >= padded) break;   // (uniform)
       auto load_rotate = [&](float (&v)[32]) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {

@@ -37,10 +37,11 @@ __device__ __forceinline__ void silu_table_to_lds(float* lds, const uint16_t* __
   }
 }
 
-// sv[i]: bf16(silu(.)) of the i-th of the bf16 values in `w`
+// sv[i]: bf16(silu(.)) of the i-th of the bf16 values in `w`.  live: whether anybody reads this lane's (other lanes get some
+// value of the table, and do not send the wave round again).
 template <int N>
 __device__ __forceinline__ void silu_lookup(const uint32_t (&w)[N], float (&sv)[2 * N], lds_f32* table,
-                                            const uint16_t* __restrict__ global) {
+                                            const uint16_t* __restrict__ global, bool live) {
   u16x2 most = u16x2{0, 0};
 #pragma unroll
   for (int k = 0; k < N; ++k) {
@@ -52,7 +53,7 @@ __device__ __forceinline__ void silu_lookup(const uint32_t (&w)[N], float (&sv)[
     sv[2 * k] = table[at.x];
     sv[2 * k + 1] = table[at.y];
   }
-  const bool outside = most.x >= kSiluLdsCount || most.y >= kSiluLdsCount;
+  const bool outside = live && (most.x >= kSiluLdsCount || most.y >= kSiluLdsCount);
   if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
 #pragma unroll
     for (int e = 0; e < 2 * N; ++e) {
