@@ -1052,6 +1052,16 @@ int gemm_fp4_stream_slabs(bool nv, const void* xq, const void* xs, const void* w
                           const float* alpha, const void* bias, const void* residual, void* y, int64_t M, int64_t N,
                           int64_t K, int64_t slab_rows, const OutSegments& seg, hipStream_t stream);
 
+// MXFP4, 256 x 128 tiles that have a CU to themselves and a long K: a ring of eight units.  Four units are 48 KB in
+// flight per CU, less than the weights' way from HBM takes at the rate one workgroup consumes them (two
+// workgroups per CU have 96 KB); weights from HBM, N = 4096, K = 14336: 1280 rows 59.6 -> 56.4 us, 1536 rows
+// 58.1 -> 53.6; N = 8192, K = 8192, 640 rows 35.3 -> 32.8; with the gated epilogue 14336 channels, K = 8192: 160 / 256 rows
+// 44.8 / 45.5 -> 40.9 / 43.3 (44.7 / 49.1 as two calls), 28672 channels, 65 / 128 rows 56.7 / 53.5 -> 54.3 / 52.7 (from the
+// caches 4-10 % slower; K = 4096 and NVFP4 measured the same either way and keep four).
+static bool deep_ring(int64_t M, int64_t N, int64_t K, int cus) {
+  return K >= 8192 && ((M + 127) / 128) * ((N + 255) / 256) <= cus;
+}
+
 // Whether gemm_packed gives a shape that it does not cut into slabs to the weight-streaming kernel.
 static bool streams(bool nv, int64_t M, int64_t N, int64_t K) {
   return stream_eligible(nv, M, N, K) && (!nv || M <= FPQ_NV_STREAM_ROWS);
@@ -1182,13 +1192,8 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
   if (plan.kind == 1)
     return launch_packed<4, 4, 4, 2, 2, NV>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream, residual, seg,
                                             plan.split, workspace);
-  // 256 x 128 tiles that have a CU to themselves and a long K: a ring of eight units.  Four units are 48 KB in
-  // flight per CU, less than the weights' way from HBM takes at the rate one workgroup consumes them (two
-  // workgroups per CU have 96 KB); weights from HBM, N = 4096, K = 14336: 1280 rows 59.6 -> 56.4 us, 1536 rows
-  // 58.1 -> 53.6; N = 8192, K = 8192, 640 rows 35.3 -> 32.8 (from the caches 4-10 % slower; K = 4096 and NVFP4
-  // measured the same either way and keep four).
   if constexpr (!NV) {
-    if (plan.kind == 2 && K >= 8192 && ((M + 127) / 128) * ((N + 255) / 256) <= cus)
+    if (plan.kind == 2 && deep_ring(M, N, K, cus))
       return launch_packed<8, 8, 4, 2, 2, false, 8>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
                                                     residual, seg);
   }
@@ -1380,6 +1385,8 @@ static int gemm_packed_gated(const void* xq, const void* xs, const void* wq, con
   out.channels = (int)channels;
   if constexpr (NV) {
     if (plan.kind == 3) return launch_gated<8, 8, NV, kRing>(xq, xs, wq, ws, alpha, M, K, stream, out);
+  } else if (deep_ring(M, N, K, device_cus())) {
+    return launch_gated<8, 4, NV, 8>(xq, xs, wq, ws, alpha, M, K, stream, out);
   }
   return launch_gated<8, 4, NV, 4>(xq, xs, wq, ws, alpha, M, K, stream, out);
 }

@@ -106,6 +106,12 @@ def test_few_rows_of_many_channels(nv, m, channels, taken):
     assert lib.fpq_gemm_packed_gated(nv, p, p, p, p, p, m, channels, 512, 0, 128, 0.1, p, p, p, 0, None) == _engine.E_UNSUPPORTED
 
 
+@pytest.mark.parametrize("nv,m,channels", [(0, 129, 8448), (0, 97, 16640), (0, 130, 16640), (1, 129, 8448)])
+def test_long_inner_dimension(nv, m, channels):
+    """K = 8192: MXFP4 at most one workgroup per CU (a ring of eight units), and more."""
+    test_gated_bytes(nv, m, channels, 8192, 0, 128, 0)
+
+
 @needs_packed
 @pytest.mark.parametrize("fmt,g,m", [("mxfp4", 128, 1037), ("mxfp4", 32, 2048), ("nvfp4", 16, 1037)])
 def test_fused_block_runs_the_gated_gemm(fmt, g, m, monkeypatch):
