@@ -219,6 +219,13 @@ __global__ __launch_bounds__(256) void gemm_mxf4_one_row_kernel(
   one_row_store(acc, part, y, bias, *alpha_p, n0, N, wave, lane);
 }
 
+// E4M3 byte `byte` of d, sign included, as fp16 (value * 2^-8) in both halves.  (From the sign-extended byte: with the sign bit
+// moved by itself one row of 28672 x 4096 took 19.8-20.3 us instead of 18.0, 1024 x 14336 14.6-15.1 instead of 13.1.)
+__device__ __forceinline__ v2h e4m3_signed_pair_f16(uint32_t d, int byte) {
+  const uint32_t h = ((uint32_t)__builtin_amdgcn_sbfe((int)d, 8 * byte, 8) << 7) & 0xbf80u;
+  return __builtin_bit_cast(v2h, h | (h << 16));
+}
+
 // NVFP4: a lane's 16 bytes of codes (32 K values) carry two E4M3 scales; dword s of every code load feeds fp16 matrix
 // instruction s of the step on both operands (K order permuted consistently), after exact dequantization to fp16.
 __global__ __launch_bounds__(256) void gemm_nvf4_one_row_kernel(
@@ -261,10 +268,11 @@ __global__ __launch_bounds__(256) void gemm_nvf4_one_row_kernel(
       const uint32_t aw[4] = {a[u].x, a[u].y, a[u].z, a[u].w}, bw[4] = {b[u].x, b[u].y, b[u].z, b[u].w};
       v8h bh[4];   // (converted ahead of the matrix instructions: 8 % faster than in turn with the weights')
 #pragma unroll
-      for (int s = 0; s < 4; ++s) bh[s] = dequant8_f16_h(bw[s], e4m3_signed_f16(tb, s >> 1));
+      for (int s = 0; s < 4; ++s) bh[s] = dequant8_f16_s(bw[s], e4m3_signed_pair_f16(tb, s >> 1));
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8_f16_h(aw[s], e4m3_signed_f16(ta, s >> 1)), bh[s], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8_f16_s(aw[s], e4m3_signed_pair_f16(ta, s >> 1)), bh[s], acc, 0, 0,
+                                                     0);
     }
   }
   one_row_store(acc, part, y, bias, *alpha_p, n0, N, wave, lane);
