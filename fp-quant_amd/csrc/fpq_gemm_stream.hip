@@ -1037,13 +1037,18 @@ static int linear_rows(const FewRows& in, int rot_kind, int g, const void* wq, c
 //   MXFP4 2 rows: 9.5 / 7.2, 16.6 / 15.7; 4 rows: K = 2048, N = 2560 8.5 / 7.2, N = 14336 9.5 / 9.4
 //   NVFP4 1 row:  12.2 / 9.2, 21.8 / 20.6; 2 rows 11.8 / 9.7, 21.3 / 21.6; 4 rows: K = 2048 9.4 / 8.4
 // Two passes (twice the registers for rows and weight) took 10.7 and 24.9 for 4 MXFP4 rows of K = 4096 (9.8, 16.8 in two kernels).
+static bool norm_rows_plan(bool nv, int64_t M, int64_t N, int64_t K, StreamPlan& plan) {
+  if (M > kFewNormRows || K > (1 << 20)) return false;
+  plan = stream_plan(M, N, K, 0, nv);
+  return few_rows_plan(plan, nv, kFewNorm, M, N, K, K);
+}
+
 template <bool NV>
 static int norm_rows_multi(const FewRows& in, int rot_kind, int g, const void* wq, const void* ws, const float* alpha,
                            const void* bias, const OutSegments& seg, int64_t M, int64_t N, int64_t K, int zero_policy,
                            hipStream_t stream) {
-  if (M > kFewNormRows || K > (1 << 20) || zero_policy != FPQ_ZERO_REFERENCE) return FPQ_E_UNSUPPORTED;
-  const StreamPlan plan = stream_plan(M, N, K, 0, NV);
-  if (!few_rows_plan(plan, NV, kFewNorm, M, N, K, K)) return FPQ_E_UNSUPPORTED;
+  StreamPlan plan;
+  if (zero_policy != FPQ_ZERO_REFERENCE || !norm_rows_plan(NV, M, N, K, plan)) return FPQ_E_UNSUPPORTED;
   return launch_few_rows<NV, kFewNorm>(in, plan, rot_kind, g, wq, ws, alpha, bias, nullptr, seg.y[0], M, N, K, nullptr, seg,
                                        stream);
 }
@@ -1154,4 +1159,9 @@ extern "C" int fpq_norm_rows_multi(int nv, const void* x, const void* norm_weigh
   const fpq::FewRows in{(const uint4*)x, (const uint4*)norm_weight, nullptr, global_scale, nullptr, nullptr, norm, (int)K, eps};
   return nv ? fpq::norm_rows_multi<true>(in, rot_kind, g, wq, ws, alpha, bias, seg, M, N, K, zero_policy, (hipStream_t)stream)
             : fpq::norm_rows_multi<false>(in, rot_kind, g, wq, ws, alpha, bias, seg, M, N, K, zero_policy, (hipStream_t)stream);
+}
+
+extern "C" int fpq_norm_rows_takes(int nv, int64_t M, int64_t N, int64_t K) {
+  fpq::StreamPlan plan;
+  return M > 0 && N > 0 && N <= (1 << 24) && fpq::norm_rows_plan(nv != 0, M, N, K, plan);
 }

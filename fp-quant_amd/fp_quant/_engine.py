@@ -61,6 +61,7 @@ _SIGNATURES = {
     "fpq_gemm_packed_gated": ([_I, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _I, _F, _P, _P, _P, _I, _P], _I),
     "fpq_gemm_packed_gated_takes": ([_I, _I64, _I64, _I64], _I),
     "fpq_norm_rows_multi": ([_I, _P, _P, _F, _I64, _I64, _I, _I, _F, _P, _P, _P, _P, _P, _P, _P, _I64, _I, _P], _I),
+    "fpq_norm_rows_takes": ([_I, _I64, _I64, _I64], _I),
     "fpq_linear_rows": ([_I, _P, _P, _I64, _I64, _I, _I, _F, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _I64, _I, _P],
                         _I),
     "fpq_unpack_mxf4": ([_P, _P, _I64, _I64, _P, _P, _I64, _P], _I),

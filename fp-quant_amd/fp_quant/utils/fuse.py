@@ -33,7 +33,7 @@ import ast
 import inspect
 import textwrap
 import types
-from typing import Dict, Optional
+from typing import Dict, Optional, Tuple
 
 import torch
 from torch import nn
@@ -229,13 +229,21 @@ def _hands_on(norm: nn.Module, reader: nn.Module) -> bool:
                      or hooks._global_forward_hooks or hooks._global_forward_pre_hooks))
 
 
-def _norm_joins(elements: int, width: int) -> bool:
-    """Row counts at which the projections' call takes the norm: with at most four rows it is part of the GEMM's launch, as long
-    as a wave holds its share of them (64 chunks of 32 elements: 4 x 2048, 1 x 8192; a call that is declined costs 3 us of host
-    time, 4 x 5120: 60.7 us a block, 64.2 with it); beyond 64 it is a launch that need not write the norm's output."""
-    if elements <= 4 * width:
-        return width % 256 == 0 and elements // width * -(-width // 1024) <= 8
-    return elements > 64 * width
+_NEVER = (0, 1 << 62)
+
+
+def _norm_bounds(layers) -> Tuple[int, int]:
+    """(few, many): the call of these projections takes the norm in front of them for inputs of at most `few` elements, where
+    it is part of the GEMM's launch, and of more than `many`, where it is a launch that need not write the norm's output.
+    Asked of the kernels' own rules, since a call that is declined costs 3 us of host time (block of 4 x 5120: 60.7 us, 64.2
+    with it): a wave holds 64 chunks of 32 elements (4 x 2048, 1 x 8192), NVFP4 converts no more than four weight tiles per
+    CU, and up to 640 rows of more than 8192 columns are two launches, which leave the norm's output anyway."""
+    width, nvfp4 = layers[0].in_features, layers[0].config.forward_dtype == FPQuantDtype.NVFP4
+    if not layers[0].qweight.is_cuda or width > 16384:
+        return _NEVER
+    takes, n = _eager()._engine.lib().fpq_norm_rows_takes, sum(layer.out_features for layer in layers)
+    few = max((m for m in range(1, 5) if width % 256 == 0 and takes(nvfp4, m, n, width)), default=0)
+    return few * width, min(640 * width, 1 << 23) if width > 8192 and width % 256 == 0 else 64 * width
 
 
 def fuse_gated_mlp(mlp: nn.Module) -> bool:
@@ -324,6 +332,7 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
         _attach_weight_group(mlp, ("gate_proj", "up_proj"))   # gate/up as one GEMM where the format allows
     mlp._fpq_unfused_forward = unfused
     mlp.forward = mlp._fpq_takes_norm = types.MethodType(forward, mlp)
+    mlp._fpq_norm_bounds = _norm_bounds(parts[:2])
     return True
 
 
@@ -416,7 +425,6 @@ def fuse_residual_adds(block: nn.Module) -> bool:
     if defaults is None:
         return False
     unfused = block.forward
-    width = o_proj.out_features
 
     def forward(self, hidden_states, *args, **kwargs):
         if args or not isinstance(hidden_states, torch.Tensor) or not _fusable_call(hidden_states):
@@ -424,8 +432,9 @@ def fuse_residual_adds(block: nn.Module) -> bool:
         attn = self.self_attn
         out_proj = attn.o_proj
         norm = self.input_layernorm
-        joins = _norm_joins(hidden_states.numel(), width)
-        if joins and _hands_on(norm, attn):
+        elements = hidden_states.numel()
+        few, many = vars(attn).get("_fpq_norm_bounds", _NEVER)
+        if (elements <= few or elements > many) and _hands_on(norm, attn):
             normed, extra = hidden_states, {"_fpq_norm": norm}
         else:
             normed, extra = norm(hidden_states), _NOTHING
@@ -439,7 +448,8 @@ def fuse_residual_adds(block: nn.Module) -> bool:
         if pending is not None:   # o_proj did not take it
             attn_out = hidden_states + attn_out
         norm, mlp = self.post_attention_layernorm, self.mlp
-        if joins and _hands_on(norm, mlp):
+        few, many = vars(mlp).get("_fpq_norm_bounds", _NEVER)
+        if (elements <= few or elements > many) and _hands_on(norm, mlp):
             return mlp(attn_out, residual=attn_out, norm=norm)
         return mlp(norm(attn_out), residual=attn_out)
 
@@ -591,6 +601,7 @@ def fuse_qkv(attn: nn.Module) -> bool:
     attn._fpq_unfused_forward = attn.forward
     attn.forward = types.MethodType(namespace["forward"], attn)
     attn._fpq_takes_norm = attn.forward if takes_norm else None
+    attn._fpq_norm_bounds = _norm_bounds(layers)
     return True
 
 
@@ -623,6 +634,7 @@ def unfuse_producers(model: nn.Module) -> None:
             module._fpq_unfused_forward = None
             vars(module).pop("_fpq_fused_forward", None)
             vars(module).pop("_fpq_takes_norm", None)
+            vars(module).pop("_fpq_norm_bounds", None)
             hook = getattr(module, "_fpq_weight_group_hook", None)
             if hook is not None:
                 hook.remove()

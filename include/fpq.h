@@ -385,6 +385,8 @@ int fpq_norm_rows_multi(int nv, const void* x, const void* norm_weight, float ep
                         float norm, const float* global_scale, const void* wq_packed, const void* ws_packed,
                         const float* alpha, const void* bias, void* const* ys, const int64_t* ns, int64_t count,
                         int zero_policy, void* stream);
+/* Whether fpq_norm_rows_multi takes these sizes (1; N: of all outputs) or answers FPQ_E_UNSUPPORTED (0). */
+int fpq_norm_rows_takes(int nv, int64_t M, int64_t N, int64_t K);
 /*
  * A gated MLP's gate and up projections and what feeds its down projection in one launch: what
  * fpq_gemm_{mxf4,nvf4}_packed_multi into gate and up [M, channels] followed by

@@ -83,15 +83,43 @@ def test_refusals():
     assert call(m=0) == 0
 
 
-@pytest.mark.parametrize("m,k", [(1, 8192), (1, 8448), (2, 4096), (2, 4352), (3, 2048), (3, 2304), (4, 2048), (4, 2304), (4, 256), (1, 384)])
-def test_rule_offers_what_the_kernel_takes(m, k):
-    from fp_quant import _engine
-    from fp_quant.utils.fuse import _norm_joins
-    p = torch.zeros(4 << 20, dtype=torch.uint8, device="cuda").data_ptr()
-    st = _engine.lib().fpq_norm_rows_multi(0, p, p, 1e-5, m, k, 0, 32, 0.1, None, p, p, p, None, (ctypes.c_void_p * 1)(p + (2 << 20)),
-                                           (ctypes.c_int64 * 1)(256), 1, 0, None)
-    assert _norm_joins(m * k, k) == (st == 0)
-    assert not _norm_joins(5 * k, k) and not _norm_joins(64 * k, k) and _norm_joins(65 * k, k)
+# (n: one weight tile, and on both sides of NVFP4's four tiles per CU)
+@pytest.mark.parametrize("nv", [0, 1])
+@pytest.mark.parametrize("m,k,n", [(1, 8192, 256), (1, 8448, 256), (2, 4096, 256), (2, 4352, 256), (3, 2048, 256), (3, 2304, 256),
+                                   (4, 2048, 256), (4, 2304, 256), (4, 256, 256), (1, 384, 256), (5, 256, 256),
+                                   (1, 1024, 32768), (1, 1024, 33024), (4, 1024, 33024)])
+def test_rule_offers_what_the_kernel_takes(nv, m, k, n):
+    from types import SimpleNamespace
+    from fp_quant import FPQuantDtype, _engine
+    from fp_quant.utils.fuse import _norm_bounds
+    buffer = torch.zeros(48 << 20, dtype=torch.uint8, device="cuda")
+    p = buffer.data_ptr()
+    st = _engine.lib().fpq_norm_rows_multi(nv, p, p, 1e-5, m, k, 0, 32, 0.1, p, p, p, p, None, (ctypes.c_void_p * 1)(p + (32 << 20)),
+                                           (ctypes.c_int64 * 1)(n), 1, 0, None)
+    config = SimpleNamespace(forward_dtype=FPQuantDtype.NVFP4 if nv else FPQuantDtype.MXFP4)
+    few, many = _norm_bounds([SimpleNamespace(in_features=k, out_features=n // 2, config=config, qweight=buffer)] * 2)
+    assert (m * k <= few) == (st == 0) and few <= 4 * k < 64 * k <= many
+
+
+@needs_packed
+@pytest.mark.parametrize("fmt,g", [("mxfp4", 128), ("nvfp4", 16)])
+@pytest.mark.parametrize("k,rows", [(2048, (1, 4, 5, 64, 65)), (8448, (1, 64, 65, 640, 641)), (16384, (1, 512, 513)), (1152, (1, 64, 65))])
+def test_rule_offers_what_the_call_takes(fmt, g, k, rows):
+    from fp_quant.utils import fuse
+    from perf.cases import BlockRMSNorm, _linear
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    layers = tuple(_linear(dict(fmt=fmt, g=g), k, 256, False, gen) for _ in range(2))
+    norm = BlockRMSNorm(k, gen)
+    assert fuse.fuse_rmsnorm(norm, layers[0])
+    group = fuse._weight_group(layers, create=True)
+    few, many = fuse._norm_bounds(layers)
+    with torch.no_grad():
+        for m in rows:
+            x = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
+            want = fuse._native_group(group, layers, norm(x))   # (the first makes the plans)
+            outs = fuse._native_group(group, layers, x, norm)
+            assert want is not None and (outs is None or all(torch.equal(a, b) for a, b in zip(outs, want)))
+            assert (outs is not None) == (m * k <= few or m * k > many), m
 
 
 @needs_packed
