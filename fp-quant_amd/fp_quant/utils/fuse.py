@@ -404,9 +404,6 @@ def _attention_call_defaults(block: nn.Module) -> Optional[Dict[str, object]]:
     return defaults
 
 
-_NOTHING: Dict[str, object] = {}
-
-
 def fuse_residual_adds(block: nn.Module) -> bool:
     """Move the two `residual + hidden_states` additions of a decoder block into the GEMMs of
     `self_attn.o_proj` and `mlp.down_proj`.  Needs the MLP patched by fuse_gated_mlp, `o_proj` an
@@ -435,13 +432,13 @@ def fuse_residual_adds(block: nn.Module) -> bool:
         elements = hidden_states.numel()
         few, many = vars(attn).get("_fpq_norm_bounds", _NEVER)
         if (elements <= few or elements > many) and _hands_on(norm, attn):
-            normed, extra = hidden_states, {"_fpq_norm": norm}
+            normed, kwargs["_fpq_norm"] = hidden_states, norm
         else:
-            normed, extra = norm(hidden_states), _NOTHING
+            normed = norm(hidden_states)
         state = vars(out_proj)   # (a plain attribute: what Module.__setattr__ does with one, without its searches)
         state["_fpq_residual"] = hidden_states
         try:
-            attn_out, _ = attn(hidden_states=normed, **{**defaults, **kwargs, **extra})
+            attn_out, _ = attn(hidden_states=normed, **{**defaults, **kwargs})
         finally:
             pending = state["_fpq_residual"]
             state["_fpq_residual"] = None
@@ -480,11 +477,10 @@ def _native_group(group, layers, x: torch.Tensor, norm=None):
     if group is None or None in layers:
         return None
     native = _native()
-    call, args = (native.group, (layers, x)) if norm is None else (native.norm_group, (layers, x, norm))
-    outs = call(group.plan, *args)
+    outs = native.group(group.plan, layers, x) if norm is None else native.norm_group(group.plan, layers, x, norm)
     if outs is False and _host().learnable():
         _host().learn_group(group, layers)
-        outs = call(group.plan, *args)
+        outs = native.group(group.plan, layers, x) if norm is None else native.norm_group(group.plan, layers, x, norm)
     return outs or None
 
 
