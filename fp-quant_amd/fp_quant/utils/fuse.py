@@ -237,11 +237,17 @@ def _norm_bounds(layers) -> Tuple[int, int]:
     it is part of the GEMM's launch, and of more than `many`, where it is a launch that need not write the norm's output.
     Asked of the kernels' own rules, since a call that is declined costs 3 us of host time (block of 4 x 5120: 60.7 us, 64.2
     with it): a wave holds 64 chunks of 32 elements (4 x 2048, 1 x 8192), NVFP4 converts no more than four weight tiles per
-    CU, and up to 640 rows of more than 8192 columns are two launches, which leave the norm's output anyway."""
+    CU, up to 640 rows of more than 8192 columns are two launches, which leave the norm's output anyway, and the norm's
+    kernels know Hadamard rotations and none."""
     width, nvfp4 = layers[0].in_features, layers[0].config.forward_dtype == FPQuantDtype.NVFP4
+    h = layers[0].forward_hadamard_matrix
     if not layers[0].qweight.is_cuda or width > 16384:
         return _NEVER
-    takes, n = _eager()._engine.lib().fpq_norm_rows_takes, sum(layer.out_features for layer in layers)
+    eager = _eager()
+    if (eager.classify_rotation(eager.as_bf16(h))[0] not in (eager._engine.ROT_HADAMARD, eager._engine.ROT_IDENTITY)
+            or width % max(h.shape[0], 32) != 0):
+        return _NEVER
+    takes, n = eager._engine.lib().fpq_norm_rows_takes, sum(layer.out_features for layer in layers)
     few = max((m for m in range(1, 5) if width % 256 == 0 and takes(nvfp4, m, n, width)), default=0)
     return few * width, min(640 * width, 1 << 23) if width > 8192 and width % 256 == 0 else 64 * width
 

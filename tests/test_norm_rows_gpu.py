@@ -97,18 +97,19 @@ def test_rule_offers_what_the_kernel_takes(nv, m, k, n):
     st = _engine.lib().fpq_norm_rows_multi(nv, p, p, 1e-5, m, k, 0, 32, 0.1, p, p, p, p, None, (ctypes.c_void_p * 1)(p + (32 << 20)),
                                            (ctypes.c_int64 * 1)(n), 1, 0, None)
     config = SimpleNamespace(forward_dtype=FPQuantDtype.NVFP4 if nv else FPQuantDtype.MXFP4)
-    few, many = _norm_bounds([SimpleNamespace(in_features=k, out_features=n // 2, config=config, qweight=buffer)] * 2)
+    few, many = _norm_bounds([SimpleNamespace(in_features=k, out_features=n // 2, config=config, qweight=buffer,
+                                              forward_hadamard_matrix=torch.eye(32, device="cuda").bfloat16())] * 2)
     assert (m * k <= few) == (st == 0) and few <= 4 * k < 64 * k <= many
 
 
 @needs_packed
-@pytest.mark.parametrize("fmt,g", [("mxfp4", 128), ("nvfp4", 16)])
+@pytest.mark.parametrize("fmt,g,init", [("mxfp4", 128, "hadamard"), ("nvfp4", 16, "identity"), ("mxfp4", 64, "gsr")])
 @pytest.mark.parametrize("k,rows", [(2048, (1, 4, 5, 64, 65)), (8448, (1, 64, 65, 640, 641)), (16384, (1, 512, 513)), (1152, (1, 64, 65))])
-def test_rule_offers_what_the_call_takes(fmt, g, k, rows):
+def test_rule_offers_what_the_call_takes(fmt, g, init, k, rows):
     from fp_quant.utils import fuse
     from perf.cases import BlockRMSNorm, _linear
     gen = torch.Generator(device="cuda").manual_seed(k)
-    layers = tuple(_linear(dict(fmt=fmt, g=g), k, 256, False, gen) for _ in range(2))
+    layers = tuple(_linear(dict(fmt=fmt, g=g, init=init), k, 256, False, gen) for _ in range(2))
     norm = BlockRMSNorm(k, gen)
     assert fuse.fuse_rmsnorm(norm, layers[0])
     group = fuse._weight_group(layers, create=True)
