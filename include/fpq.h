@@ -390,7 +390,8 @@ int fpq_norm_rows_takes(int nv, int64_t M, int64_t N, int64_t K);
 /*
  * A gated MLP's gate and up projections and what feeds its down projection in one launch: what
  * fpq_gemm_{mxf4,nvf4}_packed_multi into gate and up [M, channels] followed by
- * fpq_silu_mul_quantize_{mx,nv}_packed of the two computes, to the bit, without writing gate and up.
+ * fpq_silu_mul_quantize_{mx,nv}_packed of the two computes, to the bit, without writing gate and up (except the codes of
+ * elements that the rotation leaves NaN: of a NaN's sign, which is the compiler's order of additions, or zero).
  * Operands as fpq_gemm_{mxf4,nvf4}_packed with N = 2 * channels, gate's rows first; channels % 256 == 0; rotation,
  * global scale and packed outputs as fpq_silu_mul_quantize_{mx,nv}_packed.  FPQ_E_UNSUPPORTED, with nothing launched,
  * where the two calls are the better way (few rows) or the only one (a rotation or zero policy the kernel lacks).
