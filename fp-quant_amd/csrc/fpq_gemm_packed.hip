@@ -332,7 +332,7 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
 // small tiles spends most of a unit waiting -- for its loads, for the barrier, for its two or four matrix
 // instructions to drain -- and alone on its SIMD nothing fills that time; with a second wave there, working
 // on the other half of K, something does, and each group's loop is half as long.
-// GR = 4 (NVFP4): four groups of two waves, a quarter of K each; see tile_plan.
+// GR = 4 (NVFP4): four groups of two waves, a quarter of K each; see tile_plan.  (Both: 128 x 128 tiles.)
 //
 // WN = WM = 1, GR = 8 (kSolo), 64 x 128 tiles: every wave multiplies the whole tile over an eighth of K, with a ring of its
 // own, and the eight parts are added through LDS.  What bounded these tiles was the waves' lockstep: at every unit's barrier
@@ -1018,7 +1018,9 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_byt
   // HBM, us: NVFP4 N = 4096: K = 12288, 512 rows 51.6 -> 45.0, K = 14336, 384 rows 52.7 -> 44.5, K = 4096, 300 / 512 rows
   // 20.3 / 21.0 -> 17.7 / 19.2, K = 3328, 300 rows 21.3 -> 16.1; N = 8192, K = 8192, 256 rows 37.3 -> 34.0; N = 6144, 144 / 200
   // rows 19.8 / 19.7 -> 17.6 / 17.3; N = 14336, 128 rows 22.8 -> 21.3; K = 2048, N = 5120, 200 rows 12.5 -> 11.8.  An odd
-  // number of blocks long enough to be cut across workgroups still is: callers size their workspace for it.
+  // number of blocks from 32 on keeps the K split that callers bring the workspace of fpq_gemm_nvf4_packed_workspace_bytes for,
+  // although it is behind (split / the same without a workspace / eight waves: K = 11008, N = 4096: 300 rows 56.0 / 61.1 /
+  // 34.9, 512 rows 59.8 / 66.6 / 41.6): rule and query have to move together.
   // MXFP4, whose waves do not convert anything, has to earn the longer tail with a long K, and with weights that more than
   // one row of tiles reads: N = 4096: K = 14336, 320 / 384 / 512 rows 29.1 / 27.8 / 30.5 -> 24.5 / 26.3 / 27.8, K = 8192, 512
   // rows 18.8 -> 18.1; N = 3072, K = 10240, 400 rows 21.5 -> 18.2; N = 8192, K = 8192, 256 rows 19.6 -> 19.4.  Not K = 4096, N =
@@ -1171,10 +1173,10 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
                              (hipStream_t)stream);
     }
   }
-  // At most 128 tiles of 128 x 128 would leave half of the CUs idle: 64 x 128 tiles (twice the workgroups, the
-  // same accumulation order and bits) take 25 instead of 34.5 us for NVFP4 at 257-512 rows, N = 4096, K = 4096
-  // (K = 12288: 69 instead of 97 us) and 4-7 % less for MXFP4; with more tiles they measured 14 % slower.
-  // Either of these two kernels splits K through the caller's workspace where that fills the CUs (tile_split_plan).
+  // At most 128 tiles of 128 x 128 would leave half of the CUs idle: 64 x 128 tiles, twice the workgroups (with more tiles they
+  // measured 14 % slower); eight waves with an eighth of K each where the plan says so, whose parts are added in an order of
+  // their own, else one group of four waves that walks K as the 128 x 128 tiles do.  The kernels of one group split K through
+  // the caller's workspace where that fills the CUs (NVFP4, tile_split_plan).
   if (plan.groups == 8)
     return launch_packed<2, NV ? 2 : 4, 4, 1, 1, NV, 2, 8>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
                                                            residual, seg);

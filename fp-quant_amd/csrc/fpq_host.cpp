@@ -729,8 +729,10 @@ PyObject* group_members(const GroupPlan::Body& p, PyObject* layers, THPObjectPtr
 }
 
 // What a norm in front of a group does to the group's call: rows that one launch takes together with the GEMM, rows whose
-// norm is a launch of its own but need not leave its bf16 result (8192 x 4096: 30.2 us with it, 23.9 without), or neither
-// (the caller runs the norm module first).
+// norm is a launch of its own but need not leave its bf16 result, or neither (the caller runs the norm module first; it asks
+// for these two only, fuse._norm_bounds).  Without the bf16 result the kernel of 8192 x 4096 takes 23.9 us instead of 30.2, a
+// decoder block of 8192 / 4096 tokens 956.7 / 471.8 instead of 967.2 / 477.2; from 65 to 2048 rows the GPU's time is the
+// same within 0.3 %, and the host has one call and two allocations less (128 rows of 2048 features: 53.4 -> 48.5).
 constexpr int64_t kNormInGemmRows = 4, kNormAloneRows = 64;
 
 // The quantized output of `norm` on x where that is a launch of its own.  1: done, 0: not the plain path
@@ -877,8 +879,8 @@ PyObject* host_gated_down(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   END_HANDLE_TH_ERRORS
 }
 
-// gated_mlp(plan, (gate, up), down, x, residual, norm): norm (unless it is None), group() and gated_down() of its outputs where one GEMM forms and
-// quantizes the product in its epilogue (fpq_gemm_packed_gated: many rows); None for any other call.
+// gated_mlp(plan, (gate, up), down, x, residual, norm): norm (unless it is None), group() and gated_down() of its outputs where
+// one GEMM forms and quantizes the product in its epilogue (fpq_gemm_packed_gated: many rows); None for any other call.
 PyObject* host_gated_mlp(PyObject*, PyObject* const* args, Py_ssize_t n_args) {
   HANDLE_TH_ERRORS
   if ((n_args != 5 && n_args != 6) || Py_TYPE(args[0]) != &GroupPlanType || !PyTuple_Check(args[1])) Py_RETURN_NONE;

@@ -1,8 +1,9 @@
 """K split inside the NVFP4 tile kernels (a few hundred rows on few weight rows: at most one 64 x 128 or
-128 x 128 workgroup tile per CU).  With an even number of 256-K blocks the workgroup has eight waves in two
-groups, each multiplying one half of K, and the halves meet in LDS (no workspace).  With an odd number and a
-long K (fpq_gemm_nvf4_packed_splitk beyond 256 rows) K is cut across workgroups: fp32 parts of the workgroup
-tiles meet in the caller's workspace and the workgroup that arrives last adds them in part order.  Checked: the
+128 x 128 workgroup tile per CU).  With an even number of 256-K blocks the workgroup has eight waves, which
+multiply parts of K that meet in LDS (no workspace): an eighth each on 64 x 128 tiles, a quarter or a half in
+four or two groups on 128 x 128 tiles.  With an odd number and a long K (fpq_gemm_nvf4_packed_splitk beyond 256
+rows) K is cut across workgroups: fp32 parts of the workgroup tiles meet in the caller's workspace and the
+workgroup that arrives last adds them in part order.  Checked: the
 oracle's values (bias and residual included), the same bits on every repetition, counters left at zero, a
 smaller workspace only means fewer parts, and the layer takes the same kernel eagerly, through the traced
 operator and under a graph capture.
@@ -36,8 +37,8 @@ def _operands(m, n, k, seed):
 # edges in both directions
 SHAPES = [(300, 1024, 8448), (512, 4096, 12544), (384, 2048, 14592), (257, 200, 8448), (700, 520, 8448),
           (1000, 1024, 8448)]
-# an even number of blocks: two groups of four waves per workgroup -- 64 x 128 and 128 x 128 tiles, one block per
-# group up to 28, ragged edges, 129-256 rows on many weight rows
+# an even number of blocks -- 64 x 128 tiles, an eighth of K per wave: the first four; 128 x 128 tiles in four groups: 640 and
+# 200 rows, in two: 129 rows; 256 x 128 tiles: 513 rows; ragged edges, a single block per part
 GROUP_SHAPES = [(512, 4096, 12288), (300, 4100, 8192), (1000, 1100, 2560), (384, 4096, 14336), (640, 4096, 4096),
                 (200, 12288, 2048), (129, 16384, 2560), (513, 8190, 3072)]
 
@@ -91,7 +92,7 @@ def test_two_groups_per_workgroup_match_the_oracle(m, n, k):
     tol = 2.0 ** -7 * torch.maximum(want.double().abs(), ref.abs()) + 2.0 ** -7 * res[ri][:, ci].double().abs() + 1e-5 * mag + 1e-6
     assert ((got.double() - want.double()).abs() <= tol).all()
     assert (got.view(torch.int16) == want.view(torch.int16)).double().mean() > 0.95
-    for _ in range(3):   # the halves are added in a fixed order
+    for _ in range(3):   # the parts are added in a fixed order
         again = capi.gemm_nv_packed(xp, xsp, wp, wsp, m, n, k, ALPHA, bias=bias, residual=res)
         assert torch.equal(again.view(torch.int16), y.view(torch.int16))
     # a workspace changes nothing: these shapes need none
