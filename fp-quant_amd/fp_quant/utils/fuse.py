@@ -143,15 +143,17 @@ def _weight_group(layers, create: bool = False, previous=None):
 
 
 def _attach_weight_group(module: nn.Module, names) -> None:
-    """Build the WeightGroup of module.<names> now and keep it in `module._fpq_weight_group`; rebuilt after
-    every load_state_dict into the module (a hook), so that traced code, which cannot check tensor
-    addresses and counters, never multiplies by weights that have been replaced."""
+    """Build the WeightGroup of module.<names> now and keep it in `module._fpq_weight_group`, beside the sizes at which its
+    call takes a norm (_norm_bounds); rebuilt after every load_state_dict into the module (a hook), so that traced code, which
+    cannot check tensor addresses and counters, never multiplies by weights that have been replaced."""
     def build(*_):
         layers = [getattr(module, n) for n in names]
+        real = all(_is_real_quant_linear(l) for l in layers)
         # (built into the buffers of the group it replaces where the shapes allow: a recorded graph keeps
         # pointing at the current weights)
         module._fpq_weight_group = (_weight_group(layers, create=True, previous=getattr(module, "_fpq_weight_group", None))
-                                    if all(_is_real_quant_linear(l) for l in layers) else None)
+                                    if real else None)
+        module._fpq_norm_bounds = _norm_bounds(layers) if real else _NEVER
 
     build()
     module._fpq_weight_group_build = build   # for whoever rewrites the layers' weights by other means
@@ -338,7 +340,6 @@ def fuse_gated_mlp(mlp: nn.Module) -> bool:
         _attach_weight_group(mlp, ("gate_proj", "up_proj"))   # gate/up as one GEMM where the format allows
     mlp._fpq_unfused_forward = unfused
     mlp.forward = mlp._fpq_takes_norm = types.MethodType(forward, mlp)
-    mlp._fpq_norm_bounds = _norm_bounds(parts[:2])
     return True
 
 
@@ -603,7 +604,6 @@ def fuse_qkv(attn: nn.Module) -> bool:
     attn._fpq_unfused_forward = attn.forward
     attn.forward = types.MethodType(namespace["forward"], attn)
     attn._fpq_takes_norm = attn.forward if takes_norm else None
-    attn._fpq_norm_bounds = _norm_bounds(layers)
     return True
 
 
