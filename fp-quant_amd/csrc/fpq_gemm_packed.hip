@@ -1018,7 +1018,7 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_byt
   // HBM, us: NVFP4 N = 4096: K = 12288, 512 rows 51.6 -> 45.0, K = 14336, 384 rows 52.7 -> 44.5, K = 4096, 300 / 512 rows
   // 20.3 / 21.0 -> 17.7 / 19.2, K = 3328, 300 rows 21.3 -> 16.1; N = 8192, K = 8192, 256 rows 37.3 -> 34.0; N = 6144, 144 / 200
   // rows 19.8 / 19.7 -> 17.6 / 17.3; N = 14336, 128 rows 22.8 -> 21.3; K = 2048, N = 5120, 200 rows 12.5 -> 11.8.  An odd
-  // number of blocks from 32 on keeps the K split that callers bring the workspace of fpq_gemm_nvf4_packed_workspace_bytes for,
+  // number of blocks from 33 on keeps the K split that callers bring the workspace of fpq_gemm_nvf4_packed_workspace_bytes for,
   // although it is behind (split / the same without a workspace / eight waves: K = 11008, N = 4096: 300 rows 56.0 / 61.1 /
   // 34.9, 512 rows 59.8 / 66.6 / 41.6): rule and query have to move together.
   // MXFP4, whose waves do not convert anything, has to earn the longer tail with a long K, and with weights that more than

@@ -240,7 +240,7 @@ def _norm_bounds(layers) -> Tuple[int, int]:
     Asked of the kernels' own rules, since a call that is declined costs 3 us of host time (block of 4 x 5120: 60.7 us, 64.2
     with it): a wave holds 64 chunks of 32 elements (4 x 2048, 1 x 8192), NVFP4 converts no more than four weight tiles per
     CU, up to 640 rows of more than 8192 columns are two launches, which leave the norm's output anyway, and the norm's
-    kernels know Hadamard rotations and none."""
+    kernels know Hadamard rotations and the identity only."""
     width, nvfp4 = layers[0].in_features, layers[0].config.forward_dtype == FPQuantDtype.NVFP4
     h = layers[0].forward_hadamard_matrix
     if not layers[0].qweight.is_cuda or width > 16384:
