@@ -279,7 +279,9 @@ __device__ __forceinline__ bool quantize_chunk(const float (&v)[EPL], float gs, 
   return need_slow;
 }
 
-// UNROLL: for kernels that may not have an array in scratch memory (cw, indexed by a loop's group)
+// UNROLL: for kernels that may not have an array in scratch memory (v and cw, indexed by a loop's group): setting it up
+// costs every launch, although hardly any takes this path.  The streaming kernels, larger and longer, measured the same
+// either way (NVFP4 8192 x 4096 16.4 us) or worse unrolled (MXFP4 4096 x 5120, 64-wide, 11.3 -> 13.0) and keep the loop.
 template <int EPL, int FMT, int ZERO, bool UNROLL = false>
 __device__ __forceinline__ void quantize_chunk_slow(const float (&u)[EPL], float gs, float rg,
                                                     uint32_t (&cw)[EPL / 8], uint32_t& sbytes) {
