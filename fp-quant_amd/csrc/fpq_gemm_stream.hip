@@ -27,12 +27,10 @@
 
 #include "../../include/fpq.h"
 #include "fpq_device.h"
+#include "fpq_few_rows.h"
 #include "fpq_gemm_epilogue.h"
-#include "fpq_quantize_chunk.h"
 
 namespace fpq {
-
-typedef unsigned v4u_s __attribute__((ext_vector_type(4)));
 
 constexpr int kStreamCounters = 4096;                        // one per weight tile group
 constexpr int64_t kStreamCounterBytes = kStreamCounters * 4;  // they open the workspace
@@ -53,18 +51,6 @@ constexpr int stream_dynamic_lds(int nt, int mt) {
 //
 // IN = FewRows: the activations come as bf16 rows (few of them) and every wave rotates and quantizes the 256-K blocks it
 // multiplies, while its weights are on their way.  See few_rows_plan.
-struct Packed {};
-struct FewRows {
-  const uint4* x;            // bf16 [M, xk]; SiLU*up: gate
-  const uint4* up;           // SiLU*up: the multiplier; RMSNorm: the norm's weight [xk]
-  const uint16_t* silu;      // ... and the table of bf16(silu(g))
-  const float* gs;           // NVFP4: the activations' global scale
-  uint8_t *codes, *scales;   // optional: the quantized rows, in the packed layout (rows past M are not written)
-  float norm;
-  int xk;                    // a multiple of 32 and of the rotation's size; K is padded to whole blocks
-  float eps;                 // RMSNorm
-};
-enum { kFewPlain = 0, kFewSilu = 1, kFewNorm = 2 };   // what a few rows' chunk goes through before it is rotated
 // IN = RowMajor: both operands as the quantize operators write them, codes [rows, k / 2] and scales [rows, stride] with the
 // strides multiples of four.  A lane takes the same 16 bytes of codes of a row, and the same scale bytes, as from the
 // packed layout, so the sums are the same bit for bit; only the addresses differ.  See launch_rows.
@@ -74,10 +60,6 @@ struct RowMajor {
   int k;
   uint32_t xs_stride, ws_stride;
 };
-// 32-element chunks a wave quantizes at most: one per lane and pass
-constexpr int few_rows_passes(int pro) { return pro == kFewPlain ? 2 : 1; }
-constexpr int few_rows_chunks(int pro) { return 64 * few_rows_passes(pro); }
-constexpr int kFewNormRows = 4;   // at most, with a norm (see norm_rows_multi)
 
 template <int NT, int MT, int DB, int NW, bool NV = false, class IN = Packed, int XG = 32, int XROT = FPQ_ROT_IDENTITY,
           int XPRO = kFewPlain>
@@ -348,19 +330,18 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
       }
     }
   };
-  // Few rows: the wave's quantized chunks, 16 bytes of codes each, and their scale bytes in the order the matrix
-  // instruction takes them: [block][K half][K step].  Lanes past the last row read row 0's, as above.
-  __shared__ __attribute__((aligned(16))) uint8_t few_codes[kFew ? 4 : 1][kFew ? few_rows_chunks(XPRO) * 16 : 16];
-  __shared__ __attribute__((aligned(16))) uint8_t few_scales[kFew ? 4 : 1][kFew ? few_rows_chunks(XPRO) * (NV ? 2 : 1) : 16];
+  // (lanes past the last row read row 0's chunks, as above)
+  typedef std::conditional_t<kFew, typename FewChunks<NV, XG, XROT, XPRO, NW>::Shared, Packed> FewShared;
+  __shared__ __attribute__((aligned(16))) FewShared few_shared;
   const int few_row = (lane & 31) < M ? (lane & 31) * nblk : 0;   // first block of the lane's row
   auto run_block = [&](auto slot, int t) __attribute__((always_inline)) {
     if constexpr (kFew) {
       constexpr int s = decltype(slot)::value;
       const int blk = few_row + t, kh = lane >> 5;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) b[s][u][0] = *(const uint4*)&few_codes[wave][(blk * 8 + 2 * u + kh) * 16];
-      if constexpr (NV) sb[s][0] = *(const uint2*)&few_scales[wave][blk * 16 + kh * 8];
-      else sb[s][0].x = *(const uint32_t*)&few_scales[wave][blk * 8 + kh * 4];
+      for (int u = 0; u < 4; ++u) b[s][u][0] = *(const uint4*)&few_shared.codes[wave][(blk * 8 + 2 * u + kh) * 16];
+      if constexpr (NV) sb[s][0] = *(const uint2*)&few_shared.scales[wave][blk * 16 + kh * 8];
+      else sb[s][0].x = *(const uint32_t*)&few_shared.scales[wave][blk * 8 + kh * 4];
     }
     if constexpr (kRow) {
       constexpr int s = decltype(slot)::value;
@@ -408,171 +389,13 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // more).  With three or four activation row tiles the effect is within +-4 % either way; only four tiles
   // of NVFP4 gain throughout (128 rows, N = 4096: 15.1 -> 14.6 us).  One block in flight has nothing to order.
   constexpr bool kOrdered = NT == 1 && DB >= 2 && (MT <= 2 || (NV && MT == 4));
-  // Few rows: the wave's chunks in lane order, row by row (the eight chunks of a block are neighbours, so the lanes of
-  // a rotation block are); asked for before the weights, since loads complete in order.
-  constexpr int kFewPasses = kFew ? few_rows_passes(XPRO) : 1;
-  const int few_chunks = kFew ? M * nblk * 8 : 0;
-  uint4 xr[kFewPasses][4], ur[XPRO != kFewPlain ? kFewPasses : 1][4];
-  int few_col[kFewPasses], few_at[kFewPasses];
-  if constexpr (kFew) {
-#pragma unroll
-    for (int p = 0; p < kFewPasses; ++p) {
-      const int ci = min(p * 64 + lane, max(few_chunks - 1, 0)), blk = ci >> 3, row = nblk > 0 ? blk / nblk : 0;
-      const int kb = nblk > 0 ? first + NW * (blk - row * nblk) : 0;
-      few_col[p] = kb * 256 + (ci & 7) * 32;
-      few_at[p] = row * 0x10000 + kb;
-      // (a chunk in the padding of the last block reads the row's start and is replaced by zeros)
-      const size_t at = ((size_t)row * in.xk + (few_col[p] < in.xk ? few_col[p] : 0)) >> 3;
-      if (p == 0 || few_chunks > 64) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          xr[p][i] = in.x[at + i];
-          if constexpr (XPRO == kFewSilu) ur[p][i] = in.up[at + i];
-          if constexpr (XPRO == kFewNorm) ur[p][i] = in.up[few_col[p] / 8 + i];   // (xk is whole blocks there)
-        }
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  FewChunks<NV, XG, XROT, XPRO, NW> few;
+  if constexpr (kFew) few.load(in, M, first, nblk, lane);
   for_slots([&](auto slot) {
     load_block(slot, decltype(slot)::value);
     if constexpr (kOrdered || kFew) __builtin_amdgcn_sched_barrier(0);
   });
-  if constexpr (kFew) {
-    constexpr int FMT = NV ? kFmtNv : kFmtMx;
-    __shared__ float2 lut[NV ? 128 : 1];
-    float gs = 1.0f, rg = 1.0f;
-    bool nv_fast = true;
-    if constexpr (NV) {
-      gs = *in.gs;
-      rg = gs == 0.0f ? 0.0f : 1.0f / gs;
-      nv_fast = nv_global_scale_fast(gs);
-      if (threadIdx.x < 128) lut[threadIdx.x] = nv_division(threadIdx.x, rg, nv_fast);
-    }
-    // RMSNorm: the octets' sums of squares of all rows, added by every wave in row_inv_rms_kernel's order
-    constexpr int kOctets = few_rows_chunks(kFewNorm) * 4 * 4;   // of a workgroup's rows, at most
-    __shared__ __attribute__((aligned(16))) float octets[XPRO == kFewNorm ? kOctets : 4];
-    float row_rs[kFewNormRows] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (XPRO == kFewNorm) {
-#pragma unroll
-      for (int p = 0; p < kFewPasses; ++p) {
-        if (p * 64 + lane < few_chunks) {
-          float s[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float e[8];
-            unpack8(xr[p][i], e);
-            s[i] = e[0] * e[0];
-#pragma unroll
-            for (int k = 1; k < 8; ++k) s[i] = s[i] + e[k] * e[k];
-          }
-          *(v4f*)&octets[((few_at[p] >> 16) * in.xk + few_col[p]) / 8] = v4f{s[0], s[1], s[2], s[3]};
-        }
-      }
-    }
-    // (the weights' loads stay in flight: a barrier for LDS only)
-    if constexpr (NV || XPRO == kFewNorm) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if constexpr (XPRO == kFewNorm) {
-      const int cpr = in.xk / 8;
-      const float cols_f = (float)in.xk;
-#pragma unroll
-      for (int r = 0; r < kFewNormRows; ++r) {
-        if (r >= M) break;   // (uniform)
-        float a = 0.0f;
-        for (int c0 = 0; c0 < cpr; c0 += 512) {   // eight reads at a time (adding zero is adding nothing: a >= 0)
-          float t[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) t[i] = c0 + 64 * i + lane < cpr ? octets[r * cpr + c0 + 64 * i + lane] : 0.0f;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) a = a + t[i];
-        }
-        // the butterfly a += a[lane ^ m], m = 1, 2, ..., 32 (mirrors are lane ^ 4 and ^ 8 once a quad's lanes agree)
-        auto dpp = [](float v, auto ctrl) __attribute__((always_inline)) {
-          return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), decltype(ctrl)::value, 0xF, 0xF, true));
-        };
-        a = a + dpp(a, std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
-        a = a + dpp(a, std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
-        a = a + dpp(a, std::integral_constant<int, 0x141>{});   // row_half_mirror
-        a = a + dpp(a, std::integral_constant<int, 0x140>{});   // row_mirror
-        a = a + __shfl_xor(a, 16, 64);
-        a = a + __shfl_xor(a, 32, 64);
-        row_rs[r] = 1.0f / __builtin_sqrtf(a / cols_f + in.eps);
-      }
-    }
-#pragma unroll
-    for (int p = 0; p < kFewPasses; ++p) {
-      if (p * 64 < few_chunks) {   // (wave-uniform)
-        const int few_r = few_at[p] >> 16;
-        const float rs = few_r == 0 ? row_rs[0] : few_r == 1 ? row_rs[1] : few_r == 2 ? row_rs[2] : row_rs[3];
-        auto load_rotate = [&](float (&v)[32]) __attribute__((always_inline)) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float e[8];
-            unpack8(xr[p][i], e);
-            if constexpr (XPRO == kFewNorm) {
-              float q[8];
-              unpack8(ur[p][i], q);
-#pragma unroll
-              for (int k = 0; k < 8; k += 2) {
-                const uint32_t t = pack_bf16x2(e[k] * rs, e[k + 1] * rs);
-                const uint32_t pr = pack_bf16x2(bf16_lo(t) * q[k], bf16_hi(t) * q[k + 1]);
-                e[k] = bf16_lo(pr);
-                e[k + 1] = bf16_hi(pr);
-              }
-            }
-            if constexpr (XPRO == kFewSilu) {
-              float q[8];
-              unpack8(ur[p][i], q);
-              const uint32_t w[4] = {xr[p][i].x, xr[p][i].y, xr[p][i].z, xr[p][i].w};
-#pragma unroll
-              for (int k = 0; k < 8; ++k) {
-                const uint32_t bits = (k & 1) ? w[k >> 1] >> 16 : w[k >> 1] & 0xffffu;
-                e[k] = __uint_as_float((uint32_t)in.silu[bits] << 16);
-              }
-#pragma unroll
-              for (int k = 0; k < 8; k += 2) {
-                const uint32_t pr = pack_bf16x2(e[k] * q[k], e[k + 1] * q[k + 1]);
-                e[k] = bf16_lo(pr);
-                e[k + 1] = bf16_hi(pr);
-              }
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[8 * i + k] = e[k];
-          }
-          rotate_chunk<32, XG, XROT, false>(v, in.norm, lane);
-        };
-        float v[32];
-        load_rotate(v);
-        uint32_t cw[4], sbytes = 0u, sb_lo = 0u;
-        bool need_slow = chunk_not_finite<32>(v);
-        need_slow |= quantize_chunk<32, FMT, kZeroReference, false>(v, gs, nv_fast, lut, cw, sbytes, sb_lo);
-        if (__builtin_amdgcn_ballot_w64(need_slow) != 0ull) {
-          float u[32];
-          load_rotate(u);
-          quantize_chunk_slow<32, FMT, kZeroReference>(u, gs, rg, cw, sbytes);
-        }
-        if (few_col[p] >= in.xk) {
-          cw[0] = cw[1] = cw[2] = cw[3] = 0u;
-          sbytes = 0u;
-        }
-        const int ci = p * 64 + lane, g8 = ci & 7;
-        if (ci < few_chunks) {
-          const uint4 c4 = make_uint4(cw[0], cw[1], cw[2], cw[3]);
-          *(uint4*)&few_codes[wave][ci * 16] = c4;
-          const int sc = (ci & ~7) + (g8 & 1) * 4 + (g8 >> 1);
-          if constexpr (NV) *(uint16_t*)&few_scales[wave][sc * 2] = (uint16_t)sbytes;
-          else few_scales[wave][sc] = (uint8_t)sbytes;
-          if (in.codes && blockIdx.x == 0) {   // the first weight tile's workgroups hand the rows on
-            const int row = few_at[p] >> 16, kb = few_at[p] & 0xffff, slot = (g8 & 1) * 32 + row;
-            *(uint4*)(in.codes + ((size_t)(kb * 4 + (g8 >> 1)) * 64 + slot) * 16) = c4;
-            if constexpr (NV) *(uint16_t*)(in.scales + (size_t)kb * 512 + slot * 8 + 2 * (g8 >> 1)) = (uint16_t)sbytes;
-            else in.scales[(size_t)kb * 256 + slot * 4 + (g8 >> 1)] = (uint8_t)sbytes;
-          }
-        }
-      }
-    }
-    asm volatile("" ::: "memory");   // (a wave's LDS accesses complete in order: its chunks are there when it reads them)
-  }
+  if constexpr (kFew) few.quantize(in, M, few_shared, wave, lane, in.codes && blockIdx.x == 0);
   // Where the epilogue will store, worked out while the first loads are in flight (after the reduction
   // every instruction delays the workgroup's end).  The epilogue's lane layout: 8 consecutive columns
   // (16 bytes) of row lane / 4 and of that row + 16.  16-byte accesses need the whole tile inside N and
@@ -957,7 +780,7 @@ int gemm_fp4_rows(bool nv, const void* xq, const void* xs, int64_t xs_stride, co
 //   MXFP4 4 rows (two passes):  4096 x 4096 7.2 / 5.7, N = 14336 10.2 / 8.1, N = 28672 14.9 / 14.5, N = 128256 45.5 / 49.0
 //   NVFP4 1 row:  4096 x 4096 9.4 / 7.2, N = 14336 12.6 / 9.8, N = 28672 19.6 / 17.9, N = 128256 59.8 / 65.3
 //   NVFP4 4 rows: 4096 x 4096 9.4 / 8.2, N = 14336 12.5 / 11.5, N = 28672 19.5 / 19.9
-// SiLU*up (two more gathers per element) gains in one pass only: MXFP4, K = 14336, N = 4096: 1 row 12.1 / 11.0, 2 rows
+// SiLU*up (two more lookups per element) gains in one pass only: MXFP4, K = 14336, N = 4096: 1 row 12.1 / 11.0, 2 rows
 // 12.2 / 13.2; 4096 x 4096: 1 row 7.5 / 5.9, 4 rows 7.8 / 9.3.
 static bool few_rows_plan(const StreamPlan& plan, bool nv, int pro, int64_t M, int64_t N, int64_t K, int64_t xk) {
   const int64_t chunks = M * ((plan.bps + 3) / 4) * 8;   // of the wave with the most
