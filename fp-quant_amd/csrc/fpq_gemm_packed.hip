@@ -334,15 +334,15 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
 // on the other half of K, something does, and each group's loop is half as long.
 // GR = 4 (NVFP4): four groups of two waves, a quarter of K each; see tile_plan.  (Both: 128 x 128 tiles.)
 //
-// WN = WM = 1, GR = 8 (kSolo), 64 x 128 tiles: every wave multiplies the whole tile over an eighth of K, with a ring of its
+// WN = WM = 1, GR = 8 (kSolo, NVFP4), 64 x 128 tiles: every wave multiplies the whole tile over an eighth of K, with a ring of its
 // own, and the eight parts are added through LDS.  What bounded these tiles was the waves' lockstep: at every unit's barrier
 // all of them converted operands or waited at the same time, so the matrix pipes had the other half of the time.  Without a
 // barrier in the loop the two waves of a SIMD drift apart and one's conversions (NVFP4: 0.75 operand tiles per matrix
 // instruction instead of 1) or waits run behind the other's matrix instructions; an operand is read from LDS by one wave
 // only.  Eight rings leave room for two units each, so a slot is refilled as soon as its unit has reached the registers.  It
-// pays with a longer tail (256 KB through LDS, 2 us).  us, weights from HBM, groups of two waves (MXFP4: one of four) / this:
-//   NVFP4 512 x 4096 x 12288 51.6 / 45.0 (1.15 PFLOP/s), 512 x 4096 x 4096 21.0 / 19.2, 300 x 4096 x 3328 21.3 / 16.1
-//   MXFP4 320 x 4096 x 14336 29.1 / 24.5, 512 x 4096 x 14336 30.5 / 27.8, 512 x 4096 x 4096 10.8 / 11.6
+// pays with a longer tail (256 KB through LDS, 2 us).  us, weights from HBM, groups of two waves / this:
+//   512 x 4096 x 12288 51.6 / 45.0 (1.15 PFLOP/s), 512 x 4096 x 4096 21.0 / 19.2, 300 x 4096 x 3328 21.3 / 16.1
+// (MXFP4 goes a step further there, operands straight to registers: row slabs of the weight-streaming kernel.)
 // OUT = GatedOut: the weight rows are a gate projection's and then an up projection's, and a workgroup's tile is NT / 2 row
 // tiles of each (gated_tile_store).
 template <int NT, int KW, int MT, int WN, int WM, bool NV = false, int RING = kRing, int GR = 1, class OUT = PlainOut>
@@ -670,21 +670,12 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
     FPQ_PREP_B(Q)                                                                                   \
     _Pragma("unroll") for (int i0 = 0; i0 < kHand; ++i0) FPQ_MFMA_ROW(Q, i0)                        \
     wait_vmem_le<(ALLOWED)>();                                                                      \
-    if constexpr (!kSolo) {                                                                         \
-      barrier_lds();                                                                                \
-      if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                                 \
-    }                                                                                               \
+    barrier_lds();                                                                                  \
+    if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                                   \
     if (READ) read_unit((U) + 1, ((Q) + 1) & 1);                                                    \
     if ((Q) == 3 && (NEXT_BLOCK)) read_scales(((U) + 1) >> 2);                                      \
     __builtin_amdgcn_sched_barrier(0);                                                              \
     _Pragma("unroll") for (int i1 = kHand; i1 < TN; ++i1) FPQ_MFMA_ROW(Q, i1)                       \
-    if constexpr (kSolo) {                                                                          \
-      if (ISSUE) {                                                                                  \
-        wait_lds();                                                                                 \
-        issue_unit((U) + 3, (Q) == 1);                                                              \
-        __builtin_amdgcn_sched_barrier(0);                                                          \
-      }                                                                                             \
-    }                                                                                               \
   }
 #define FPQ_TAKE_SCALES_NOW()                                                                       \
   {                                                                                                 \
@@ -1021,12 +1012,8 @@ static TilePlan tile_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_byt
   // number of blocks from 33 on keeps the K split that callers bring the workspace of fpq_gemm_nvf4_packed_workspace_bytes for,
   // although it is behind (split / the same without a workspace / eight waves: K = 11008, N = 4096: 300 rows 56.0 / 61.1 /
   // 34.9, 512 rows 59.8 / 66.6 / 41.6): rule and query have to move together.
-  // MXFP4, whose waves do not convert anything, has to earn the longer tail with a long K, and with weights that more than
-  // one row of tiles reads: N = 4096: K = 14336, 320 / 384 / 512 rows 29.1 / 27.8 / 30.5 -> 24.5 / 26.3 / 27.8, K = 8192, 512
-  // rows 18.8 -> 18.1; N = 3072, K = 10240, 400 rows 21.5 -> 18.2; N = 8192, K = 8192, 256 rows 19.6 -> 19.4.  Not K = 4096, N =
-  // 4096, 512 rows 10.8 -> 11.6; not one row of tiles, 128 rows, N = 14336: K = 4096 11.8 -> 13.4, K = 14336 32.2 -> 33.8.
   const int64_t nkb = K / 256;
-  if (plan.kind == 0 && (NV ? nkb >= 8 && (nkb % 2 == 0 || nkb < 2 * kTileSplitMinBlocks) : nkb >= 32 && M > 128)) {
+  if (NV && plan.kind == 0 && nkb >= 8 && (nkb % 2 == 0 || nkb < 2 * kTileSplitMinBlocks)) {
     plan.groups = 8;
     return plan;
   }
@@ -1052,7 +1039,7 @@ int gemm_fp4_stream(bool nv, const void* xq, const void* xs, const void* wq, con
                     void* workspace, int64_t workspace_bytes, const OutSegments& seg, hipStream_t stream);
 int gemm_fp4_stream_slabs(bool nv, const void* xq, const void* xs, const void* wq, const void* ws,
                           const float* alpha, const void* bias, const void* residual, void* y, int64_t M, int64_t N,
-                          int64_t K, int64_t slab_rows, const OutSegments& seg, hipStream_t stream);
+                          int64_t K, int64_t slab_rows, int nt, const OutSegments& seg, hipStream_t stream);
 
 // MXFP4, 256 x 128 tiles that have a CU to themselves and a long K: a ring of eight units.  Four units are 48 KB in
 // flight per CU, less than the weights' way from HBM takes at the rate one workgroup consumes them (two
@@ -1129,16 +1116,33 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
   const bool tile_splits = FPQ_TILE_SPLIT_OVER_SLABS && plan.split.ksplit > 1;
   {
     const int64_t tiles = (N + 31) / 32;
+    bool one_slab = false;
     const bool splits = tile_splits || (workspace && workspace_bytes > 16384 && M <= 96 &&
                                         gemm_mxf4_stream_workspace_bytes(M, N, K) > 0);
-    for (int64_t cap = 32; cap <= 128 && !splits; cap += 32) {
+    for (int64_t cap = 32; cap <= (NV ? 128 : 96) && !splits; cap += 32) {
       const int64_t slabs = (M + cap - 1) / cap;
       if (slabs * tiles > slab_workgroups(cus)) continue;
       const int64_t rows = ((M + slabs - 1) / slabs + 31) / 32 * 32;   // rows of a slab, whole 32-row tiles
       if (slabs > 1 && rows < M && stream_eligible(NV, rows, N, K))
-        return gemm_fp4_stream_slabs(NV, xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, rows, seg,
+        return gemm_fp4_stream_slabs(NV, xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, rows, 1, seg,
                                      (hipStream_t)stream);
+      one_slab = true;
       break;   // one slab, or a shape the kernel does not take: the paths below
+    }
+    // MXFP4: two weight tiles per workgroup.  The time follows what a workgroup loads per K step (weight tiles + activation
+    // tiles): two and two (or three) beat one and four, and the 64 x 128 tiles of the tile kernel.  Two and four do from K =
+    // 4096 on (below, the longer tail shows: 512 x 4096 x 1024 5.5 / 6.5).  us, weights from HBM, those / this: K = 4096:
+    // 160 rows, N = 8192 12.2 / 10.2, 200 rows, N = 4096 / 6144 8.4 / 7.8, 12.1 / 11.1, 333 rows, N = 4096 11.7 / 9.6; K = 8192,
+    // N = 8192: 128 / 160 / 256 rows 15.3 / 14.0, 19.2 / 15.5, 20.9 / 18.9; K = 14336, N = 4096: 200 / 384 / 512 rows 21.0 / 18.1,
+    // 28.5 / 22.8, 31.2 / 27.6.
+    for (int64_t cap = 64; cap <= (K >= 8192 ? 128 : 96) && !NV && !splits && !one_slab && K >= 1024; cap += 32) {
+      const int64_t slabs = (M + cap - 1) / cap;
+      if (slabs * ((tiles + 1) / 2) > slab_workgroups(cus)) continue;
+      const int64_t rows = ((M + slabs - 1) / slabs + 31) / 32 * 32;
+      if (slabs > 1 && rows > 32 && rows < M && stream_eligible(false, rows, N, K))
+        return gemm_fp4_stream_slabs(false, xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, rows, 2, seg,
+                                     (hipStream_t)stream);
+      break;
     }
   }
   if (streams(NV, M, N, K))
@@ -1174,13 +1178,12 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
     }
   }
   // At most 128 tiles of 128 x 128 would leave half of the CUs idle: 64 x 128 tiles, twice the workgroups (with more tiles they
-  // measured 14 % slower); eight waves with an eighth of K each where the plan says so, whose parts are added in an order of
-  // their own, else one group of four waves that walks K as the 128 x 128 tiles do.  The kernels of one group split K through
+  // measured 14 % slower); NVFP4 with eight waves and an eighth of K each where the plan says so, whose parts are added in an
+  // order of their own, else one group of four waves that walks K as the 128 x 128 tiles do.  The kernels of one group split K through
   // the caller's workspace where that fills the CUs (NVFP4, tile_split_plan).
-  if (plan.groups == 8)
-    return launch_packed<2, NV ? 2 : 4, 4, 1, 1, NV, 2, 8>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
-                                                           residual, seg);
   if constexpr (NV) {
+    if (plan.groups == 8)
+      return launch_packed<2, 2, 4, 1, 1, true, 2, 8>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream, residual, seg);
     if (plan.groups == 4)
       return launch_packed<4, 4, 4, 1, 2, true, 4, 4>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
                                                       residual, seg);

@@ -36,21 +36,37 @@ constexpr int kStreamCounters = 4096;                        // one per weight t
 constexpr int64_t kStreamCounterBytes = kStreamCounters * 4;  // they open the workspace
 constexpr int kStreamMaxRows = 128;
 
+// Output tiles whose parts of K are in LDS at a time: all, or half where all of them would not fit
+constexpr int stream_lds_tiles(int nt, int mt) { return nt * mt <= 8 ? nt * mt : (nt * mt + 1) / 2; }
 // Dynamic LDS of a workgroup with more than four output tiles (0: the kernel's own arrays hold them)
 constexpr int stream_dynamic_lds(int nt, int mt) {
-  return nt * mt > 4 ? 4 * nt * mt * 3 * 64 * 16 + nt * mt * 32 * 20 * 4 : 0;
+  return nt * mt > 4 ? 4 * stream_lds_tiles(nt, mt) * 3 * 64 * 16 + nt * mt * 32 * 20 * 4 : 0;
 }
 
 // NT weight row tiles per workgroup, MT activation row tiles (exactly ceil(M / 32)), DB 256-K blocks
 // of loads in flight per wave, NW waves.  Every workgroup re-reads all activations (NT = 2 halves
 // that, at a register cost that stream_plan explains).  Two weight tiles per workgroup are compiled for
 // two workgroups per CU (at most 256 registers).
+//
+// What bounds it.  A CU takes in about 60 bytes per nanosecond of a mix of weights from HBM and activations from the L2,
+// whatever number of loads a wave has outstanding (one or two blocks per wave, measured the same): they complete in order,
+// so an activation that the L2 would serve at once waits behind a weight, and some 64 KB are under way at a time (the
+// activations and weights of 512 x 4096 x 14336 take 26 us with the matrix instructions left out and 14 us the other way
+// round).  So the time follows the kilobytes that a workgroup loads per K step, NT + MT, as long as one round of the
+// CUs holds all workgroups; and MXFP4 with several weight tiles per workgroup (kUnits) streams K step by K step: a step's
+// registers are asked for again, one load behind each matrix instruction of the step after it, and not a whole block
+// at a time, which left the matrix pipes idle while the loads went out.  us, weights from HBM, block by block with one
+// weight tile per workgroup or two (or the tile kernels) / step by step: 64 x 14336 x 4096 11.2 / 10.3, 64 x 24576 x 4096
+// 15.8 / 13.0, 96 x 14336 x 4096 13.4 / 11.8, 32 x 28672 x 4096 15.2 / 12.9.
 // NV: NVFP4 operands (two E4M3 scale bytes per lane and K step, 512-byte scale blocks): a lane's dword s
 // of a 64-K unit, times its group's scale, is its fp16 operand of the s-th 32x32x16 matrix instruction
 // of the unit on both sides, so the K order is permuted consistently and the sum is complete.
 //
 // IN = FewRows: the activations come as bf16 rows (few of them) and every wave rotates and quantizes the 256-K blocks it
 // multiplies, while its weights are on their way.  See few_rows_plan.
+// IN = PackedSlabs: more than 32 MT activation rows in slabs of that many.  Dispatch goes round the XCDs workgroup by
+// workgroup: in a grid of 8 x slabs x eighths of the groups of weight tiles the slabs (blockIdx.y) of a group
+// (8 blockIdx.z + blockIdx.x) run on one XCD at about the same time, and all but one find the weights in its L2.
 // IN = RowMajor: both operands as the quantize operators write them, codes [rows, k / 2] and scales [rows, stride] with the
 // strides multiples of four.  A lane takes the same 16 bytes of codes of a row, and the same scale bytes, as from the
 // packed layout, so the sums are the same bit for bit; only the addresses differ.  See launch_rows.
@@ -70,25 +86,28 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
     float* partial, unsigned* counters, const OutSegments seg, const IN in) {
   constexpr bool kFew = std::is_same_v<IN, FewRows>;
   constexpr bool kRagged = std::is_same_v<IN, RowMajor<true>>, kRow = kRagged || std::is_same_v<IN, RowMajor<false>>;
+  constexpr bool kSlabs = std::is_same_v<IN, PackedSlabs>;
   static_assert(!kFew || (NT == 1 && MT == 1), "few rows: one tile");
+  constexpr bool kUnits = !NV && NT >= 2;   // K step by K step (see above)
   static_assert(NW == 4, "a wave owns a quarter of every tile");
-  // More than 32 MT activation rows: blockIdx.z numbers slabs of 32 MT rows, each a product of its own
-  // (the last may have fewer rows, even fewer row tiles).
-  const int slab = blockIdx.z, m0 = slab * (MT * 32);
+  // Slabs of 32 MT rows, each a product of its own (the last may have fewer rows, even fewer row tiles).
+  const int slab = kSlabs ? blockIdx.y : 0, m0 = slab * (MT * 32);
+  const int rtg = kSlabs ? blockIdx.z * 8 + blockIdx.x : blockIdx.x, split = kSlabs ? 0 : blockIdx.y;
   const int M = min(M_all - m0, MT * 32);
   const uint8_t* xq = xq_all + (size_t)slab * MT * (K >> 6) * 1024;
   const uint8_t* xs = xs_all + (size_t)slab * MT * (K >> 8) * (NV ? 512 : 256);
   const uint16_t* residual = residual_all ? residual_all + (size_t)m0 * N : nullptr;
-  const int tile_id = slab * gridDim.x + blockIdx.x;   // numbers the output tile groups for the K split
+  const int tile_id = rtg;   // numbers the output tile groups for the K split (slabs never come with one)
   constexpr int kStageRow = 20;             // dwords: 16 of a row's 32 bf16 + 4, rows stay 16-byte aligned
   constexpr int kStageTile = 32 * kStageRow;
   // part: [owning wave][tile][the other waves in order][lane]; stage: the rounded tiles on their way out.  More
   // than four tiles per workgroup need more than the 64 KB a kernel may declare: those take them from the
   // launch's dynamic LDS.
-  typedef v4f PartOf[NT * MT][3][64];
+  constexpr int kLdsTiles = stream_lds_tiles(NT, MT);
+  typedef v4f PartOf[kLdsTiles][3][64];
   typedef uint32_t StageOf[kStageTile];
   constexpr bool kDynLds = stream_dynamic_lds(NT, MT) > 0;
-  __shared__ v4f part_fixed[kDynLds ? 1 : 4][kDynLds ? 1 : NT * MT][3][64];
+  __shared__ v4f part_fixed[kDynLds ? 1 : 4][kDynLds ? 1 : kLdsTiles][3][64];
   __shared__ __attribute__((aligned(16))) uint32_t stage_fixed[kDynLds ? 1 : NT * MT][kStageTile];
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dynamic[];
   PartOf* const part = kDynLds ? (PartOf*)lds_dynamic : (PartOf*)part_fixed;
@@ -97,12 +116,14 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   constexpr int kSB = NV ? 512 : 256;    // scale bytes per row tile and 256-K block
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int nu = K >> 6, nkb = K >> 8;
-  const int rtg = blockIdx.x, split = blockIdx.y;
   const float alpha = *alpha_p;   // asked for now: the epilogue, on the critical path of every workgroup, finds it there
   const int rt_n = (N + 31) >> 5;
   const int kb_begin = split * bps, kb_end = min(nkb, kb_begin + bps);
   const int first = kb_begin + wave;                                   // this wave: first, first + NW, ...
-  const int nblk = kb_end > first ? (kb_end - first + NW - 1) / NW : 0;
+  // (Slabs: the groups of weight tiles may be rounded up to eights.  The ones past the last have no blocks and store nothing;
+  // a return at the top would have every workgroup wait for N before it asks for its other arguments, 0.2 us.)
+  const bool exists = !kSlabs || rtg * (NT * 32) < N;
+  const int nblk = kb_end > first && exists ? (kb_end - first + NW - 1) / NW : 0;
 
   // A weight tile past the last one (odd tile count, NT = 2) re-reads the last: nothing of it is stored.
   const uint8_t* wcode[NT];
@@ -181,6 +202,10 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
     else return kb * 128 + u * 32;
   };
   const int t_last = nblk > 0 ? nblk - 1 : 0;
+  auto load_weights = [&](const uint8_t* from) __attribute__((always_inline)) {
+    const v4u_s ld = __builtin_nontemporal_load((const v4u_s*)from);
+    return make_uint4(ld.x, ld.y, ld.z, ld.w);
+  };
   // (the lambdas must be inlined whatever their size: a call would pin the register arrays they capture
   // to memory)
   auto load_block = [&](auto slot, int t) __attribute__((always_inline)) {
@@ -205,8 +230,7 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
     for (int i = 0; i < NT; ++i) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const v4u_s ld = __builtin_nontemporal_load((const v4u_s*)(wcode[i] + (size_t)(kb * 4 + u) * 1024));
-        a[s][u][i] = make_uint4(ld.x, ld.y, ld.z, ld.w);
+        a[s][u][i] = load_weights(wcode[i] + (size_t)(kb * 4 + u) * 1024);
       }
       if constexpr (NV) sa[s][i] = *(const uint2*)(wscale[i] + (size_t)kb * kSB);
       else sa[s][i].x = *(const uint32_t*)(wscale[i] + (size_t)kb * kSB);
@@ -389,11 +413,79 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // more).  With three or four activation row tiles the effect is within +-4 % either way; only four tiles
   // of NVFP4 gain throughout (128 rows, N = 4096: 15.1 -> 14.6 us).  One block in flight has nothing to order.
   constexpr bool kOrdered = NT == 1 && DB >= 2 && (MT <= 2 || (NV && MT == 4));
+  // K step by K step (kUnits): the steps of the blocks in flight are a ring of 4 DB steps in a[] and b[].  While the matrix
+  // instructions of a step issue, the step before it is asked for again, 4 DB - 1 steps ahead; a block's scales go with its
+  // first step and are taken into registers of their own when the block begins.
+  constexpr int kLoads = NT + MT;     // operands loaded per step: the weights' first
+  uint32_t now_a[NT], now_b[MT];
+  auto block_at = [&](int t) __attribute__((always_inline)) { return min(first + NW * min(t, t_last), nkb - 1); };
+  auto load_operand = [&](auto slot, int u, int l, int kb) __attribute__((always_inline)) {
+    constexpr int s = decltype(slot)::value;
+    const size_t at = (size_t)(kb * 4 + u) * 1024;
+    if (l < NT) a[s][u][l] = load_weights(wcode[l] + at);
+    else b[s][u][l - NT] = *(const uint4*)(xcode[l - NT] + at);
+  };
+  auto load_scale = [&](auto slot, int l, int kb) __attribute__((always_inline)) {
+    constexpr int s = decltype(slot)::value;
+    if (l < NT) sa[s][l].x = *(const uint32_t*)(wscale[l] + (size_t)kb * kSB);
+    else sb[s][l - NT].x = *(const uint32_t*)(xscale[l - NT] + (size_t)kb * kSB);
+  };
+  // Block t of the wave; the first ASK of its steps ask for one further ahead (which has to exist: the last blocks ask for less)
+  auto run_units = [&](auto slot, int t, auto ask) __attribute__((always_inline)) {
+    constexpr int s = decltype(slot)::value, ASK = decltype(ask)::value;
+    // (moves that the compiler may not turn into copies at the end of the loop, where it would wait for every load)
+#pragma unroll
+    for (int l = 0; l < kLoads; ++l) {
+      if (l < NT) asm volatile("v_mov_b32 %0, %1" : "=v"(now_a[l]) : "v"(sa[s][l].x));
+      else asm volatile("v_mov_b32 %0, %1" : "=v"(now_b[l - NT]) : "v"(sb[s][l - NT].x));
+    }
+    const int kb_before = block_at(t - 1 + DB), kb_next = block_at(t + DB);
+    auto step = [&](auto step_u) __attribute__((always_inline)) {   // (which byte of the scales an instruction takes is a constant)
+      constexpr int U = decltype(step_u)::value;
+#pragma unroll
+      for (int p = 0; p < NT * MT; ++p) {
+        const int i = p / MT, j = p % MT;
+        const uint4 aq = a[s][U][i], bq = b[s][U][j];
+        acc[p] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+            v8i{(int)aq.x, (int)aq.y, (int)aq.z, (int)aq.w, 0, 0, 0, 0}, v8i{(int)bq.x, (int)bq.y, (int)bq.z, (int)bq.w, 0, 0, 0, 0},
+            acc[p], 4, 4, U, (int)now_a[i], U, (int)now_b[j]);
+        if constexpr (U < ASK) {
+#pragma unroll
+          for (int l = p * kLoads / (NT * MT); l < (p + 1) * kLoads / (NT * MT); ++l) {
+            if constexpr (U == 0) {
+              load_operand(std::integral_constant<int, (s + DB - 1) % DB>{}, 3, l, kb_before);
+            } else {
+              if constexpr (U == 1) load_scale(slot, l, kb_next);
+              load_operand(slot, U - 1, l, kb_next);
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    step(std::integral_constant<int, 0>{});
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 3>{});
+  };
   FewChunks<NV, XG, XROT, XPRO, NW> few;
   if constexpr (kFew) few.load(in, M, first, nblk, lane);
   for_slots([&](auto slot) {
-    load_block(slot, decltype(slot)::value);
-    if constexpr (kOrdered || kFew) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kUnits) {
+      constexpr int s = decltype(slot)::value;
+      const int kb = block_at(s);
+#pragma unroll
+      for (int l = 0; l < kLoads; ++l) load_scale(slot, l, kb);
+#pragma unroll
+      for (int u = 0; u < (s == DB - 1 ? 3 : 4); ++u) {
+#pragma unroll
+        for (int l = 0; l < kLoads; ++l) load_operand(slot, u, l, kb);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      load_block(slot, decltype(slot)::value);
+      if constexpr (kOrdered || kFew) __builtin_amdgcn_sched_barrier(0);
+    }
   });
   if constexpr (kFew) few.quantize(in, M, few_shared, wave, lane, in.codes && blockIdx.x == 0);
   // Where the epilogue will store, worked out while the first loads are in flight (after the reduction
@@ -419,7 +511,31 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   }
   if constexpr (NT == 1) asm volatile("" : "+s"(res_rows), "+v"(res_src));
   int t0 = 0;
-  for (; t0 + 2 * DB <= nblk; t0 += DB) {   // steady state: the block DB ahead exists
+  if constexpr (kUnits) {
+    static_assert(DB <= 2, "one or two blocks of K steps in flight");
+    typedef std::integral_constant<int, 0> S0;
+    typedef std::integral_constant<int, DB - 1> S1;
+    typedef std::integral_constant<int, 1> Ask1;   // (the step that completes the ring)
+    typedef std::integral_constant<int, 4> Ask4;
+    for (; t0 + 2 * DB <= nblk; t0 += DB)
+      for_slots([&](auto slot) { run_units(slot, t0 + decltype(slot)::value, Ask4{}); });
+    if constexpr (DB == 1) {
+      if (t0 < nblk) run_units(S0{}, t0, Ask1{});
+    } else {
+      if (nblk - t0 == 3) {
+        run_units(S0{}, t0, Ask4{});
+        run_units(S1{}, t0 + 1, Ask1{});
+        run_units(S0{}, t0 + 2, std::integral_constant<int, 0>{});
+      } else if (nblk - t0 == 2) {
+        run_units(S0{}, t0, Ask1{});
+        run_units(S1{}, t0 + 1, std::integral_constant<int, 0>{});
+      } else if (nblk - t0 == 1) {
+        run_units(S0{}, t0, std::integral_constant<int, 0>{});
+      }
+    }
+    t0 = nblk;
+  }
+  for (; !kUnits && t0 + 2 * DB <= nblk; t0 += DB) {   // steady state: the block DB ahead exists
     for_slots([&](auto slot) {
       run_block(slot, t0 + decltype(slot)::value);
       if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
@@ -427,11 +543,11 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
       if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
     });
   }
-  for_slots([&](auto slot) {                // the ring's last full or partial content
+  if constexpr (!kUnits) for_slots([&](auto slot) {   // the ring's last full or partial content
     if (t0 + decltype(slot)::value < nblk) run_block(slot, t0 + decltype(slot)::value);
     if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
   });
-  if (nblk - t0 > DB) {                     // up to DB - 1 blocks more
+  if (!kUnits && nblk - t0 > DB) {          // up to DB - 1 blocks more
     for_slots([&](auto slot) { load_block(slot, t0 + DB + decltype(slot)::value); });
     for_slots([&](auto slot) {
       if (t0 + DB + decltype(slot)::value < nblk) run_block(slot, t0 + DB + decltype(slot)::value);
@@ -442,14 +558,6 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // Whatever follows the last matrix instruction delays the workgroup's end, so all four waves share it:
   // wave g owns quarter g of every tile (registers 4g .. 4g + 3: columns 8g .. 8g + 7), gets that
   // quarter from the three others through LDS and carries it through the rest of the kernel.
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    if (g == wave) continue;
-    const int from = wave < g ? wave : wave - 1;
-#pragma unroll
-    for (int t = 0; t < NT * MT; ++t)
-      part[g][t][from][lane] = v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
-  }
   // The rows of the residual this wave will add are asked for now: they arrive during the reduction.
   // (Store pass 2 t + p -- rows 16 p .. 16 p + 15 of tile t -- belongs to wave (2 t + p) % 4.)
   uint4 rv[(2 * NT * MT + 3) / 4];
@@ -463,20 +571,32 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
                                      : make_uint4(0, 0, 0, 0);
     }
   }
-  __syncthreads();
   v4f sum[NT * MT];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    if (g != wave) continue;
+  for (int c0 = 0; c0 < NT * MT; c0 += kLdsTiles) {
+    if (c0 > 0) __syncthreads();   // (the tiles before have been read)
 #pragma unroll
-    for (int t = 0; t < NT * MT; ++t) {
-      v4f k[4];   // the quarter as each wave computed it
+    for (int g = 0; g < 4; ++g) {
+      if (g == wave) continue;
+      const int from = wave < g ? wave : wave - 1;
 #pragma unroll
-      for (int w = 0; w < 4; ++w)
-        k[w] = w == g ? v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]}
-                      : part[g][t][w < g ? w : w - 1][lane];
+      for (int t = c0; t < NT * MT && t < c0 + kLdsTiles; ++t)
+        part[g][t - c0][from][lane] = v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
+    }
+    __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 4; ++q) sum[t][q] = (k[0][q] + k[2][q]) + (k[1][q] + k[3][q]);
+    for (int g = 0; g < 4; ++g) {
+      if (g != wave) continue;
+#pragma unroll
+      for (int t = c0; t < NT * MT && t < c0 + kLdsTiles; ++t) {
+        v4f k[4];   // the quarter as each wave computed it
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          k[w] = w == g ? v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]}
+                        : part[g][t - c0][w < g ? w : w - 1][lane];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sum[t][q] = (k[0][q] + k[2][q]) + (k[1][q] + k[3][q]);
+      }
     }
   }
 
@@ -614,7 +734,13 @@ static StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int64_t workspace
   if (rt_m == 3 && !nv && tiles > 2 * cus) return plan;
   if (rt_m == 4 && tiles > cus) return plan;
   plan.use = true;
-  if (rt_m == 2 && tiles >= (nv ? 3 * cus / 2 : 3 * cus)) plan.nt = 2;
+  // MXFP4: as many weight tiles per workgroup as bring the workgroups into one round of the CUs, up to four.  A second
+  // round, full or not, costs its start and its end, and all activations once more per weight tile (us, weights from HBM,
+  // K = 4096, one tile per workgroup, from 768 tiles at 33-64 rows two / this: 32 rows: N = 10240 8.5 / 7.6, N = 14336 9.5 /
+  // 8.6, N = 28672 15.2 / 12.9; 64 rows: N = 10240 10.5 / 9.1, N = 16384 12.3 / 10.6, N = 20480 15.0 / 12.0, N = 24576
+  // 15.8 / 13.0, N = 28672 16.7 / 15.3; 96 rows: N = 10240 12.2 / 10.7, N = 16384 13.6 / 12.3).
+  if (!nv && tiles > cus && tiles <= 4 * cus) plan.nt = (int)((tiles + cus - 1) / cus);
+  else if (rt_m == 2 && tiles >= (nv ? 3 * cus / 2 : 3 * cus)) plan.nt = 2;
   // NVFP4, 33-64 rows, between two and three weight tiles per CU: three per workgroup, one workgroup per CU in
   // a single round instead of a round and a half of pairs (N = 24576: K = 4096 22.2 -> 21.2 us, K = 12288 56.0 ->
   // 48.0; N = 20480 21.0 -> 19.7; four tiles per workgroup for the next range measured 4 % slower than pairs).
@@ -646,63 +772,82 @@ int64_t gemm_mxf4_stream_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 
 // Arguments are validated by the caller (gemm_packed); `workspace` is null or 256-byte aligned with
 // its first kStreamCounterBytes zero.  NV: NVFP4 operands.  slab_rows > 0 (a multiple of 32, at most 128):
-// M exceeds what one workgroup takes and is cut into slabs of that many rows, one grid plane each, K whole.
+// M exceeds what one workgroup takes and is cut into slabs of that many rows, slab_nt weight tiles per workgroup, K whole.
 template <bool NV>
 static int launch_stream(const void* xq, const void* xs, const void* wq, const void* ws, const float* alpha,
                          const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K,
                          void* workspace, int64_t workspace_bytes, const OutSegments& seg, hipStream_t stream,
-                         int64_t slab_rows = 0) {
+                         int64_t slab_rows = 0, int slab_nt = 1) {
   if (slab_rows) workspace = nullptr;
   const int64_t rows = slab_rows ? slab_rows : M;   // what one workgroup sees
-  const StreamPlan plan = stream_plan(rows, N, K, workspace ? workspace_bytes : 0, NV);
+  StreamPlan plan = stream_plan(rows, N, K, workspace ? workspace_bytes : 0, NV);
   if (!plan.use) return FPQ_E_UNSUPPORTED;
-  const dim3 grid((unsigned)(((N + 31) / 32 + plan.nt - 1) / plan.nt), (unsigned)plan.ksplit,
-                  (unsigned)(slab_rows ? (M + slab_rows - 1) / slab_rows : 1));
+  if (slab_rows) plan.nt = slab_nt;
+  const unsigned groups = (unsigned)(((N + 31) / 32 + plan.nt - 1) / plan.nt);
+  const unsigned slabs = (unsigned)(slab_rows ? (M + slab_rows - 1) / slab_rows : 1);
+  // (slabs: eights of groups unless that gives an XCD more workgroups than CUs, two on one of them)
+  const bool eights = 8u * ((groups + 7) / 8) * slabs <= (unsigned)device_cus();
+  const dim3 grid = !slab_rows ? dim3(groups, (unsigned)plan.ksplit)
+                    : eights   ? dim3(8, slabs, (groups + 7) / 8) : dim3(groups, slabs);
   unsigned* counters = (unsigned*)workspace;
   float* partial = workspace ? (float*)((uint8_t*)workspace + kStreamCounterBytes) : nullptr;
-#define FPQ_STREAM(NTT, MTT, DBB)                                                                       \
-  hipLaunchKernelGGL((gemm_fp4_stream_kernel<NTT, MTT, DBB, 4, NV>), grid, dim3(256), 0, stream,        \
-                     (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws, alpha, \
-                     (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N,    \
-                     (int)K, plan.bps, plan.ksplit, partial, counters, seg, Packed{})
-  const int mt = (int)((rows + 31) / 32);
-#define FPQ_STREAM_BIG(NTT, MTT, DBB)                                                                   \
-  {                                                                                                     \
-    constexpr int kLds = stream_dynamic_lds(NTT, MTT);                                                  \
-    static LdsLimitOnce lds_limit;                                                                      \
-    if (const int st = lds_limit.ensure((const void*)gemm_fp4_stream_kernel<NTT, MTT, DBB, 4, NV>, kLds)) return st; \
-    hipLaunchKernelGGL((gemm_fp4_stream_kernel<NTT, MTT, DBB, 4, NV>), grid, dim3(256), kLds, stream,   \
-                       (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq, (const uint8_t*)ws, alpha, \
-                       (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N,  \
-                       (int)K, plan.bps, plan.ksplit, partial, counters, seg, Packed{});                          \
-    return (int)hipGetLastError();                                                                      \
-  }
-  if constexpr (NV) {
-    if (plan.nt == 3 && mt == 2) FPQ_STREAM_BIG(3, 2, 2)
-  }
-#undef FPQ_STREAM_BIG
-  if (plan.nt > 2) return FPQ_E_UNSUPPORTED;
-  if (plan.nt == 2) {   // 33-64 rows only
-    if (mt != 2) return FPQ_E_UNSUPPORTED;
-    FPQ_STREAM(2, 2, 1);
+  auto go = [&](auto nt, auto mt, auto db, auto in) {
+    constexpr int NT = decltype(nt)::value, MT = decltype(mt)::value, DB = decltype(db)::value;
+    constexpr int kLds = stream_dynamic_lds(NT, MT);
+    constexpr auto kernel = &gemm_fp4_stream_kernel<NT, MT, DB, 4, NV, decltype(in)>;
+    if constexpr (kLds > 0) {
+      static LdsLimitOnce lds_limit;
+      if (const int st = lds_limit.ensure((const void*)kernel, kLds)) return st;
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(256), kLds, stream, (const uint8_t*)xq, (const uint8_t*)xs, (const uint8_t*)wq,
+                       (const uint8_t*)ws, alpha, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M,
+                       (int)N, (int)K, plan.bps, plan.ksplit, partial, counters, seg, in);
     return (int)hipGetLastError();
+  };
+  typedef std::integral_constant<int, 1> I1;
+  typedef std::integral_constant<int, 2> I2;
+  typedef std::integral_constant<int, 3> I3;
+  typedef std::integral_constant<int, 4> I4;
+  const int mt = (int)((rows + 31) / 32);
+  // enough workgroups for three per CU: two blocks in flight per wave beat four by 3-5 %; with fewer
+  // workgroups the deeper ring of each wave is what keeps the memory system busy
+  const bool many = (int64_t)groups * plan.ksplit * slabs >= 3 * device_cus() / 2;
+  // (65-128 rows: one block in flight per wave, which fits two workgroups into a CU, measured 1-2 %
+  // slower for MXFP4 and 6-12 % slower for NVFP4 than two blocks -- 96 rows of NVFP4, N = 4096:
+  // K = 4096 12.4 against 11.5 us, K = 14336 33.7 against 29.5 us)
+  if (slab_rows) {
+    if (plan.nt == 1) {
+      if (mt == 1) return many ? go(I1{}, I1{}, I2{}, PackedSlabs{}) : go(I1{}, I1{}, I4{}, PackedSlabs{});
+      if (mt == 2) return go(I1{}, I2{}, I2{}, PackedSlabs{});
+      if (mt == 3) return go(I1{}, I3{}, I2{}, PackedSlabs{});
+      if constexpr (NV) return go(I1{}, I4{}, I2{}, PackedSlabs{});
+    }
+    if constexpr (!NV) {
+      if (plan.nt == 2 && mt == 2) return go(I2{}, I2{}, I1{}, PackedSlabs{});
+      if (plan.nt == 2 && mt == 3) return go(I2{}, I3{}, I1{}, PackedSlabs{});
+      if (plan.nt == 2 && mt == 4) return go(I2{}, I4{}, I1{}, PackedSlabs{});
+    }
+    return FPQ_E_UNSUPPORTED;
   }
-  switch (mt) {
-    case 1:
-      // enough workgroups for three per CU: two blocks in flight per wave beat four by 3-5 %; with fewer
-      // workgroups the deeper ring of each wave is what keeps the memory system busy
-      if ((int64_t)grid.x * grid.y * grid.z >= 3 * device_cus() / 2) FPQ_STREAM(1, 1, 2);
-      else FPQ_STREAM(1, 1, 4);
-      break;
-    case 2: FPQ_STREAM(1, 2, 2); break;
-    // (65-128 rows: one block in flight per wave, which fits two workgroups into a CU, measured 1-2 %
-    // slower for MXFP4 and 6-12 % slower for NVFP4 than two blocks -- 96 rows of NVFP4, N = 4096:
-    // K = 4096 12.4 against 11.5 us, K = 14336 33.7 against 29.5 us)
-    case 3: FPQ_STREAM(1, 3, 2); break;
-    default: FPQ_STREAM(1, 4, 2); break;
+  if (plan.nt == 1) {
+    if (mt == 1) return many ? go(I1{}, I1{}, I2{}, Packed{}) : go(I1{}, I1{}, I4{}, Packed{});
+    if (mt == 2) return go(I1{}, I2{}, I2{}, Packed{});
+    if (mt == 3) return go(I1{}, I3{}, I2{}, Packed{});
+    return go(I1{}, I4{}, I2{}, Packed{});
   }
-#undef FPQ_STREAM
-  return (int)hipGetLastError();
+  if constexpr (NV) {   // 33-64 rows
+    if (mt != 2) return FPQ_E_UNSUPPORTED;
+    if (plan.nt == 3) return go(I3{}, I2{}, I2{}, Packed{});
+    return go(I2{}, I2{}, I1{}, Packed{});
+  } else {
+    if (plan.nt == 2) {
+      if (mt == 1) return go(I2{}, I1{}, I2{}, Packed{});
+      return mt == 2 ? go(I2{}, I2{}, I1{}, Packed{}) : mt == 3 ? go(I2{}, I3{}, I1{}, Packed{}) : (int)FPQ_E_UNSUPPORTED;
+    }
+    if (plan.nt == 3)
+      return mt == 1 ? go(I3{}, I1{}, I2{}, Packed{}) : mt == 2 ? go(I3{}, I2{}, I1{}, Packed{}) : (int)FPQ_E_UNSUPPORTED;
+    return mt == 1 ? go(I4{}, I1{}, I1{}, Packed{}) : mt == 2 ? go(I4{}, I2{}, I1{}, Packed{}) : (int)FPQ_E_UNSUPPORTED;
+  }
 }
 
 int gemm_fp4_stream(bool nv, const void* xq, const void* xs, const void* wq, const void* ws, const float* alpha,
@@ -714,13 +859,14 @@ int gemm_fp4_stream(bool nv, const void* xq, const void* xs, const void* wq, con
                                    stream);
 }
 
-// M rows in slabs of slab_rows (a multiple of 32 for which stream_eligible holds), all in one launch.
+// M rows in slabs of slab_rows (a multiple of 32 for which stream_eligible holds), all in one launch; nt weight tiles per
+// workgroup (NVFP4: one).
 int gemm_fp4_stream_slabs(bool nv, const void* xq, const void* xs, const void* wq, const void* ws,
                           const float* alpha, const void* bias, const void* residual, void* y, int64_t M, int64_t N,
-                          int64_t K, int64_t slab_rows, const OutSegments& seg, hipStream_t stream) {
+                          int64_t K, int64_t slab_rows, int nt, const OutSegments& seg, hipStream_t stream) {
   if (slab_rows < 32 || slab_rows > kStreamMaxRows || slab_rows % 32 != 0 || M <= slab_rows) return FPQ_E_UNSUPPORTED;
-  return nv ? launch_stream<true>(xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, nullptr, 0, seg, stream, slab_rows)
-            : launch_stream<false>(xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, nullptr, 0, seg, stream, slab_rows);
+  return nv ? launch_stream<true>(xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, nullptr, 0, seg, stream, slab_rows, nt)
+            : launch_stream<false>(xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, nullptr, 0, seg, stream, slab_rows, nt);
 }
 
 
@@ -784,7 +930,7 @@ int gemm_fp4_rows(bool nv, const void* xq, const void* xs, int64_t xs_stride, co
 // 12.2 / 13.2; 4096 x 4096: 1 row 7.5 / 5.9, 4 rows 7.8 / 9.3.
 static bool few_rows_plan(const StreamPlan& plan, bool nv, int pro, int64_t M, int64_t N, int64_t K, int64_t xk) {
   const int64_t chunks = M * ((plan.bps + 3) / 4) * 8;   // of the wave with the most
-  if (!plan.use || plan.nt != 1 || M > 32 || chunks > few_rows_chunks(pro) || K >= ((int64_t)1 << 22) || xk > K) return false;
+  if (!plan.use || (nv && plan.nt != 1) || M > 32 || chunks > few_rows_chunks(pro) || K >= ((int64_t)1 << 22) || xk > K) return false;
   const int64_t tiles = (N + 31) / 32, cus = device_cus();
   return chunks <= 64 ? !nv || tiles <= 4 * cus : tiles <= (nv ? 2 : 4) * cus;
 }
@@ -798,6 +944,9 @@ static int launch_few_rows(const FewRows& in, const StreamPlan& plan, int rot_ki
                            void* workspace, const OutSegments& seg, hipStream_t stream) {
   if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
   else if (rot_kind != FPQ_ROT_HADAMARD || in.xk % g != 0) return FPQ_E_UNSUPPORTED;
+  // (One weight tile per workgroup whatever plan.nt says, for the same sums: there are no activations to load once more per
+  // workgroup, and a workgroup's quantization hides behind other workgroups' weights: a decoder block's token, whose gate and
+  // up projections have 896 weight tiles, 38.0 us with one, 40.2 with four.)
   const dim3 grid((unsigned)((N + 31) / 32), (unsigned)plan.ksplit);
   const bool many = (int64_t)grid.x * grid.y >= 3 * device_cus() / 2;   // (as launch_stream)
   unsigned* counters = (unsigned*)workspace;

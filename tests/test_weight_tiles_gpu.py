@@ -1,0 +1,44 @@
+"""MXFP4 with several weight tiles per workgroup of the weight-streaming kernel, K step by K step, against the oracle: two,
+three and four weight tiles and up to three activation tiles in one round of the CUs; row slabs of two weight tiles by two,
+three and four; every number of 256-K blocks that a wave's loop takes on a way of its own (none to six); an odd last weight
+tile, groups of weight tiles that are no multiple of eight, a short last slab, N that ends inside a tile."""
+import pytest
+import torch
+
+from oracle import fpq_oracle as O
+from tests import capi
+from tests.conftest import needs_packed
+from tests.test_packed_gpu import pack_by_definition
+
+pytestmark = [pytest.mark.gpu, needs_packed]
+
+# 256 CUs: 257 to 512, 768, 1024 weight tiles of 32 are two, three, four per workgroup
+ROWS = [(m, n, k) for m, n in ((5, 8200), (32, 16384), (33, 8296), (64, 16390), (96, 8264), (80, 16384),
+                               (31, 16448), (64, 24576), (3, 24584), (40, 32768)) for k in (256, 1280, 2304, 3328, 4352, 6144)]
+SLABS = [(129, 4104, 1024), (250, 4096, 1536), (463, 2200, 1280), (333, 4096, 1024), (160, 8192, 2048), (161, 8000, 1024),
+         (700, 2048, 1280), (512, 4096, 8192), (257, 8100, 8448), (400, 4000, 9984)]
+
+
+@pytest.mark.parametrize("m,n,k", ROWS + SLABS)
+def test_against_the_oracle(m, n, k):
+    g = torch.Generator().manual_seed(m + n + k)
+    xq = torch.randint(0, 256, (m, k // 2), dtype=torch.uint8, generator=g)
+    wq = torch.randint(0, 256, (n, k // 2), dtype=torch.uint8, generator=g)
+    xs = torch.randint(118, 134, (m, k // 32), dtype=torch.uint8, generator=g)
+    ws = torch.randint(118, 134, (n, k // 32), dtype=torch.uint8, generator=g)
+    xp, xsp = pack_by_definition(xq, xs, k)
+    wp, wsp = pack_by_definition(wq, ws, k)
+    bias = torch.randn(n, generator=g).to(torch.bfloat16) if k % 512 else None
+    residual = torch.randn(m, n, generator=g).to(torch.bfloat16) if k % 512 and m % 2 else None
+    y = capi.gemm_packed(xp, xsp, wp, wsp, m, n, k, 0.111328125, bias=bias, residual=residual)
+    ref, mag = O.gemm_ref(xq, xs, wq, ws, 0.111328125, "mxfp4")
+    want = ref.to(torch.bfloat16)
+    big = want.double().abs()
+    for add in (bias, residual):
+        if add is not None:
+            want = want + add
+            big = torch.maximum(big, want.double().abs())
+    # 2^-8 for each rounding to bf16 (up to three, of values no larger than `big`), twice that where a sum next to a tie
+    # rounds the other way; 1e-5 of the sum of magnitudes for fp32 sums in another order
+    tol = 2.0 ** -8 * 2 * (1 + (bias is not None) + (residual is not None)) * big + 1e-5 * mag + 1e-6
+    assert ((y.double() - want.double()).abs() <= tol).all()
