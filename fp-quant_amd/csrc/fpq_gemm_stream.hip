@@ -3,7 +3,7 @@
 //
 // With so few rows the time is the one pass over the weights (31 MB for the Llama-3-8B up/gate
 // projection: 3.9 us at 8 TB/s), so the kernel is built around bytes in flight, not around tiles:
-//   * a workgroup owns ONE 32-row weight tile and a range of K; nothing is staged through LDS:
+//   * a workgroup owns one 32-row weight tile (up to four: stream_plan) and a range of K; nothing is staged through LDS:
 //     in the packed layout one operand of one 32x32x64 matrix instruction is one contiguous
 //     kilobyte, lane by lane, so a wave loads it straight into the registers the instruction reads;
 //   * the four waves take the 256-K blocks of the range in turn (wave w: blocks w, w + 4, ...) and
@@ -36,11 +36,9 @@ constexpr int kStreamCounters = 4096;                        // one per weight t
 constexpr int64_t kStreamCounterBytes = kStreamCounters * 4;  // they open the workspace
 constexpr int kStreamMaxRows = 128;
 
-// Output tiles whose parts of K are in LDS at a time: all, or half where all of them would not fit
-constexpr int stream_lds_tiles(int nt, int mt) { return nt * mt <= 8 ? nt * mt : (nt * mt + 1) / 2; }
 // Dynamic LDS of a workgroup with more than four output tiles (0: the kernel's own arrays hold them)
 constexpr int stream_dynamic_lds(int nt, int mt) {
-  return nt * mt > 4 ? 4 * stream_lds_tiles(nt, mt) * 3 * 64 * 16 + nt * mt * 32 * 20 * 4 : 0;
+  return nt * mt > 4 ? 4 * nt * mt * 3 * 64 * 16 + nt * mt * 32 * 20 * 4 : 0;
 }
 
 // NT weight row tiles per workgroup, MT activation row tiles (exactly ceil(M / 32)), DB 256-K blocks
@@ -103,11 +101,10 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // part: [owning wave][tile][the other waves in order][lane]; stage: the rounded tiles on their way out.  More
   // than four tiles per workgroup need more than the 64 KB a kernel may declare: those take them from the
   // launch's dynamic LDS.
-  constexpr int kLdsTiles = stream_lds_tiles(NT, MT);
-  typedef v4f PartOf[kLdsTiles][3][64];
+  typedef v4f PartOf[NT * MT][3][64];
   typedef uint32_t StageOf[kStageTile];
   constexpr bool kDynLds = stream_dynamic_lds(NT, MT) > 0;
-  __shared__ v4f part_fixed[kDynLds ? 1 : 4][kDynLds ? 1 : kLdsTiles][3][64];
+  __shared__ v4f part_fixed[kDynLds ? 1 : 4][kDynLds ? 1 : NT * MT][3][64];
   __shared__ __attribute__((aligned(16))) uint32_t stage_fixed[kDynLds ? 1 : NT * MT][kStageTile];
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dynamic[];
   PartOf* const part = kDynLds ? (PartOf*)lds_dynamic : (PartOf*)part_fixed;
@@ -558,6 +555,14 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // Whatever follows the last matrix instruction delays the workgroup's end, so all four waves share it:
   // wave g owns quarter g of every tile (registers 4g .. 4g + 3: columns 8g .. 8g + 7), gets that
   // quarter from the three others through LDS and carries it through the rest of the kernel.
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    if (g == wave) continue;
+    const int from = wave < g ? wave : wave - 1;
+#pragma unroll
+    for (int t = 0; t < NT * MT; ++t)
+      part[g][t][from][lane] = v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
+  }
   // The rows of the residual this wave will add are asked for now: they arrive during the reduction.
   // (Store pass 2 t + p -- rows 16 p .. 16 p + 15 of tile t -- belongs to wave (2 t + p) % 4.)
   uint4 rv[(2 * NT * MT + 3) / 4];
@@ -571,32 +576,20 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
                                      : make_uint4(0, 0, 0, 0);
     }
   }
+  __syncthreads();
   v4f sum[NT * MT];
 #pragma unroll
-  for (int c0 = 0; c0 < NT * MT; c0 += kLdsTiles) {
-    if (c0 > 0) __syncthreads();   // (the tiles before have been read)
+  for (int g = 0; g < 4; ++g) {
+    if (g != wave) continue;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (g == wave) continue;
-      const int from = wave < g ? wave : wave - 1;
+    for (int t = 0; t < NT * MT; ++t) {
+      v4f k[4];   // the quarter as each wave computed it
 #pragma unroll
-      for (int t = c0; t < NT * MT && t < c0 + kLdsTiles; ++t)
-        part[g][t - c0][from][lane] = v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]};
-    }
-    __syncthreads();
+      for (int w = 0; w < 4; ++w)
+        k[w] = w == g ? v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]}
+                      : part[g][t][w < g ? w : w - 1][lane];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (g != wave) continue;
-#pragma unroll
-      for (int t = c0; t < NT * MT && t < c0 + kLdsTiles; ++t) {
-        v4f k[4];   // the quarter as each wave computed it
-#pragma unroll
-        for (int w = 0; w < 4; ++w)
-          k[w] = w == g ? v4f{acc[t][4 * g], acc[t][4 * g + 1], acc[t][4 * g + 2], acc[t][4 * g + 3]}
-                        : part[g][t - c0][w < g ? w : w - 1][lane];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sum[t][q] = (k[0][q] + k[2][q]) + (k[1][q] + k[3][q]);
-      }
+      for (int q = 0; q < 4; ++q) sum[t][q] = (k[0][q] + k[2][q]) + (k[1][q] + k[3][q]);
     }
   }
 
@@ -707,19 +700,17 @@ struct StreamPlan {
 };
 
 // Which shapes run here and how (all thresholds are measured break-even points on Llama-3-8B and
-// Qwen3-8B layer shapes).  Up to 64 activation rows: always, one weight tile per workgroup.  More
+// Qwen3-8B layer shapes).  Up to 64 activation rows: always.  More
 // rows: up to a number of weight tiles beyond which the 128x128 tile kernel, which shares activations
 // through LDS, is faster -- 65-96 rows: 512 tiles for MXFP4, one round of this kernel's workgroups (with the
 // weights from HBM, this kernel against the tiles: N = 14336 12.0 / 12.3 us, N = 16384 12.5 / 12.5, N = 18432
 // 15.6 / 14.3, N = 24576 17.1 / 15.3, N = 28672 20.7 / 16.5, N = 32768 21.9 / 18.0), any number for NVFP4 (N = 14336: 22.1
 // against 35.9 us, N = 128256: 165 against 215); 97-128 rows (276-346 registers, one workgroup per
 // CU): one round of the 256 CUs for both formats (NVFP4 took two until its tile kernels ran eight waves per
-// workgroup: N = 8192 15.0 against 22.9 us for the tiles, N = 10240 26.7 against 22.7, N = 16384 27.7 against 23.9).  (Two weight tiles per workgroup halve what the L2 has to
-// deliver for 33-64 rows, but need so many registers that one workgroup fills a CU; one tile per
-// workgroup with two blocks in flight, two workgroups per CU, measured 5-13 % faster -- except from
-// 768 weight tiles on, where two tiles per workgroup with ONE block in flight, held to 256 registers,
-// are 12-16 % faster: MXFP4, N = 28672 at 64 rows 20.1 -> 17.0 us, N = 128256 73.5 -> 61.6 us; NVFP4 -- where the
-// two weight tiles also share the activations' conversion to fp16 -- N = 28672 26.2 -> 22.6 us, N = 57344 45.6 -> 40.8, and already from 384 tiles on 1-4 %.)
+// workgroup: N = 8192 15.0 against 22.9 us for the tiles, N = 10240 26.7 against 22.7, N = 16384 27.7 against 23.9).  (One tile per workgroup with two blocks in flight, two workgroups per CU, is the
+// better one for NVFP4 at 33-64 rows -- except from 384 weight tiles on, where two tiles per workgroup with ONE block in
+// flight, held to 256 registers, share the activations' conversion to fp16: N = 28672 26.2 -> 22.6 us, N = 57344 45.6 ->
+// 40.8, 1-4 % up to 767 tiles.  MXFP4: see below.)
 // K is split across workgroups when the weight tiles leave at least half of the CUs idle and every
 // part keeps at least 4096 of K (the exchange of partial tiles through the workspace costs about as
 // much as streaming 16 blocks); fewer parts if the workspace is small.  (While one wave did the
