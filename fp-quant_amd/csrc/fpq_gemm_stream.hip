@@ -85,7 +85,7 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   constexpr bool kFew = std::is_same_v<IN, FewRows>;
   constexpr bool kRagged = std::is_same_v<IN, RowMajor<true>>, kRow = kRagged || std::is_same_v<IN, RowMajor<false>>;
   constexpr bool kSlabs = std::is_same_v<IN, PackedSlabs>;
-  static_assert(!kFew || (NT == 1 && MT == 1), "few rows: one tile");
+  static_assert(!kFew || MT == 1, "few rows: one activation tile");
   constexpr bool kUnits = !NV && NT >= 2;   // K step by K step (see above)
   static_assert(NW == 4, "a wave owns a quarter of every tile");
   // Slabs of 32 MT rows, each a product of its own (the last may have fewer rows, even fewer row tiles).
@@ -412,8 +412,8 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   constexpr bool kOrdered = NT == 1 && DB >= 2 && (MT <= 2 || (NV && MT == 4));
   // K step by K step (kUnits): the steps of the blocks in flight are a ring of 4 DB steps in a[] and b[].  While the matrix
   // instructions of a step issue, the step before it is asked for again, 4 DB - 1 steps ahead; a block's scales go with its
-  // first step and are taken into registers of their own when the block begins.
-  constexpr int kLoads = NT + MT;     // operands loaded per step: the weights' first
+  // first step and are taken into registers of their own when the block begins.  Few rows: theirs come from LDS then.
+  constexpr int kLoads = NT + (kFew ? 0 : MT);     // operands loaded per step: the weights' first
   uint32_t now_a[NT], now_b[MT];
   auto block_at = [&](int t) __attribute__((always_inline)) { return min(first + NW * min(t, t_last), nkb - 1); };
   auto load_operand = [&](auto slot, int u, int l, int kb) __attribute__((always_inline)) {
@@ -430,6 +430,12 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   // Block t of the wave; the first ASK of its steps ask for one further ahead (which has to exist: the last blocks ask for less)
   auto run_units = [&](auto slot, int t, auto ask) __attribute__((always_inline)) {
     constexpr int s = decltype(slot)::value, ASK = decltype(ask)::value;
+    if constexpr (kFew) {
+      const int blk = few_row + t, kh = lane >> 5;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) b[s][u][0] = *(const uint4*)&few_shared.codes[wave][(blk * 8 + 2 * u + kh) * 16];
+      now_b[0] = *(const uint32_t*)&few_shared.scales[wave][blk * 8 + kh * 4];
+    }
     // (moves that the compiler may not turn into copies at the end of the loop, where it would wait for every load)
 #pragma unroll
     for (int l = 0; l < kLoads; ++l) {
@@ -935,10 +941,13 @@ static int launch_few_rows(const FewRows& in, const StreamPlan& plan, int rot_ki
                            void* workspace, const OutSegments& seg, hipStream_t stream) {
   if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
   else if (rot_kind != FPQ_ROT_HADAMARD || in.xk % g != 0) return FPQ_E_UNSUPPORTED;
-  // (One weight tile per workgroup whatever plan.nt says, for the same sums: there are no activations to load once more per
-  // workgroup, and a workgroup's quantization hides behind other workgroups' weights: a decoder block's token, whose gate and
-  // up projections have 896 weight tiles, 38.0 us with one, 40.2 with four.)
-  const dim3 grid((unsigned)((N + 31) / 32), (unsigned)plan.ksplit);
+  // Beyond two weight tiles per CU (up to four) a workgroup takes two of them, and the rows are quantized, and a norm's sums
+  // added up, half as often; the sums are those of any plan.nt.  There are no activations to load, so that fewer workgroups
+  // than that gain nothing (us, one / two / four weight tiles; graph replays, weights from HBM: a token's decoder block with
+  // 896 of them for gate and up 41.5 / 39.0 / 41.8, 1 x 28672 x 4096 14.4 / 13.9 / 14.3; 1 x 14336 x 4096, 448 of them, 8.2 /
+  // 8.7).  SiLU*up's projections have a hidden size of features, too few for it.
+  const int nt = !NV && PRO != kFewSilu && plan.nt >= 3 ? 2 : 1;
+  const dim3 grid((unsigned)(((N + 31) / 32 + nt - 1) / nt), (unsigned)plan.ksplit);
   const bool many = (int64_t)grid.x * grid.y >= 3 * device_cus() / 2;   // (as launch_stream)
   unsigned* counters = (unsigned*)workspace;
   float* partial = workspace ? (float*)((uint8_t*)workspace + kStreamCounterBytes) : nullptr;
@@ -949,6 +958,12 @@ static int launch_few_rows(const FewRows& in, const StreamPlan& plan, int rot_ki
                          (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, plan.bps,
                          plan.ksplit, partial, counters, seg, in);
     };
+    if constexpr (!NV && PRO != kFewSilu) {
+      if (nt == 2) {
+        launch(gemm_fp4_stream_kernel<2, 1, 2, 4, NV, FewRows, G, ROT, PRO>);
+        return (int)hipGetLastError();
+      }
+    }
     if (many) launch(gemm_fp4_stream_kernel<1, 1, 2, 4, NV, FewRows, G, ROT, PRO>);
     else launch(gemm_fp4_stream_kernel<1, 1, 4, 4, NV, FewRows, G, ROT, PRO>);
     return (int)hipGetLastError();

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import fpq_oracle as O
-from tests import capi
+from tests import capi, test_few_rows_gpu, test_norm_rows_gpu
 from tests.conftest import needs_packed
 from tests.test_packed_gpu import pack_by_definition
 
@@ -42,3 +42,15 @@ def test_against_the_oracle(m, n, k):
     # rounds the other way; 1e-5 of the sum of magnitudes for fp32 sums in another order
     tol = 2.0 ** -8 * 2 * (1 + (bias is not None) + (residual is not None)) * big + 1e-5 * mag + 1e-6
     assert ((y.double() - want.double()).abs() <= tol).all()
+
+
+# 513 to 1024 weight tiles: two per workgroup that quantizes its rows itself, the bits of the two kernels
+@pytest.mark.parametrize("init,g", [("hadamard", 32), ("hadamard", 128), ("identity", 64)])
+def test_few_rows(init, g, monkeypatch):
+    monkeypatch.setattr(test_few_rows_gpu, "SHAPES", [(1, 256, 16392), (3, 768, 24584), (2, 2304, 16456), (1, 5120, 32768)])
+    test_few_rows_gpu.test_same_bits_as_two_kernels("mxfp4", init, g, False)
+
+
+@pytest.mark.parametrize("m,k,ns", [(1, 768, (16640,)), (4, 2048, (8448, 8192)), (2, 3328, (24832,)), (1, 4096, (14336, 14336))])
+def test_few_rows_with_a_norm(m, k, ns):
+    test_norm_rows_gpu.test_bits(0, m, k, ns, 0, 128, m % 2)
