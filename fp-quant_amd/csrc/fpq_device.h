@@ -170,6 +170,15 @@ __device__ __forceinline__ void lds_dma4(const uint8_t* gbase, uint32_t voff, ui
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2"
                :: "s"(lds_base), "v"(voff), "s"(gbase) : "memory");
 }
+// A matrix instruction may read a register two wait states after a vector instruction wrote it.  The compiler sees to that for
+// instructions of its own but does not look into assembly: behind assembly that writes matrix operands (or their scales), before
+// the first matrix instruction.  for_each hands every register written to its argument.
+template <class F>
+__device__ __forceinline__ void wait_states_before_mfma(F&& for_each) {
+  asm volatile("s_nop 1");
+  for_each([](uint32_t& r) __attribute__((always_inline)) { asm volatile("" : "+v"(r)); });   // (read no earlier than here)
+}
+
 __device__ __forceinline__ void wait_vmem() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // a / 6 correctly rounded (the reference writes fl(fl(2a)/12), the same number): Markstein's

@@ -693,6 +693,10 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
       asm volatile("v_mov_b32 %0, %1" : "=v"(sa[i].x) : "v"(sa_next[i].x));                         \
     _Pragma("unroll") for (int j = 0; j < TM; ++j)                                                  \
       asm volatile("v_mov_b32 %0, %1" : "=v"(sb[j].x) : "v"(sb_next[j].x));                         \
+    wait_states_before_mfma([&](auto&& pass) __attribute__((always_inline)) {                       \
+      _Pragma("unroll") for (int i = 0; i < TN; ++i) pass(sa[i].x);                                 \
+      _Pragma("unroll") for (int j = 0; j < TM; ++j) pass(sb[j].x);                                 \
+    });                                                                                             \
   }
 
   // steady state: every unit of these blocks still has a unit RING ahead of it to issue

@@ -442,6 +442,10 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
       if (l < NT) asm volatile("v_mov_b32 %0, %1" : "=v"(now_a[l]) : "v"(sa[s][l].x));
       else asm volatile("v_mov_b32 %0, %1" : "=v"(now_b[l - NT]) : "v"(sb[s][l - NT].x));
     }
+    wait_states_before_mfma([&](auto&& pass) __attribute__((always_inline)) {
+#pragma unroll
+      for (int l = 0; l < kLoads; ++l) pass(l < NT ? now_a[l] : now_b[l - NT]);
+    });
     const int kb_before = block_at(t - 1 + DB), kb_next = block_at(t + DB);
     auto step = [&](auto step_u) __attribute__((always_inline)) {   // (which byte of the scales an instruction takes is a constant)
       constexpr int U = decltype(step_u)::value;
