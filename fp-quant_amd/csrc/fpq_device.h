@@ -156,18 +156,19 @@ __device__ __forceinline__ float scale_element(float x, const GroupScale& g) {
 // ---------------------------------------------------------------------------------------------
 // Direct global -> LDS loads: 16 (4) bytes per lane land at lds_base + lane * 16 (4).  Written as
 // inline assembly so that the compiler does not serialise every later LDS read behind them;
-// completion is awaited explicitly with wait_vmem().  Nothing else in these kernels uses M0.
+// completion is awaited explicitly with wait_vmem().  Nothing else in these kernels uses M0; one wait
+// state has to pass between its write and the load that takes its LDS address from it.
 __device__ __forceinline__ void lds_dma16(const uint8_t* gbase, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :: "s"(lds_base), "v"(voff), "s"(gbase) : "memory");
 }
 // Same, marked non-temporal: for data that is read exactly once (streaming kernels).
 __device__ __forceinline__ void lds_dma16_nt(const uint8_t* gbase, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
                :: "s"(lds_base), "v"(voff), "s"(gbase) : "memory");
 }
 __device__ __forceinline__ void lds_dma4(const uint8_t* gbase, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :: "s"(lds_base), "v"(voff), "s"(gbase) : "memory");
 }
 // A matrix instruction may read a register two wait states after a vector instruction wrote it.  The compiler sees to that for

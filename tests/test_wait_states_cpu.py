@@ -63,6 +63,13 @@ def matrix_operands_too_early(code, into):
                                       and bool(registers(args.split(",")[0]) & read))
 
 
+def lds_address_too_early(code, into):
+    """M0, from which a load to LDS takes its address: one wait state."""
+    for i, (opcode, _) in enumerate(code):
+        if opcode.startswith("global_load_lds"):
+            yield from writers_within(code, into, i, 1, lambda op, args: args.split(",")[0].strip() == "m0")
+
+
 @pytest.fixture(scope="module")
 def built(tmp_path_factory):
     if not os.path.exists(LIB) or not os.path.exists(os.path.join(BIN, "llvm-objdump")):
@@ -75,7 +82,8 @@ def built(tmp_path_factory):
                                    capture_output=True, text=True).stdout.split("\n"))]
 
 
-@pytest.mark.parametrize("rule,reads,at_least", [(matrix_operands_too_early, "v_mfma", 10000)])
+@pytest.mark.parametrize("rule,reads,at_least", [(matrix_operands_too_early, "v_mfma", 10000),
+                                                 (lds_address_too_early, "global_load_lds", 1000)])
 def test_wait_states(built, rule, reads, at_least):
     assert sum(op.startswith(reads) for _, code, _ in built for op, _ in code) >= at_least
     early = {name: found for name, code, into in built if (found := list(rule(code, into)))}
