@@ -16,6 +16,7 @@ typedef unsigned v4u_s __attribute__((ext_vector_type(4)));
 
 struct Packed {};
 struct PackedSlabs {};
+struct PackedSlabsInARow {};
 struct FewRows {
   const uint4* x;            // bf16 [M, xk]; SiLU*up: gate
   const uint4* up;           // SiLU*up: the multiplier; RMSNorm: the norm's weight [xk]

@@ -65,6 +65,10 @@ constexpr int stream_dynamic_lds(int nt, int mt) {
 // IN = PackedSlabs: more than 32 MT activation rows in slabs of that many.  Dispatch goes round the XCDs workgroup by
 // workgroup: in a grid of 8 x slabs x eighths of the groups of weight tiles the slabs (blockIdx.y) of a group
 // (8 blockIdx.z + blockIdx.x) run on one XCD at about the same time, and all but one find the weights in its L2.
+// IN = PackedSlabsInARow: where that grid would give an XCD more workgroups than CUs (groups rounded up to eights), every XCD
+// takes a row of the workgroups numbered slab by slab within a group: most groups are still one XCD's.  Slabs by a grid of
+// groups x slabs, on eight XCDs, / this (two weight tiles per workgroup; us, weights from HBM): 400 x 3200 x 4096 11.5 / 9.7,
+// 280 x 5400 x 10240 22.5 / 18.7, 1100 x 700 x 4096 11.2 / 8.9, 500 x 2688 x 14336 28.8 / 23.9.
 // IN = RowMajor: both operands as the quantize operators write them, codes [rows, k / 2] and scales [rows, stride] with the
 // strides multiples of four.  A lane takes the same 16 bytes of codes of a row, and the same scale bytes, as from the
 // packed layout, so the sums are the same bit for bit; only the addresses differ.  See launch_rows.
@@ -84,13 +88,19 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
     float* partial, unsigned* counters, const OutSegments seg, const IN in) {
   constexpr bool kFew = std::is_same_v<IN, FewRows>;
   constexpr bool kRagged = std::is_same_v<IN, RowMajor<true>>, kRow = kRagged || std::is_same_v<IN, RowMajor<false>>;
-  constexpr bool kSlabs = std::is_same_v<IN, PackedSlabs>;
+  constexpr bool kSlabsInARow = std::is_same_v<IN, PackedSlabsInARow>, kSlabs = kSlabsInARow || std::is_same_v<IN, PackedSlabs>;
   static_assert(!kFew || MT == 1, "few rows: one activation tile");
   constexpr bool kUnits = !NV && NT >= 2;   // K step by K step (see above)
   static_assert(NW == 4, "a wave owns a quarter of every tile");
   // Slabs of 32 MT rows, each a product of its own (the last may have fewer rows, even fewer row tiles).
-  const int slab = kSlabs ? blockIdx.y : 0, m0 = slab * (MT * 32);
-  const int rtg = kSlabs ? blockIdx.z * 8 + blockIdx.x : blockIdx.x, split = kSlabs ? 0 : blockIdx.y;
+  int slab = kSlabs ? blockIdx.y : 0, rtg = kSlabs ? blockIdx.z * 8 + blockIdx.x : blockIdx.x;
+  if constexpr (kSlabsInARow) {
+    const unsigned slabs = (unsigned)(M_all + MT * 32 - 1) / (MT * 32), each = gridDim.x >> 3, xcd = blockIdx.x & 7;
+    const unsigned at = xcd * each + min(xcd, gridDim.x & 7) + (blockIdx.x >> 3);   // (the first XCDs have one more)
+    rtg = at / slabs;
+    slab = at - rtg * slabs;
+  }
+  const int m0 = slab * (MT * 32), split = kSlabs ? 0 : blockIdx.y;
   const int M = min(M_all - m0, MT * 32);
   const uint8_t* xq = xq_all + (size_t)slab * MT * (K >> 6) * 1024;
   const uint8_t* xs = xs_all + (size_t)slab * MT * (K >> 8) * (NV ? 512 : 256);
@@ -786,10 +796,11 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
   if (slab_rows) plan.nt = slab_nt;
   const unsigned groups = (unsigned)(((N + 31) / 32 + plan.nt - 1) / plan.nt);
   const unsigned slabs = (unsigned)(slab_rows ? (M + slab_rows - 1) / slab_rows : 1);
-  // (slabs: eights of groups unless that gives an XCD more workgroups than CUs, two on one of them)
+  // (slabs: eights of groups unless that gives an XCD more workgroups than CUs, two on one of them; then in a row)
   const bool eights = 8u * ((groups + 7) / 8) * slabs <= (unsigned)device_cus();
-  const dim3 grid = !slab_rows ? dim3(groups, (unsigned)plan.ksplit)
-                    : eights   ? dim3(8, slabs, (groups + 7) / 8) : dim3(groups, slabs);
+  const dim3 grid = !slab_rows        ? dim3(groups, (unsigned)plan.ksplit)
+                    : eights          ? dim3(8, slabs, (groups + 7) / 8)
+                    : plan.nt == 1    ? dim3(groups, slabs) : dim3(groups * slabs);
   unsigned* counters = (unsigned*)workspace;
   float* partial = workspace ? (float*)((uint8_t*)workspace + kStreamCounterBytes) : nullptr;
   auto go = [&](auto nt, auto mt, auto db, auto in) {
@@ -824,9 +835,10 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
       if constexpr (NV) return go(I1{}, I4{}, I2{}, PackedSlabs{});
     }
     if constexpr (!NV) {
-      if (plan.nt == 2 && mt == 2) return go(I2{}, I2{}, I1{}, PackedSlabs{});
-      if (plan.nt == 2 && mt == 3) return go(I2{}, I3{}, I1{}, PackedSlabs{});
-      if (plan.nt == 2 && mt == 4) return go(I2{}, I4{}, I1{}, PackedSlabs{});
+      auto go_slabs = [&](auto mt_c) { return eights ? go(I2{}, mt_c, I1{}, PackedSlabs{}) : go(I2{}, mt_c, I1{}, PackedSlabsInARow{}); };
+      if (plan.nt == 2 && mt == 2) return go_slabs(I2{});
+      if (plan.nt == 2 && mt == 3) return go_slabs(I3{});
+      if (plan.nt == 2 && mt == 4) return go_slabs(I4{});
     }
     return FPQ_E_UNSUPPORTED;
   }
