@@ -796,11 +796,14 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
   if (slab_rows) plan.nt = slab_nt;
   const unsigned groups = (unsigned)(((N + 31) / 32 + plan.nt - 1) / plan.nt);
   const unsigned slabs = (unsigned)(slab_rows ? (M + slab_rows - 1) / slab_rows : 1);
-  // (slabs: eights of groups unless that gives an XCD more workgroups than CUs, two on one of them; then in a row)
+  // Slabs: eights of groups unless that gives an XCD more workgroups than CUs, two on one of them; then in a row.  A multiple of
+  // four groups has each on two XCDs at most in a grid of groups x slabs, which measured the same or better (us, that / in a row:
+  // 590 x 2304 x 10240 17.8 / 18.4, 1300 x 768 x 10240 14.9 / 15.8), and the weights of few groups are little to share.
   const bool eights = 8u * ((groups + 7) / 8) * slabs <= (unsigned)device_cus();
-  const dim3 grid = !slab_rows        ? dim3(groups, (unsigned)plan.ksplit)
-                    : eights          ? dim3(8, slabs, (groups + 7) / 8)
-                    : plan.nt == 1    ? dim3(groups, slabs) : dim3(groups * slabs);
+  const bool in_a_row = !NV && slab_rows && plan.nt == 2 && !eights && groups > 8 && groups % 4 != 0;
+  const dim3 grid = !slab_rows ? dim3(groups, (unsigned)plan.ksplit)
+                    : eights   ? dim3(8, slabs, (groups + 7) / 8)
+                    : in_a_row ? dim3(groups * slabs) : dim3(groups, slabs);
   unsigned* counters = (unsigned*)workspace;
   float* partial = workspace ? (float*)((uint8_t*)workspace + kStreamCounterBytes) : nullptr;
   auto go = [&](auto nt, auto mt, auto db, auto in) {
@@ -835,7 +838,7 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
       if constexpr (NV) return go(I1{}, I4{}, I2{}, PackedSlabs{});
     }
     if constexpr (!NV) {
-      auto go_slabs = [&](auto mt_c) { return eights ? go(I2{}, mt_c, I1{}, PackedSlabs{}) : go(I2{}, mt_c, I1{}, PackedSlabsInARow{}); };
+      auto go_slabs = [&](auto mt_c) { return in_a_row ? go(I2{}, mt_c, I1{}, PackedSlabsInARow{}) : go(I2{}, mt_c, I1{}, PackedSlabs{}); };
       if (plan.nt == 2 && mt == 2) return go_slabs(I2{});
       if (plan.nt == 2 && mt == 3) return go_slabs(I3{});
       if (plan.nt == 2 && mt == 4) return go_slabs(I4{});
