@@ -334,7 +334,7 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
 // on the other half of K, something does, and each group's loop is half as long.
 // GR = 4 (NVFP4): four groups of two waves, a quarter of K each; see tile_plan.  (Both: 128 x 128 tiles.)
 //
-// WN = WM = 1, GR = 8 (kSolo, NVFP4), 64 x 128 tiles: every wave multiplies the whole tile over an eighth of K, with a ring of its
+// WN = WM = 1, GR = 8 (kSolo), 64 x 128 tiles: every wave multiplies the whole tile over an eighth of K, with a ring of its
 // own, and the eight parts are added through LDS.  What bounded these tiles was the waves' lockstep: at every unit's barrier
 // all of them converted operands or waited at the same time, so the matrix pipes had the other half of the time.  Without a
 // barrier in the loop the two waves of a SIMD drift apart and one's conversions (NVFP4: 0.75 operand tiles per matrix
@@ -342,7 +342,8 @@ __device__ __forceinline__ void gated_tile_store(const v16f (&acc)[TN][TM], uint
 // only.  Eight rings leave room for two units each, so a slot is refilled as soon as its unit has reached the registers.  It
 // pays with a longer tail (256 KB through LDS, 2 us).  us, weights from HBM, groups of two waves / this:
 //   512 x 4096 x 12288 51.6 / 45.0 (1.15 PFLOP/s), 512 x 4096 x 4096 21.0 / 19.2, 300 x 4096 x 3328 21.3 / 16.1
-// (MXFP4 goes a step further there, operands straight to registers: row slabs of the weight-streaming kernel.)
+// (MXFP4 goes a step further in most of that range, operands straight to registers: row slabs of the weight-streaming kernel;
+// these tiles keep a long K in many slabs or with a short last one, see gemm_packed.)
 // OUT = GatedOut: the weight rows are a gate projection's and then an up projection's, and a workgroup's tile is NT / 2 row
 // tiles of each (gated_tile_store).
 template <int NT, int KW, int MT, int WN, int WM, bool NV = false, int RING = kRing, int GR = 1, class OUT = PlainOut>
@@ -670,12 +671,21 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
     FPQ_PREP_B(Q)                                                                                   \
     _Pragma("unroll") for (int i0 = 0; i0 < kHand; ++i0) FPQ_MFMA_ROW(Q, i0)                        \
     wait_vmem_le<(ALLOWED)>();                                                                      \
-    barrier_lds();                                                                                  \
-    if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                                   \
+    if constexpr (!kSolo) {                                                                         \
+      barrier_lds();                                                                                \
+      if (ISSUE) issue_unit((U) + RING, (Q) == 0);                                                 \
+    }                                                                                               \
     if (READ) read_unit((U) + 1, ((Q) + 1) & 1);                                                    \
     if ((Q) == 3 && (NEXT_BLOCK)) read_scales(((U) + 1) >> 2);                                      \
     __builtin_amdgcn_sched_barrier(0);                                                              \
     _Pragma("unroll") for (int i1 = kHand; i1 < TN; ++i1) FPQ_MFMA_ROW(Q, i1)                       \
+    if constexpr (kSolo) {                                                                          \
+      if (ISSUE) {                                                                                  \
+        wait_lds();                                                                                 \
+        issue_unit((U) + 3, (Q) == 1);                                                              \
+        __builtin_amdgcn_sched_barrier(0);                                                          \
+      }                                                                                             \
+    }                                                                                               \
   }
 #define FPQ_TAKE_SCALES_NOW()                                                                       \
   {                                                                                                 \
@@ -1143,6 +1153,23 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
       const int64_t slabs = (M + cap - 1) / cap;
       if (slabs * ((tiles + 1) / 2) > slab_workgroups(cus)) continue;
       const int64_t rows = ((M + slabs - 1) / slabs + 31) / 32 * 32;
+      // From K = 8192 the 64 x 128 tiles of eight waves (kSolo) are ahead of slabs of 128 rows where the last slab is short (up to
+      // 32 rows from K = 10240, 64 from 12288: it runs ahead of the others, which then find fewer weights in the L2), in six
+      // slabs and more from K = 14336, in 14 from 10240, in six that are no eights (fpq_gemm_stream.hip; five from 12288); and in
+      // 24 of 96 or 128 rows, where every group of weight tiles reads more activations than weights.  us, weights from HBM, slabs / tiles:
+      // 416 x 4096 x 10240 19.9 / 19.9, 416 x 4096 x 12288 22.9 / 22.5, x 14336 26.7 / 25.2, 513 x 3072 x 12288 22.5 / 21.9, 900 x 2048
+      // x 14336 27.4 / 25.2, 1200 x 1536 x 14336 27.1 / 25.4, 800 x 2304 x 8192 18.2 / 17.1, 700 x 2688 x 14336 28.2 / 25.8, 1700 x
+      // 1024 x 10240 20.3 / 18.9, 3000 x 512 x 8192 19.4 / 15.9, 3700 x 512 x 8192 23.2 / 17.2; on this side of the line 448 x 4096 x
+      // 10240 19.4 / 20.4, 640 x 3072 x 14336 25.8 / 26.8, 1024 x 2048 x 10240 20.1 / 21.1, 1700 x 1024 x 8192 16.2 / 16.0.
+      if constexpr (!NV) {
+        const int64_t last = M - (slabs - 1) * rows;
+        const bool eights = 8 * (((tiles + 1) / 2 + 7) / 8) * slabs <= cus;
+        const bool long_k = (last <= 64 && K >= 8192 + 64 * last) || (slabs >= 6 && (K >= 14336 || !eights)) ||
+                            (slabs >= 5 && K >= 12288 && !eights) || (slabs >= 14 && K >= 10240);
+        if (K >= 8192 && rows >= 96 && slabs > 1 && (slabs >= 24 || (rows == 128 && long_k)))
+          return launch_packed<2, 4, 4, 1, 1, false, 2, 8>(xq, xs, wq, ws, alpha, bias, y, M, N, K, (hipStream_t)stream,
+                                                           residual, seg);
+      }
       if (slabs > 1 && rows > 32 && rows < M && stream_eligible(false, rows, N, K))
         return gemm_fp4_stream_slabs(false, xq, xs, wq, ws, alpha, bias, residual, y, M, N, K, rows, 2, seg,
                                      (hipStream_t)stream);

@@ -1,6 +1,7 @@
 """64 x 128 workgroup tiles of eight waves that multiply an eighth of K each: the oracle's values, bias and residual
 included, and the same bits on every repetition.  NVFP4 from eight 256-K blocks on (one per wave; two for some and one for
-the others; an odd number), MXFP4 from 32 blocks and 129 rows on; rows and columns cut off inside the last tile."""
+the others; an odd number), MXFP4 where row slabs of the weight-streaming kernel fall behind (a long K with a short last slab or
+with many slabs; the other MXFP4 shapes here are such slabs); rows and columns cut off inside the last tile."""
 import pytest
 import torch
 
@@ -20,7 +21,11 @@ def test_nvfp4_matches_the_oracle(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(129, 8190, 8192), (300, 4100, 8448), (512, 4096, 14336), (511, 2500, 10240), (1025, 1025, 8192),
-                                   (257, 4000, 9984)])
+                                   (257, 4000, 9984),
+                                   # eight waves: 1 to 64 rows in the last slab, numbers of blocks that eight do and do not
+                                   # divide; five slabs; six and seven that are no eights of groups of weight tiles; 14; 27 of 96 rows
+                                   (385, 4090, 8448), (416, 4096, 10496), (448, 4000, 12544), (320, 5110, 12288), (600, 3190, 14592),
+                                   (760, 2680, 8192), (833, 2300, 9984), (1700, 1020, 10240), (2500, 500, 8448)])
 def test_mxfp4_matches_the_oracle(m, n, k):
     xq, _, wq, _, bias, res, g = _operands(m, n, k, m + n + k)
     xs = torch.randint(120, 131, (m, k // 32), dtype=torch.uint8, generator=g)
