@@ -1149,7 +1149,12 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
     // 160 rows, N = 8192 12.2 / 10.2, 200 rows, N = 4096 / 6144 8.4 / 7.8, 12.1 / 11.1, 333 rows, N = 4096 11.7 / 9.6; K = 8192,
     // N = 8192: 128 / 160 / 256 rows 15.3 / 14.0, 19.2 / 15.5, 20.9 / 18.9; K = 14336, N = 4096: 200 / 384 / 512 rows 21.0 / 18.1,
     // 28.5 / 22.8, 31.2 / 27.6.
-    for (int64_t cap = 64; cap <= (K >= 8192 ? 128 : 96) && !NV && !splits && !one_slab && K >= 1024; cap += 32) {
+    // Below K = 1024 where slabs of 128 rows by one weight tile would fit a round of the CUs, of more than two weight tiles (us,
+    // weights from HBM, tiles / those / this: 256 x 2790 x 768 10.0 / 7.3 / 6.1, 512 x 2048 x 512 4.7 / 5.7 / 4.5, 1000 x 1000 x 768
+    // 6.1 / 6.2 / 4.8, 128 x 8192 x 768 6.0 / 6.0 / 4.8; two: 16000 x 64 x 256 4.4 / 5.9 / 5.4).  Any other short K keeps the tile
+    // kernels and with them the bits of the row-major operator, which slabs do not give.
+    const bool short_k_slabs = tiles > 2 && (M + 127) / 128 * tiles <= slab_workgroups(cus);
+    for (int64_t cap = 64; cap <= (K >= 8192 ? 128 : 96) && !NV && !splits && !one_slab && (K >= 1024 || short_k_slabs); cap += 32) {
       const int64_t slabs = (M + cap - 1) / cap;
       if (slabs * ((tiles + 1) / 2) > slab_workgroups(cus)) continue;
       const int64_t rows = ((M + slabs - 1) / slabs + 31) / 32 * 32;
