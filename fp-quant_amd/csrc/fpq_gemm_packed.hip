@@ -1133,7 +1133,8 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
     bool one_slab = false;
     const bool splits = tile_splits || (workspace && workspace_bytes > 16384 && M <= 96 &&
                                         gemm_mxf4_stream_workspace_bytes(M, N, K) > 0);
-    for (int64_t cap = 32; cap <= (NV ? 128 : 96) && !splits; cap += 32) {
+    // (128 rows by one weight tile: MXFP4 for a single one only, two being better below)
+    for (int64_t cap = 32; cap <= (NV || (tiles == 1 && K >= 1024) ? 128 : 96) && !splits; cap += 32) {
       const int64_t slabs = (M + cap - 1) / cap;
       if (slabs * tiles > slab_workgroups(cus)) continue;
       const int64_t rows = ((M + slabs - 1) / slabs + 31) / 32 * 32;   // rows of a slab, whole 32-row tiles

@@ -835,7 +835,7 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
       if (mt == 1) return many ? go(I1{}, I1{}, I2{}, PackedSlabs{}) : go(I1{}, I1{}, I4{}, PackedSlabs{});
       if (mt == 2) return go(I1{}, I2{}, I2{}, PackedSlabs{});
       if (mt == 3) return go(I1{}, I3{}, I2{}, PackedSlabs{});
-      if constexpr (NV) return go(I1{}, I4{}, I2{}, PackedSlabs{});
+      if (mt == 4) return go(I1{}, I4{}, I2{}, PackedSlabs{});
     }
     if constexpr (!NV) {
       auto go_slabs = [&](auto mt_c) { return in_a_row ? go(I2{}, mt_c, I1{}, PackedSlabsInARow{}) : go(I2{}, mt_c, I1{}, PackedSlabs{}); };

@@ -46,14 +46,15 @@ def test_against_the_oracle(m, n, k):
 
 
 # A row's sums are those of a few rows by themselves wherever both are slabs (K in four parts, in one order)
-@pytest.mark.parametrize("m,n,k", [(512, 2048, 768), (1000, 1000, 768), (256, 2790, 512), (256, 4090, 768)])
+@pytest.mark.parametrize("m,n,k", [(512, 2048, 768), (1000, 1000, 768), (256, 2790, 512), (256, 4090, 768),
+                                   (24577, 32, 1024), (32740, 24, 1280)])
 def test_bits_of_fewer_rows(m, n, k):
     g = torch.Generator().manual_seed(m + n + k)
     xq, wq = (torch.randint(0, 256, (r, k // 2), dtype=torch.uint8, generator=g) for r in (m, n))
     xs, ws = (torch.randint(118, 134, (r, k // 32), dtype=torch.uint8, generator=g) for r in (m, n))
     w = pack_by_definition(wq, ws, k)
-    few = capi.gemm_packed(*pack_by_definition(xq[:50], xs[:50], k), *w, 50, n, k, 0.111328125)
-    assert torch.equal(capi.gemm_packed(*pack_by_definition(xq, xs, k), *w, m, n, k, 0.111328125)[:50], few)
+    few = capi.gemm_packed(*pack_by_definition(xq[:m // 4], xs[:m // 4], k), *w, m // 4, n, k, 0.111328125)
+    assert torch.equal(capi.gemm_packed(*pack_by_definition(xq, xs, k), *w, m, n, k, 0.111328125)[:m // 4], few)
 
 
 # 513 to 1024 weight tiles: two per workgroup that quantizes its rows itself, the bits of the two kernels
