@@ -90,6 +90,11 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   constexpr bool kRagged = std::is_same_v<IN, RowMajor<true>>, kRow = kRagged || std::is_same_v<IN, RowMajor<false>>;
   constexpr bool kSlabsInARow = std::is_same_v<IN, PackedSlabsInARow>, kSlabs = kSlabsInARow || std::is_same_v<IN, PackedSlabs>;
   static_assert(!kFew || MT == 1, "few rows: one activation tile");
+  // The arguments lie in four cache lines, and none of them is near when a kernel starts: what the rows and the weights are asked
+  // for with comes from all four at once.  Left alone, the compiler asks for the weights' addresses behind the rows (us, a
+  // line later / at once, weights from HBM: 1 x 4096 x 4096 5.7 / 5.5, 1 x 6144 x 4096 6.1 / 5.9, 1 x 14336 x 4096 8.0 / 7.7).
+  if constexpr (kFew)
+    asm volatile("" :: "s"(wq), "s"(ws), "s"(M_all), "s"(N), "s"(K), "s"(bps), "s"(in.x), "s"(in.up), "s"(in.xk));
   constexpr bool kUnits = !NV && NT >= 2;   // K step by K step (see above)
   static_assert(NW == 4, "a wave owns a quarter of every tile");
   // Slabs of 32 MT rows, each a product of its own (the last may have fewer rows, even fewer row tiles).
