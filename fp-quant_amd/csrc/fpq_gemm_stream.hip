@@ -965,12 +965,22 @@ static int launch_few_rows(const FewRows& in, const StreamPlan& plan, int rot_ki
                            void* workspace, const OutSegments& seg, hipStream_t stream) {
   if (rot_kind == FPQ_ROT_IDENTITY) g = 32;
   else if (rot_kind != FPQ_ROT_HADAMARD || in.xk % g != 0) return FPQ_E_UNSUPPORTED;
-  // Beyond two weight tiles per CU (up to four) a workgroup takes two of them, and the rows are quantized, and a norm's sums
-  // added up, half as often; the sums are those of any plan.nt.  There are no activations to load, so that fewer workgroups
-  // than that gain nothing (us, one / two / four weight tiles; graph replays, weights from HBM: a token's decoder block with
-  // 896 of them for gate and up 41.5 / 39.0 / 41.8, 1 x 28672 x 4096 14.4 / 13.9 / 14.3; 1 x 14336 x 4096, 448 of them, 8.2 /
-  // 8.7).  SiLU*up's projections have a hidden size of features, too few for it.
-  const int nt = !NV && PRO != kFewSilu && plan.nt >= 3 ? 2 : 1;
+  // Two weight tiles per workgroup: the rows are quantized, and a norm's sums added up, half as often; the sums of the products
+  // are those of any plan.nt.  There are no activations to load, so that it pays for the vector work alone: with three to four
+  // weight tiles per CU, of which a CU holds three at a time; with two to three where a wave has two passes, of two rows
+  // over up to five blocks or of three and more, or, in one pass for three to five blocks, a norm in front or blocks that the
+  // waves do not share evenly.  us, one
+  // / two tiles, weights from HBM: 1 row, K = 4096: N = 24832 12.2 / 12.1, N = 32768 14.5 / 13.7, N = 20480 10.5 / 11.5; N = 20480: 1 row,
+  // K = 8192 16.8 / 18.8, K = 2560 9.2 / 8.7, 2 rows, K = 8192 17.5 / 18.4, 4 rows, K = 4096 11.4 / 10.9; with a norm, 1 row: N = 28672, K =
+  // 4096 14.8 / 12.5, N = 24576, K = 4096 12.0 / 11.4, N = 20480: K = 2048 9.2 / 9.6, K = 3072 11.3 / 10.1, K = 6144 13.8 / 14.9.  Four tiles
+  // measured as one does, and 448 tiles lose (1 x 14336 x 4096 8.2 / 8.7).  SiLU*up's projections have a hidden size of features,
+  // too few for it.
+  const int64_t nkb = K / 256, blocks = (nkb + 3) / 4;
+  const bool three_to_five = blocks >= 3 && blocks <= 5;
+  const bool pays = plan.nt >= 4 || (plan.nt == 3 && (PRO == kFewNorm ? three_to_five
+                                                      : (M * blocks > 8 && (M >= 3 || three_to_five)) ||
+                                                        (three_to_five && nkb % 4 != 0)));
+  const int nt = !NV && PRO != kFewSilu && pays ? 2 : 1;
   const dim3 grid((unsigned)(((N + 31) / 32 + nt - 1) / nt), (unsigned)plan.ksplit);
   const bool many = (int64_t)grid.x * grid.y >= 3 * device_cus() / 2;   // (as launch_stream)
   unsigned* counters = (unsigned*)workspace;

@@ -57,13 +57,16 @@ def test_bits_of_fewer_rows(m, n, k):
     assert torch.equal(capi.gemm_packed(*pack_by_definition(xq, xs, k), *w, m, n, k, 0.111328125)[:m // 4], few)
 
 
-# 513 to 1024 weight tiles: two per workgroup that quantizes its rows itself, the bits of the two kernels
+# 513 to 1024 weight tiles: two per workgroup that quantizes its rows itself or, where that does not pay, one: the bits of the
+# two kernels.  One block per wave and up, in one pass and in two (4 x 4096)
 @pytest.mark.parametrize("init,g", [("hadamard", 32), ("hadamard", 128), ("identity", 64)])
 def test_few_rows(init, g, monkeypatch):
-    monkeypatch.setattr(test_few_rows_gpu, "SHAPES", [(1, 256, 16392), (3, 768, 24584), (2, 2304, 16456), (1, 5120, 32768)])
+    monkeypatch.setattr(test_few_rows_gpu, "SHAPES", [(1, 256, 16392), (3, 768, 24584), (2, 2304, 16456), (1, 5120, 32768),
+                                                     (1, 256, 24680), (4, 4096, 16456), (1, 4096, 20488), (2, 5120, 16456)])
     test_few_rows_gpu.test_same_bits_as_two_kernels("mxfp4", init, g, False)
 
 
-@pytest.mark.parametrize("m,k,ns", [(1, 768, (16640,)), (4, 2048, (8448, 8192)), (2, 3328, (24832,)), (1, 4096, (14336, 14336))])
+@pytest.mark.parametrize("m,k,ns", [(1, 768, (16640,)), (4, 2048, (8448, 8192)), (2, 3328, (24832,)), (1, 4096, (14336, 14336)),
+                                    (1, 768, (24832,)), (4, 2048, (16640, 8448)), (2, 4096, (16640,)), (1, 6144, (20480,))])
 def test_few_rows_with_a_norm(m, k, ns):
     test_norm_rows_gpu.test_bits(0, m, k, ns, 0, 128, m % 2)
