@@ -755,8 +755,18 @@ static StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int64_t workspace
   // K = 4096, one tile per workgroup, from 768 tiles at 33-64 rows two / this: 32 rows: N = 10240 8.5 / 7.6, N = 14336 9.5 /
   // 8.6, N = 28672 15.2 / 12.9; 64 rows: N = 10240 10.5 / 9.1, N = 16384 12.3 / 10.6, N = 20480 15.0 / 12.0, N = 24576
   // 15.8 / 13.0, N = 28672 16.7 / 15.3; 96 rows: N = 10240 12.2 / 10.7, N = 16384 13.6 / 12.3).
-  if (!nv && tiles > cus && tiles <= 4 * cus) plan.nt = (int)((tiles + cus - 1) / cus);
-  else if (rt_m == 2 && tiles >= (nv ? 3 * cus / 2 : 3 * cus)) plan.nt = 2;
+  // Not where one tile per workgroup fills its rounds to the last sixteenth, its waves have whole pairs of blocks, as many as
+  // they keep in flight, and up to 16 rows (24 in place of four tiles) leave few activations to load again (one tile / this: 16 x
+  // 24576 x 8192 18.0 / 19.1, 5 x 32768 x 4096 13.3 / 14.4; 24 x 24576 x 8192 18.9 / 19.2; 5 x 15360 x 5120 9.7 / 8.8); nor four in place
+  // of a single pair (8 x 28672 x 2048 8.2 / 8.7), nor three for a single block (5 x 16640 x 256 4.8 / 5.1).  33-64 rows: two instead of four for a short K, with two workgroups to a CU (four / two: 64 x
+  // 24832 x 1024 7.7 / 6.7, 33 x 32768 x 2048 11.1 / 10.1, 64 x 30720 x 3072 12.9 / 12.6).
+  if (!nv && tiles > cus && tiles <= 4 * cus) {
+    plan.nt = (int)((tiles + cus - 1) / cus);
+    if (rt_m == 2 && plan.nt == 4 && K <= 3072) plan.nt = 2;
+    if (M <= (plan.nt == 4 ? 24 : 16) && nkb % 8 == 0 && (16 * tiles >= 15 * plan.nt * cus || (plan.nt == 4 && nkb == 8)))
+      plan.nt = 1;
+    if (rt_m == 1 && plan.nt == 3 && nkb == 1) plan.nt = 1;
+  } else if (rt_m == 2 && tiles >= (nv ? 3 * cus / 2 : 3 * cus)) plan.nt = 2;
   // NVFP4, 33-64 rows, between two and three weight tiles per CU: three per workgroup, one workgroup per CU in
   // a single round instead of a round and a half of pairs (N = 24576: K = 4096 22.2 -> 21.2 us, K = 12288 56.0 ->
   // 48.0; N = 20480 21.0 -> 19.7; four tiles per workgroup for the next range measured 4 % slower than pairs).
@@ -975,11 +985,12 @@ static int launch_few_rows(const FewRows& in, const StreamPlan& plan, int rot_ki
   // 4096 14.8 / 12.5, N = 24576, K = 4096 12.0 / 11.4, N = 20480: K = 2048 9.2 / 9.6, K = 3072 11.3 / 10.1, K = 6144 13.8 / 14.9.  Four tiles
   // measured as one does, and 448 tiles lose (1 x 14336 x 4096 8.2 / 8.7).  SiLU*up's projections have a hidden size of features,
   // too few for it.
-  const int64_t nkb = K / 256, blocks = (nkb + 3) / 4;
+  const int64_t nkb = K / 256, blocks = (nkb + 3) / 4, tiles = (N + 31) / 32, cus = device_cus();
   const bool three_to_five = blocks >= 3 && blocks <= 5;
-  const bool pays = plan.nt >= 4 || (plan.nt == 3 && (PRO == kFewNorm ? three_to_five
-                                                      : (M * blocks > 8 && (M >= 3 || three_to_five)) ||
-                                                        (three_to_five && nkb % 4 != 0)));
+  const bool pays = tiles > 3 * cus ? tiles <= 4 * cus
+                                    : tiles > 2 * cus && (PRO == kFewNorm ? three_to_five
+                                                          : (M * blocks > 8 && (M >= 3 || three_to_five)) ||
+                                                            (three_to_five && nkb % 4 != 0));
   const int nt = !NV && PRO != kFewSilu && pays ? 2 : 1;
   const dim3 grid((unsigned)(((N + 31) / 32 + nt - 1) / nt), (unsigned)plan.ksplit);
   const bool many = (int64_t)grid.x * grid.y >= 3 * device_cus() / 2;   // (as launch_stream)

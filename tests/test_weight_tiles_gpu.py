@@ -15,6 +15,7 @@ pytestmark = [pytest.mark.gpu, needs_packed]
 # 256 CUs: 257 to 512, 768, 1024 weight tiles of 32 are two, three, four per workgroup
 ROWS = [(m, n, k) for m, n in ((5, 8200), (32, 16384), (33, 8296), (64, 16390), (96, 8264), (80, 16384),
                                (31, 16448), (64, 24576), (3, 24584), (40, 32768)) for k in (256, 1280, 2304, 3328, 4352, 6144)]
+ROWS += [(16, 15360, 2048), (24, 32760, 4096), (24, 26000, 2048), (7, 24570, 4096)]   # one again, where that fills its rounds
 SLABS = [(129, 4104, 1024), (250, 4096, 1536), (463, 2200, 1280), (333, 4096, 1024), (160, 8192, 2048), (161, 8000, 1024),
          (700, 2048, 1280), (512, 4096, 8192), (257, 8100, 8448), (400, 4000, 9984),
          (1100, 690, 1024), (200, 5390, 1024), (500, 2680, 1280), (600, 3190, 8192)]   # (the XCDs' rows of workgroups)
