@@ -11,15 +11,7 @@ from tests.conftest import SINGLE_WEIGHT_COPY, needs_packed
 pytestmark = pytest.mark.gpu
 
 
-# (256, 512, 768: waves without a block; 4 x 2048 and 1 x 8192: as many chunks as a wave holds; 5120: blocks that the waves
-# do not share evenly; 14336 columns: the GEMM's variant for many workgroups; 3 x 5120, 1 x 16384: refused)
-@pytest.mark.parametrize("nv", [0, 1])
-@pytest.mark.parametrize("m,k,ns,kind,g,bias", [
-    (1, 256, (256,), 0, 128, 0), (4, 512, (256, 512), 0, 64, 1), (3, 768, (256, 256, 256), 0, 32, 0),
-    (4, 2048, (512, 256), 1, 32, 1), (1, 4096, (4096, 1024, 1024), 0, 128, 0), (2, 4096, (14336,), 0, 16, 0),
-    (2, 4096, (4096, 256), 0, 128, 1), (1, 8192, (512,), 0, 64, 0), (1, 5120, (1024, 256), 0, 128, 0), (3, 5120, (256,), 0, 64, 0), (1, 16384, (256,), 0, 128, 0),
-])
-def test_bits(nv, m, k, ns, kind, g, bias):
+def check_bits(nv, m, k, ns, kind, g, bias):
     from fp_quant import _engine
     lib = _engine.lib()
     if not nv and g == 16:
@@ -68,6 +60,18 @@ def test_bits(nv, m, k, ns, kind, g, bias):
         _engine.check(st, "norm_rows_multi")
         for a, c in zip(got, want):
             assert torch.equal(a.view(torch.int16), c.view(torch.int16)), special
+
+
+# (256, 512, 768: waves without a block; 4 x 2048 and 1 x 8192: as many chunks as a wave holds; 5120: blocks that the waves
+# do not share evenly; 14336 columns: the GEMM's variant for many workgroups; 3 x 5120, 1 x 16384: refused)
+@pytest.mark.parametrize("nv", [0, 1])
+@pytest.mark.parametrize("m,k,ns,kind,g,bias", [
+    (1, 256, (256,), 0, 128, 0), (4, 512, (256, 512), 0, 64, 1), (3, 768, (256, 256, 256), 0, 32, 0),
+    (4, 2048, (512, 256), 1, 32, 1), (1, 4096, (4096, 1024, 1024), 0, 128, 0), (2, 4096, (14336,), 0, 16, 0),
+    (2, 4096, (4096, 256), 0, 128, 1), (1, 8192, (512,), 0, 64, 0), (1, 5120, (1024, 256), 0, 128, 0), (3, 5120, (256,), 0, 64, 0), (1, 16384, (256,), 0, 128, 0),
+])
+def test_bits(nv, m, k, ns, kind, g, bias):
+    check_bits(nv, m, k, ns, kind, g, bias)
 
 
 def test_refusals():

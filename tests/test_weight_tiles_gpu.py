@@ -6,9 +6,11 @@ import pytest
 import torch
 
 from oracle import fpq_oracle as O
-from tests import capi, test_few_rows_gpu, test_norm_rows_gpu
-from tests.conftest import needs_packed
-from tests.test_packed_gpu import pack_by_definition
+import capi
+from conftest import needs_packed
+from test_few_rows_gpu import check_same_bits_as_two_kernels
+from test_norm_rows_gpu import check_bits
+from test_packed_gpu import pack_by_definition
 
 pytestmark = [pytest.mark.gpu, needs_packed]
 
@@ -16,8 +18,10 @@ pytestmark = [pytest.mark.gpu, needs_packed]
 ROWS = [(m, n, k) for m, n in ((5, 8200), (32, 16384), (33, 8296), (64, 16390), (96, 8264), (80, 16384),
                                (31, 16448), (64, 24576), (3, 24584), (40, 32768)) for k in (256, 1280, 2304, 3328, 4352, 6144)]
 ROWS += [(16, 15360, 2048), (24, 32760, 4096), (24, 26000, 2048), (7, 24570, 4096)]   # one again, where that fills its rounds
+FEW_ROWS = [(1, 256, 16392), (3, 768, 24584), (2, 2304, 16456), (1, 5120, 32768), (1, 256, 24680), (4, 4096, 16456),
+            (1, 4096, 20488), (2, 5120, 16456)]
 SLABS = [(129, 4104, 1024), (250, 4096, 1536), (463, 2200, 1280), (333, 4096, 1024), (160, 8192, 2048), (161, 8000, 1024),
-         (700, 2048, 1280), (512, 4096, 8192), (257, 8100, 8448), (400, 4000, 9984),
+         (700, 2048, 1280), (512, 4096, 8192), (257, 8100, 8448), (250, 8100, 8448), (400, 4000, 9984),
          (1100, 690, 1024), (200, 5390, 1024), (500, 2680, 1280), (600, 3190, 8192)]   # (the XCDs' rows of workgroups)
 
 
@@ -61,13 +65,11 @@ def test_bits_of_fewer_rows(m, n, k):
 # 513 to 1024 weight tiles: two per workgroup that quantizes its rows itself or, where that does not pay, one: the bits of the
 # two kernels.  One block per wave and up, in one pass and in two (4 x 4096)
 @pytest.mark.parametrize("init,g", [("hadamard", 32), ("hadamard", 128), ("identity", 64)])
-def test_few_rows(init, g, monkeypatch):
-    monkeypatch.setattr(test_few_rows_gpu, "SHAPES", [(1, 256, 16392), (3, 768, 24584), (2, 2304, 16456), (1, 5120, 32768),
-                                                     (1, 256, 24680), (4, 4096, 16456), (1, 4096, 20488), (2, 5120, 16456)])
-    test_few_rows_gpu.test_same_bits_as_two_kernels("mxfp4", init, g, False)
+def test_few_rows(init, g):
+    check_same_bits_as_two_kernels("mxfp4", init, g, False, FEW_ROWS)
 
 
 @pytest.mark.parametrize("m,k,ns", [(1, 768, (16640,)), (4, 2048, (8448, 8192)), (2, 3328, (24832,)), (1, 4096, (14336, 14336)),
                                     (1, 768, (24832,)), (4, 2048, (16640, 8448)), (2, 4096, (16640,)), (1, 6144, (20480,))])
 def test_few_rows_with_a_norm(m, k, ns):
-    test_norm_rows_gpu.test_bits(0, m, k, ns, 0, 128, m % 2)
+    check_bits(0, m, k, ns, 0, 128, m % 2)
