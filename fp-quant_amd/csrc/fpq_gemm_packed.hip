@@ -454,9 +454,10 @@ __global__ __launch_bounds__(64 * WN * WM * GR, (NT * MT <= 32 && GR == 1 ? 2 : 
                   smem_base + kScaleBase + (blk % kSlots) * kSlotBytes + (wave * kScLoads + j) * 1024);
     }
     const uint32_t dst = smem_base + (u % RING) * kUnitBytes + wave * kPer * 1024;
+    // (the unit's place in the lane's offset, one addition for all loads, and not in the bases, two for each)
+    const uint32_t at = lane16 + (uint32_t)u * 1024u;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j)
-      lds_dma16(op_base[j] + (size_t)u * 1024, lane16, dst + (kSolo && j >= NT ? KW + j - NT : j) * 1024);
+    for (int j = 0; j < kPer; ++j) lds_dma16(op_base[j], at, dst + (kSolo && j >= NT ? KW + j - NT : j) * 1024);
   };
 
   v16f acc[TN][TM];
