@@ -92,8 +92,10 @@ __global__ __launch_bounds__(64 * NW, NT == 2 && NT * MT <= 4 ? 2 : 1) void gemm
   static_assert(!kFew || MT == 1, "few rows: one activation tile");
   // The arguments lie in four cache lines, and none of them is near when a kernel starts: what the rows and the weights are asked
   // for with comes from all four at once.  Left alone, the compiler asks for the weights' addresses behind the rows (us, a
-  // line later / at once, weights from HBM: 1 x 4096 x 4096 5.7 / 5.5, 1 x 6144 x 4096 6.1 / 5.9, 1 x 14336 x 4096 8.0 / 7.7).
-  if constexpr (kFew)
+  // line later / at once, weights from HBM, rows not handed on: 1 x 4096 x 4096 5.7 / 5.5, 1 x 6144 x 4096 6.1 / 5.9, 1 x 14336 x
+  // 4096 8.0 / 7.7; handed on 5.6 / 5.6, 6.0 / 6.0, 8.0 / 7.9).  With a norm or SiLU*up, whose rows take longer than the line,
+  // and with two weight tiles a token's block measured 0.2 slower that way.
+  if constexpr (kFew && XPRO == kFewPlain && NT == 1)
     asm volatile("" :: "s"(wq), "s"(ws), "s"(M_all), "s"(N), "s"(K), "s"(bps), "s"(in.x), "s"(in.up), "s"(in.xk));
   constexpr bool kUnits = !NV && NT >= 2;   // K step by K step (see above)
   static_assert(NW == 4, "a wave owns a quarter of every tile");
