@@ -1,4 +1,4 @@
-// A GEMM that quantizes its few activation rows itself: what the weight-streaming and the sixteen-row kernels share.
+// A GEMM that quantizes its few activation rows itself: a part of the weight-streaming kernel.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -118,7 +118,8 @@ struct FewChunks {
           }
           // (A 24-bit product.  The 64-bit multiply-add that the compiler takes otherwise reads a register pair whose upper half
           // it had given to a weight scale on its way: the wave waited for all its weights here.  us, a token's norm with q, k
-          // and v / gate and up: 7.8 / 16.6 -> 7.1 / 15.5.)
+          // and v / gate and up: 7.8 / 16.6 -> 7.1 / 15.5; 7.0 / 15.0 with other code around it, by whose chance
+          // the pair was free.)
           *(v4f*)&sh.octets[(__umul24(at[p] >> 16, in.xk) + col[p]) / 8] = v4f{s[0], s[1], s[2], s[3]};
         }
       }

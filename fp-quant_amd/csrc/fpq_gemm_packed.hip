@@ -1114,15 +1114,14 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
       ((uintptr_t)y & 15u) || ((uintptr_t)residual & 15u))
     return FPQ_E_ALIGN;
   if ((uintptr_t)workspace & 255u) return FPQ_E_ALIGN;
-  // Few weight tiles: the rows are cut into slabs, one grid plane of the weight-streaming kernel each, as low as
+  // Few weight tiles: the rows are cut into slabs, one launch of the weight-streaming kernel for all, as low as
   // keeps slabs x weight tiles within one round of the 256 CUs -- more workgroups that each hold fewer
   // activation row tiles (fewer registers, less to re-read per weight tile, a shorter tail) and that, unlike
   // the tile kernels', share nothing through LDS and meet at no barrier in their K loop.  Slabs of 32 / 64 /
-  // 96 / 128 rows measured best exactly where they are the lowest that fit (us, K = 4096, against one
-  // workgroup per weight tile or the tile kernels): N = 4096: 64 rows 6.3 -> 5.3, 128 rows 8.0 -> 6.2, 256
-  // rows 9.9 -> 8.0; N = 2048: 128 rows 7.8 -> 5.1, 256 rows 7.6 -> 6.0 (tiles: 9.5), 384 rows 9.6 -> 6.9;
-  // N = 1024: 512 rows 9.5 -> 5.5; NVFP4 N = 4096: 128 rows 14.1 -> 9.3, 256 rows 28 -> 14.1; K = 14336, 256
-  // rows: 32 -> 19.  (More slabs than one round -- two or three workgroups per CU -- measured slower.)  K
+  // 96 rows (NVFP4: 128 too) measured best exactly where they are the lowest that fit (us, K = 4096, against one
+  // workgroup per weight tile or the tile kernels): N = 4096: 64 rows 6.3 -> 5.3, 128 rows 8.0 -> 6.2;
+  // N = 2048: 128 rows 7.8 -> 5.1, 256 rows 7.6 -> 6.0 (tiles: 9.5), 384 rows 9.6 -> 6.9;
+  // N = 1024: 512 rows 9.5 -> 5.5; NVFP4 N = 4096: 128 rows 14.1 -> 9.3, 256 rows 28 -> 14.1.  (More slabs than one round -- two or three workgroups per CU -- measured slower.)  K
   // stays whole in slabs, so a shape whose K the caller's workspace lets split keeps the split up to 96 rows
   // (N = 4096, K = 14336: 64 rows 11.7 split / 11.9 us in slabs, 96 rows 13.9 / 13.9, 128 rows 15.4 / 14.1).
   const int cus = device_cus();
@@ -1147,7 +1146,7 @@ static int gemm_packed(const void* xq, const void* xs, const void* wq, const voi
     }
     // MXFP4: two weight tiles per workgroup.  The time follows what a workgroup loads per K step (weight tiles + activation
     // tiles): two and two (or three) beat one and four, and the 64 x 128 tiles of the tile kernel.  Two and four do from K =
-    // 4096 on (below, the longer tail shows: 512 x 4096 x 1024 5.5 / 6.5).  us, weights from HBM, those / this: K = 4096:
+    // 8192 on (with a short K the longer tail shows: 512 x 4096 x 1024 5.5 / 6.5).  us, weights from HBM, those / this: K = 4096:
     // 160 rows, N = 8192 12.2 / 10.2, 200 rows, N = 4096 / 6144 8.4 / 7.8, 12.1 / 11.1, 333 rows, N = 4096 11.7 / 9.6; K = 8192,
     // N = 8192: 128 / 160 / 256 rows 15.3 / 14.0, 19.2 / 15.5, 20.9 / 18.9; K = 14336, N = 4096: 200 / 384 / 512 rows 21.0 / 18.1,
     // 28.5 / 22.8, 31.2 / 27.6.

@@ -959,8 +959,9 @@ int gemm_fp4_rows(bool nv, const void* xq, const void* xs, int64_t xs_stride, co
 //   MXFP4 4 rows (two passes):  4096 x 4096 7.2 / 5.7, N = 14336 10.2 / 8.1, N = 28672 14.9 / 14.5, N = 128256 45.5 / 49.0
 //   NVFP4 1 row:  4096 x 4096 9.4 / 7.2, N = 14336 12.6 / 9.8, N = 28672 19.6 / 17.9, N = 128256 59.8 / 65.3
 //   NVFP4 4 rows: 4096 x 4096 9.4 / 8.2, N = 14336 12.5 / 11.5, N = 28672 19.5 / 19.9
-// SiLU*up (two more lookups per element) gains in one pass only: MXFP4, K = 14336, N = 4096: 1 row 12.1 / 11.0, 2 rows
-// 12.2 / 13.2; 4096 x 4096: 1 row 7.5 / 5.9, 4 rows 7.8 / 9.3.
+// SiLU*up (two more lookups per element) gains in one pass only (weights from HBM, two passes built for it): MXFP4, N = 4096, K =
+// 14336: 1 row 13.8 / 12.1, 2 rows (two passes) 13.9 / 13.7; K = 12288: 13.2 / 11.4, 13.3 / 13.6; K = 4096: 1 row 8.7 / 6.6, 2 rows
+// 8.7 / 7.1, 4 rows (two) 8.8 / 9.2; NVFP4, K = 14336: 16.5 / 15.8, 16.7 / 17.8; K = 4096: 10.8 / 10.1, 4 rows 10.9 / 12.1.
 static bool few_rows_plan(const StreamPlan& plan, bool nv, int pro, int64_t M, int64_t N, int64_t K, int64_t xk) {
   const int64_t chunks = M * ((plan.bps + 3) / 4) * 8;   // of the wave with the most
   if (!plan.use || (nv && plan.nt != 1) || M > 32 || chunks > few_rows_chunks(pro) || K >= ((int64_t)1 << 22) || xk > K) return false;

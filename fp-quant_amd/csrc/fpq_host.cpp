@@ -3,7 +3,7 @@
 // What bounds a decode step is the host: one layer is 8 us of kernels behind 25 us of Python (attribute lookups on the
 // module, tensor constructors, two foreign calls of eleven to fourteen arguments, the checks of every cached constant),
 // a fused decoder block of one token 52 us of kernels behind 170, a quantize operator 6 us behind 18 (most of it
-// operator dispatch).  On this path they take 8.7, 46 and 6.9 us from call to call: a layer of few rows is one launch
+// operator dispatch).  On this path they take 8.7, 36 and 6.9 us from call to call: a layer of few rows is one launch
 // (fpq_linear_rows, 4.8 us), the rest of its time three allocations, what publish() makes and the module call around
 // them; with more rows it is two launches of 3.3 us (32 rows, 14336 -> 4096: 13.2 us).  Here the same sequence -- checks,
 // allocations, launches, the hand-over of quantized activations between layers that share an input -- runs as native code

@@ -188,7 +188,8 @@ int fpq_quantize_mx_packed(const void* x, int64_t rows, int64_t cols, int rot_ki
                            void* packed_codes, void* packed_scales, int zero_policy, void* stream);
 
 /*
- * fpq_gemm_mxf4 on packed operands (same arithmetic, bit-identical y): the kernel for large M.
+ * fpq_gemm_mxf4 on packed operands: the same arithmetic, with the fp32 sums over K in an order of its own for sizes that the
+ * weight-streaming kernel or workgroups with K in parts take (the same on every call).
  * Stands in for qutlass.matmul_mxf4_bf16_tn (qutlass_ops.py:111-128) like fpq_gemm_mxf4.
  */
 int fpq_gemm_mxf4_packed(const void* xq_packed, const void* xs_packed, const void* wq_packed,
