@@ -816,7 +816,11 @@ static int launch_stream(const void* xq, const void* xs, const void* wq, const v
   // Slabs: eights of groups unless that gives an XCD more workgroups than CUs, two on one of them; then in a row.  A multiple of
   // four groups has each on two XCDs at most in a grid of groups x slabs, which measured the same or better (us, that / in a row:
   // 590 x 2304 x 10240 17.8 / 18.4, 1300 x 768 x 10240 14.9 / 15.8), and the weights of few groups are little to share.
-  const bool eights = 8u * ((groups + 7) / 8) * slabs <= (unsigned)device_cus();
+  // MXFP4 with one tile and up to one block per wave: not eights either that are half empty or more, whose workgroups without a
+  // tile cost 0.2 to 0.5 (eights / groups x slabs: 34 x 2112 x 512 4.6 / 4.2, 84 x 128 x 256 4.2 / 4.0, 132 x 3336 x 768 5.8 / 5.5; 100 x 1470 x
+  // 1024, 46 groups, 4.7 / 5.1; 34 x 2112 x 1280 4.7 / 4.8; NVFP4 level).
+  const bool half_empty = !NV && plan.nt == 1 && K <= 1024 && groups % 8 >= 1 && groups % 8 <= 4;
+  const bool eights = !half_empty && 8u * ((groups + 7) / 8) * slabs <= (unsigned)device_cus();
   const bool in_a_row = !NV && slab_rows && plan.nt == 2 && !eights && groups > 8 && groups % 4 != 0;
   const dim3 grid = !slab_rows ? dim3(groups, (unsigned)plan.ksplit)
                     : eights   ? dim3(8, slabs, (groups + 7) / 8)
